@@ -10,6 +10,8 @@
 #include <cmath>
 #include <cstdio>
 #include <mutex>
+#include <system_error>
+#include <thread>
 #include <utility>
 
 #include "common.h"
@@ -559,6 +561,39 @@ int choose_tile(int N, int H, int W, int C, int K, int ks, int stride, int pad, 
   return fail(TETRIS_EINVAL, "no tile shape the kernel accepts for this layer");
 }
 
+namespace {
+// The two inner loops of the channel order, over plain arrays, in the widest vectors the host has (a 512 x 512 3x3 filter:
+// 2.4 million weights to test and some million loads to compare).
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+#define TETRIS_HOST_VECTORS __attribute__((target_clones("avx2", "default")))
+#else
+#define TETRIS_HOST_VECTORS
+#endif
+TETRIS_HOST_VECTORS int count_nonzero(const float* w, int n) {
+  int sum = 0;
+  for (int i = 0; i < n; ++i) sum += w[i] != 0.f;
+  return sum;
+}
+// sum over the stages of max(busiest, load + add): what a stage would cost
+TETRIS_HOST_VECTORS int raised(const int32_t* busiest, const int32_t* load, const int32_t* add, int n) {
+  int sum = 0;
+  for (int s = 0; s < n; ++s) sum += std::max(busiest[s], load[s] + add[s]);
+  return sum;
+}
+TETRIS_HOST_VECTORS void raise(int32_t* busiest, int32_t* load, const int32_t* add, int n) {
+  for (int s = 0; s < n; ++s) {
+    load[s] += add[s];
+    busiest[s] = std::max(busiest[s], load[s]);
+  }
+}
+TETRIS_HOST_VECTORS void add_to(int32_t* sum, const int32_t* add, int n) {
+  for (int s = 0; s < n; ++s) sum[s] += add[s];
+}
+TETRIS_HOST_VECTORS void max_to(int32_t* worst, const int32_t* v, int n) {
+  for (int s = 0; s < n; ++s) worst[s] = std::max(worst[s], v[s]);
+}
+}  // namespace
+
 // Output-channel order that evens out the work inside a workgroup.  A wave walks the entries of its
 // `oc_per_wave` slots stage by stage and the waves of a workgroup meet at a barrier after every stage.  Waves
 // w, w + 4, w + 8, ... run on the same SIMD and share its issue slots, so what a stage costs is the entry count of
@@ -576,16 +611,35 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
   const int G = t.oc_per_wave, waves = t.waves, tile_ic = t.tile_ic;
   if (G <= 0 || waves <= 0 || tile_ic <= 0) return fail(TETRIS_EINVAL, "bad tile");
   const int S = ceil_div(C, tile_ic), B = G * waves, nblocks = ceil_div(K, B), taps = ks * ks;
-  std::vector<int32_t> per((size_t)K * S, 0);
-  std::vector<int64_t> total(K, 0);
-  for (int k = 0; k < K; ++k)
-    for (int c = 0; c < C; ++c) {
-      const float* w = filter + ((size_t)k * C + c) * taps;
-      int n = 0;
-      for (int i = 0; i < taps; ++i) n += w[i] != 0.f;
-      per[(size_t)k * S + c / tile_ic] += n;
-      total[k] += n;
+  if ((long long)C * K * taps > INT_MAX) return fail(TETRIS_EINVAL, "%d x %d filters of %d weights are too many to order", K, C, taps);
+  // non-zeros per channel and stage: the weights of a stage lie side by side
+  std::vector<int32_t> per((size_t)K * S);
+  std::vector<int32_t> total(K, 0);
+  auto count = [&](int k0, int k1) {
+    for (int k = k0; k < k1; ++k)
+      for (int s = 0; s < S; ++s) {
+        const int c0 = s * tile_ic, c1 = std::min(C, c0 + tile_ic);
+        const int n = count_nonzero(filter + ((size_t)k * C + c0) * taps, (c1 - c0) * taps);
+        per[(size_t)k * S + s] = n;
+        total[k] += n;
+      }
+  };
+  // Past a million weights (0.15 ms of reading on one core) the count is shared by four threads, 25 us each to start.
+  if ((long long)C * K * taps >= (1 << 20) && K >= 4) {
+    std::vector<std::thread> helpers;
+    for (int i = 1; i < 4; ++i) {
+      const int k0 = (int)((long long)K * i / 4), k1 = (int)((long long)K * (i + 1) / 4);
+      try {
+        helpers.emplace_back(count, k0, k1);
+      } catch (const std::system_error&) {  // no more threads: counted here
+        count(k0, k1);
+      }
     }
+    count(0, K / 4);
+    for (std::thread& h : helpers) h.join();
+  } else {
+    count(0, K);
+  }
   std::vector<int32_t> sorted(K);
   for (int k = 0; k < K; ++k) sorted[k] = k;
   std::stable_sort(sorted.begin(), sorted.end(), [&](int32_t a, int32_t b) { return total[a] > total[b]; });
@@ -604,7 +658,7 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
     }
   }
   const int nsimd = std::min(4, waves);  // wave w runs on SIMD w % 4
-  std::vector<int64_t> load((size_t)waves * S), busiest(S), simd_load((size_t)nsimd * S), busiest_simd(S);
+  std::vector<int32_t> load((size_t)waves * S), busiest(S), simd_load((size_t)nsimd * S), busiest_simd(S), sum(waves);
   std::vector<std::vector<int32_t>> members(waves);
   int32_t* o = order;
   for (const std::vector<int32_t>& blk : blocks) {
@@ -612,35 +666,34 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
     std::fill(busiest.begin(), busiest.end(), 0);
     std::fill(simd_load.begin(), simd_load.end(), 0);
     std::fill(busiest_simd.begin(), busiest_simd.end(), 0);
+    std::fill(sum.begin(), sum.end(), 0);
     for (auto& m : members) m.clear();
     const int len = (int)blk.size();
+    auto takes = [&](int w) {  // slots of this wave that hold a channel: is one free?
+      return (int)members[w].size() < std::min(G, std::max(0, len - w * G));
+    };
     for (int32_t k : blk) {
-      int best = -1;
-      int64_t best_simd = 0, best_wave = 0, best_sum = 0;
+      const int32_t* add = &per[(size_t)k * S];
+      // least added to the busiest SIMD; of the waves on such SIMDs, to the busiest wave; of those the least loaded, the first
+      int cost_simd[4], best_simd = INT_MAX;
+      for (int sd = 0; sd < nsimd; ++sd) {
+        cost_simd[sd] = INT_MAX;
+        bool any = false;
+        for (int w = sd; w < waves && !any; w += nsimd) any = takes(w);
+        if (any) cost_simd[sd] = raised(busiest_simd.data(), &simd_load[(size_t)sd * S], add, S);
+        best_simd = std::min(best_simd, cost_simd[sd]);
+      }
+      int best = -1, best_wave = 0;
       for (int w = 0; w < waves; ++w) {
-        const int cap = std::min(G, std::max(0, len - w * G));  // slots of this wave that hold a channel
-        if ((int)members[w].size() >= cap) continue;
-        const int sd = w % nsimd;
-        int64_t cost_simd = 0, cost_wave = 0, sum = 0;
-        for (int s = 0; s < S; ++s) {
-          const int64_t add = per[(size_t)k * S + s];
-          cost_simd += std::max(busiest_simd[s], simd_load[(size_t)sd * S + s] + add);
-          cost_wave += std::max(busiest[s], load[(size_t)w * S + s] + add);
-          sum += load[(size_t)w * S + s];
-        }
-        if (best < 0 || cost_simd < best_simd || (cost_simd == best_simd && (cost_wave < best_wave ||
-            (cost_wave == best_wave && sum < best_sum)))) {
-          best = w; best_simd = cost_simd; best_wave = cost_wave; best_sum = sum;
+        if (cost_simd[w % nsimd] != best_simd || !takes(w)) continue;
+        const int cost_wave = raised(busiest.data(), &load[(size_t)w * S], add, S);
+        if (best < 0 || cost_wave < best_wave || (cost_wave == best_wave && sum[w] < sum[best])) {
+          best = w; best_wave = cost_wave;
         }
       }
-      const int sd = best % nsimd;
-      for (int s = 0; s < S; ++s) {
-        const int64_t add = per[(size_t)k * S + s];
-        load[(size_t)best * S + s] += add;
-        busiest[s] = std::max(busiest[s], load[(size_t)best * S + s]);
-        simd_load[(size_t)sd * S + s] += add;
-        busiest_simd[s] = std::max(busiest_simd[s], simd_load[(size_t)sd * S + s]);
-      }
+      raise(busiest.data(), &load[(size_t)best * S], add, S);
+      raise(busiest_simd.data(), &simd_load[(size_t)(best % nsimd) * S], add, S);
+      sum[best] += total[k];
       members[best].push_back(k);
     }
     for (int w = 0; w < waves; ++w)
@@ -648,22 +701,22 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
   }
   // The deal is a heuristic: keep the file order when it is no worse by the measure the deal aims at (what the waves
   // of a workgroup wait for: per block and stage the busiest wave's entries, summed).
+  std::vector<int32_t> wave_load(S), worst(S);
   auto wait_cost = [&](auto channel_at) {
-    int64_t sum = 0;
-    for (int b = 0; b < nblocks; ++b)
-      for (int s = 0; s < S; ++s) {
-        int64_t worst = 0;
-        for (int w = 0; w < waves; ++w) {
-          int64_t n = 0;
-          for (int i = 0; i < G; ++i) {
-            const int slot = b * B + w * G + i;
-            if (slot < K) n += per[(size_t)channel_at(slot) * S + s];
-          }
-          worst = std::max(worst, n);
+    int64_t cost = 0;
+    for (int b = 0; b < nblocks; ++b) {
+      std::fill(worst.begin(), worst.end(), 0);
+      for (int w = 0; w < waves; ++w) {
+        std::fill(wave_load.begin(), wave_load.end(), 0);
+        for (int i = 0; i < G; ++i) {
+          const int slot = b * B + w * G + i;
+          if (slot < K) add_to(wave_load.data(), &per[(size_t)channel_at(slot) * S], S);
         }
-        sum += worst;
+        max_to(worst.data(), wave_load.data(), S);
       }
-    return sum;
+      for (int s = 0; s < S; ++s) cost += worst[s];
+    }
+    return cost;
   };
   if (wait_cost([&](int slot) { return slot; }) <= wait_cost([&](int slot) { return order[slot]; }))
     for (int k = 0; k < K; ++k) order[k] = k;
