@@ -179,6 +179,10 @@ int tetris_measure_peaks(void* stream, float* copy_gbs_out, float* fma_tflops_ou
  * `order_out` receives a permutation of 0..out_channel-1.  Pure host code. */
 int tetris_oc_order_balanced(const float* h_filter_oihw, int in_channel, int out_channel, int kernel_size,
                              const tetris_tile* tile, int32_t* order_out);
+/* Same as tetris_g950_create with the channel order of tetris_oc_order_balanced for `tile` (and the tile's tile_ic and
+ * oc_per_wave); the order is made while the filter is uploaded. */
+int tetris_g950_create_balanced(const float* h_filter_oihw, int in_channel, int out_channel, int kernel_size,
+                                const tetris_tile* tile, void* stream, tetris_g950** out);
 
 /* Measured selection, the counterpart of GetTetrisSparseConv2dTime (Tetris/spconv2d.cc:72-329): packs the filter
  * for the `max_candidates` (0 = 24) tile shapes the model of tetris_tile_select ranks best (each in the

@@ -449,14 +449,8 @@ int conv_host(const float* h_in, const float* h_filter, float* h_out, int N, int
     if (rc) return done(rc);
     // apply_reorder: the reference regroups output channels for its warps (ReorderOutChannel); the kernel here
     // gets the order that balances its own waves instead.  The results do not depend on the order.
-    std::vector<int32_t> order;
-    if (apply_reorder) {
-      order.resize(K);
-      rc = balance_oc_order(h_filter, C, K, ks, tile, order.data());
-      if (rc) return done(rc);
-    }
-    rc = tetris_g950_create(h_filter, C, K, ks, tile.tile_ic, tile.oc_per_wave, apply_reorder ? order.data() : nullptr,
-                            stream, &pack);
+    rc = apply_reorder ? tetris_g950_create_balanced(h_filter, C, K, ks, &tile, stream, &pack)
+                       : tetris_g950_create(h_filter, C, K, ks, tile.tile_ic, tile.oc_per_wave, nullptr, stream, &pack);
     if (rc) return done(rc);
     run = pack;
   }

@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -177,11 +178,12 @@ struct tetris_g950 {
   int slots = 0;            // K rounded up to a multiple of kSlotPad
   int groups = 0;           // slots / g
   int64_t n_entries = 0, nnz = 0;
-  int32_t* d_grp_off = nullptr;   // [groups*stages+1] entry index, multiples of 8
+  // two allocations: grp_off, grp_nnz and oc_order; position and values
+  int32_t* d_grp_off = nullptr;   // [groups*stages+1] entry index, multiples of 8; then the number of non-zeros
   int32_t* d_grp_nnz = nullptr;   // [groups*stages]
-  int32_t* d_position = nullptr;  // [n_entries] s | r<<3 | ic_local<<6 | slot-in-group<<24
-  float* d_values = nullptr;      // [n_entries]
   int32_t* d_oc_order = nullptr;  // [slots], -1 for padding slots
+  int32_t* d_position = nullptr;  // [n_entries + 8] s | r<<3 | ic_local<<6 | slot-in-group<<24
+  float* d_values = nullptr;      // [n_entries + 8]
   // (LDS byte offset | accumulator index << 16 | 0xC << 28, value) pairs for one tile geometry, made on first use
   std::map<tetris::BoundKey, int2*> bound;
   // Paired arrangement of the streams (made on the first paired bind; depends on the pack only): two consecutive
@@ -203,8 +205,7 @@ struct tetris_g950 {
   std::vector<float*> retired;
   std::mutex mu;
   // host mirrors, filled by tetris_g950_host_arrays
-  std::vector<int32_t> h_grp_off, h_grp_nnz, h_position, h_oc_order;
-  std::vector<float> h_values;
+  std::unique_ptr<int32_t[]> h_fixed, h_entries;  // the two allocations as they lie
 };
 
 struct tetris_spf {

@@ -10,6 +10,9 @@
 // wave-uniform.  A stream lists the non-zeros of the group's G channels position by position (channel,
 // row, column ascending; within a position by slot), carries the slot's index inside the group in bits
 // 24..31, and is padded with zero entries to a multiple of 8 (one 64-byte scalar fetch).
+#include <system_error>
+#include <thread>
+
 #include "common.h"
 
 namespace tetris {
@@ -39,9 +42,9 @@ __global__ __launch_bounds__(256) void count_kernel(const float* __restrict__ fi
   }
 }
 
-// exclusive scan of grp_pad into grp_off[0..n], single workgroup
+// exclusive scan of grp_pad into grp_off[0..n], single workgroup; nnz != nullptr: grp_off[n + 1] = the sum of nnz[0..n)
 __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ grp_pad, int32_t* __restrict__ grp_off,
-                                                    int n) {
+                                                    int n, const int32_t* __restrict__ nnz = nullptr) {
   __shared__ int part[1024];
   const int tid = threadIdx.x;
   const int chunk = (n + 1023) / 1024;
@@ -62,6 +65,18 @@ __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ 
     run += grp_pad[i];
   }
   if (tid == 1023) grp_off[n] = part[1023];
+  if (!nnz) return;
+  s = 0;
+  for (int i = tid; i < n; i += 1024) s += nnz[i];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  __syncthreads();  // part has been read
+  if ((tid & 63) == 0) part[tid >> 6] = s;
+  __syncthreads();
+  if (tid == 0) {
+    s = 0;
+    for (int i = 0; i < 16; ++i) s += part[i];
+    grp_off[n + 1] = s;
+  }
 }
 
 __global__ __launch_bounds__(256) void scatter_kernel(const float* __restrict__ filter,
@@ -97,7 +112,8 @@ __global__ __launch_bounds__(256) void scatter_kernel(const float* __restrict__ 
     }
     written += __popcll(m);
   }
-  for (int i = beg + written + lane; i < end; i += 64) {  // padding entries
+  const int last = sid == nstream - 1 ? end + kBatch : end;  // the spare batch follows the last stream
+  for (int i = beg + written + lane; i < last; i += 64) {  // padding entries
     position[i] = 0;
     values[i] = 0.f;
   }
@@ -145,9 +161,7 @@ int pack_device(const float* d_filter, int C, int K, int ks, int tile_ic, int G,
     seen[oc] = 1;
     order[i] = oc;
   }
-  int32_t* d_pad = nullptr;
   auto cleanup = [&](int rc) {
-    if (d_pad) (void)hipFree(d_pad);
     if (rc != TETRIS_OK) tetris_g950_destroy(p);
     return rc;
   };
@@ -157,34 +171,32 @@ int pack_device(const float* d_filter, int C, int K, int ks, int tile_ic, int G,
     if (e_ != hipSuccess)                                                                                       \
       return cleanup(fail(TETRIS_EHIP, "%s failed at %s:%d: %s", #call, __FILE__, __LINE__, hipGetErrorString(e_))); \
   } while (0)
-  HIPC(hipMalloc(&p->d_oc_order, sizeof(int32_t) * p->slots));
-  HIPC(hipMalloc(&p->d_grp_off, sizeof(int32_t) * (nseg + 1)));
-  HIPC(hipMalloc(&p->d_grp_nnz, sizeof(int32_t) * nseg));
-  HIPC(hipMalloc(&d_pad, sizeof(int32_t) * nseg));
+  // One allocation for what the layer's shape fixes -- offsets (and, after the last, the number of non-zeros), counts,
+  // channel order, and the padded counts that only packing needs -- and one for the entries; tetris_g950_host_arrays
+  // copies each back as a whole.
+  HIPC(hipMalloc(&p->d_grp_off, sizeof(int32_t) * (3 * (size_t)nseg + 2 + p->slots)));
+  p->d_grp_nnz = p->d_grp_off + nseg + 2;
+  p->d_oc_order = p->d_grp_nnz + nseg;
+  int32_t* const d_pad = p->d_oc_order + p->slots;
   HIPC(hipMemcpyAsync(p->d_oc_order, order.data(), sizeof(int32_t) * p->slots, hipMemcpyHostToDevice, stream));
   const int blocks = (nseg + 3) / 4;
   hipLaunchKernelGGL(count_kernel, dim3(blocks), dim3(256), 0, stream, d_filter, p->d_oc_order, p->d_grp_nnz, d_pad, C,
                      ks, tile_ic, p->stages, G, nseg);
-  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, stream, d_pad, p->d_grp_off, nseg);
+  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, stream, d_pad, p->d_grp_off, nseg, p->d_grp_nnz);
   HIPC(hipGetLastError());
-  int32_t total = 0;
-  HIPC(hipMemcpyAsync(&total, p->d_grp_off + nseg, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+  int32_t total[2] = {0, 0};  // entries, non-zeros
+  HIPC(hipMemcpyAsync(total, p->d_grp_off + nseg, sizeof total, hipMemcpyDeviceToHost, stream));
   HIPC(hipStreamSynchronize(stream));
-  p->n_entries = total;
+  p->n_entries = total[0];
+  p->nnz = total[1];
   // one spare batch so that a kernel may prefetch the batch after the last one
-  HIPC(hipMalloc(&p->d_position, sizeof(int32_t) * (size_t)(total + kBatch)));
-  HIPC(hipMalloc(&p->d_values, sizeof(float) * (size_t)(total + kBatch)));
-  HIPC(hipMemsetAsync(p->d_position + total, 0, sizeof(int32_t) * kBatch, stream));
-  HIPC(hipMemsetAsync(p->d_values + total, 0, sizeof(float) * kBatch, stream));
+  const size_t room = (size_t)total[0] + kBatch;
+  HIPC(hipMalloc(&p->d_position, 2 * sizeof(int32_t) * room));
+  p->d_values = reinterpret_cast<float*>(p->d_position + room);
   hipLaunchKernelGGL(scatter_kernel, dim3(blocks), dim3(256), 0, stream, d_filter, p->d_oc_order, p->d_grp_off,
                      p->d_position, p->d_values, C, ks, tile_ic, p->stages, G, nseg);
   HIPC(hipGetLastError());
-  // nnz = sum of seg_nnz, summed on the host (small)
-  std::vector<int32_t> nz(nseg);
-  HIPC(hipMemcpyAsync(nz.data(), p->d_grp_nnz, sizeof(int32_t) * nseg, hipMemcpyDeviceToHost, stream));
-  HIPC(hipStreamSynchronize(stream));
-  p->nnz = 0;
-  for (int v : nz) p->nnz += v;
+  HIPC(hipStreamSynchronize(stream));  // the caller may free or rewrite the filter
 #undef HIPC
   *out = p;
   return cleanup(TETRIS_OK);
@@ -474,30 +486,68 @@ int tetris_g950_create_device(const float* d_filter, int C, int K, int ks, int t
   return tetris::pack_device(d_filter, C, K, ks, tile_ic, oc_per_wave, oc_order, static_cast<hipStream_t>(stream), out);
 }
 
-int tetris_g950_create(const float* h_filter, int C, int K, int ks, int tile_ic, int oc_per_wave,
-                       const int32_t* oc_order, void* stream, tetris_g950** out) {
+}  // extern "C"
+
+// From a filter in host memory.  `tile`: pack in the balanced order for it, which is made while the filter is uploaded
+// (both take some 0.2 ms for 2.4 million weights).
+static int create_from_host(const float* h_filter, int C, int K, int ks, int tile_ic, int oc_per_wave, const int32_t* oc_order,
+                            const tetris_tile* tile, hipStream_t stream, tetris_g950** out) {
   if (!h_filter) return tetris::fail(TETRIS_EINVAL, "null filter");
   if (C <= 0 || K <= 0 || ks <= 0) return tetris::fail(TETRIS_EINVAL, "bad filter shape C=%d K=%d ks=%d", C, K, ks);
-  float* d = nullptr;
   const size_t bytes = sizeof(float) * (size_t)C * K * ks * ks;
-  TETRIS_HIP(hipMalloc(&d, bytes));
-  hipError_t e = hipMemcpyAsync(d, h_filter, bytes, hipMemcpyHostToDevice, static_cast<hipStream_t>(stream));
+  std::vector<int32_t> order;
+  int order_rc = TETRIS_OK;
+  std::string order_error;
+  std::thread helper;
+  if (tile) {
+    order.resize(K);
+    auto make = [&] {
+      order_rc = tetris::balance_oc_order(h_filter, C, K, ks, *tile, order.data());
+      if (order_rc != TETRIS_OK) order_error = tetris_last_error();  // this thread's
+    };
+    if (bytes >= (1u << 18)) {  // below, the order takes less than the thread
+      try {
+        helper = std::thread(make);
+      } catch (const std::system_error&) {
+        make();
+      }
+    } else {
+      make();
+    }
+  }
+  float* d = nullptr;
+  hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&d), bytes, stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(d, h_filter, bytes, hipMemcpyHostToDevice, stream);
+  if (helper.joinable()) helper.join();
   int rc = e == hipSuccess ? TETRIS_OK : tetris::fail(TETRIS_EHIP, "filter upload failed: %s", hipGetErrorString(e));
+  if (rc == TETRIS_OK && order_rc != TETRIS_OK) rc = tetris::fail(order_rc, "%s", order_error.c_str());
   if (rc == TETRIS_OK)
-    rc = tetris::pack_device(d, C, K, ks, tile_ic, oc_per_wave, oc_order, static_cast<hipStream_t>(stream), out);
-  (void)hipStreamSynchronize(static_cast<hipStream_t>(stream));
-  (void)hipFree(d);
+    rc = tetris::pack_device(d, C, K, ks, tile_ic, oc_per_wave, tile ? order.data() : oc_order, stream, out);
+  else
+    (void)hipStreamSynchronize(stream);
+  if (d) (void)hipFreeAsync(d, stream);
   return rc;
+}
+
+extern "C" {
+
+int tetris_g950_create(const float* h_filter, int C, int K, int ks, int tile_ic, int oc_per_wave,
+                       const int32_t* oc_order, void* stream, tetris_g950** out) {
+  return create_from_host(h_filter, C, K, ks, tile_ic, oc_per_wave, oc_order, nullptr, static_cast<hipStream_t>(stream), out);
+}
+
+int tetris_g950_create_balanced(const float* h_filter, int C, int K, int ks, const tetris_tile* tile, void* stream,
+                                tetris_g950** out) {
+  if (!tile) return tetris::fail(TETRIS_EINVAL, "null argument");
+  return create_from_host(h_filter, C, K, ks, tile->tile_ic, tile->oc_per_wave, nullptr, tile,
+                          static_cast<hipStream_t>(stream), out);
 }
 
 void tetris_g950_destroy(tetris_g950* p) {
   if (!p) return;
   for (auto& kv : p->bound) (void)hipFree(kv.second);
-  (void)hipFree(p->d_grp_off);
-  (void)hipFree(p->d_grp_nnz);
-  (void)hipFree(p->d_position);
-  (void)hipFree(p->d_values);
-  (void)hipFree(p->d_oc_order);
+  (void)hipFree(p->d_grp_off);   // with the counts and the channel order
+  (void)hipFree(p->d_position);  // with the values
   (void)hipFree(p->d_pgrp_off);
   (void)hipFree(p->d_pgrp_pair);
   (void)hipFree(p->d_zero_pair);
@@ -510,25 +560,20 @@ int tetris_g950_host_arrays(tetris_g950* p, tetris_g950_arrays* out) {
   if (!p || !out) return tetris::fail(TETRIS_EINVAL, "null argument");
   const int nseg = p->groups * p->stages;
   std::lock_guard<std::mutex> lock(p->mu);
-  if (p->h_grp_off.empty()) {
-    p->h_grp_off.resize(nseg + 1);
-    p->h_grp_nnz.resize(nseg);
-    p->h_position.resize(p->n_entries);
-    p->h_values.resize(p->n_entries);
-    p->h_oc_order.resize(p->slots);
-    TETRIS_HIP(hipMemcpy(p->h_grp_off.data(), p->d_grp_off, sizeof(int32_t) * (nseg + 1), hipMemcpyDeviceToHost));
-    TETRIS_HIP(hipMemcpy(p->h_grp_nnz.data(), p->d_grp_nnz, sizeof(int32_t) * nseg, hipMemcpyDeviceToHost));
-    if (p->n_entries) {
-      TETRIS_HIP(hipMemcpy(p->h_position.data(), p->d_position, sizeof(int32_t) * p->n_entries, hipMemcpyDeviceToHost));
-      TETRIS_HIP(hipMemcpy(p->h_values.data(), p->d_values, sizeof(float) * p->n_entries, hipMemcpyDeviceToHost));
-    }
-    TETRIS_HIP(hipMemcpy(p->h_oc_order.data(), p->d_oc_order, sizeof(int32_t) * p->slots, hipMemcpyDeviceToHost));
+  const size_t fixed = 2 * (size_t)nseg + 2 + p->slots, room = (size_t)p->n_entries + tetris::kBatch;
+  if (!p->h_fixed) {
+    std::unique_ptr<int32_t[]> h(new int32_t[fixed]), e(new int32_t[2 * room]);
+    TETRIS_HIP(hipMemcpy(h.get(), p->d_grp_off, sizeof(int32_t) * fixed, hipMemcpyDeviceToHost));
+    TETRIS_HIP(hipMemcpy(e.get(), p->d_position, sizeof(int32_t) * 2 * room, hipMemcpyDeviceToHost));
+    p->h_fixed = std::move(h);
+    p->h_entries = std::move(e);
   }
-  out->grp_offsets = p->h_grp_off.data(); out->n_grp_offsets = nseg + 1;
-  out->grp_nnz = p->h_grp_nnz.data();     out->n_grp_nnz = nseg;
-  out->position = p->h_position.data();   out->n_entries = p->n_entries;
-  out->values = p->h_values.data();
-  out->oc_order = p->h_oc_order.data();   out->n_slots = p->slots;
+  const int32_t* h = p->h_fixed.get();
+  out->grp_offsets = h; out->n_grp_offsets = nseg + 1;
+  out->grp_nnz = h + nseg + 2; out->n_grp_nnz = nseg;
+  out->position = p->h_entries.get(); out->n_entries = p->n_entries;
+  out->values = reinterpret_cast<const float*>(p->h_entries.get() + room);
+  out->oc_order = h + 2 * (size_t)nseg + 2; out->n_slots = p->slots;
   out->stages = p->stages; out->tile_ic = p->tile_ic; out->oc_per_wave = p->g; out->nnz = p->nnz;
   return TETRIS_OK;
 }

@@ -108,6 +108,8 @@ _lib.tetris_spf_host_arrays.argtypes = [C.c_void_p, C.POINTER(_SpfArrays)]
 _lib.tetris_spf_device_arrays.argtypes = [C.c_void_p, C.POINTER(_SpfArrays)]
 _lib.tetris_g950_create.argtypes = [_f32p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _i32p_opt, C.c_void_p,
                                     C.POINTER(C.c_void_p)]
+_lib.tetris_g950_create_balanced.argtypes = [_f32p, C.c_int, C.c_int, C.c_int, C.POINTER(Tile), C.c_void_p,
+                                             C.POINTER(C.c_void_p)]
 _lib.tetris_g950_create_device.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _i32p_opt,
                                            C.c_void_p, C.POINTER(C.c_void_p)]
 _lib.tetris_g950_destroy.argtypes = [C.c_void_p]
@@ -246,9 +248,16 @@ class G950Filter:
         """oc_order: None or "file" (file order), an int32 permutation, "balanced" (oc_order_balanced for this tile) or
         "reference" (the order the reference's ReorderOutChannel pass gives, spconv2d_utils.h:249-289)."""
         if isinstance(oc_order, str):
-            if oc_order == "balanced":
-                oc_order = oc_order_balanced(filter, tile)
-            elif oc_order == "reference":
+            if oc_order == "balanced":  # ordered while the filter is uploaded
+                w = np.ascontiguousarray(filter, np.float32)
+                self = cls.__new__(cls)
+                self._h = C.c_void_p()
+                self.K, self.C, self.ks = w.shape[:3]
+                self.tile_ic, self.oc_per_wave = tile.tile_ic, tile.oc_per_wave
+                _check(_lib.tetris_g950_create_balanced(w, self.C, self.K, self.ks, C.byref(tile), C.c_void_p(stream),
+                                                        C.byref(self._h)))
+                return self
+            if oc_order == "reference":
                 oc_order = oc_order_reference(filter, tile.tile_ic)
             elif oc_order == "file":
                 oc_order = None
