@@ -88,10 +88,13 @@ int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const te
   return TETRIS_OK;
 }
 
-// scratch of a split layer: the tickets, then csplit copies of the output
+// scratch a split layer needs: the tickets, then csplit copies of the output
 size_t partial_bytes_of(const Geom& g) {
   return g.csplit > 1 ? (size_t)kTicketBytes + sizeof(float) * (size_t)g.csplit * g.N * g.K * g.OH * g.OW : 0;
 }
+
+// ... and what it gets where the library allocates it: room for the waves' sums as well, which idle lanes make longer
+size_t scratch_bytes_of(const Geom& g) { return std::max(partial_bytes_of(g), kTicketBytes + sum_bytes_of(g)); }
 
 // Partial-sum buffer of a split layer: one per (pack, stream), so that launches of one pack on different streams do
 // not share it.  A buffer that has to grow is replaced, and the old one is kept until the pack is destroyed: a HIP
@@ -133,11 +136,12 @@ int run_launch(tetris_g950* p, const float* d_in, float* d_out, int N, int H, in
   int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, &plan);
   if (rc) return rc;
   float* d_partial = nullptr;
+  const size_t scratch = scratch_bytes_of(plan.geom);
   if (plan.geom.csplit > 1) {
-    rc = partial_buffer(p, stream, partial_bytes_of(plan.geom), true, &d_partial);
+    rc = partial_buffer(p, stream, scratch, true, &d_partial);
     if (rc) return rc;
   }
-  return launch_conv(plan.geom, d_in, d_out, d_partial, plan.entries, plan.grp_off, plan.grp_pair, p->d_oc_order, act,
+  return launch_conv(plan.geom, d_in, d_out, d_partial, scratch, plan.entries, plan.grp_off, plan.grp_pair, p->d_oc_order, act,
                      stream);
 }
 
@@ -762,7 +766,7 @@ int tetris_g950_prepare(tetris_g950* p, int N, int H, int W, int stride, int pad
   if (rc) return rc;
   if (plan.geom.csplit > 1) {
     float* d_partial = nullptr;
-    rc = partial_buffer(p, stream, partial_bytes_of(plan.geom), true, &d_partial);
+    rc = partial_buffer(p, stream, scratch_bytes_of(plan.geom), true, &d_partial);
     if (rc) return rc;
   }
   float* s = nullptr;
@@ -803,10 +807,10 @@ int tetris_spconv2d_launch_noalloc(tetris_g950* p, const float* d_in, float* d_o
     rc = static_scratch(&d_partial);
     if (rc) return rc;
   }
-  // Every element of the partial sums that reduce_kernel reads is written by this launch's conv kernel first, so
+  // Every element of the partial sums that are added is written by this launch's conv kernel first, so
   // what an earlier call left in the array needs no clearing.
-  return launch_conv(plan.geom, d_in, d_out, d_partial, plan.entries, plan.grp_off, plan.grp_pair, p->d_oc_order, 0,
-                     stream);
+  return launch_conv(plan.geom, d_in, d_out, d_partial, g_scratch_limit.load(), plan.entries, plan.grp_off, plan.grp_pair,
+                     p->d_oc_order, 0, stream);
 }
 
 int tetris_spconv2d_launch_spf_arrays(const float* d_in, const int32_t* d_offsets, const int32_t* d_stage_len,

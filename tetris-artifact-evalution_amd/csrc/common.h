@@ -50,6 +50,7 @@ constexpr int kMaxSplit = 8;      // most workgroups that may share an output ti
 // the partial sums follow.
 constexpr int kTicketBytes = 65536;
 constexpr int kMaxTickets = kTicketBytes / 4;
+constexpr size_t kMaxWaveSums = 16u << 20;  // most bytes of sums that a launch keeps in its waves' order (see launch_conv)
 
 inline int out_extent(int in, int pad, int ks, int stride) { return (in + 2 * pad - ks) / stride + 1; }
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
@@ -101,7 +102,7 @@ struct Geom {
   int cpp, nchunks, ni;
   int buf_bytes;       // size of one of the three LDS buffers: kBufBytes, or kHalfBufBytes (8 waves of <= 64 accumulators)
   int csplit;          // workgroups that share an output tile, each reducing a slice of the stages into its own copy
-                       // of the output (a scratch buffer); reduce_kernel adds the copies.  1 = no split
+                       // of the output or of its waves' sums (a scratch buffer), which are added afterwards.  1 = no split
   // A 1x1 convolution of stride s without padding only reads every s-th row and column: it is run as a stride-1
   // layer on that sub-grid (H, W, stride above then describe the sub-grid) and the staging loads step through the
   // real image: element (row, col) of the sub-grid lies at row*step*in_w + col*step of a plane of in_hw floats.
@@ -128,14 +129,22 @@ struct Geom {
   // What a kernel does to a finished sum before it writes it (set per launch): 0 nothing, 1 ReLU, 2 ReLU and 2x2
   // max-pooling inside the halo'd kernels (the output tensor is then N x K x OH/2 x OW/2).
   int act;
-  // Split layers (csplit > 1), set per launch: 1 = every wave, once its partial sums are stored, takes a ticket of its
+  // Split layers (csplit > 1), set per launch.  1 = every wave, once its partial sums are stored, takes a ticket of its
   // (output tile, wave) pair, and the wave that draws the last one adds the slices itself, in slice order, and writes
-  // the finished sums (through `act` 0 or 1); 0 = a second kernel adds the slices.
+  // the finished sums (through `act`); 2 = add_kernel does, from the same order of the sums; 0 = every slice writes a copy
+  // of the output and reduce_kernel or reduce_pool_kernel adds the copies.
   int fused;
+  // the sums a wave keeps for one of its channels and quads: 16 bytes per lane that owns pixels, to a multiple of 128
+  int sum_bytes;
   // multiply-high reciprocals, floor(2^32 / d) + 1: x / d == umulhi(x, m) whenever x * d < 2^32
   unsigned m_per_unit, m_cpp, m_pitch, m_par, m_upi, m_units_w, m_lr, m_thi, m_kblocks, m_csplit;
   unsigned m_fill_slots, m_slots_per_unit, m_per_img, m_per_row, m_ng;  // single-tile kernel's staging plan
 };
+
+// what the waves of a split layer keep: every slice's sums
+inline size_t sum_bytes_of(const Geom& g) {
+  return g.csplit > 1 ? (size_t)g.ugroups * g.kblocks * g.csplit * g.waves * g.g * g.nq * g.sum_bytes : 0;
+}
 
 // how many images a tile of `lw` lanes per row places side by side on an output OW pixels wide
 inline int fold_of(int lw, int OW) { return lw >= OW ? 4 : 2 * lw >= OW ? 2 : 1; }
@@ -260,14 +269,14 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
 
 // spconv2d_kernel.hip
 // launches the conv; when the geometry splits the channel reduction (csplit > 1) the workgroups write their partial
-// sums to the scratch ([csplit] outputs) and the slices are added, in slice order, into d_out: by the last wave of
-// every (tile, wave) pair to finish (TETRIS_OPT_ADD_IN_KERNEL, on a device whose workgroup placement keeps a tile's
-// slices on one XCD, no pooling), or else by a second kernel
-// act: 0 = d_out gets the sums; 1 = their ReLU; 2 = ReLU and 2x2 max-pooling (d_out is N x K x OH/2 x OW/2), done by
-// the adding kernel of a split layer and otherwise inside the conv kernel where geom_pools_in_kernel allows (else
+// sums to the scratch and the slices are added, in slice order, into d_out: by the last wave of every (tile, wave) pair
+// to finish (TETRIS_OPT_ADD_IN_KERNEL, on a device whose workgroup placement keeps a tile's slices on one XCD), or else by a second kernel
+// act: 0 = d_out gets the sums; 1 = their ReLU; 2 = ReLU and 2x2 max-pooling (d_out is N x K x OH/2 x OW/2), done where
+// the slices are added and otherwise inside the conv kernel where geom_pools_in_kernel allows (else
 // TETRIS_EUNSUPPORTED, nothing launched)
-// d_scratch (split layers): kTicketBytes of tickets, all zero between launches, then room for csplit outputs
-int launch_conv(const Geom& g, const float* d_in, float* d_out, float* d_scratch, const int2* entries,
+// d_scratch (split layers): kTicketBytes of tickets, all zero between launches, then room for csplit outputs; where
+// scratch_bytes says that sum_bytes_of fits as well, the sums may be kept in the waves' order
+int launch_conv(const Geom& g, const float* d_in, float* d_out, float* d_scratch, size_t scratch_bytes, const int2* entries,
                 const int32_t* grp_off, const int32_t* grp_pair, const int32_t* oc_order, int act, hipStream_t stream);
 // whether workgroups with the same blockIdx.x % 8 run on one XCD of the current device (probed once per device):
 // what lets the slices of a split layer exchange their partial sums through that XCD's L2

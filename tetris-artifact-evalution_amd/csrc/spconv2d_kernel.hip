@@ -248,20 +248,29 @@ __device__ __forceinline__ void read_accumulators4(int i, float (&v)[4]) {
                  : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "s"(i) : "m0");
 }
 
-// Writes a wave's accumulators: slot k of the wave goes to the output channel lane k holds in lane_oc, quad q of a lane to
-// the lane's four pixels of unit u0 + q.  The per-pixel byte offsets (inside the image block that starts at
-// n_base, channel 0) are formed once; a channel then only adds a scalar offset, and out-of-range pixels carry an
-// offset the buffer hardware drops.
-template <int NQ, int VARIANT>
-__device__ __forceinline__ void store_outputs(float* __restrict__ out, int lane_oc, const Geom& g, int u0, int n_base,
-                                              int limg, int lrow, int lx, bool lane_ok) {
-  constexpr unsigned kInvalid = 0x80000000u;
+// acc[i .. i+3] added to v (i wave-uniform).
+template <int VARIANT>
+__device__ __forceinline__ void add_accumulators4(int i, float (&v)[4]) {
+  if constexpr (small_acc(VARIANT))
+    asm volatile("s_set_gpr_idx_on %4, 0x1\n v_add_f32 %0, v64, %0\n v_add_f32 %1, v65, %1\n v_add_f32 %2, v66, %2\n"
+                 "v_add_f32 %3, v67, %3\n s_set_gpr_idx_off\n"
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : "s"(i) : "m0");
+  else
+    asm volatile("s_set_gpr_idx_on %4, 0x1\n v_add_f32 %0, v128, %0\n v_add_f32 %1, v129, %1\n v_add_f32 %2, v130, %2\n"
+                 "v_add_f32 %3, v131, %3\n s_set_gpr_idx_off\n"
+                 : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : "s"(i) : "m0");
+}
+
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+constexpr unsigned kNoPixel = 0x80000000u;  // a byte offset the buffer hardware drops (loads read zero)
+
+// Byte offsets, inside the image block that starts at n_base and channel 0, of the pixels a lane owns: quad q, pixel j.
+// SHIFT 1: of the 2x2-pooled output instead, for the lanes of even row and column (see store_pooled).
+template <int NQ, int SHIFT>
+__device__ __forceinline__ void pixel_offsets(unsigned (&ooff)[NQ][4], const Geom& g, int u0, int n_base, int limg,
+                                              int lrow, int lx, bool lane_ok) {
   const int upi = g.units_w * g.units_h;
-  const int ohw = g.OH * g.OW;
-  const long long rec = (long long)(g.N - n_base) * g.K * (long long)ohw * 4;
-  const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(
-      out + (size_t)n_base * g.K * ohw, 0, rec > 0x7fffffffll ? 0x7fffffff : (int)rec, 0x00020000);
-  unsigned ooff[NQ][4];
+  const int oh_end = g.OH >> SHIFT, ow_end = g.OW >> SHIFT;
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     const int u = u0 + q;
@@ -272,29 +281,72 @@ __device__ __forceinline__ void store_outputs(float* __restrict__ out, int lane_
     const int n0 = (ub_n * g.nb + limg) * g.fold;  // first of the images this lane's quads belong to
     const int oh = ub_h * g.thi + lrow;
     const int ow = ub_w * (1 << g.jsh) * g.lw + lx;
-    const bool ok = lane_ok && u < g.units && oh < g.OH;
+    const bool ok = lane_ok && u < g.units && (oh >> SHIFT) < oh_end && !(SHIFT && ((lrow | lx) & 1));
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + (j >> g.jsh);
       const int col = ow + (j & ((1 << g.jsh) - 1)) * g.lw;
-      ooff[q][j] = (ok && n < g.N && col < g.OW) ? 4u * (unsigned)(((n - n_base) * g.K * g.OH + oh) * g.OW + col) : kInvalid;
+      ooff[q][j] = (ok && n < g.N && (col >> SHIFT) < ow_end)
+                       ? 4u * (unsigned)(((n - n_base) * g.K * oh_end + (oh >> SHIFT)) * ow_end + (col >> SHIFT)) : kNoPixel;
     }
   }
-  const bool relu = g.act != 0 && g.csplit == 1;  // a slice's partial sums are stored as they are
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t block_of(float* out, int n_base, const Geom& g, int plane) {
+  const long long rec = (long long)(g.N - n_base) * g.K * (long long)plane * 4;
+  return __builtin_amdgcn_make_buffer_rsrc(out + (size_t)n_base * g.K * plane, 0, rec > 0x7fffffffll ? 0x7fffffff : (int)rec,
+                                           0x00020000);
+}
+
+__device__ __forceinline__ void store_quad(const float (&v)[4], bool relu, __amdgpu_buffer_rsrc_t orsrc,
+                                           const unsigned (&ooff)[4], int soff) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (ooff[j] != kNoPixel)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(v[j], 0.f) : v[j]), orsrc, (int)ooff[j], soff, 0);
+}
+
+// A quad of consecutive pixels, 16-byte aligned.
+__device__ __forceinline__ void store_consecutive(const float (&v)[4], bool relu, __amdgpu_buffer_rsrc_t orsrc, unsigned ooff, int soff) {
+  u4 d;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) d[j] = (unsigned)__float_as_int(relu ? fmaxf(v[j], 0.f) : v[j]);
+  if (ooff != kNoPixel) __builtin_amdgcn_raw_buffer_store_b128(d, orsrc, (int)ooff, soff, 0);
+}
+
+// ReLU and 2x2 max-pooling (see store_pooled); right, below: byte addresses of the neighbour lanes for ds_bpermute.
+__device__ __forceinline__ void store_quad_pooled(const float (&v)[4], int right, int below, __amdgpu_buffer_rsrc_t orsrc,
+                                                  const unsigned (&ooff)[4], int soff) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float m = fmaxf(v[j], 0.f);
+    m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(right, __builtin_bit_cast(int, m))));
+    m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(below, __builtin_bit_cast(int, m))));
+    if (ooff[j] != kNoPixel)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, m), orsrc, (int)ooff[j], soff, 0);
+  }
+}
+
+// Writes a wave's accumulators: slot k of the wave goes to the output channel lane k holds in lane_oc, quad q of a lane to
+// the lane's four pixels of unit u0 + q.  The per-pixel byte offsets are formed once; a channel then only adds a
+// scalar offset.
+template <int NQ, int VARIANT, bool SPLIT>
+__device__ __forceinline__ void store_outputs(float* __restrict__ out, int lane_oc, const Geom& g, int u0, int n_base,
+                                              int limg, int lrow, int lx, bool lane_ok) {
+  const int ohw = g.OH * g.OW;
+  const __amdgpu_buffer_rsrc_t orsrc = block_of(out, n_base, g, ohw);
+  unsigned ooff[NQ][4];
+  pixel_offsets<NQ, 0>(ooff, g, u0, n_base, limg, lrow, lx, lane_ok);
+  const bool relu = !SPLIT && g.act != 0;  // a slice's partial sums are stored as they are
   for (int k = 0; k < g.g; ++k) {
     const int oc = __builtin_amdgcn_readlane(lane_oc, k);  // lane k fetched the slot's channel when the kernel began
     if (oc < 0) continue;  // padding slot
-    const int soff = oc * ohw * 4;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-      {
-        float v = read_accumulator<VARIANT>((k * NQ + q) * 4 + j);
-        if (relu) v = fmaxf(v, 0.f);
-        if (ooff[q][j] != kInvalid)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), orsrc, (int)ooff[q][j], soff, 0);
-      }
+    for (int q = 0; q < NQ; ++q) {
+      float v[4];
+      read_accumulators4<VARIANT>((k * NQ + q) * 4, v);
+      store_quad(v, relu, orsrc, ooff[q], oc * ohw * 4);
+    }
   }
 }
 
@@ -306,135 +358,149 @@ __device__ __forceinline__ void store_outputs(float* __restrict__ out, int lane_
 template <int NQ, int VARIANT>
 __device__ __forceinline__ void store_pooled(float* __restrict__ out, int lane_oc, const Geom& g, int u0, int n_base,
                                              int limg, int lrow, int lx, bool lane_ok) {
-  constexpr unsigned kInvalid = 0x80000000u;
-  const int upi = g.units_w * g.units_h;
-  const int poh = g.OH >> 1, pow_ = g.OW >> 1;
-  const int phw = poh * pow_;
-  const long long rec = (long long)(g.N - n_base) * g.K * (long long)phw * 4;
-  const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(
-      out + (size_t)n_base * g.K * phw, 0, rec > 0x7fffffffll ? 0x7fffffff : (int)rec, 0x00020000);
+  const int phw = (g.OH >> 1) * (g.OW >> 1);
+  const __amdgpu_buffer_rsrc_t orsrc = block_of(out, n_base, g, phw);
   const int lane = threadIdx.x & 63;
-  const int right = 4 * min(lane + 1, 63), below = 4 * min(lane + g.lr, 63);  // byte addresses for ds_bpermute
+  const int right = 4 * min(lane + 1, 63), below = 4 * min(lane + g.lr, 63);
   unsigned ooff[NQ][4];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int u = u0 + q;
-    const int ub_n = fast_div(u, g.m_upi);
-    const int ur = u - ub_n * upi;
-    const int ub_h = fast_div(ur, g.m_units_w);
-    const int ub_w = ur - ub_h * g.units_w;
-    const int n0 = (ub_n * g.nb + limg) * g.fold;
-    const int oh = ub_h * g.thi + lrow;
-    const int ow = ub_w * (1 << g.jsh) * g.lw + lx;
-    const bool ok = lane_ok && u < g.units && !(lrow & 1) && !(lx & 1) && (oh >> 1) < poh;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + (j >> g.jsh);
-      const int col = ow + (j & ((1 << g.jsh) - 1)) * g.lw;
-      ooff[q][j] = (ok && n < g.N && (col >> 1) < pow_)
-                       ? 4u * (unsigned)(((n - n_base) * g.K * poh + (oh >> 1)) * pow_ + (col >> 1)) : kInvalid;
-    }
-  }
+  pixel_offsets<NQ, 1>(ooff, g, u0, n_base, limg, lrow, lx, lane_ok);
   for (int k = 0; k < g.g; ++k) {
     const int oc = __builtin_amdgcn_readlane(lane_oc, k);
     if (oc < 0) continue;  // padding slot
-    const int soff = oc * phw * 4;
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-      {
-        float v = fmaxf(read_accumulator<VARIANT>((k * NQ + q) * 4 + j), 0.f);
-        v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(right, __builtin_bit_cast(int, v))));
-        v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(below, __builtin_bit_cast(int, v))));
-        if (ooff[q][j] != kInvalid)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), orsrc, (int)ooff[q][j], soff, 0);
-      }
+    for (int q = 0; q < NQ; ++q) {
+      float v[4];
+      read_accumulators4<VARIANT>((k * NQ + q) * 4, v);
+      store_quad_pooled(v, right, below, orsrc, ooff[q], oc * phw * 4);
+    }
   }
 }
 
 
-// ---- split layers: the last wave to finish adds the slices ---------------------------------------------------------
-// The workgroups that share an output tile (the slices of its channel reduction) have consecutive logical ids inside
-// one XCD's range, so they run on one XCD and meet in its L2.  Wave w of every slice holds the same output channels
-// and pixels.  Once its partial sums are stored and acknowledged by L2 (vmcnt(0)), a wave takes a ticket of the
-// (tile, wave) pair with an atomic add that L2 executes; the wave that draws ticket csplit - 1 knows that the same
-// wave of every other slice has stored its sums before taking its ticket, reads all slices back with loads that
-// bypass the CU's vector cache (sc1) and adds them in slice order.  Nobody waits for anybody.  The ticket is put
-// back to zero by the wave that used it up.
-__device__ __forceinline__ bool drew_last_ticket(int* __restrict__ tickets, int tile_id, int wave, const Geom& g) {
+// ---- split layers ---------------------------------------------------------------------------------------------------
+// Wave w of every slice of a tile holds the same output channels and pixels, so the slices can be added wave by wave,
+// and the sums need no other order in memory than the one the waves hold them in (sums_of).
+//
+// add_kernel adds them, or (TETRIS_OPT_ADD_IN_KERNEL) the wave that finishes last.  The workgroups that share an output tile have consecutive
+// logical ids inside one XCD's range, so they run on one XCD and meet in its L2.  Once its sums are stored and
+// acknowledged by L2 (vmcnt(0)), a wave takes a ticket of the (tile, wave) pair with an atomic add that L2 executes
+// (workgroup scope: the tickets of an XCD share no line with another's); the wave that draws ticket csplit - 1 knows
+// that the same wave of every other slice has stored its sums before taking its ticket, reads all slices back with
+// loads that bypass the CU's vector cache (sc0) and adds them in slice order.  Nobody waits for anybody.  The ticket is
+// put back to zero by the wave that used it up.
+//
+// What bounds the adding wave is the round trip to L2, with nothing left in the kernel to hide it.  Its accumulators
+// are in memory by then, so their registers are where the sums land: 64 or 128 of them, filled in one round trip.
+__device__ __forceinline__ bool drew_last_ticket(int* __restrict__ tickets, int wave, const Geom& g) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partial sums have reached L2
-  int* t = tickets + tile_id * g.waves + wave;
+  int* t = tickets + (blockIdx.x & 7) * (kMaxTickets / 8) + fast_div(blockIdx.x >> 3, g.m_csplit) * g.waves + wave;
   int old = 0;
-  if ((threadIdx.x & 63) == 0) old = __hip_atomic_fetch_add(t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((threadIdx.x & 63) == 0) old = __hip_atomic_fetch_add(t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   old = __builtin_amdgcn_readfirstlane(old);
   if (old != g.csplit - 1) return false;
-  if ((threadIdx.x & 63) == 0) __hip_atomic_store(t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((threadIdx.x & 63) == 0) __hip_atomic_store(t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   return true;
 }
-constexpr int kBypassL1 = 16;  // cache policy of a buffer load: sc1 (agent scope), never served by the CU's vector cache
 
-// The halo'd kernels' counterpart of store_outputs for the wave that drew the last ticket: out[...] = act(sum over the
-// slices, in slice order, of the partial sums at the same offsets).
-template <int NQ>
-__device__ __forceinline__ void add_slices(const float* __restrict__ partial, float* __restrict__ out, int lane_oc,
-                                           const Geom& g, int u0, int n_base, int limg, int lrow, int lx, bool lane_ok) {
-  constexpr unsigned kInvalid = 0x80000000u;
-  const int upi = g.units_w * g.units_h;
-  const int ohw = g.OH * g.OW;
-  const size_t out_elems = (size_t)g.N * g.K * ohw;
-  const long long rec = (long long)(g.N - n_base) * g.K * (long long)ohw * 4;
-  const int records = rec > 0x7fffffffll ? 0x7fffffff : (int)rec;
-  const __amdgpu_buffer_rsrc_t orsrc =
-      __builtin_amdgcn_make_buffer_rsrc(out + (size_t)n_base * g.K * ohw, 0, records, 0x00020000);
-  unsigned ooff[NQ][4];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int u = u0 + q;
-    const int ub_n = fast_div(u, g.m_upi);
-    const int ur = u - ub_n * upi;
-    const int ub_h = fast_div(ur, g.m_units_w);
-    const int ub_w = ur - ub_h * g.units_w;
-    const int n0 = (ub_n * g.nb + limg) * g.fold;
-    const int oh = ub_h * g.thi + lrow;
-    const int ow = ub_w * (1 << g.jsh) * g.lw + lx;
-    const bool ok = lane_ok && u < g.units && oh < g.OH;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + (j >> g.jsh);
-      const int col = ow + (j & ((1 << g.jsh) - 1)) * g.lw;
-      ooff[q][j] = (ok && n < g.N && col < g.OW) ? 4u * (unsigned)(((n - n_base) * g.K * g.OH + oh) * g.OW + col) : kInvalid;
+template <int VARIANT>
+constexpr int kFirstAcc = small_acc(VARIANT) ? 64 : 128;
+template <int VARIANT>
+constexpr int kAccs = small_acc(VARIANT) ? 64 : 128;
+
+// Where a wave keeps its sums for the wave that adds: 16 bytes per lane and quad, a channel's quads and the wave's
+// channels one after another; bytes `slice` apart for the slices of a tile.
+struct SliceSums { float* base; u4 rsrc; int slice_bytes; };
+__device__ __forceinline__ SliceSums sums_of(float* partial, int tile_id, int wave, int nq, const Geom& g) {
+  const int wave_bytes = g.g * nq * g.sum_bytes;
+  const unsigned long long base = reinterpret_cast<unsigned long long>(partial) +
+                                  ((size_t)tile_id * g.csplit * g.waves + wave) * (size_t)wave_bytes;
+  SliceSums s;
+  s.base = reinterpret_cast<float*>(base);
+  s.slice_bytes = g.waves * wave_bytes;
+  s.rsrc = u4{(unsigned)uniform((int)base), (unsigned)uniform((int)(base >> 32)),
+              (unsigned)((g.csplit - 1) * s.slice_bytes + wave_bytes), 0x00020000u};
+  asm volatile("s_nop 4" : "+s"(s.rsrc));  // five wait states between a vector instruction's write of it and a load
+  return s;
+}
+
+// Loads of (channel, slice) pairs into the accumulators, four registers each: B-th load to accumulators 4 B ..., `k` the
+// running (channel, quad), `s` the slice.
+template <int VARIANT, int B = 0>
+__device__ __forceinline__ void land_slices(const SliceSums& p, int lane16, int kq, int s, int loads, const Geom& g) {
+  if constexpr (B < kAccs<VARIANT> / 4) {
+    if (B >= loads) return;
+    constexpr int R = kFirstAcc<VARIANT> + 4 * B;
+    int soff;
+    asm volatile("s_mov_b32 %0, %1" : "=s"(soff) : "s"(uniform(kq * g.sum_bytes + s * p.slice_bytes)));  // a scalar write needs no wait states
+    asm volatile("buffer_load_dwordx4 v[%0:%1], %2, %3, %4 offen sc0" ::"n"(R), "n"(R + 3), "v"(lane16), "s"(p.rsrc), "s"(soff)
+                 : "memory");
+    const bool next = s + 1 == g.csplit;
+    land_slices<VARIANT, B + 1>(p, lane16, next ? kq + 1 : kq, next ? 0 : s + 1, loads, g);
+  }
+}
+
+template <int VARIANT, int NQ>
+__device__ __forceinline__ void store_sums(const SliceSums& p, int lane16, int slice, const Geom& g) {
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(p.base, 0, (int)p.rsrc.z, 0x00020000);
+  for (int kq = 0; kq < g.g * NQ; ++kq) {
+    float v[4];
+    read_accumulators4<VARIANT>(kq * 4, v);
+    store_consecutive(v, false, rsrc, (unsigned)lane16, slice * p.slice_bytes + kq * g.sum_bytes);
+  }
+}
+
+// Reads back, adds and hands on the sums of all of the wave's channels: finish(channel, q, v) once per channel and quad.
+template <int VARIANT, int NQ, class Finish>
+__device__ __forceinline__ void add_slices(const SliceSums& p, int lane16, int lane_oc, const Geom& g, Finish finish) {
+  const int fit = fast_div(kAccs<VARIANT> / 4, g.m_csplit);  // (channel, quad)s per round trip, at least one
+  for (int kq0 = 0; kq0 < g.g * NQ; kq0 += fit) {
+    const int n = min(fit, g.g * NQ - kq0);
+    land_slices<VARIANT>(p, lane16, kq0, 0, n * g.csplit, g);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (int i = 0; i < n; ++i) {
+      const int k = (kq0 + i) / NQ, q = (kq0 + i) % NQ;
+      const int oc = __builtin_amdgcn_readlane(lane_oc, k);
+      if (oc < 0) continue;  // padding slot
+      int r = i * g.csplit * 4;
+      float v[4];
+      read_accumulators4<VARIANT>(r, v);
+      for (int s = 1; s < g.csplit; ++s) add_accumulators4<VARIANT>(r += 4, v);
+      finish(oc, q, v);
     }
   }
-  const bool relu = g.act != 0;
-  for (int k = 0; k < g.g; ++k) {
-    const int oc = __builtin_amdgcn_readlane(lane_oc, k);
-    if (oc < 0) continue;  // padding slot
-    const int soff = oc * ohw * 4;
-    float sum[NQ][4];
-    for (int s = 0; s < g.csplit; ++s) {
-      const __amdgpu_buffer_rsrc_t prsrc = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<float*>(partial) + (size_t)s * out_elems + (size_t)n_base * g.K * ohw, 0, records, 0x00020000);
+}
+
+// The halo'd kernels' output for the wave that drew the last ticket.
+template <int NQ, int VARIANT>
+__device__ __forceinline__ void add_and_store(const SliceSums& p, int lane16, float* __restrict__ out, int lane_oc, const Geom& g, int u0,
+                                              int n_base, int limg, int lrow, int lx, bool lane_ok) {
+  unsigned ooff[NQ][4];
+  if (g.act == 2) {
+    pixel_offsets<NQ, 1>(ooff, g, u0, n_base, limg, lrow, lx, lane_ok);
+    const int phw = (g.OH >> 1) * (g.OW >> 1);
+    const __amdgpu_buffer_rsrc_t orsrc = block_of(out, n_base, g, phw);
+    const int lane = threadIdx.x & 63;
+    const int right = 4 * min(lane + 1, 63), below = 4 * min(lane + g.lr, 63);
+    add_slices<VARIANT, NQ>(p, lane16, lane_oc, g, [&](int oc, int q, const float(&v)[4]) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q)
+      for (int i = 0; i < NQ; ++i)
+        if (i == q) store_quad_pooled(v, right, below, orsrc, ooff[i], oc * phw * 4);
+    });
+  } else {
+    pixel_offsets<NQ, 0>(ooff, g, u0, n_base, limg, lrow, lx, lane_ok);
+    const int ohw = g.OH * g.OW;
+    const __amdgpu_buffer_rsrc_t orsrc = block_of(out, n_base, g, ohw);
+    const bool relu = g.act != 0;
+    add_slices<VARIANT, NQ>(p, lane16, lane_oc, g, [&](int oc, int q, const float(&v)[4]) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {  // an offset out of range reads as zero
-          const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(prsrc, (int)ooff[q][j], soff, kBypassL1));
-          sum[q][j] = s == 0 ? v : sum[q][j] + v;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (ooff[q][j] != kInvalid)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, relu ? fmaxf(sum[q][j], 0.f) : sum[q][j]), orsrc,
-                                                (int)ooff[q][j], soff, 0);
+      for (int i = 0; i < NQ; ++i)
+        if (i == q) store_quad(v, relu, orsrc, ooff[i], oc * ohw * 4);
+    });
   }
 }
 
 // SPT: 16-byte LDS slots of the unit group a thread stages (1 or 2)
-template <int NQ, int SPT>
+template <int NQ, int SPT, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(88))) void spconv2d_kernel(
     const float* __restrict__ in, float* __restrict__ out, const int2* __restrict__ entries,
     const int32_t* __restrict__ grp_off, const int32_t* __restrict__ grp_pair,
@@ -451,17 +517,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(88))) void spco
   // Workgroup -> (unit group, channel block).  Consecutive workgroup ids go round-robin to the eight XCDs;
   // give each XCD a contiguous range of logical ids so that the channel blocks of one unit group, which read
   // the same input, share an L2.
-  const int total = g.ugroups * g.kblocks * g.csplit;
+  const int total = g.ugroups * g.kblocks * (SPLIT ? g.csplit : 1);
   const int per_xcd = gridDim.x >> 3;
   const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (logical >= total) return;
-  const int tile_id = fast_div(logical, g.m_csplit);  // slices of one output tile are neighbours: same XCD, same L2
-  const int slice = logical - tile_id * g.csplit;
+  const int tile_id = SPLIT ? fast_div(logical, g.m_csplit) : logical;  // slices of one output tile are neighbours: same XCD, same L2
+  const int slice = SPLIT ? logical - tile_id * g.csplit : 0;
   const int ugroup = fast_div(tile_id, g.m_kblocks);
   const int kblock = tile_id - ugroup * g.kblocks;
   const int u0 = ugroup * NQ;
   // this workgroup's stages (multiply-high division: make_geom checks its range)
-  const int st0 = fast_div(slice * g.stages, g.m_csplit), st1 = fast_div((slice + 1) * g.stages, g.m_csplit);
+  const int st0 = SPLIT ? fast_div(slice * g.stages, g.m_csplit) : 0;
+  const int st1 = SPLIT ? fast_div((slice + 1) * g.stages, g.m_csplit) : g.stages;
   // a slice of a split reduction writes its partial sums to its own copy of the output (`out` is then that scratch)
   const size_t out_elems = (size_t)g.N * g.K * g.OH * g.OW;
   const int upi = g.units_w * g.units_h;  // units per image block
@@ -610,10 +677,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(88))) void spco
 
   // ---- write the outputs -------------------------------------------------------------------------------------
   if (g.N < 0) out[0] = __builtin_bit_cast(float, sink ^ touched);  // never true: keeps the touching loads alive
-  if (g.act == 2) store_pooled<NQ, 2>(out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
-  else store_outputs<NQ, 2>(out + (size_t)slice * out_elems, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
-  if (g.fused && drew_last_ticket(tickets, tile_id, wave, g))
-    add_slices<NQ>(out, final_out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  if (SPLIT && g.fused) {
+    const SliceSums sums = sums_of(out, tile_id, wave, NQ, g);
+    const int lane16 = lane_ok ? 16 * (ly * g.lw + lx) : (int)kNoPixel;  // idle lanes keep no sums
+    store_sums<2, NQ>(sums, lane16, slice, g);
+    if (g.fused == 1 && drew_last_ticket(tickets, wave, g))
+      add_and_store<NQ, 2>(sums, lane16, final_out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  } else if (!SPLIT && g.act == 2) {
+    store_pooled<NQ, 2>(out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  } else {
+    store_outputs<NQ, 2, SPLIT>(out + (size_t)slice * out_elems, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  }
   TETRIS_STAMP_END();
 }
 
@@ -633,7 +707,7 @@ static_assert(TETRIS_WALK_TILE_BYTES == kTileBytes && TETRIS_WALK_BUF_BYTES == k
 //     end of the stage; every SIMD holds a wave of each half, so one computes while the other issues loads.
 // WAVES == 8: 128 accumulators per wave, two waves per SIMD.  WAVES == 16: 64 accumulators and at most 128 VGPRs
 // per wave, four waves per SIMD, which hides more of the LDS latency (the loop alone runs about 1.3x faster).
-template <int NQ, int WAVES, int VARIANT>
+template <int NQ, int WAVES, int VARIANT, bool SPLIT>
 __device__ __forceinline__ void conv3_body(const float* __restrict__ in, float* __restrict__ out,
                                            const int2* __restrict__ entries, const int32_t* __restrict__ grp_off,
                                            const int32_t* __restrict__ grp_pair, const int32_t* __restrict__ oc_order,
@@ -648,17 +722,18 @@ __device__ __forceinline__ void conv3_body(const float* __restrict__ in, float* 
   const int lane = tid & 63;
   const int wave = uniform(tid >> 6);
 
-  const int total = g.ugroups * g.kblocks * g.csplit;
+  const int total = g.ugroups * g.kblocks * (SPLIT ? g.csplit : 1);
   const int per_xcd = gridDim.x >> 3;
   const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (logical >= total) return;
-  const int tile_id = fast_div(logical, g.m_csplit);  // slices of one output tile are neighbours: same XCD, same L2
-  const int slice = logical - tile_id * g.csplit;
+  const int tile_id = SPLIT ? fast_div(logical, g.m_csplit) : logical;  // slices of one output tile are neighbours: same XCD, same L2
+  const int slice = SPLIT ? logical - tile_id * g.csplit : 0;
   const int ugroup = fast_div(tile_id, g.m_kblocks);
   const int kblock = tile_id - ugroup * g.kblocks;
   const int u0 = ugroup * NQ;
   // this workgroup's stages (multiply-high division: make_geom checks its range)
-  const int st0 = fast_div(slice * g.stages, g.m_csplit), st1 = fast_div((slice + 1) * g.stages, g.m_csplit);
+  const int st0 = SPLIT ? fast_div(slice * g.stages, g.m_csplit) : 0;
+  const int st1 = SPLIT ? fast_div((slice + 1) * g.stages, g.m_csplit) : g.stages;
   // a slice of a split reduction writes its partial sums to its own copy of the output (`out` is then that scratch)
   const size_t out_elems = (size_t)g.N * g.K * g.OH * g.OW;
   const int upi = g.units_w * g.units_h;
@@ -821,35 +896,42 @@ __device__ __forceinline__ void conv3_body(const float* __restrict__ in, float* 
 
   // ---- write the outputs -------------------------------------------------------------------------------------
   if (g.N < 0) out[0] = __builtin_bit_cast(float, sink);  // never true: keeps the touching loads alive
-  if (g.act == 2) store_pooled<NQ, VARIANT>(out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
-  else store_outputs<NQ, VARIANT>(out + (size_t)slice * out_elems, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
-  if (g.fused && drew_last_ticket(tickets, tile_id, wave, g))
-    add_slices<NQ>(out, final_out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  if (SPLIT && g.fused) {
+    const SliceSums sums = sums_of(out, tile_id, wave, NQ, g);
+    const int lane16 = lane_ok ? 16 * (ly * g.lw + lx) : (int)kNoPixel;  // idle lanes keep no sums
+    store_sums<VARIANT, NQ>(sums, lane16, slice, g);
+    if (g.fused == 1 && drew_last_ticket(tickets, wave, g))
+      add_and_store<NQ, VARIANT>(sums, lane16, final_out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  } else if (!SPLIT && g.act == 2) {
+    store_pooled<NQ, VARIANT>(out, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  } else {
+    store_outputs<NQ, VARIANT, SPLIT>(out + (size_t)slice * out_elems, lane_oc, g, u0, n_base, limg, lrow, lx, lane_ok);
+  }
   TETRIS_STAMP_END();
 }
 
-template <int NQ>
+template <int NQ, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(TETRIS_WALK3_FIRST_RESERVED_4))) void spconv2d_kernel3(
     const float* __restrict__ in, float* __restrict__ out, const int2* __restrict__ entries,
     const int32_t* __restrict__ grp_off, const int32_t* __restrict__ grp_pair,
     const int32_t* __restrict__ oc_order, float* __restrict__ final_out, int* __restrict__ tickets, const Geom g) {
-  conv3_body<NQ, 8, 3>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
+  conv3_body<NQ, 8, 3, SPLIT>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
 }
 
-template <int NQ>
+template <int NQ, bool SPLIT>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_num_vgpr(TETRIS_WALK4_FIRST_RESERVED_2))) void spconv2d_kernel4(
     const float* __restrict__ in, float* __restrict__ out, const int2* __restrict__ entries,
     const int32_t* __restrict__ grp_off, const int32_t* __restrict__ grp_pair,
     const int32_t* __restrict__ oc_order, float* __restrict__ final_out, int* __restrict__ tickets, const Geom g) {
-  conv3_body<NQ, 16, 4>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
+  conv3_body<NQ, 16, 4, SPLIT>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
 }
 
-template <int NQ>
+template <int NQ, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(TETRIS_WALK5_FIRST_RESERVED_2))) void spconv2d_kernel5(
     const float* __restrict__ in, float* __restrict__ out, const int2* __restrict__ entries,
     const int32_t* __restrict__ grp_off, const int32_t* __restrict__ grp_pair,
     const int32_t* __restrict__ oc_order, float* __restrict__ final_out, int* __restrict__ tickets, const Geom g) {
-  conv3_body<NQ, 8, 5>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
+  conv3_body<NQ, 8, 5, SPLIT>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
 }
 
 // Pointwise layers (1x1, stride 1, no padding) with flat tiles: a lane owns four consecutive pixels of one image
@@ -864,7 +946,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(TETRIS_WALK5_FI
 //     output channel when H*W is a multiple of four.
 // VARIANT 6: 16 waves, 64 accumulators; 7: 8 waves, 128 accumulators (64 KiB buffers, one workgroup per CU);
 // 8: 8 waves, 64 accumulators, 32 KiB buffers, two workgroups per CU.
-template <int NQ, int WAVES, int VARIANT>
+template <int NQ, int WAVES, int VARIANT, bool SPLIT>
 __device__ __forceinline__ void flat_body(const float* __restrict__ in, float* __restrict__ out,
                                           const int2* __restrict__ entries, const int32_t* __restrict__ grp_off,
                                           const int32_t* __restrict__ grp_pair, const int32_t* __restrict__ oc_order,
@@ -878,16 +960,17 @@ __device__ __forceinline__ void flat_body(const float* __restrict__ in, float* _
   const int lane = tid & 63;
   const int wave = uniform(tid >> 6);
 
-  const int total = g.ugroups * g.kblocks * g.csplit;
+  const int total = g.ugroups * g.kblocks * (SPLIT ? g.csplit : 1);
   const int per_xcd = gridDim.x >> 3;
   const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (logical >= total) return;
-  const int tile_id = fast_div(logical, g.m_csplit);
-  const int slice = logical - tile_id * g.csplit;
+  const int tile_id = SPLIT ? fast_div(logical, g.m_csplit) : logical;
+  const int slice = SPLIT ? logical - tile_id * g.csplit : 0;
   const int ugroup = fast_div(tile_id, g.m_kblocks);
   const int kblock = tile_id - ugroup * g.kblocks;
   const int u0 = ugroup * NQ;
-  const int st0 = fast_div(slice * g.stages, g.m_csplit), st1 = fast_div((slice + 1) * g.stages, g.m_csplit);
+  const int st0 = SPLIT ? fast_div(slice * g.stages, g.m_csplit) : 0;
+  const int st1 = SPLIT ? fast_div((slice + 1) * g.stages, g.m_csplit) : g.stages;
   const size_t out_elems = (size_t)g.N * g.K * g.OH * g.OW;
   const int hw = g.in_hw;        // floats per (image, channel) plane of the input in memory
   const int ohw = g.OH * g.OW;   // ... of the output: the same, unless the layer is strided
@@ -1019,15 +1102,37 @@ __device__ __forceinline__ void flat_body(const float* __restrict__ in, float* _
 
   // ---- write the outputs ------------------------------------------------------------------------------------------
   if (g.N < 0) out[0] = __builtin_bit_cast(float, sink);  // never true: keeps the touching loads alive
+  if (SPLIT && g.fused) {
+    const SliceSums sums = sums_of(out, tile_id, wave, NQ, g);
+    store_sums<VARIANT, NQ>(sums, 16 * lane, slice, g);
+    if (g.fused != 1 || !drew_last_ticket(tickets, wave, g)) {
+      TETRIS_STAMP_END();
+      return;
+    }
+    const bool vec = (ohw & 3) == 0 && (reinterpret_cast<size_t>(final_out) & 15) == 0;
+    const __amdgpu_buffer_rsrc_t frsrc = block_of(final_out, n_base, g, ohw);
+    add_slices<VARIANT, NQ>(sums, 16 * lane, lane_oc, g, [&](int oc, int q, const float(&v)[4]) {
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        if (i != q) continue;
+        unsigned poff[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) poff[j] = j < npx[i] ? ooff[i] + 4 * j : kNoPixel;
+        if (vec) store_consecutive(v, g.act != 0, frsrc, ooff[i], oc * ohw * 4);
+        else store_quad(v, g.act != 0, frsrc, poff, oc * ohw * 4);
+      }
+    });
+    TETRIS_STAMP_END();
+    return;
+  }
   float* obase = out + (size_t)slice * out_elems + (size_t)n_base * g.K * ohw;
   const long long orec = (long long)(g.N - n_base) * g.K * (long long)ohw * 4;
   const __amdgpu_buffer_rsrc_t orsrc =
       __builtin_amdgcn_make_buffer_rsrc(obase, 0, orec > 0x7fffffffll ? 0x7fffffff : (int)orec, 0x00020000);
   // 16-byte stores need every quad whole and 16-byte aligned addresses
   const bool vec = (ohw & 3) == 0 && (reinterpret_cast<size_t>(out) & 15) == 0;
-  const bool relu = g.act != 0 && g.csplit == 1;  // a slice's partial sums are stored as they are
+  const bool relu = !SPLIT && g.act != 0;  // a slice's partial sums are stored as they are
   typedef float f4 __attribute__((ext_vector_type(4)));
-  typedef unsigned u4 __attribute__((ext_vector_type(4)));
   for (int k = 0; k < g.g; ++k) {
     const int oc = __builtin_amdgcn_readlane(lane_oc, k);
     if (oc < 0) continue;  // padding slot
@@ -1052,82 +1157,98 @@ __device__ __forceinline__ void flat_body(const float* __restrict__ in, float* _
       }
     }
   }
-  if (!(g.fused && drew_last_ticket(tickets, tile_id, wave, g))) {
-    TETRIS_STAMP_END();
-    return;
-  }
-  // This wave adds the slices (see drew_last_ticket): the same quads and channels at the same offsets of every slice.
-  const bool fvec = vec && (reinterpret_cast<size_t>(final_out) & 15) == 0;
-  const __amdgpu_buffer_rsrc_t frsrc = __builtin_amdgcn_make_buffer_rsrc(
-      final_out + (size_t)n_base * g.K * ohw, 0, orec > 0x7fffffffll ? 0x7fffffff : (int)orec, 0x00020000);
-  const bool frelu = g.act != 0;
-  for (int k = 0; k < g.g; ++k) {
-    const int oc = __builtin_amdgcn_readlane(lane_oc, k);
-    if (oc < 0) continue;
-    const int soff = oc * ohw * 4;
-    float sum[NQ][4];
-    for (int s = 0; s < g.csplit; ++s) {
-      const __amdgpu_buffer_rsrc_t prsrc = __builtin_amdgcn_make_buffer_rsrc(
-          out + (size_t)s * out_elems + (size_t)n_base * g.K * ohw, 0, orec > 0x7fffffffll ? 0x7fffffff : (int)orec, 0x00020000);
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        float v[4];
-        if (vec) {  // an offset out of range reads as zero
-          const f4 d = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(prsrc, (int)ooff[q], soff, kBypassL1));
-          v[0] = d.x; v[1] = d.y; v[2] = d.z; v[3] = d.w;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            v[j] = j < npx[q] ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                    prsrc, (int)ooff[q] + 4 * j, soff, kBypassL1)) : 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sum[q][j] = s == 0 ? v[j] : sum[q][j] + v[j];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      if (ooff[q] == kInvalid) continue;
-      if (frelu) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sum[q][j] = fmaxf(sum[q][j], 0.f);
-      }
-      if (fvec) {
-        const f4 d = {sum[q][0], sum[q][1], sum[q][2], sum[q][3]};
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, d), frsrc, (int)ooff[q], soff, 0);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (j < npx[q])
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sum[q][j]), frsrc, (int)ooff[q] + 4 * j, soff, 0);
-      }
-    }
-  }
   TETRIS_STAMP_END();
 }
 
-template <int NQ>
+template <int NQ, bool SPLIT>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_num_vgpr(TETRIS_WALK6_FIRST_RESERVED_2))) void spconv2d_flat6(
     const float* __restrict__ in, float* __restrict__ out, const int2* __restrict__ entries,
     const int32_t* __restrict__ grp_off, const int32_t* __restrict__ grp_pair,
     const int32_t* __restrict__ oc_order, float* __restrict__ final_out, int* __restrict__ tickets, const Geom g) {
-  flat_body<NQ, 16, 6>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
+  flat_body<NQ, 16, 6, SPLIT>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
 }
 
-template <int NQ>
+template <int NQ, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(TETRIS_WALK7_FIRST_RESERVED_4))) void spconv2d_flat7(
     const float* __restrict__ in, float* __restrict__ out, const int2* __restrict__ entries,
     const int32_t* __restrict__ grp_off, const int32_t* __restrict__ grp_pair,
     const int32_t* __restrict__ oc_order, float* __restrict__ final_out, int* __restrict__ tickets, const Geom g) {
-  flat_body<NQ, 8, 7>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
+  flat_body<NQ, 8, 7, SPLIT>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
 }
 
-template <int NQ>
+template <int NQ, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_num_vgpr(TETRIS_WALK8_FIRST_RESERVED_2))) void spconv2d_flat8(
     const float* __restrict__ in, float* __restrict__ out, const int2* __restrict__ entries,
     const int32_t* __restrict__ grp_off, const int32_t* __restrict__ grp_pair,
     const int32_t* __restrict__ oc_order, float* __restrict__ final_out, int* __restrict__ tickets, const Geom g) {
-  flat_body<NQ, 8, 8>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
+  flat_body<NQ, 8, 8, SPLIT>(in, out, entries, grp_off, grp_pair, oc_order, final_out, tickets, g);
+}
+
+// Adds the slices of a split layer whose waves kept their sums in the order of sums_of: a wave per (tile, wave of the
+// tile, channel of the wave, quad).  A launch of a few microseconds is a chain of round trips, so nothing is serial that
+// need not be: the kernel arguments are touched at once, all slices' loads (1 KiB of consecutive bytes each) are on
+// their way before the channel and the pixels are worked out, and a wave has one sum per lane and slice only (two or
+// four: 5 ... 25 % slower).  Workgroups are mapped to tiles as in the conv kernel, so that a tile's sums are read on the
+// XCD that wrote them.
+__global__ __launch_bounds__(256) void add_kernel(const float* __restrict__ partial, float* __restrict__ out,
+                                                  const int32_t* __restrict__ oc_order, unsigned m_per_wave, unsigned m_nq,
+                                                  const Geom g) {
+  touch_kernel_arguments();
+  const int tiles = g.ugroups * g.kblocks;
+  const int tile_id = (blockIdx.x & 7) * ((tiles + 7) >> 3) + (blockIdx.x >> 3);  // eight ranges of tiles, one per XCD
+  const int lane = threadIdx.x & 63;
+  const int item = uniform(blockIdx.y * 4 + (threadIdx.x >> 6));
+  const int per_wave = g.g * g.nq;
+  if (tile_id >= tiles || item >= g.waves * per_wave) return;
+  const bool flat = g.ver == 4;
+  const int ly = flat ? 0 : fast_div(lane, g.m_lr);
+  const int lx = lane - ly * g.lr;
+  const int limg = flat ? 0 : fast_div(ly, g.m_thi);
+  const int lrow = ly - limg * g.thi;
+  const bool lane_ok = flat || (ly < g.lh && limg < g.nb && lx < g.lw);
+  const size_t slice = (size_t)g.waves * per_wave * g.sum_bytes;
+  const char* src = reinterpret_cast<const char*>(partial) + (size_t)tile_id * g.csplit * slice + (size_t)item * g.sum_bytes +
+                    (lane_ok ? 16 * (ly * g.lw + lx) : 0);
+  float4 p[kMaxSplit];
+#pragma unroll
+  for (int s = 0; s < kMaxSplit; ++s)
+    if (s < g.csplit) p[s] = *reinterpret_cast<const float4*>(src + s * slice);
+  const int wave = fast_div(item, m_per_wave), kq = item - wave * per_wave;
+  const int k = fast_div(kq, m_nq), q = kq - k * g.nq;
+  const int ugroup = fast_div(tile_id, g.m_kblocks);
+  const int kblock = tile_id - ugroup * g.kblocks;
+  const int oc = oc_order[uniform((kblock * g.waves + wave) * g.g + k)];
+  if (oc < 0) return;  // padding slot
+  const int u0 = ugroup * g.nq;
+  const int ohw = g.OH * g.OW;
+  const int n_base = flat ? fast_div(u0 * 64, g.m_qi) : fast_div(u0, g.m_upi) * g.nb * g.fold;
+  unsigned ooff[1][4];
+  if (flat) {
+    const int qd = (u0 + q) * 64 + lane;
+    const int n = fast_div(qd, g.m_qi);
+    const int qq = qd - n * g.qi;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      ooff[0][j] = qd < g.quads_total && 4 * qq + j < ohw ? 4u * (unsigned)((n - n_base) * g.K * ohw + 4 * qq + j) : kNoPixel;
+  } else if (g.act == 2) {
+    pixel_offsets<1, 1>(ooff, g, u0 + q, n_base, limg, lrow, lx, lane_ok);
+  } else {
+    pixel_offsets<1, 0>(ooff, g, u0 + q, n_base, limg, lrow, lx, lane_ok);
+  }
+  float v[4] = {p[0].x, p[0].y, p[0].z, p[0].w};
+#pragma unroll
+  for (int s = 1; s < kMaxSplit; ++s)
+    if (s < g.csplit) {
+      v[0] += p[s].x; v[1] += p[s].y; v[2] += p[s].z; v[3] += p[s].w;
+    }
+  if (g.act == 2) {
+    const int phw = (g.OH >> 1) * (g.OW >> 1);
+    store_quad_pooled(v, 4 * min(lane + 1, 63), 4 * min(lane + g.lr, 63), block_of(out, n_base, g, phw), ooff[0], oc * phw * 4);
+  } else if (flat && (ohw & 3) == 0 && (reinterpret_cast<size_t>(out) & 15) == 0) {
+    store_consecutive(v, g.act != 0, block_of(out, n_base, g, ohw), ooff[0][0], oc * ohw * 4);
+  } else {
+    store_quad(v, g.act != 0, block_of(out, n_base, g, ohw), ooff[0], oc * ohw * 4);
+  }
 }
 
 // Adds the `slices` partial outputs of a split reduction, in slice order (so the result does not depend on timing);
@@ -1214,18 +1335,18 @@ int grid_size(const Geom& g) {
   return 8 * ((tiles + 7) / 8) * g.csplit;
 }
 
-template <int NQ, int WAVES, int VARIANT>
+template <int NQ, int WAVES, int VARIANT, bool SPLIT>
 int launch_three(const Geom& g, const float* d_in, float* d_out, const int2* entries, const int32_t* grp_off,
                  const int32_t* grp_pair, const int32_t* oc_order, float* d_final, int* d_tickets, hipStream_t stream) {
   void (*kern)(const float*, float*, const int2*, const int32_t*, const int32_t*, const int32_t*, float*, int*, const Geom);
   constexpr int LDS = VARIANT == 5 ? kBufs * kHalfBufBytes : VARIANT == 8 ? 2 * kFlatHalfBufBytes
                       : VARIANT >= 6 ? 2 * kFlatBufBytes : kBufs * kBufBytes;
-  if constexpr (VARIANT == 4) kern = spconv2d_kernel4<NQ>;
-  else if constexpr (VARIANT == 5) kern = spconv2d_kernel5<NQ>;
-  else if constexpr (VARIANT == 6) kern = spconv2d_flat6<NQ>;
-  else if constexpr (VARIANT == 7) kern = spconv2d_flat7<NQ>;
-  else if constexpr (VARIANT == 8) kern = spconv2d_flat8<NQ>;
-  else kern = spconv2d_kernel3<NQ>;
+  if constexpr (VARIANT == 4) kern = spconv2d_kernel4<NQ, SPLIT>;
+  else if constexpr (VARIANT == 5) kern = spconv2d_kernel5<NQ, SPLIT>;
+  else if constexpr (VARIANT == 6) kern = spconv2d_flat6<NQ, SPLIT>;
+  else if constexpr (VARIANT == 7) kern = spconv2d_flat7<NQ, SPLIT>;
+  else if constexpr (VARIANT == 8) kern = spconv2d_flat8<NQ, SPLIT>;
+  else kern = spconv2d_kernel3<NQ, SPLIT>;
   static std::atomic<bool> lds_set{false};  // per instantiation; setting the attribute twice is harmless
   if (!lds_set.load(std::memory_order_acquire)) {
     TETRIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
@@ -1237,10 +1358,10 @@ int launch_three(const Geom& g, const float* d_in, float* d_out, const int2* ent
   return TETRIS_OK;
 }
 
-template <int NQ, int SPT>
+template <int NQ, int SPT, bool SPLIT>
 int launch_one(const Geom& g, const float* d_in, float* d_out, const int2* entries, const int32_t* grp_off,
                const int32_t* grp_pair, const int32_t* oc_order, float* d_final, int* d_tickets, hipStream_t stream) {
-  auto kern = spconv2d_kernel<NQ, SPT>;
+  auto kern = spconv2d_kernel<NQ, SPT, SPLIT>;
   static std::atomic<bool> lds_set{false};  // per instantiation; setting the attribute twice is harmless
   if (!lds_set.load(std::memory_order_acquire)) {
     TETRIS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1255,6 +1376,7 @@ int launch_one(const Geom& g, const float* d_in, float* d_out, const int2* entri
 
 }  // namespace
 
+template <bool SPLIT>
 static int launch_kernel(const Geom& g, const float* d_in, float* d_out, const int2* entries, const int32_t* grp_off,
                          const int32_t* grp_pair, const int32_t* oc_order, float* d_final, int* d_tickets,
                          hipStream_t stream) {
@@ -1266,15 +1388,15 @@ static int launch_kernel(const Geom& g, const float* d_in, float* d_out, const i
         g.stagers > g.waves || g.ugroups * g.nq * 64ll < g.quads_total)
       return fail(TETRIS_EINVAL, "inconsistent kernel geometry (flat kernel)");
     if (g.waves == 16) {
-      if (g.nq == 1) return launch_three<1, 16, 6>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 2) return launch_three<2, 16, 6>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 1) return launch_three<1, 16, 6, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 2) return launch_three<2, 16, 6, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
     } else if (g.buf_bytes == kFlatHalfBufBytes) {
-      if (g.nq == 1) return launch_three<1, 8, 8>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 2) return launch_three<2, 8, 8>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 1) return launch_three<1, 8, 8, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 2) return launch_three<2, 8, 8, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
     } else {
-      if (g.nq == 1) return launch_three<1, 8, 7>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 2) return launch_three<2, 8, 7>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 4) return launch_three<4, 8, 7>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 1) return launch_three<1, 8, 7, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 2) return launch_three<2, 8, 7, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 4) return launch_three<4, 8, 7, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
     }
     return fail(TETRIS_EINVAL, "no flat kernel for quads=%d waves=%d", g.nq, g.waves);
   }
@@ -1285,22 +1407,22 @@ static int launch_kernel(const Geom& g, const float* d_in, float* d_out, const i
         g.stagers < 4 || g.stagers > g.waves || g.ni * g.stagers < g.nchunks || g.ni > (g.waves == 16 || g.buf_bytes == kHalfBufBytes ? kMaxChunks16 : kMaxChunks))
       return fail(TETRIS_EINVAL, "inconsistent kernel geometry (triple-buffered kernel)");
     if (g.waves == 16) {
-      if (g.nq == 1) return launch_three<1, 16, 4>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 2) return launch_three<2, 16, 4>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 1) return launch_three<1, 16, 4, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 2) return launch_three<2, 16, 4, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
     } else if (g.buf_bytes == kHalfBufBytes) {
-      if (g.nq == 1) return launch_three<1, 8, 5>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 2) return launch_three<2, 8, 5>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 1) return launch_three<1, 8, 5, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 2) return launch_three<2, 8, 5, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
     } else {
-      if (g.nq == 1) return launch_three<1, 8, 3>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 2) return launch_three<2, 8, 3>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
-      if (g.nq == 4) return launch_three<4, 8, 3>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 1) return launch_three<1, 8, 3, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 2) return launch_three<2, 8, 3, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+      if (g.nq == 4) return launch_three<4, 8, 3, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
     }
     return fail(TETRIS_EINVAL, "no kernel for quads=%d waves=%d", g.nq, g.waves);
   }
   if (g.region * g.nq != kTileBytes || g.spt * g.fill_iters > kFillItems || g.fill_slots > g.spt * g.waves * 64)
     return fail(TETRIS_EINVAL, "inconsistent kernel geometry");
 #define TETRIS_CASE(NQ, SPT) \
-  if (g.nq == NQ && g.spt == SPT) return launch_one<NQ, SPT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
+  if (g.nq == NQ && g.spt == SPT) return launch_one<NQ, SPT, SPLIT>(g, d_in, d_out, entries, grp_off, grp_pair, oc_order, d_final, d_tickets, stream);
   TETRIS_CASE(1, 1)
   TETRIS_CASE(1, 2)
   TETRIS_CASE(2, 1)
@@ -1317,7 +1439,7 @@ bool geom_walks_pairs(const Geom& g) { return (options() & TETRIS_OPT_PAIRS) && 
 
 // whether the kernel of geometry `g` can pool its own outputs (store_pooled's conditions)
 bool geom_pools_in_kernel(const Geom& g) {
-  return g.ver != 4 && g.csplit == 1 && (g.thi & 1) == 0 && ((g.lw & 1) == 0 || g.jsh == 0);
+  return g.ver != 4 && (g.thi & 1) == 0 && ((g.lw & 1) == 0 || g.jsh == 0);
 }
 
 // ---- which XCD a workgroup runs on ---------------------------------------------------------------------------------
@@ -1363,8 +1485,8 @@ int same_xcd_by_residue(bool* ok) {
   return TETRIS_OK;
 }
 
-int launch_conv(const Geom& g0, const float* d_in, float* d_user_out, float* d_scratch, const int2* entries,
-                const int32_t* grp_off, const int32_t* grp_pair, const int32_t* oc_order, int act, hipStream_t stream) {
+int launch_conv(const Geom& g0, const float* d_in, float* d_user_out, float* d_scratch, size_t scratch_bytes,
+                const int2* entries, const int32_t* grp_off, const int32_t* grp_pair, const int32_t* oc_order, int act, hipStream_t stream) {
   // what the kernel's indexing assumes, checked once more before anything is launched
   if (g0.g * 4 * g0.nq > kAccRegs || g0.nb * g0.img_stride * 4 > g0.region || g0.lr * g0.lh > 64 || g0.lw > g0.lr ||
       g0.kblocks * g0.kb > g0.slots || g0.waves < 1 || g0.waves > 16 || g0.csplit < 1 || g0.csplit > kMaxSplit ||
@@ -1379,21 +1501,41 @@ int launch_conv(const Geom& g0, const float* d_in, float* d_user_out, float* d_s
   g.fused = 0;
   if (g.csplit == 1) {
     g.act = act;
-    return launch_kernel(g, d_in, d_user_out, entries, grp_off, grp_pair, oc_order, nullptr, nullptr, stream);
+    return launch_kernel<false>(g, d_in, d_user_out, entries, grp_off, grp_pair, oc_order, nullptr, nullptr, stream);
   }
-  // A split layer.  Its scratch: the tickets, then one copy of the output per slice.
+  // A split layer.  Its scratch: the tickets, then the sums of every slice.  Who adds them, and how they are kept:
+  //   * up to 16 MiB of sums: add_kernel, the sums in the order the waves hold them -- 16-byte stores of consecutive bytes
+  //     instead of four-byte ones of a quarter of a row each, 0.5 instead of 1.5 ... 1.8 us at the end of the conv kernel
+  //     (ResNet-50 at batch 16: 0.4 ... 2.4 us less per split layer; VGG19 at batch 1: 0.5 ... 1.8);
+  //   * beyond that the padding of partly filled waves (a quarter of a 7x7 layer's sums) costs the adding kernel what the
+  //     stores give (27 MB: between 4.6 us less and 2.0 us more): one copy of the output per slice and reduce_kernel.
+  //     So does a pooled layer whose tile cannot pool, which needs neighbours that other waves hold;
+  //   * the wave that finishes last (TETRIS_OPT_ADD_IN_KERNEL): less time for a layer launched again and again where two
+  //     slices meet (16x128x28x28 -> 128, 3x3: 30.7 us, add_kernel 32.8), more with four or eight, which one wave then
+  //     reads alone (1x512x14x14 -> 512, 1x1: 11.5 and 8.6), and between other layers up to 2 us more everywhere.
   int* d_tickets = reinterpret_cast<int*>(d_scratch);
   float* d_partial = d_scratch + kTicketBytes / sizeof(float);
-  if (act != 2 && (options() & TETRIS_OPT_ADD_IN_KERNEL) &&
-      (long long)g.ugroups * g.kblocks * g.waves <= kMaxTickets) {
-    bool ok = false;
-    const int rc = same_xcd_by_residue(&ok);  // asked once per device (the first time from tetris_g950_prepare or an
-    if (rc) return rc;                        // eager launch, never under capture: planning a split layer allocates)
-    g.fused = ok ? 1 : 0;
+  const size_t sums = sum_bytes_of(g);
+  if ((act != 2 || geom_pools_in_kernel(g)) && kTicketBytes + sums <= scratch_bytes) {
+    if (options() & TETRIS_OPT_ADD_IN_KERNEL) {
+      bool ok = false;
+      // asked once per device (the first time from tetris_g950_prepare or an eager launch, never under capture: planning
+      // a split layer allocates)
+      if (const int rc = same_xcd_by_residue(&ok)) return rc;
+      if (ok && (long long)ceil_div(g.ugroups * g.kblocks, 8) * g.waves <= kMaxTickets / 8) g.fused = 1;
+    }
+    if (!g.fused && sums <= kMaxWaveSums) g.fused = 2;
   }
   g.act = g.fused ? act : 0;  // otherwise the sums are finished by the adding kernel
-  const int rc = launch_kernel(g, d_in, d_partial, entries, grp_off, grp_pair, oc_order, d_user_out, d_tickets, stream);
-  if (rc != TETRIS_OK || g.fused) return rc;
+  const int rc = launch_kernel<true>(g, d_in, d_partial, entries, grp_off, grp_pair, oc_order, d_user_out, d_tickets, stream);
+  if (rc != TETRIS_OK || g.fused == 1) return rc;
+  if (g.fused == 2) {
+    const int per_wave = g.g * g.nq;
+    hipLaunchKernelGGL(add_kernel, dim3(8 * ceil_div(g.ugroups * g.kblocks, 8), ceil_div(g.waves * per_wave, 4)), dim3(256), 0,
+                       stream, d_partial, d_user_out, oc_order, magic_reciprocal(per_wave), magic_reciprocal(g.nq), g);
+    TETRIS_HIP(hipGetLastError());
+    return TETRIS_OK;
+  }
   const long long n = (long long)g.N * g.K * g.OH * g.OW;
   if (act == 2) {
     const int vec = (g.OW & 3) == 0 && (reinterpret_cast<size_t>(d_user_out) & 15) == 0;

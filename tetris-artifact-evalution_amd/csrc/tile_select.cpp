@@ -172,6 +172,7 @@ static int make_flat_geom(const tetris_g950* p, Geom g, const tetris_tile& t, Ge
     return fail(TETRIS_EINVAL, "%d slices of this layer's output are more than 1 GiB of partial sums", g.csplit);
   g.m_kblocks = magic_reciprocal(g.kblocks);
   g.m_csplit = magic_reciprocal(g.csplit);
+  g.sum_bytes = ceil_div(16 * g.nb * g.thi * g.lw, 128) * 128;
   // Every load a wave issues waits its turn at the CU's address unit, and a wave that issues does not walk.  In a
   // 16-wave workgroup the eight oldest waves (two per SIMD, served first) stage for all: the other eight walk meanwhile
   // (MobileNet pass -1.9 %, ResNet-50 -1.0 % against all sixteen staging; four stagers: +4 % and 0 %).
@@ -272,6 +273,7 @@ int make_geom(const tetris_g950* p, int N, int H, int W, int stride, int pad, co
       return fail(TETRIS_EINVAL, "%d slices of this layer's output are more than 1 GiB of partial sums", g.csplit);
     g.m_kblocks = magic_reciprocal(g.kblocks);
     g.m_csplit = magic_reciprocal(g.csplit);
+    g.sum_bytes = ceil_div(16 * g.nb * g.thi * g.lw, 128) * 128;
   }
   if (g.ver == 3) {
     g.cpp = ceil_div(g.plane, 64);
