@@ -238,7 +238,7 @@ typedef struct tetris_launch_shape {
   int32_t csplit;         /* workgroups that share an output tile (the tile's value, or the rule's when that is 0) */
   int32_t stages;         /* input-channel stages of the whole reduction: ceil(in_channel / tile_ic) */
   int32_t lanes_used;     /* lanes of a wave that own pixels, out of 64 */
-  int32_t kernel;         /* 2 single LDS tile, 3 three LDS buffers, 4 flat tile of pointwise layers */
+  int32_t kernel;         /* 2 single LDS tile, 3 three LDS buffers, 4 flat tile of pointwise layers; 5 matrix cores */
   int32_t lds_bytes;      /* dynamic LDS of a workgroup */
   int64_t scratch_bytes;  /* tickets + partial sums a split layer needs (0 when csplit is 1) */
 } tetris_launch_shape;

@@ -41,6 +41,42 @@ int upload(const std::vector<T>& v, T** d) {
   return TETRIS_OK;
 }
 
+// Whether the matrix kernel runs the layer, and how.  Only where the choice is the library's: no tile given, or the one that
+// tetris_tile_select names; a tile of the caller's own is obeyed, and so is an option that picks a form of the walking
+// kernels.
+bool choose_matrix(const tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile* tile, const Geom& walk,
+                   MatGeom* g, MatGeom* pool) {
+  if (options() & (TETRIS_OPT_PAIRS | TETRIS_OPT_NO_BANK_RULE | TETRIS_OPT_ADD_IN_KERNEL)) return false;
+  if (tile) {
+    tetris_tile own{};
+    if (choose_tile(N, H, W, p->C, p->K, p->ks, stride, pad, &own) != TETRIS_OK || tile->lanes_w != own.lanes_w ||
+        tile->quads != own.quads || tile->oc_per_wave != own.oc_per_wave || tile->waves != own.waves ||
+        tile->tile_ic != own.tile_ic || tile->csplit != own.csplit)
+      return false;
+  }
+  return choose_mat_geom(N, p->C, H, W, p->K, p->ks, stride, pad, walk, p->nnz, g, pool);
+}
+
+// the weights of pack `p` as the matrix kernel loads them, made on first use
+int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const void** out) {
+  std::lock_guard<std::mutex> lock(p->mu);
+  auto it = p->parts.find(g.kgs);
+  if (it == p->parts.end()) {
+    void* d = nullptr;
+    TETRIS_HIP(hipMalloc(&d, mat_weight_bytes(g)));
+    int rc = mat_weights(p, g, stream, d);
+    // launches on other streams may follow at once
+    if (rc == TETRIS_OK && hipStreamSynchronize(stream) != hipSuccess) rc = fail(TETRIS_EHIP, "making a matrix plan failed");
+    if (rc) {
+      (void)hipFree(d);
+      return rc;
+    }
+    it = p->parts.emplace(g.kgs, d).first;
+  }
+  *out = it->second;
+  return TETRIS_OK;
+}
+
 // The launch plan of (input shape, tile) for pack `p`: looked up, or -- when `create` allows it -- made (geometry,
 // bound entries: one device allocation and one small kernel on `stream`) and remembered.
 int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile* tile, hipStream_t stream,
@@ -77,8 +113,12 @@ int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const te
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
     return fail(TETRIS_EINVAL, "the first launch of a shape allocates: call tetris_g950_prepare before capturing");
-  rc = g950_bind(p, plan.geom, geom_walks_pairs(plan.geom), stream, &plan.entries, &plan.grp_off, &plan.grp_pair,
-                 &plan.geom.heads_off);
+  if (choose_matrix(p, N, H, W, stride, pad, given ? tile : nullptr, plan.geom, &plan.mat, &plan.mat_pool)) {
+    rc = matrix_weights(p, plan.mat, stream, &plan.parts);
+  } else {
+    rc = g950_bind(p, plan.geom, geom_walks_pairs(plan.geom), stream, &plan.entries, &plan.grp_off, &plan.grp_pair,
+                   &plan.geom.heads_off);
+  }
   if (rc) return rc;
   memcpy(plan.key, key, sizeof key);
   std::lock_guard<std::mutex> lock(p->mu);
@@ -88,13 +128,39 @@ int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const te
   return TETRIS_OK;
 }
 
+// how many workgroups share an output tile
+int slices_of(const Plan& p) { return p.parts ? p.mat.csplit : p.geom.csplit; }
+
 // scratch a split layer needs: the tickets, then csplit copies of the output
+size_t partial_bytes_of(const MatGeom& g) {
+  return g.csplit > 1 ? (size_t)kTicketBytes + sizeof(float) * (size_t)g.csplit * g.out_floats : 0;
+}
 size_t partial_bytes_of(const Geom& g) {
   return g.csplit > 1 ? (size_t)kTicketBytes + sizeof(float) * (size_t)g.csplit * g.N * g.K * g.OH * g.OW : 0;
 }
 
 // ... and what it gets where the library allocates it: room for the waves' sums as well, which idle lanes make longer
-size_t scratch_bytes_of(const Geom& g) { return std::max(partial_bytes_of(g), kTicketBytes + sum_bytes_of(g)); }
+size_t scratch_bytes_of(const Plan& p) {
+  return p.parts ? partial_bytes_of(p.mat) : std::max(partial_bytes_of(p.geom), kTicketBytes + sum_bytes_of(p.geom));
+}
+
+// launches a layer as its plan says
+int launch_plan(const Plan& p, const float* d_in, float* d_out, float* d_scratch, size_t scratch_bytes,
+                const int32_t* oc_order, int act, hipStream_t stream) {
+  if (!p.parts)
+    return launch_conv(p.geom, d_in, d_out, d_scratch, scratch_bytes, p.entries, p.grp_off, p.grp_pair, oc_order, act, stream);
+  if (act < 0 || act > 2) return fail(TETRIS_EINVAL, "unknown activation %d", act);
+  if (act == 2 && (p.mat.OH < 2 || p.mat.OW < 2))
+    return fail(TETRIS_EINVAL, "2x2 pooling needs an output of at least 2 x 2");
+  if (p.mat.csplit == 1) {
+    if (act == 2 && !p.mat_pool.N) return fail(TETRIS_EUNSUPPORTED, "this layer cannot pool its outputs");
+    return launch_matrix(act == 2 ? p.mat_pool : p.mat, d_in, d_out, p.parts, act != 0, stream);
+  }
+  float* copies = d_scratch + kTicketBytes / sizeof(float);
+  const int rc = launch_matrix(p.mat, d_in, copies, p.parts, 0, stream);
+  if (rc) return rc;
+  return add_copies(copies, d_out, p.mat.N, p.mat.K, p.mat.OH, p.mat.OW, p.mat.csplit, act, stream);
+}
 
 // Partial-sum buffer of a split layer: one per (pack, stream), so that launches of one pack on different streams do
 // not share it.  A buffer that has to grow is replaced, and the old one is kept until the pack is destroyed: a HIP
@@ -136,13 +202,12 @@ int run_launch(tetris_g950* p, const float* d_in, float* d_out, int N, int H, in
   int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, &plan);
   if (rc) return rc;
   float* d_partial = nullptr;
-  const size_t scratch = scratch_bytes_of(plan.geom);
-  if (plan.geom.csplit > 1) {
+  const size_t scratch = scratch_bytes_of(plan);
+  if (slices_of(plan) > 1) {
     rc = partial_buffer(p, stream, scratch, true, &d_partial);
     if (rc) return rc;
   }
-  return launch_conv(plan.geom, d_in, d_out, d_partial, scratch, plan.entries, plan.grp_off, plan.grp_pair, p->d_oc_order, act,
-                     stream);
+  return launch_plan(plan, d_in, d_out, d_partial, scratch, p->d_oc_order, act, stream);
 }
 
 // ---- scratch of the entry point that allocates nothing ------------------------------------------------------------
@@ -735,8 +800,10 @@ int tetris_spconv2d_act_supported(tetris_g950* p, int N, int H, int W, int strid
   Geom g;
   const int rc = make_geom(p, N, H, W, stride, pad, *tile, &g);
   if (rc) return rc;
+  MatGeom m, pool;
+  const bool matrix = choose_matrix(p, N, H, W, stride, pad, tile, g, &m, &pool);
   *supported = activation != TETRIS_ACT_RELU_POOL2 ||
-               (g.OH >= 2 && g.OW >= 2 && (g.csplit > 1 || geom_pools_in_kernel(g)));
+               (g.OH >= 2 && g.OW >= 2 && (matrix ? m.csplit > 1 || pool.N : g.csplit > 1 || geom_pools_in_kernel(g)));
   return TETRIS_OK;
 }
 
@@ -746,6 +813,12 @@ int tetris_launch_shape_of(tetris_g950* p, int N, int H, int W, int stride, int 
   Geom g;
   const int rc = make_geom(p, N, H, W, stride, pad, *tile, &g);
   if (rc) return rc;
+  MatGeom m, pool;
+  if (choose_matrix(p, N, H, W, stride, pad, tile, g, &m, &pool)) {
+    *out = {m.ptiles * m.mtiles * m.csplit, m.ptiles, m.mtiles, m.csplit, m.chunks, 64, 5, mat_lds_bytes(m),
+            (int64_t)partial_bytes_of(m)};
+    return TETRIS_OK;
+  }
   out->unit_groups = g.ugroups;
   out->channel_blocks = g.kblocks;
   out->csplit = g.csplit;
@@ -764,9 +837,9 @@ int tetris_g950_prepare(tetris_g950* p, int N, int H, int W, int stride, int pad
   Plan plan;
   int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, &plan);
   if (rc) return rc;
-  if (plan.geom.csplit > 1) {
+  if (slices_of(plan) > 1) {
     float* d_partial = nullptr;
-    rc = partial_buffer(p, stream, scratch_bytes_of(plan.geom), true, &d_partial);
+    rc = partial_buffer(p, stream, scratch_bytes_of(plan), true, &d_partial);
     if (rc) return rc;
   }
   float* s = nullptr;
@@ -798,8 +871,8 @@ int tetris_spconv2d_launch_noalloc(tetris_g950* p, const float* d_in, float* d_o
   int rc = find_plan(p, N, H, W, stride, pad, tile, stream, false, &plan);
   if (rc) return rc;
   float* d_partial = nullptr;
-  if (plan.geom.csplit > 1) {
-    const size_t need = partial_bytes_of(plan.geom);
+  if (slices_of(plan) > 1) {
+    const size_t need = plan.parts ? partial_bytes_of(plan.mat) : partial_bytes_of(plan.geom);
     const size_t limit = g_scratch_limit.load();
     if (need > limit)
       return fail(TETRIS_EINVAL, "this layer needs %zu bytes of tickets and partial sums, the static scratch holds %zu: "
@@ -809,8 +882,7 @@ int tetris_spconv2d_launch_noalloc(tetris_g950* p, const float* d_in, float* d_o
   }
   // Every element of the partial sums that are added is written by this launch's conv kernel first, so
   // what an earlier call left in the array needs no clearing.
-  return launch_conv(plan.geom, d_in, d_out, d_partial, g_scratch_limit.load(), plan.entries, plan.grp_off, plan.grp_pair,
-                     p->d_oc_order, 0, stream);
+  return launch_plan(plan, d_in, d_out, d_partial, g_scratch_limit.load(), p->d_oc_order, 0, stream);
 }
 
 int tetris_spconv2d_launch_spf_arrays(const float* d_in, const int32_t* d_offsets, const int32_t* d_stage_len,

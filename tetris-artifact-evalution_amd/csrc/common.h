@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <array>
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -170,6 +171,26 @@ struct BoundKey {
 }  // namespace tetris
 
 namespace tetris {
+// How the matrix kernel (matrix_conv.hip) cuts a layer into workgroups.  Its output pixels are numbered strip by strip
+// (a strip: up to 64 columns of an image), row by row -- in 2x2 blocks when pooling -- and a tile is consecutive ones.
+struct MatDiv { unsigned m; int shift; };  // x / d == x * m >> shift for x < 2^30
+struct MatGeom {
+  int N, C, H, W, K, OH, OW, ks, stride, pad, sub;  // stride, in staged pixels, of the outputs; sub, in input pixels, of the staged ones
+  int in_bytes, out_floats;  // input bytes; floats of the output, or of one slice's copy of it
+  int pool, relu;
+  int strips, ws, wp, ihs;   // strips per image; output columns of one; staged columns and rows of one
+  int uw, uh, upq, npix;     // columns, rows and pixels of a strip's outputs (2x2 blocks when pooling); all outputs
+  int kgs, chunks, steps;    // groups of 8 channels staged together; such chunks; products of 16 k-values
+  int mblocks, mtiles, ptiles, csplit, cfg;
+  int lpad;                  // staged pixels of a tile, to a multiple of 64
+  unsigned m_uw, m_uh, m_wp, m_ihs, m_strips;
+  MatDiv d_tiles, d_mtiles, d_upq, d_uw, d_blocks;
+};
+constexpr int kMatConfigs = 11;
+constexpr int kMatTasks = 4;        // most blocks of 64 staged pixels x 8 channels that a wave holds at a time
+constexpr int kMatLds = 160 * 1024;
+constexpr long long kMatCopies = 32 << 20;  // most bytes of partial sums of a split layer
+
 // A launch plan: everything run_launch derives from (input shape, tile) for one pack, kept for the next call.
 struct Plan {
   int key[11];  // N, H, W, stride, pad, lanes_w, quads, oc_per_wave, waves, tile_ic, csplit
@@ -177,6 +198,8 @@ struct Plan {
   const int2* entries;        // the pack's entries bound to the geometry
   const int32_t* grp_off;     // [groups*stages+1] first entry of every stream in `entries`
   const int32_t* grp_pair;    // [groups*stages] entries of the stream's leading segment of pairs (0 when unpaired)
+  const void* parts = nullptr;  // the weights of the matrix kernel: set where it runs the layer instead
+  MatGeom mat, mat_pool;
 };
 }  // namespace tetris
 
@@ -195,6 +218,7 @@ struct tetris_g950 {
   float* d_values = nullptr;      // [n_entries + 8]
   // (LDS byte offset | accumulator index << 16 | 0xC << 28, value) pairs for one tile geometry, made on first use
   std::map<tetris::BoundKey, int2*> bound;
+  std::map<int, void*> parts;  // the weights as the matrix kernel loads them, by MatGeom::kgs
   // Paired arrangement of the streams (made on the first paired bind; depends on the pack only): two consecutive
   // entries of a stream that share their position become a pair; per stream first all pairs, padded to a multiple
   // of 8 entries, then the entries left single, padded likewise.
@@ -278,6 +302,18 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
 // scratch_bytes says that sum_bytes_of fits as well, the sums may be kept in the waves' order
 int launch_conv(const Geom& g, const float* d_in, float* d_out, float* d_scratch, size_t scratch_bytes, const int2* entries,
                 const int32_t* grp_off, const int32_t* grp_pair, const int32_t* oc_order, int act, hipStream_t stream);
+// adds the copies of the output that the slices of a split layer wrote, in slice order, through `act`
+int add_copies(const float* d_copies, float* d_out, int N, int K, int OH, int OW, int slices, int act, hipStream_t stream);
+
+// matrix_conv.hip
+bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out);
+bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
+                     MatGeom* g, MatGeom* pool);
+int mat_lds_bytes(const MatGeom& g);
+size_t mat_weight_bytes(const MatGeom& g);
+int mat_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* dst);
+int launch_matrix(const MatGeom& g, const float* d_in, float* d_out, const void* weights, int relu, hipStream_t stream);
+
 // whether workgroups with the same blockIdx.x % 8 run on one XCD of the current device (probed once per device):
 // what lets the slices of a split layer exchange their partial sums through that XCD's L2
 int same_xcd_by_residue(bool* ok);

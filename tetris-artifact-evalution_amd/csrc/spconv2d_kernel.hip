@@ -1485,6 +1485,22 @@ int same_xcd_by_residue(bool* ok) {
   return TETRIS_OK;
 }
 
+int add_copies(const float* d_copies, float* d_out, int N, int K, int OH, int OW, int slices, int act, hipStream_t stream) {
+  const long long n = (long long)N * K * OH * OW;
+  if (act == 2) {
+    const int vec = (OW & 3) == 0 && (reinterpret_cast<size_t>(d_out) & 15) == 0;
+    const long long items = (long long)N * K * (OH / 2) * (vec ? OW / 4 : OW / 2);
+    const int blocks = (int)std::min<long long>((items + 255) / 256, 2048);
+    hipLaunchKernelGGL(reduce_pool_kernel, dim3(blocks), dim3(256), 0, stream, d_copies, d_out,
+                       (long long)N * K, OH, OW, slices, vec);
+  } else {
+    const int blocks = (int)std::min<long long>(((n + 3) / 4 + 255) / 256, 2048);
+    hipLaunchKernelGGL(reduce_kernel, dim3(blocks), dim3(256), 0, stream, d_copies, d_out, n, slices, act);
+  }
+  TETRIS_HIP(hipGetLastError());
+  return TETRIS_OK;
+}
+
 int launch_conv(const Geom& g0, const float* d_in, float* d_user_out, float* d_scratch, size_t scratch_bytes,
                 const int2* entries, const int32_t* grp_off, const int32_t* grp_pair, const int32_t* oc_order, int act, hipStream_t stream) {
   // what the kernel's indexing assumes, checked once more before anything is launched
@@ -1536,19 +1552,7 @@ int launch_conv(const Geom& g0, const float* d_in, float* d_user_out, float* d_s
     TETRIS_HIP(hipGetLastError());
     return TETRIS_OK;
   }
-  const long long n = (long long)g.N * g.K * g.OH * g.OW;
-  if (act == 2) {
-    const int vec = (g.OW & 3) == 0 && (reinterpret_cast<size_t>(d_user_out) & 15) == 0;
-    const long long items = (long long)g.N * g.K * (g.OH / 2) * (vec ? g.OW / 4 : g.OW / 2);
-    const int blocks = (int)std::min<long long>((items + 255) / 256, 2048);
-    hipLaunchKernelGGL(reduce_pool_kernel, dim3(blocks), dim3(256), 0, stream, d_partial, d_user_out,
-                       (long long)g.N * g.K, g.OH, g.OW, g.csplit, vec);
-  } else {
-    const int blocks = (int)std::min<long long>(((n + 3) / 4 + 255) / 256, 2048);
-    hipLaunchKernelGGL(reduce_kernel, dim3(blocks), dim3(256), 0, stream, d_partial, d_user_out, n, g.csplit, act);
-  }
-  TETRIS_HIP(hipGetLastError());
-  return TETRIS_OK;
+  return add_copies(d_partial, d_user_out, g.N, g.K, g.OH, g.OW, g.csplit, act, stream);
 }
 
 }  // namespace tetris
