@@ -280,7 +280,8 @@ size_t tetris_noalloc_scratch_limit(size_t bytes);
 /* The reference launcher on the five device arrays of a SparseFilter (Tetris/spconv2d_kernel.cuh:14-21,
  * Tetris/spconv2d_kernel.cu:91-156): the convolution is computed FROM THE ARRAYS PASSED -- offsets, positions, values
  * and the output-channel permutation -- not from anything a handle remembers.  The arrays are hashed on the device at
- * every call (one pass over them and a stream synchronisation); the first call, and any call after their content has
+ * every call (one pass over them, whose result the host waits for; the launch is already behind it, so a call that finds
+ * the arrays changed, or in error, may have written the output before it writes it again or fails); the first call, and any call after their content has
  * changed (a caller that rewrites d_values in place), decodes them on the device into the kernel's own pack, whose
  * slots follow d_oc_permutation.  Decoded packs are cached per set of addresses (16 sets, least recently used first
  * out).  d_stage_len is accepted and not read, as in the reference's kernel.  tile_ic and vec_width are the

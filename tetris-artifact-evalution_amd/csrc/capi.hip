@@ -300,6 +300,7 @@ struct SpfView {
   const void* ptrs[4];  // offsets, permutation, position, values
   int C, K, ks, tile_ic, vec;
   unsigned long long hash = 0;
+  long long n_ent = 0;  // entries the hash covers
   float* d_filter = nullptr;
   std::vector<int32_t> order;                              // oc_permutation copied to the host: the packs' slot order
   std::map<std::array<int, 2>, tetris_g950*> packs;        // by (tile_ic of the kernel, oc_per_wave)
@@ -316,6 +317,8 @@ constexpr size_t kMaxViews = 16;
 std::mutex g_views_mu;
 std::vector<SpfView*> g_views;  // most recently used last
 unsigned long long* g_hash_scratch = nullptr;
+unsigned long long* g_hash_shares = nullptr;  // pinned: what spf_arrays_rehash leaves
+unsigned g_hash_tag = 0;
 
 void drop_views(const void* d_values) {
   std::lock_guard<std::mutex> lock(g_views_mu);
@@ -325,6 +328,21 @@ void drop_views(const void* d_values) {
       delete g_views[i];
       g_views.erase(g_views.begin() + (long)i);
     }
+}
+
+// the view of these addresses and this shape, if there is one
+SpfView* find_view(const int32_t* d_offsets, const int32_t* d_perm, const int32_t* d_position, const float* d_values, int C,
+                   int K, int ks, int tile_ic, int vec) {
+  for (SpfView* c : g_views)
+    if (c->ptrs[0] == d_offsets && c->ptrs[1] == d_perm && c->ptrs[2] == d_position && c->ptrs[3] == d_values &&
+        c->C == C && c->K == K && c->ks == ks && c->tile_ic == tile_ic && c->vec == vec)
+      return c;
+  return nullptr;
+}
+
+// what the hash of a view's arrays is mixed with
+unsigned long long hash_salt(int C, int ks, int tile_ic, int vec) {
+  return 0x5bd1e995ull * (unsigned long long)(C * 131 + ks) + (unsigned long long)tile_ic * 7919ull + (unsigned)vec;
 }
 
 // The kernel pack (and tile) for a convolution whose weights are the arrays at these addresses, rebuilt when the
@@ -342,16 +360,10 @@ int view_pack(const int32_t* d_offsets, const int32_t* d_perm, const int32_t* d_
   if (C <= 0 || K <= 0 || ks <= 0 || ks > kMaxKs || tile_ic <= 0 || (vec != 0 && vec != 1 && vec != 4))
     return fail(TETRIS_EINVAL, "bad filter shape C=%d K=%d ks=%d tile_ic=%d vector width=%d", C, K, ks, tile_ic, vec);
   if (capacity < 0) return fail(TETRIS_EINVAL, "negative entry capacity");
-  auto find = [&]() -> SpfView* {  // the view of these addresses and this shape, if there is one
-    for (SpfView* c : g_views)
-      if (c->ptrs[0] == d_offsets && c->ptrs[1] == d_perm && c->ptrs[2] == d_position && c->ptrs[3] == d_values &&
-          c->C == C && c->K == K && c->ks == ks && c->tile_ic == tile_ic && c->vec == vec)
-        return c;
-    return nullptr;
-  };
-  SpfView* v = find();
+  SpfView* v = find_view(d_offsets, d_perm, d_position, d_values, C, K, ks, tile_ic, vec);
   const bool trusted = v && v->d_filter && (options() & TETRIS_OPT_TRUST_SPF_ARRAYS);
   unsigned long long hash = v ? v->hash : 0;
+  long long n_entries = v ? v->n_ent : 0;
   int rc = TETRIS_OK;
   if (!trusted) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -373,7 +385,8 @@ int view_pack(const int32_t* d_offsets, const int32_t* d_perm, const int32_t* d_
     rc = spf_arrays_hash(d_offsets, n_off, d_perm, vec == 0 ? 0 : K, d_position, d_values, n_ent, g_hash_scratch, stream,
                          &hash);
     if (rc) return rc;
-    hash ^= 0x5bd1e995ull * (unsigned long long)(C * 131 + ks) + (unsigned long long)tile_ic * 7919ull + (unsigned)vec;
+    hash ^= hash_salt(C, ks, tile_ic, vec);
+    n_entries = n_ent;
   }
   if (v) g_views.erase(std::find(g_views.begin(), g_views.end(), v));  // moves to the most-recently-used end below
   if (!v) {
@@ -407,6 +420,7 @@ int view_pack(const int32_t* d_offsets, const int32_t* d_perm, const int32_t* d_
       for (int k = 0; k < K; ++k) v->order[k] = k;
     }
     v->hash = hash;
+    v->n_ent = n_entries;
   }
   tetris_tile t{};
   if (tile && tile->lanes_w > 0) {
@@ -433,6 +447,70 @@ int view_pack(const int32_t* d_offsets, const int32_t* d_perm, const int32_t* d_
   *pack_out = it->second;
   *tile_out = t;
   return TETRIS_OK;
+}
+
+// A launch on arrays whose view, pack and tile were made before: the arrays are hashed again and the convolution is launched
+// right behind, while the host waits for the hash only, so the GPU is not idle between the two or between calls (hash
+// and offsets read back one after the other, then the launch: 86 us for 4 x 256 x 28 x 28 -> 256).  *done: the arrays were
+// what the view was made from, and the launch stands.  Otherwise nothing is known, and the caller goes the long
+// way, whose launch on this stream overwrites the output.  The caller holds g_views_mu.
+int launch_seen_arrays(const float* d_in, float* d_out, const int32_t* d_offsets, const int32_t* d_perm,
+                       const int32_t* d_position, const float* d_values, int N, int H, int W, int C, int K, int ks,
+                       int stride, int pad, int tile_ic, int vec, long long capacity, const tetris_tile* tile,
+                       hipStream_t stream, bool* done) {
+  *done = false;
+  SpfView* v = find_view(d_offsets, d_perm, d_position, d_values, C, K, ks, tile_ic, vec);
+  if (!v || !v->d_filter || !d_in || !d_out || (capacity > 0 && v->n_ent > capacity) ||
+      (options() & TETRIS_OPT_TRUST_SPF_ARRAYS))
+    return TETRIS_OK;
+  tetris_tile t{};
+  if (tile && tile->lanes_w > 0) {
+    t = *tile;
+  } else {
+    const auto it = v->tiles.find({N, H, W, stride, pad});
+    if (it == v->tiles.end()) return TETRIS_OK;
+    t = it->second;
+  }
+  const auto pk = v->packs.find({t.tile_ic, t.oc_per_wave});
+  if (pk == v->packs.end()) return TETRIS_OK;
+  Plan plan;
+  if (find_plan(pk->second, N, H, W, stride, pad, &t, stream, false, &plan) != TETRIS_OK) return TETRIS_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) return TETRIS_OK;
+  if (!g_hash_shares) {
+    TETRIS_HIP(hipHostMalloc(&g_hash_shares, 16 * kRehashBlocks, hipHostMallocPortable | hipHostMallocMapped));
+    memset(g_hash_shares, 0, 16 * kRehashBlocks);
+  }
+  const int stages = (C - 1) / tile_ic + 1;
+  const int n_off = (vec == 0 ? K : (K + kRefLanes - 1) / kRefLanes) * stages + 1;
+  if (++g_hash_tag == 0) ++g_hash_tag;
+  const unsigned tag = g_hash_tag;
+  int rc = spf_arrays_rehash(d_offsets, n_off, d_perm, vec == 0 ? 0 : K, d_position, d_values, v->n_ent,
+                             vec == 0 ? 1 : kRefLanes, tag, g_hash_shares, stream);
+  if (rc) return rc;
+  rc = run_launch(pk->second, d_in, d_out, N, H, W, stride, pad, &t, stream);
+  // every share has to arrive before the next call may reuse the buffer, whatever the launch said
+  unsigned long long sum = 0;
+  for (int i = 0; i < kRehashBlocks; ++i) {
+    unsigned long long word[2];
+    long long spins = 0;
+    for (int k = 0; k < 2; ++k)
+      while ((unsigned)(word[k] = __atomic_load_n(g_hash_shares + 2 * i + k, __ATOMIC_ACQUIRE)) != tag) {
+        if (++spins % 65536) continue;
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return fail(TETRIS_EHIP, "hashing the arrays failed: %s", hipGetErrorString(e));
+        if ((unsigned)__atomic_load_n(g_hash_shares + 2 * i + k, __ATOMIC_ACQUIRE) != tag)
+          return fail(TETRIS_EHIP, "the arrays' hash did not arrive");
+      }
+    sum += word[0] >> 32 | (word[1] & 0xffffffff00000000ull);
+  }
+  *done = rc != TETRIS_OK || (sum ^ hash_salt(C, ks, tile_ic, vec)) == v->hash;
+  if (*done) {  // moves to the most-recently-used end
+    g_views.erase(std::find(g_views.begin(), g_views.end(), v));
+    g_views.push_back(v);
+  }
+  return rc;
 }
 
 // Shared body of the two host-to-host entry points.
@@ -896,8 +974,12 @@ int tetris_spconv2d_launch_spf_arrays(const float* d_in, const int32_t* d_offset
   tetris_tile t{};
   // held until the launch is issued: the pack belongs to a view that another thread's call may evict or drop
   std::lock_guard<std::mutex> lock(g_views_mu);
-  int rc = view_pack(d_offsets, d_perm, d_position, d_values, N, H, W, C, K, ks, stride, pad, tile_ic, vec_width,
-                     (long long)n_entries, tile, stream, &pack, &t);
+  bool done = false;
+  int rc = launch_seen_arrays(d_in, d_out, d_offsets, d_perm, d_position, d_values, N, H, W, C, K, ks, stride, pad, tile_ic,
+                              vec_width, (long long)n_entries, tile, stream, &done);
+  if (rc || done) return rc;
+  rc = view_pack(d_offsets, d_perm, d_position, d_values, N, H, W, C, K, ks, stride, pad, tile_ic, vec_width,
+                 (long long)n_entries, tile, stream, &pack, &t);
   if (rc) return rc;
   return run_launch(pack, d_in, d_out, N, H, W, stride, pad, &t, stream);
 }

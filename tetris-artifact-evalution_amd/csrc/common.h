@@ -270,6 +270,11 @@ int g950_bind(tetris_g950* p, const Geom& g, bool paired, hipStream_t stream, co
 int spf_arrays_hash(const int32_t* d_offsets, int n_off, const int32_t* d_perm, int K, const int32_t* d_position,
                     const float* d_values, long long n_ent, unsigned long long* d_scratch2, hipStream_t stream,
                     unsigned long long* hash_out);
+// ... of arrays hashed before: kRehashBlocks shares, whose sum is the hash, left in host memory (spf_rehash_kernel)
+constexpr int kRehashBlocks = 128;
+int spf_arrays_rehash(const int32_t* d_offsets, int n_off, const int32_t* d_perm, int K, const int32_t* d_position,
+                      const float* d_values, long long n_ent, int lanes, unsigned tag, unsigned long long* shares,
+                      hipStream_t stream);
 int spf_arrays_decode(const int32_t* d_offsets, const int32_t* d_perm, const int32_t* d_position, const float* d_values,
                       float* d_filter, int C, int K, int ks, int tile_ic, int vec, hipStream_t stream);
 

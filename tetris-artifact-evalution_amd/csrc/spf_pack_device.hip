@@ -389,12 +389,11 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
   return z ^ (z >> 31);
 }
 
-// out[0] += order-independent hash of (array id, index, word) over the four arrays, n_ent entries of the last two
-__global__ __launch_bounds__(256) void spf_hash_kernel(const int32_t* __restrict__ offsets, int n_off,
-                                                       const int32_t* __restrict__ perm, int K,
-                                                       const int32_t* __restrict__ position,
-                                                       const float* __restrict__ values, long long n_ent,
-                                                       unsigned long long* __restrict__ out) {
+// a wave's share of the order-independent hash of (array id, index, word) over the four arrays, n_ent entries of the last two
+__device__ __forceinline__ unsigned long long hash_share(const int32_t* __restrict__ offsets, int n_off,
+                                                         const int32_t* __restrict__ perm, int K,
+                                                         const int32_t* __restrict__ position,
+                                                         const float* __restrict__ values, long long n_ent) {
   const long long total = n_off + K + 2 * n_ent;
   unsigned long long h = 0;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long long)gridDim.x * blockDim.x) {
@@ -406,7 +405,37 @@ __global__ __launch_bounds__(256) void spf_hash_kernel(const int32_t* __restrict
     h += mix64(((unsigned long long)i << 32) ^ word ^ 0x9E3779B97F4A7C15ull);
   }
   for (int off = 32; off > 0; off >>= 1) h += __shfl_xor(h, off);
+  return h;
+}
+
+// out[0] += the hash
+__global__ __launch_bounds__(256) void spf_hash_kernel(const int32_t* __restrict__ offsets, int n_off,
+                                                       const int32_t* __restrict__ perm, int K,
+                                                       const int32_t* __restrict__ position,
+                                                       const float* __restrict__ values, long long n_ent,
+                                                       unsigned long long* __restrict__ out) {
+  const unsigned long long h = hash_share(offsets, n_off, perm, K, position, values, n_ent);
   if ((threadIdx.x & 63) == 0) atomicAdd(out, h);
+}
+
+// The same, for arrays that were hashed before with `n_ent` entries: every block leaves its share in host memory, in two
+// words whose lower halves carry `tag`, which tells the host that they have arrived.  Arrays whose offsets end elsewhere
+// by now are not read (and hash to 0).
+__global__ __launch_bounds__(1024) void spf_rehash_kernel(const int32_t* __restrict__ offsets, int n_off,
+                                                          const int32_t* __restrict__ perm, int K,
+                                                          const int32_t* __restrict__ position,
+                                                          const float* __restrict__ values, long long n_ent, int lanes,
+                                                          unsigned tag, unsigned long long* __restrict__ out) {
+  __shared__ unsigned long long part[16];
+  unsigned long long h = 0;
+  if ((long long)lanes * offsets[n_off - 1] == n_ent) h = hash_share(offsets, n_off, perm, K, position, values, n_ent);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = h;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  h = 0;
+  for (int i = 0; i < 16; ++i) h += part[i];
+  __hip_atomic_store(out + 2 * blockIdx.x, h << 32 | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(out + 2 * blockIdx.x + 1, (h & 0xffffffff00000000ull) | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // vec > 0: the reorder path's layout (Tetris/spconv2d_utils.h:206-244): one workgroup per (32-lane group, stage);
@@ -461,6 +490,15 @@ int spf_arrays_hash(const int32_t* d_offsets, int n_off, const int32_t* d_perm, 
   TETRIS_HIP(hipMemcpyAsync(h, d_scratch2, sizeof h, hipMemcpyDeviceToHost, stream));
   TETRIS_HIP(hipStreamSynchronize(stream));
   *hash_out = h[0];
+  return TETRIS_OK;
+}
+
+int spf_arrays_rehash(const int32_t* d_offsets, int n_off, const int32_t* d_perm, int K, const int32_t* d_position,
+                      const float* d_values, long long n_ent, int lanes, unsigned tag, unsigned long long* shares,
+                      hipStream_t stream) {
+  hipLaunchKernelGGL(spf_rehash_kernel, dim3(kRehashBlocks), dim3(1024), 0, stream, d_offsets, n_off, d_perm, K, d_position,
+                     d_values, n_ent, lanes, tag, shares);
+  TETRIS_HIP(hipGetLastError());
   return TETRIS_OK;
 }
 
