@@ -56,3 +56,17 @@ def test_order_is_the_stated_deal(K, C, ks, g, waves, tile_ic):
     w = (rng.random((K, C, ks, ks), dtype=np.float32) * (rng.random((K, C, ks, ks), dtype=np.float32) < density[:, None, None, None]))
     got = T.oc_order_balanced(w.astype(np.float32), T.Tile(7, 1, g, waves, tile_ic))
     assert got.tolist() == deal(w, g, waves, tile_ic)
+
+
+def test_order_of_more_weights_than_32_bits_count():
+    """2^31 weights and some (nearly all zero: pages that are never written take no memory) are ordered as any others."""
+    K, C = 32769, 65540
+    w = np.zeros((K, C, 1, 1), np.float32)
+    dense = np.arange(K) // 64 < 128
+    dense &= np.arange(K) % 64 < 8  # in file order one wave of a workgroup holds all that the workgroup has
+    w[dense, :40, 0, 0] = 1.0
+    got = T.oc_order_balanced(w, T.Tile(7, 1, 8, 8, 32768))
+    assert np.array_equal(np.sort(got), np.arange(K))
+    # 1024 channels dealt to 513 blocks of 64, forth and back, and there to different waves of eight
+    waves = dense[got[:64 * 512]].reshape(512, 8, 8).sum(2)
+    assert waves.max() == 1 and waves.sum(1).min() == 1 and waves.sum(1).max() == 2

@@ -613,7 +613,6 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
   const int G = t.oc_per_wave, waves = t.waves, tile_ic = t.tile_ic;
   if (G <= 0 || waves <= 0 || tile_ic <= 0) return fail(TETRIS_EINVAL, "bad tile");
   const int S = ceil_div(C, tile_ic), B = G * waves, nblocks = ceil_div(K, B), taps = ks * ks;
-  if ((long long)C * K * taps > INT_MAX) return fail(TETRIS_EINVAL, "%d x %d filters of %d weights are too many to order", K, C, taps);
   // non-zeros per channel and stage: the weights of a stage lie side by side
   std::vector<int32_t> per((size_t)K * S);
   std::vector<int32_t> total(K, 0);
@@ -662,6 +661,14 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
   const int nsimd = std::min(4, waves);  // wave w runs on SIMD w % 4
   std::vector<int32_t> load((size_t)waves * S), busiest(S), simd_load((size_t)nsimd * S), busiest_simd(S), sum(waves);
   std::vector<std::vector<int32_t>> members(waves);
+  // A stage of one workgroup holds at most B * tile_ic * taps non-zeros, so that the 32-bit sums of `run` stages do not
+  // overflow: all stages at once unless a block of channels has more than 2^31 weights.
+  const int run = (int)std::max(1ll, std::min((long long)S, INT_MAX / std::max(1ll, (long long)std::min(B, K) * std::min(tile_ic, C) * taps)));
+  auto cost = [&](const int32_t* most, const int32_t* held, const int32_t* add) {
+    int64_t sum = 0;
+    for (int s = 0; s < S; s += run) sum += raised(most + s, held + s, add + s, std::min(run, S - s));
+    return sum;
+  };
   int32_t* o = order;
   for (const std::vector<int32_t>& blk : blocks) {
     std::fill(load.begin(), load.end(), 0);
@@ -677,18 +684,19 @@ int balance_oc_order(const float* filter, int C, int K, int ks, const tetris_til
     for (int32_t k : blk) {
       const int32_t* add = &per[(size_t)k * S];
       // least added to the busiest SIMD; of the waves on such SIMDs, to the busiest wave; of those the least loaded, the first
-      int cost_simd[4], best_simd = INT_MAX;
+      int64_t cost_simd[4], best_simd = INT64_MAX;
       for (int sd = 0; sd < nsimd; ++sd) {
-        cost_simd[sd] = INT_MAX;
+        cost_simd[sd] = INT64_MAX;
         bool any = false;
         for (int w = sd; w < waves && !any; w += nsimd) any = takes(w);
-        if (any) cost_simd[sd] = raised(busiest_simd.data(), &simd_load[(size_t)sd * S], add, S);
+        if (any) cost_simd[sd] = cost(busiest_simd.data(), &simd_load[(size_t)sd * S], add);
         best_simd = std::min(best_simd, cost_simd[sd]);
       }
-      int best = -1, best_wave = 0;
+      int best = -1;
+      int64_t best_wave = 0;
       for (int w = 0; w < waves; ++w) {
         if (cost_simd[w % nsimd] != best_simd || !takes(w)) continue;
-        const int cost_wave = raised(busiest.data(), &load[(size_t)w * S], add, S);
+        const int64_t cost_wave = cost(busiest.data(), &load[(size_t)w * S], add);
         if (best < 0 || cost_wave < best_wave || (cost_wave == best_wave && sum[w] < sum[best])) {
           best = w; best_wave = cost_wave;
         }
