@@ -26,3 +26,16 @@ def test_one_call_equals_order_then_pack(K, C, ks, tile_ic, g, waves, oracle):
     assert np.array_equal(a["oc_order"][:K], order) and np.array_equal(a["position"], ref.position)
     with pytest.raises(T.TetrisError):
         T.G950Filter.for_tile(w, T.Tile(7, 1, 0, waves, tile_ic), oc_order="balanced")
+
+
+def test_refused_pack_has_let_go_of_the_filter():
+    """A pack that is refused for its arguments returns only when the upload no longer reads the caller's (pinned) filter."""
+    import torch
+    import tetris_amd as T
+
+    w = torch.zeros((4096, 4096, 2, 2), pin_memory=True)  # 256 MiB: some milliseconds of upload
+    torch.cuda.synchronize()
+    with pytest.raises(T.TetrisError) as e:
+        T.G950Filter(w.numpy(), 8, 3)  # three channels to a wave
+    assert torch.cuda.default_stream().query()
+    assert e.value.code == T.EINVAL

@@ -561,8 +561,8 @@ static int create_from_host(const float* h_filter, int C, int K, int ks, int til
   if (rc == TETRIS_OK && order_rc != TETRIS_OK) rc = tetris::fail(order_rc, "%s", order_error.c_str());
   if (rc == TETRIS_OK)
     rc = tetris::pack_device(d, C, K, ks, tile_ic, oc_per_wave, tile ? order.data() : oc_order, stream, out);
-  else
-    (void)hipStreamSynchronize(stream);
+  // the caller may free or rewrite the filter once this returns, whatever went wrong on the way
+  if (rc != TETRIS_OK) (void)hipStreamSynchronize(stream);
   if (d) (void)hipFreeAsync(d, stream);
   return rc;
 }
