@@ -388,6 +388,29 @@ def test_raw_launcher_refuses_arrays_that_do_not_fit_the_shape(env):
     assert e.value.code == T.EINVAL
 
 
+def test_raw_launcher_refuses_a_negative_capacity_also_on_arrays_it_has_seen(env):
+    T, torch, O = env
+    N, C, H, W, K, ks = 1, 40, 9, 9, 70, 3
+    w = sparse_filter(np.random.default_rng(68), K, C, ks, 0.8)
+    p = O.SpfPack(w, 16, True, True, True, True)
+    offsets, stage_len, position, values, perm = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in p.arrays()]
+    dx, dy = torch.zeros((N, C, H, W), device="cuda"), torch.zeros((N, K, H, W), device="cuda")
+
+    def call(n_entries):
+        T.SparseConv2d(dx.data_ptr(), offsets.data_ptr(), stage_len.data_ptr(), perm.data_ptr(), position.data_ptr(),
+                       values.data_ptr(), dy.data_ptr(), N, H, W, C, K, ks, 1, 1, TILE_IC=16, vec_width=4, n_entries=n_entries)
+        torch.cuda.synchronize()
+
+    for n_entries in (-1, values.numel(), values.numel(), -1, 0):  # not seen yet; then seen, with and without a plan
+        if n_entries < 0:
+            with pytest.raises(T.TetrisError) as e:
+                call(n_entries)
+            assert e.value.code == T.EINVAL
+        else:
+            call(n_entries)
+    T.spf_invalidate(values.data_ptr())
+
+
 def test_raw_launcher_trusting_arrays_it_has_seen(env):
     # TETRIS_OPT_TRUST_SPF_ARRAYS: a set of arrays decoded once is launched again without a read-back (so an in-place
     # rewrite goes unseen) until tetris_spf_invalidate says the arrays have changed.

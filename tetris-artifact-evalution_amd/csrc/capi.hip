@@ -460,7 +460,7 @@ int launch_seen_arrays(const float* d_in, float* d_out, const int32_t* d_offsets
                        hipStream_t stream, bool* done) {
   *done = false;
   SpfView* v = find_view(d_offsets, d_perm, d_position, d_values, C, K, ks, tile_ic, vec);
-  if (!v || !v->d_filter || !d_in || !d_out || (capacity > 0 && v->n_ent > capacity) ||
+  if (!v || !v->d_filter || !d_in || !d_out || capacity < 0 || (capacity > 0 && v->n_ent > capacity) ||
       (options() & TETRIS_OPT_TRUST_SPF_ARRAYS))
     return TETRIS_OK;
   tetris_tile t{};
