@@ -48,3 +48,50 @@ def test_slices_added_by_a_kernel(N, C, H, W, K, ks, t5, slices, oracle):
         want = np.maximum(got, 0)[:, :, :2 * ph, :2 * pw].reshape(N, K, ph, 2, pw, 2).max(axis=(3, 5))
         assert p.cpu().numpy().tobytes() == want.tobytes(), cs
         pk.close()
+
+
+def test_room_for_the_sums_is_taken_where_they_are_kept(oracle):
+    """33 of 128 channel slots used: the waves' order of the sums (51 MB) takes four times the room of the slices' copies
+    of the output (13 MB), and beyond 16 MiB only TETRIS_OPT_ADD_IN_KERNEL keeps it."""
+    import torch
+    import tetris_amd as T
+
+    N, C, H, K = 1024, 32, 7, 33
+    rng = np.random.default_rng(9)
+    w, x = sparse_filter(rng, K, C, 3, 0.8), relu_like(rng, (N, C, H, H))
+    tile = T.Tile(7, 1, 8, 16, 4, 2)
+    pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+    copies = pk.launch_shape(N, H, H, 1, 1, tile).scratch_bytes
+    assert 13e6 < copies < 14e6
+    dx, y = torch.from_numpy(x).cuda(), torch.empty((N, K, H, H), device="cuda")
+    pk.prepare(1, H, H, 1, 1, tile)  # what any first plan on a device allocates
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    pk.prepare(N, H, H, 1, 1, tile)
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] < copies + (8 << 20)
+    outs, options = [], T.options_get()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    pk.prepare(N, H, H, 1, 1, tile, stream=side.cuda_stream)
+    try:
+        pk.launch(dx.data_ptr(), y.data_ptr(), N, H, H, 1, 1, tile)
+        torch.cuda.synchronize()
+        outs.append(y.cpu().numpy())
+        T.options_set(options | T.OPT_ADD_IN_KERNEL)
+        with torch.cuda.graph(graph, stream=side):  # the buffer was made without the option: the copies are added instead
+            pk.launch(dx.data_ptr(), y.data_ptr(), N, H, H, 1, 1, tile, stream=torch.cuda.current_stream().cuda_stream)
+        for _ in range(2):
+            y.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            outs.append(y.cpu().numpy())
+        y.fill_(float("nan"))
+        pk.launch(dx.data_ptr(), y.data_ptr(), N, H, H, 1, 1, tile)  # grows
+        torch.cuda.synchronize()
+        outs.append(y.cpu().numpy())
+    finally:
+        T.options_set(options)
+    assert max_rel_err(outs[0][:32], oracle.host_conv2d(x[:32], w, 1, 1, threads=8)) <= 1e-4
+    assert all(o.tobytes() == outs[0].tobytes() for o in outs)
+    del graph
+    pk.close()

@@ -139,9 +139,13 @@ size_t partial_bytes_of(const Geom& g) {
   return g.csplit > 1 ? (size_t)kTicketBytes + sizeof(float) * (size_t)g.csplit * g.N * g.K * g.OH * g.OW : 0;
 }
 
-// ... and what it gets where the library allocates it: room for the waves' sums as well, which idle lanes make longer
+// ... and what it gets where the library allocates it: room for the waves' sums as well, which idle lanes make longer,
+// where the launcher keeps the sums so
 size_t scratch_bytes_of(const Plan& p) {
-  return p.parts ? partial_bytes_of(p.mat) : std::max(partial_bytes_of(p.geom), kTicketBytes + sum_bytes_of(p.geom));
+  if (p.parts) return partial_bytes_of(p.mat);
+  const size_t sums = sum_bytes_of(p.geom);
+  const bool kept = sums <= kMaxWaveSums || (options() & TETRIS_OPT_ADD_IN_KERNEL);
+  return std::max(partial_bytes_of(p.geom), kept ? kTicketBytes + sums : 0);
 }
 
 // launches a layer as its plan says
@@ -164,18 +168,21 @@ int launch_plan(const Plan& p, const float* d_in, float* d_out, float* d_scratch
 
 // Partial-sum buffer of a split layer: one per (pack, stream), so that launches of one pack on different streams do
 // not share it.  A buffer that has to grow is replaced, and the old one is kept until the pack is destroyed: a HIP
-// graph captured earlier may still hold its address.
-int partial_buffer(tetris_g950* p, hipStream_t stream, size_t need, bool grow, float** out) {
+// graph captured earlier may still hold its address.  Under capture nothing can grow, and a buffer of `least` bytes
+// will do (one made before TETRIS_OPT_ADD_IN_KERNEL was set).  *bytes: what the buffer holds.
+int partial_buffer(tetris_g950* p, hipStream_t stream, size_t need, size_t least, float** out, size_t* bytes) {
   std::lock_guard<std::mutex> lock(p->mu);
   tetris_g950::Partial& b = p->partial[stream];
   if (b.bytes < need) {
-    if (!grow)
-      return fail(TETRIS_ENOTFOUND, "no partial-sum buffer of %zu bytes on this stream: call tetris_g950_prepare first",
-                  need);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
-      return fail(TETRIS_EINVAL, "this launch would allocate its partial-sum buffer: call tetris_g950_prepare before "
-                  "capturing");
+    if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+      if (b.bytes < least)
+        return fail(TETRIS_EINVAL, "this launch would allocate its partial-sum buffer: call tetris_g950_prepare before "
+                    "capturing");
+      *out = b.ptr;
+      *bytes = b.bytes;
+      return TETRIS_OK;
+    }
     bool same_xcd = false;  // asked here, where allocating and synchronising is allowed, so that launches find the answer
     int rc = same_xcd_by_residue(&same_xcd);
     if (rc) return rc;
@@ -192,7 +199,17 @@ int partial_buffer(tetris_g950* p, hipStream_t stream, size_t need, bool grow, f
     b.bytes = need;
   }
   *out = b.ptr;
+  *bytes = b.bytes;
   return TETRIS_OK;
+}
+
+// the same for a plan: nothing where the layer is not split
+int plan_scratch(tetris_g950* p, const Plan& plan, hipStream_t stream, float** out, size_t* bytes) {
+  *out = nullptr;
+  *bytes = 0;
+  if (slices_of(plan) == 1) return TETRIS_OK;
+  return partial_buffer(p, stream, scratch_bytes_of(plan), plan.parts ? partial_bytes_of(plan.mat) : partial_bytes_of(plan.geom),
+                        out, bytes);
 }
 
 int run_launch(tetris_g950* p, const float* d_in, float* d_out, int N, int H, int W, int stride, int pad,
@@ -202,11 +219,9 @@ int run_launch(tetris_g950* p, const float* d_in, float* d_out, int N, int H, in
   int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, &plan);
   if (rc) return rc;
   float* d_partial = nullptr;
-  const size_t scratch = scratch_bytes_of(plan);
-  if (slices_of(plan) > 1) {
-    rc = partial_buffer(p, stream, scratch, true, &d_partial);
-    if (rc) return rc;
-  }
+  size_t scratch = 0;
+  rc = plan_scratch(p, plan, stream, &d_partial, &scratch);
+  if (rc) return rc;
   return launch_plan(plan, d_in, d_out, d_partial, scratch, p->d_oc_order, act, stream);
 }
 
@@ -915,11 +930,10 @@ int tetris_g950_prepare(tetris_g950* p, int N, int H, int W, int stride, int pad
   Plan plan;
   int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, &plan);
   if (rc) return rc;
-  if (slices_of(plan) > 1) {
-    float* d_partial = nullptr;
-    rc = partial_buffer(p, stream, scratch_bytes_of(plan), true, &d_partial);
-    if (rc) return rc;
-  }
+  float* d_partial = nullptr;
+  size_t bytes = 0;
+  rc = plan_scratch(p, plan, stream, &d_partial, &bytes);
+  if (rc) return rc;
   float* s = nullptr;
   return static_scratch(&s);  // looks the static scratch array of this GPU up, for tetris_spconv2d_launch_noalloc
 }
