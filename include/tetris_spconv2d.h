@@ -130,7 +130,9 @@ int tetris_tile_select(int batch, int img_h, int img_w, int in_channel, int out_
  * tetris_tile_autotune runs; other lines are skipped) and makes tetris_tile_select, and every entry point that
  * chooses the tile itself, answer from them before the built-in table.  Plays the part of the reference's static
  * per-layer cache of the exhaustive search (Tetris/spconv2d.cc:90, 285-329), kept across processes.  A row whose
- * tile the kernel's checks refuse is ignored at look-up.  *rows_out (may be NULL) receives the rows read.
+ * tile the kernel's checks refuse is ignored at look-up.  A loaded row is obeyed: the kernel that walks the non-zeros
+ * runs the layer with that tile, also where the library by itself would predict the matrix cores to be faster.
+ * *rows_out (may be NULL) receives the rows read.
  * Process-wide; may be called several times (later files win). */
 int tetris_tile_table_load(const char* path, int* rows_out);
 
@@ -188,7 +190,8 @@ int tetris_g950_create_balanced(const float* h_filter_oihw, int in_channel, int 
  * for the `max_candidates` (0 = 24) tile shapes the model of tetris_tile_select ranks best (each in the
  * output-channel order of tetris_oc_order_balanced for that tile), times each on the device with the real
  * weights (1 warm-up + 3 launches on zero-filled input), times the four fastest again (2 + 10 launches) and
- * returns the fastest and its milliseconds per launch.  Allocates and frees its own device buffers;
+ * returns the fastest and its milliseconds per launch.  Every candidate is timed on the kernel that walks the
+ * non-zeros, which is what a row loaded with tetris_tile_table_load runs.  Allocates and frees its own device buffers;
  * synchronises `stream`. */
 int tetris_tile_autotune(const float* h_filter_oihw, int batch, int img_h, int img_w, int in_channel, int out_channel,
                          int kernel_size, int stride, int padding, int max_candidates, void* stream,

@@ -75,3 +75,37 @@ def test_parts_keep_every_bit():
     torch.cuda.synchronize()
     assert np.array_equal(y.cpu().numpy(), x[:, np.arange(K) % C])
     pk.close()
+
+
+def test_loaded_row_is_obeyed(oracle, tmp_path):
+    """A walking tile that the caller loaded runs as such, given or chosen, where the library would take the matrix cores."""
+    import torch
+    import tetris_amd as T
+
+    N, C, H, W, K, ks = 3, 50, 22, 31, 90, 3
+    rng = np.random.default_rng(12)
+    w, x = sparse_filter(rng, K, C, ks, 0.7), relu_like(rng, (N, C, H, W))
+    tile = T.tile_select(N, H, W, C, K, ks, 1, 1)
+    before, after = (T.G950Filter.for_tile(w, tile, oc_order="balanced") for _ in range(2))
+    dx = torch.from_numpy(x).cuda()
+
+    def conv(pk, t):
+        y = torch.full((N, K, H, W), float("nan"), device="cuda")
+        pk.launch(dx.data_ptr(), y.data_ptr(), N, H, W, 1, 1, t)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    assert before.launch_shape(N, H, W, 1, 1, tile).kernel == 5
+    matrix = conv(before, tile)
+    table = tmp_path / "tiles.inc"
+    table.write_text("    {%d, %d, %d, %d, %d, %d, 1, 1, {%s}},\n" % (N, H, W, C, K, ks, ", ".join(map(str, tile.as_list()))))
+    assert T.tile_table_load(str(table)) == 1
+    shape = after.launch_shape(N, H, W, 1, 1, tile)
+    assert shape.kernel != 5
+    walk = conv(after, T.Tile(*tile.as_list()[:5], shape.csplit))
+    assert walk.tobytes() != matrix.tobytes()  # sums in another order: tells the two kernels apart
+    assert conv(after, tile).tobytes() == walk.tobytes() and conv(after, None).tobytes() == walk.tobytes()
+    ref = oracle.host_conv2d(x, w, 1, 1, threads=8)
+    assert max_rel_err(walk, ref) <= 1e-4 and max_rel_err(matrix, ref) <= 1e-4
+    before.close()
+    after.close()

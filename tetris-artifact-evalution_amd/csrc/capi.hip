@@ -42,18 +42,17 @@ int upload(const std::vector<T>& v, T** d) {
 }
 
 // Whether the matrix kernel runs the layer, and how.  Only where the choice is the library's: no tile given, or the one that
-// tetris_tile_select names; a tile of the caller's own is obeyed, and so is an option that picks a form of the walking
-// kernels.
+// tetris_tile_select names; a tile of the caller's own is obeyed, and so are a row that the caller loaded (a walking
+// tile that was measured, where this is a prediction) and an option that picks a form of the walking kernels.
 bool choose_matrix(const tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile* tile, const Geom& walk,
                    MatGeom* g, MatGeom* pool) {
   if (options() & (TETRIS_OPT_PAIRS | TETRIS_OPT_NO_BANK_RULE | TETRIS_OPT_ADD_IN_KERNEL)) return false;
-  if (tile) {
-    tetris_tile own{};
-    if (choose_tile(N, H, W, p->C, p->K, p->ks, stride, pad, &own) != TETRIS_OK || tile->lanes_w != own.lanes_w ||
-        tile->quads != own.quads || tile->oc_per_wave != own.oc_per_wave || tile->waves != own.waves ||
-        tile->tile_ic != own.tile_ic || tile->csplit != own.csplit)
-      return false;
-  }
+  tetris_tile own{};
+  bool loaded = false;
+  if (choose_tile(N, H, W, p->C, p->K, p->ks, stride, pad, &own, &loaded) != TETRIS_OK || loaded) return false;
+  if (tile && (tile->lanes_w != own.lanes_w || tile->quads != own.quads || tile->oc_per_wave != own.oc_per_wave ||
+               tile->waves != own.waves || tile->tile_ic != own.tile_ic || tile->csplit != own.csplit))
+    return false;
   return choose_mat_geom(N, p->C, H, W, p->K, p->ks, stride, pad, walk, p->nnz, g, pool);
 }
 
@@ -79,13 +78,15 @@ int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const v
 
 // The launch plan of (input shape, tile) for pack `p`: looked up, or -- when `create` allows it -- made (geometry,
 // bound entries: one device allocation and one small kernel on `stream`) and remembered.
+// walk: the kernel that walks the non-zeros, also where the library would take the matrix kernel -- for what times or
+// runs walking tiles as such (autotune, the rungs of the ablation ladder).
 int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile* tile, hipStream_t stream,
-              bool create, Plan* out) {
+              bool create, bool walk, Plan* out) {
   const bool given = tile && tile->lanes_w > 0;
   // a NULL tile is remembered under a key of zeros, so that the library's own choice is made once per shape
   const tetris_tile none{};
   const tetris_tile& kt = given ? *tile : none;
-  const int key[11] = {N, H, W, stride, pad, kt.lanes_w, kt.quads, kt.oc_per_wave, kt.waves, kt.tile_ic, kt.csplit};
+  const int key[12] = {N, H, W, stride, pad, kt.lanes_w, kt.quads, kt.oc_per_wave, kt.waves, kt.tile_ic, kt.csplit, walk};
   {
     std::lock_guard<std::mutex> lock(p->mu);
     for (size_t i = p->plans.size(); i-- > 0;)
@@ -113,7 +114,7 @@ int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const te
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
     return fail(TETRIS_EINVAL, "the first launch of a shape allocates: call tetris_g950_prepare before capturing");
-  if (choose_matrix(p, N, H, W, stride, pad, given ? tile : nullptr, plan.geom, &plan.mat, &plan.mat_pool)) {
+  if (!walk && choose_matrix(p, N, H, W, stride, pad, given ? tile : nullptr, plan.geom, &plan.mat, &plan.mat_pool)) {
     rc = matrix_weights(p, plan.mat, stream, &plan.parts);
   } else {
     rc = g950_bind(p, plan.geom, geom_walks_pairs(plan.geom), stream, &plan.entries, &plan.grp_off, &plan.grp_pair,
@@ -213,10 +214,10 @@ int plan_scratch(tetris_g950* p, const Plan& plan, hipStream_t stream, float** o
 }
 
 int run_launch(tetris_g950* p, const float* d_in, float* d_out, int N, int H, int W, int stride, int pad,
-               const tetris_tile* tile, hipStream_t stream, int act = 0) {
+               const tetris_tile* tile, hipStream_t stream, int act = 0, bool walk = false) {
   if (!p || !d_in || !d_out) return fail(TETRIS_EINVAL, "null argument");
   Plan plan;
-  int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, &plan);
+  int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, walk, &plan);
   if (rc) return rc;
   float* d_partial = nullptr;
   size_t scratch = 0;
@@ -256,7 +257,7 @@ int static_scratch(float** out) {
 }
 
 int time_launches(tetris_g950* p, const float* d_in, float* d_out, int N, int H, int W, int stride, int pad,
-                  const tetris_tile* tile, hipStream_t stream, int warm, int repeat, float* ms_out) {
+                  const tetris_tile* tile, hipStream_t stream, int warm, int repeat, float* ms_out, bool walk = false) {
   if (repeat <= 0 || warm < 0) return fail(TETRIS_EINVAL, "bad warm/repeat");
   hipEvent_t a = nullptr, b = nullptr;
   auto done = [&](int code) {
@@ -273,7 +274,7 @@ int time_launches(tetris_g950* p, const float* d_in, float* d_out, int N, int H,
   HIPT(hipEventCreate(&a));
   HIPT(hipEventCreate(&b));
   for (int i = 0; i < warm; ++i) {
-    const int rc = run_launch(p, d_in, d_out, N, H, W, stride, pad, tile, stream);
+    const int rc = run_launch(p, d_in, d_out, N, H, W, stride, pad, tile, stream, 0, walk);
     if (rc) return done(rc);
   }
   HIPT(hipStreamSynchronize(stream));
@@ -285,7 +286,7 @@ int time_launches(tetris_g950* p, const float* d_in, float* d_out, int N, int H,
       int rc = sweep_caches(stream);
       if (rc) return done(rc);
       HIPT(hipEventRecord(a, stream));
-      rc = run_launch(p, d_in, d_out, N, H, W, stride, pad, tile, stream);
+      rc = run_launch(p, d_in, d_out, N, H, W, stride, pad, tile, stream, 0, walk);
       if (rc) return done(rc);
       HIPT(hipEventRecord(b, stream));
       HIPT(hipEventSynchronize(b));
@@ -296,7 +297,7 @@ int time_launches(tetris_g950* p, const float* d_in, float* d_out, int N, int H,
   } else {
     HIPT(hipEventRecord(a, stream));
     for (int i = 0; i < repeat; ++i) {
-      const int rc = run_launch(p, d_in, d_out, N, H, W, stride, pad, tile, stream);
+      const int rc = run_launch(p, d_in, d_out, N, H, W, stride, pad, tile, stream, 0, walk);
       if (rc) return done(rc);
     }
     HIPT(hipEventRecord(b, stream));
@@ -489,7 +490,7 @@ int launch_seen_arrays(const float* d_in, float* d_out, const int32_t* d_offsets
   const auto pk = v->packs.find({t.tile_ic, t.oc_per_wave});
   if (pk == v->packs.end()) return TETRIS_OK;
   Plan plan;
-  if (find_plan(pk->second, N, H, W, stride, pad, &t, stream, false, &plan) != TETRIS_OK) return TETRIS_OK;
+  if (find_plan(pk->second, N, H, W, stride, pad, &t, stream, false, false, &plan) != TETRIS_OK) return TETRIS_OK;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) return TETRIS_OK;
   if (!g_hash_shares) {
@@ -626,7 +627,7 @@ int conv_host(const float* h_in, const float* h_filter, float* h_out, int N, int
   HIPD(hipMalloc(&d_out, out_bytes));
   HIPD(hipMemcpyAsync(d_in, h_in, in_bytes, hipMemcpyHostToDevice, stream));
   float ms = 0;
-  rc = time_launches(run, d_in, d_out, N, H, W, stride, pad, &tile, stream, 30, 100, &ms);
+  rc = time_launches(run, d_in, d_out, N, H, W, stride, pad, &tile, stream, 30, 100, &ms, spf_path);
   if (views_lock.owns_lock()) views_lock.unlock();
   if (rc) return done(rc);
   HIPD(hipMemcpyAsync(h_out, d_out, out_bytes, hipMemcpyDeviceToHost, stream));
@@ -789,7 +790,8 @@ int tetris_tile_autotune_list(const float* h_filter, int N, int H, int W, int C,
   HIPA(hipMemsetAsync(d_in, 0, in_bytes, stream));  // timing does not depend on the values
   HIPA(hipMemcpyAsync(d_f, h_filter, f_bytes, hipMemcpyHostToDevice, stream));
 #undef HIPA
-  // first pass: a quick look at every candidate; second pass: the four fastest again, with more launches
+  // first pass: a quick look at every candidate; second pass: the four fastest again, with more launches; the walking
+  // kernels throughout, also for the tile with which the library would take the matrix kernel
   std::vector<std::pair<float, tetris_tile>> timed;
   for (const tetris_tile& t : ranked) {
     if ((int)timed.size() >= max_candidates) break;
@@ -803,7 +805,7 @@ int tetris_tile_autotune_list(const float* h_filter, int N, int H, int W, int C,
       it = packs.emplace(key, p).first;
     }
     float ms = 0;
-    rc = time_launches(it->second, d_in, d_out, N, H, W, stride, pad, &t, stream, timed.empty() ? 8 : 1, 3, &ms);
+    rc = time_launches(it->second, d_in, d_out, N, H, W, stride, pad, &t, stream, timed.empty() ? 8 : 1, 3, &ms, true);
     if (rc == TETRIS_EINVAL) continue;  // the model ranks shapes make_geom may still refuse
     if (rc) return done(rc);
     if (timed.empty() && ms > 0) {
@@ -811,7 +813,7 @@ int tetris_tile_autotune_list(const float* h_filter, int N, int H, int W, int C,
       // reach the 2.3-2.4 GHz it holds under load, a tenth in time that would otherwise count against the candidates
       // the model ranks first.  Some 30 ms of launches, then the candidate's time again.
       const int settle = (int)std::min(3000.0f, 30.0f / ms);
-      rc = time_launches(it->second, d_in, d_out, N, H, W, stride, pad, &t, stream, settle, 3, &ms);
+      rc = time_launches(it->second, d_in, d_out, N, H, W, stride, pad, &t, stream, settle, 3, &ms, true);
       if (rc) return done(rc);
     }
     timed.emplace_back(ms, t);
@@ -839,7 +841,7 @@ int tetris_tile_autotune_list(const float* h_filter, int N, int H, int W, int C,
         // more slices than wave slots to run them at once only add partial sums
         if (cs > g0.csplit && (long long)gv.ugroups * gv.kblocks * cs * v.waves > 16ll * 256 * 2) continue;
         float ms = 0;
-        rc = time_launches(pk, d_in, d_out, N, H, W, stride, pad, &v, stream, 1, 3, &ms);
+        rc = time_launches(pk, d_in, d_out, N, H, W, stride, pad, &v, stream, 1, 3, &ms, true);
         if (rc == TETRIS_EINVAL) continue;
         if (rc) return done(rc);
         extra.emplace_back(ms, v);
@@ -853,7 +855,7 @@ int tetris_tile_autotune_list(const float* h_filter, int N, int H, int W, int C,
     const tetris_tile& t = timed[i].second;
     float ms = 0;
     rc = time_launches(packs[{t.tile_ic, t.oc_per_wave, t.waves}], d_in, d_out, N, H, W, stride, pad, &t, stream, 2, 10,
-                       &ms);
+                       &ms, true);
     if (rc) return done(rc);
     timed[i].first = ms;
   }
@@ -928,7 +930,7 @@ int tetris_g950_prepare(tetris_g950* p, int N, int H, int W, int stride, int pad
   if (!p) return fail(TETRIS_EINVAL, "null argument");
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   Plan plan;
-  int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, &plan);
+  int rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, false, &plan);
   if (rc) return rc;
   float* d_partial = nullptr;
   size_t bytes = 0;
@@ -960,7 +962,7 @@ int tetris_spconv2d_launch_noalloc(tetris_g950* p, const float* d_in, float* d_o
   if (!p || !d_in || !d_out) return fail(TETRIS_EINVAL, "null argument");
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   Plan plan;
-  int rc = find_plan(p, N, H, W, stride, pad, tile, stream, false, &plan);
+  int rc = find_plan(p, N, H, W, stride, pad, tile, stream, false, false, &plan);
   if (rc) return rc;
   float* d_partial = nullptr;
   if (slices_of(plan) > 1) {

@@ -193,7 +193,7 @@ constexpr long long kMatCopies = 32 << 20;  // most bytes of partial sums of a s
 
 // A launch plan: everything run_launch derives from (input shape, tile) for one pack, kept for the next call.
 struct Plan {
-  int key[11];  // N, H, W, stride, pad, lanes_w, quads, oc_per_wave, waves, tile_ic, csplit
+  int key[12];  // N, H, W, stride, pad, lanes_w, quads, oc_per_wave, waves, tile_ic, csplit, walk (see find_plan)
   Geom geom;
   const int2* entries;        // the pack's entries bound to the geometry
   const int32_t* grp_off;     // [groups*stages+1] first entry of every stream in `entries`
@@ -282,7 +282,8 @@ int spf_arrays_decode(const int32_t* d_offsets, const int32_t* d_perm, const int
 unsigned options();  // TETRIS_OPT_* flags in force (tetris_options_set, or the environment variable TETRIS_OPTIONS)
 void set_options(unsigned flags);
 int make_geom(const tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile& t, Geom* g);
-int choose_tile(int N, int H, int W, int C, int K, int ks, int stride, int pad, tetris_tile* t);
+// loaded (may be null): whether the tile is that of a row the caller loaded (tetris_tile_table_load)
+int choose_tile(int N, int H, int W, int C, int K, int ks, int stride, int pad, tetris_tile* t, bool* loaded = nullptr);
 // reads rows in the format of tuned_tiles.inc; choose_tile looks them up before the built-in table
 int load_tile_table(const char* path, int* rows_out);
 // every tile shape the kernel can run for the layer, cheapest first by the selector's time model

@@ -502,12 +502,14 @@ int load_tile_table(const char* path, int* rows_out) {
   return TETRIS_OK;
 }
 
-int choose_tile(int N, int H, int W, int C, int K, int ks, int stride, int pad, tetris_tile* t) {
+int choose_tile(int N, int H, int W, int C, int K, int ks, int stride, int pad, tetris_tile* t, bool* loaded) {
+  if (loaded) *loaded = false;
   {
     std::lock_guard<std::mutex> lock(g_loaded_mu);
     for (const Tuned& e : g_loaded)
       if (same_shape(e, N, H, W, C, K, ks, stride, pad) && usable(e)) {
         *t = e.tile;
+        if (loaded) *loaded = true;
         return TETRIS_OK;
       }
   }

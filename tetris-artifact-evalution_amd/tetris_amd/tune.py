@@ -28,6 +28,10 @@ of the pass at batch 16, 5.9 % at batch 1; the built-in table keeps the faster t
 times, for every shape on which two tables disagree, both tiles head to head (three alternating rounds of 30 launches;
 from cold caches for the suites named) and keeps OLD's row unless NEW's tile is faster by more than --margin.
 
+A table other than the built-in one is for tetris_tile_table_load, whose rows are obeyed: a layer that the library runs
+faster on the matrix cores than the best walking tile does gets no row there.  All times of tiles are those of the
+walking kernels.
+
 Rebuild the library afterwards.  tetris_tile_select consults the table before its cycle model; a shape that is not
 listed, or whose tile the kernel's checks refuse, falls back to the model.
 """
@@ -37,9 +41,29 @@ import glob
 import json
 import os
 import sys
+import tempfile
 
 import tetris_amd as T
 from tetris_amd import workloads as W
+
+
+BUILT_IN = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc", "tuned_tiles.inc")
+
+
+def own_choice_ms(w, L, n, cold):
+    """Milliseconds per launch where the library runs the layer on the matrix cores, else None."""
+    import torch
+
+    tile = T.tile_select(n, L.H, L.W, L.C, L.K, L.ks, L.stride, L.pad)
+    pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+    try:
+        if pk.launch_shape(n, L.H, L.W, L.stride, L.pad, tile).kernel != 5:
+            return None
+        x = torch.zeros((n, L.C, L.H, L.W), device="cuda")
+        y = torch.empty((n, L.K) + tuple(W.out_hw(L)), device="cuda")
+        return pk.time(x.data_ptr(), y.data_ptr(), n, L.H, L.W, L.stride, L.pad, tile, warm=2 if cold else 5, repeat=10)
+    finally:
+        pk.close()
 
 
 def shapes(args):
@@ -85,9 +109,18 @@ def write_table(path, rows):
     print("wrote %d shapes to %s" % (len(rows), path), file=sys.stderr)
 
 
+def obey(key, tile):
+    """From now on `tile` is a loaded row for this shape: its launches run the walking kernel it describes, not the matrix
+    kernel that the library may predict to be faster where a tile is the one it would choose itself."""
+    with tempfile.NamedTemporaryFile("w", suffix=".inc") as f:
+        f.write("    {%d, %d, %d, %d, %d, %d, %d, %d, %s},\n" % (tuple(key) + (tile_text(tile),)))
+        f.flush()
+        T.tile_table_load(f.name)
+
+
 def counter_sums(directory, names):
-    """Per conv launch, in dispatch order: the sum of the named counters over the conv kernel and the reduce kernel
-    that may follow it."""
+    """Per conv launch, in dispatch order: the sum of the named counters over the conv kernel and the kernel that may
+    follow it to add the slices (reduce_kernel or add_kernel)."""
     files = glob.glob(os.path.join(directory, "**", "*counter_collection.csv"), recursive=True)
     if not files:
         sys.exit("no counter_collection.csv under %s" % directory)
@@ -101,7 +134,7 @@ def counter_sums(directory, names):
         name, vals = per[did]
         if "spconv2d_" in name:
             out.append(dict(vals))
-        elif "reduce_kernel" in name and out:
+        elif ("reduce_kernel" in name or "add_kernel" in name) and out:
             for k, v in vals.items():
                 out[-1][k] = out[-1].get(k, 0.0) + v
     return out
@@ -138,8 +171,7 @@ def main():
                     "vector units (0: they take their fastest tile)")
     ap.add_argument("--within", type=float, default=0.02, help="how much slower than the fastest a tile may be and still "
                     "win on bytes moved")
-    ap.add_argument("--out", default=os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc",
-                                                  "tuned_tiles.inc"))
+    ap.add_argument("--out", default=BUILT_IN)
     args = ap.parse_args()
 
     if args.replay:
@@ -157,6 +189,7 @@ def main():
             y = torch.empty((n, K, oh, ow), device="cuda")
             for c in it["candidates"]:
                 tile = T.Tile(*c["tile"])
+                obey(it["key"], c["tile"])
                 pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
                 pk.prepare(n, H, Wd, stride, pad, tile)
                 pk.launch(x.data_ptr(), y.data_ptr(), n, H, Wd, stride, pad, tile)
@@ -254,6 +287,7 @@ def main():
             packs = {t: T.G950Filter.for_tile(w, T.Tile(*t), oc_order="balanced") for t in (tile_old, tile_new)}
             for _ in range(3):
                 for t, pk in packs.items():
+                    obey(key, t)
                     ms = pk.time(x.data_ptr(), y.data_ptr(), n, L.H, L.W, L.stride, L.pad, T.Tile(*t), warm=2 if cold else 5,
                                  repeat=10 if cold else 30)
                     best[t] = min(best.get(t, 1e9), ms)
@@ -293,6 +327,7 @@ def main():
             if inc and all(tuple(t.as_list()) != inc for t, _ in cands):
                 try:  # the incumbent, timed like the tuner's second pass (2 + 10 launches)
                     tile = T.Tile(*inc)
+                    obey(key, inc)
                     pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
                     oh, ow = W.out_hw(L)
                     x = torch.zeros((n, L.C, L.H, L.W), device="cuda")
@@ -307,6 +342,11 @@ def main():
             tile, ms = cands[0]
         else:
             tile, ms = T.tile_autotune(w, n, L.H, L.W, L.stride, L.pad, args.candidates)
+            own = own_choice_ms(w, L, n, args.cold) if args.out != BUILT_IN else None
+            if own is not None and own < ms:
+                print("%-10s %-26s N=%-2d %8.1f us  %r, left out: the library runs it in %.1f us on the matrix cores" % (
+                    suite, L.name, n, ms * 1e3, tile, own * 1e3), file=sys.stderr, flush=True)
+                continue
         rows.append((key, tuple(tile.as_list()),
                      "%s %s: %.1f us" % (suite, L.name, ms * 1e3)))
         print("%-10s %-26s N=%-2d %8.1f us  %r" % (suite, L.name, n, ms * 1e3, tile), file=sys.stderr, flush=True)
