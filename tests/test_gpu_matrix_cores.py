@@ -109,3 +109,45 @@ def test_loaded_row_is_obeyed(oracle, tmp_path):
     assert max_rel_err(walk, ref) <= 1e-4 and max_rel_err(matrix, ref) <= 1e-4
     before.close()
     after.close()
+
+
+@pytest.mark.parametrize("C,matrix", [(24, True), (15, False)])
+def test_queries_tell_what_launches_run(C, matrix, oracle):
+    """Options set after a plan was made change neither what the plan runs nor what the queries say of it; a shape that has
+    no plan yet is answered for under the options in force."""
+    import torch
+    import tetris_amd as T
+
+    N, H, W, K, ks = 2, 20, 26, 40, 3
+    rng = np.random.default_rng(13)
+    w, x = sparse_filter(rng, K, C, ks, 0.6), relu_like(rng, (N, C, H, W))
+    tile = T.tile_select(N, H, W, C, K, ks, 1, 1)
+    pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+    dx, y = torch.from_numpy(x).cuda(), torch.empty((N, K, H, W), device="cuda")
+
+    def ask():
+        s = pk.launch_shape(N, H, W, 1, 1, tile)
+        acts = [pk.act_supported(N, H, W, 1, 1, tile, a) for a in (T.ACT_NONE, T.ACT_RELU, T.ACT_RELU_POOL2)]
+        return [getattr(s, f) for f, _ in T.LaunchShape._fields_], acts
+
+    def conv():
+        y.fill_(float("nan"))
+        pk.launch(dx.data_ptr(), y.data_ptr(), N, H, W, 1, 1, tile)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    options = T.options_get()
+    try:
+        T.options_set(options | T.OPT_PAIRS)
+        assert ask()[0][6] != 5  # the option picks a walking kernel, and no plan says otherwise
+        T.options_set(options)
+        before = ask()
+        assert (before[0][6] == 5) == matrix
+        out = conv()
+        assert ask() == before
+        T.options_set(options | T.OPT_PAIRS | T.OPT_NO_BANK_RULE)
+        assert ask() == before and conv().tobytes() == out.tobytes()
+    finally:
+        T.options_set(options)
+    assert max_rel_err(out, oracle.host_conv2d(x, w, 1, 1, threads=8)) <= 1e-4
+    pk.close()

@@ -76,6 +76,64 @@ int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const v
   return TETRIS_OK;
 }
 
+// what a plan or a choice is remembered under; a NULL tile under zeros, so that the library's own choice is made once
+using Key = std::array<int, 12>;
+Key plan_key(int N, int H, int W, int stride, int pad, const tetris_tile* tile, bool walk) {
+  const tetris_tile none{};
+  const tetris_tile& t = tile && tile->lanes_w > 0 ? *tile : none;
+  return {N, H, W, stride, pad, t.lanes_w, t.quads, t.oc_per_wave, t.waves, t.tile_ic, t.csplit, walk};
+}
+
+bool known_plan(tetris_g950* p, const Key& key, Plan* out) {
+  std::lock_guard<std::mutex> lock(p->mu);
+  for (size_t i = p->plans.size(); i-- > 0;)
+    if (memcmp(p->plans[i].key, key.data(), sizeof key) == 0) {
+      *out = p->plans[i];
+      return true;
+    }
+  return false;
+}
+
+// Decides which kernel runs (input shape, tile); `t`: the tile, given or chosen.  Remembered, so that a query and the
+// plan that follows it decide once (0.3 ms for an image of 211 x 223).
+int choose_kernel(tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile& t, bool given, bool walk,
+                  Choice* out) {
+  const Key shape = plan_key(N, H, W, stride, pad, given ? &t : nullptr, walk);
+  int key[14];
+  std::copy(shape.begin(), shape.end(), key);
+  key[12] = (int)options();
+  key[13] = (int)loaded_tables();
+  {
+    std::lock_guard<std::mutex> lock(p->mu);
+    for (size_t i = p->chosen.size(); i-- > 0;)
+      if (memcmp(p->chosen[i].key, key, sizeof key) == 0) {
+        *out = p->chosen[i].choice;
+        return TETRIS_OK;
+      }
+  }
+  Chosen c;
+  memcpy(c.key, key, sizeof key);
+  const int rc = make_geom(p, N, H, W, stride, pad, t, &c.choice.geom);
+  if (rc) return rc;
+  c.choice.matrix = !walk && choose_matrix(p, N, H, W, stride, pad, given ? &t : nullptr, c.choice.geom, &c.choice.mat,
+                                           &c.choice.mat_pool);
+  std::lock_guard<std::mutex> lock(p->mu);
+  if (p->chosen.size() >= 64) p->chosen.erase(p->chosen.begin());
+  p->chosen.push_back(c);
+  *out = c.choice;
+  return TETRIS_OK;
+}
+
+// What a launch of (input shape, tile) would run, for queries: the plan's own choice where there is a plan.
+int find_choice(tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile& tile, Choice* out) {
+  Plan plan;
+  if (tile.lanes_w > 0 && known_plan(p, plan_key(N, H, W, stride, pad, &tile, false), &plan)) {
+    *out = {plan.geom, plan.parts != nullptr, plan.mat, plan.mat_pool};
+    return TETRIS_OK;
+  }
+  return choose_kernel(p, N, H, W, stride, pad, tile, true, false, out);
+}
+
 // The launch plan of (input shape, tile) for pack `p`: looked up, or -- when `create` allows it -- made (geometry,
 // bound entries: one device allocation and one small kernel on `stream`) and remembered.
 // walk: the kernel that walks the non-zeros, also where the library would take the matrix kernel -- for what times or
@@ -83,18 +141,8 @@ int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const v
 int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile* tile, hipStream_t stream,
               bool create, bool walk, Plan* out) {
   const bool given = tile && tile->lanes_w > 0;
-  // a NULL tile is remembered under a key of zeros, so that the library's own choice is made once per shape
-  const tetris_tile none{};
-  const tetris_tile& kt = given ? *tile : none;
-  const int key[12] = {N, H, W, stride, pad, kt.lanes_w, kt.quads, kt.oc_per_wave, kt.waves, kt.tile_ic, kt.csplit, walk};
-  {
-    std::lock_guard<std::mutex> lock(p->mu);
-    for (size_t i = p->plans.size(); i-- > 0;)
-      if (memcmp(p->plans[i].key, key, sizeof key) == 0) {
-        *out = p->plans[i];
-        return TETRIS_OK;
-      }
-  }
+  const Key key = plan_key(N, H, W, stride, pad, tile, walk);
+  if (known_plan(p, key, out)) return TETRIS_OK;
   if (!create)
     return fail(TETRIS_ENOTFOUND, "no launch plan for N=%d H=%d W=%d stride=%d pad=%d with this tile: call "
                 "tetris_g950_prepare first", N, H, W, stride, pad);
@@ -108,20 +156,24 @@ int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const te
   if (t.tile_ic != p->tile_ic || t.oc_per_wave != p->g)
     return fail(TETRIS_EINVAL, "tile (tile_ic=%d, oc_per_wave=%d) does not match the pack (tile_ic=%d, oc_per_wave=%d)",
                 t.tile_ic, t.oc_per_wave, p->tile_ic, p->g);
-  Plan plan;
-  int rc = make_geom(p, N, H, W, stride, pad, t, &plan.geom);
+  Choice choice;
+  int rc = choose_kernel(p, N, H, W, stride, pad, t, given, walk, &choice);
   if (rc) return rc;
+  Plan plan;
+  plan.geom = choice.geom;
+  plan.mat = choice.mat;
+  plan.mat_pool = choice.mat_pool;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
     return fail(TETRIS_EINVAL, "the first launch of a shape allocates: call tetris_g950_prepare before capturing");
-  if (!walk && choose_matrix(p, N, H, W, stride, pad, given ? tile : nullptr, plan.geom, &plan.mat, &plan.mat_pool)) {
+  if (choice.matrix) {
     rc = matrix_weights(p, plan.mat, stream, &plan.parts);
   } else {
     rc = g950_bind(p, plan.geom, geom_walks_pairs(plan.geom), stream, &plan.entries, &plan.grp_off, &plan.grp_pair,
                    &plan.geom.heads_off);
   }
   if (rc) return rc;
-  memcpy(plan.key, key, sizeof key);
+  std::copy(key.begin(), key.end(), plan.key);
   std::lock_guard<std::mutex> lock(p->mu);
   if (p->plans.size() >= 64) p->plans.erase(p->plans.begin());
   p->plans.push_back(plan);
@@ -892,24 +944,24 @@ int tetris_spconv2d_act_supported(tetris_g950* p, int N, int H, int W, int strid
   if (!p || !tile || !supported) return fail(TETRIS_EINVAL, "null argument");
   if (activation < TETRIS_ACT_NONE || activation > TETRIS_ACT_RELU_POOL2)
     return fail(TETRIS_EINVAL, "unknown activation %d", activation);
-  Geom g;
-  const int rc = make_geom(p, N, H, W, stride, pad, *tile, &g);
+  Choice c;
+  const int rc = find_choice(p, N, H, W, stride, pad, *tile, &c);
   if (rc) return rc;
-  MatGeom m, pool;
-  const bool matrix = choose_matrix(p, N, H, W, stride, pad, tile, g, &m, &pool);
   *supported = activation != TETRIS_ACT_RELU_POOL2 ||
-               (g.OH >= 2 && g.OW >= 2 && (matrix ? m.csplit > 1 || pool.N : g.csplit > 1 || geom_pools_in_kernel(g)));
+               (c.geom.OH >= 2 && c.geom.OW >= 2 &&
+                (c.matrix ? c.mat.csplit > 1 || c.mat_pool.N : c.geom.csplit > 1 || geom_pools_in_kernel(c.geom)));
   return TETRIS_OK;
 }
 
 int tetris_launch_shape_of(tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile* tile,
                            tetris_launch_shape* out) {
   if (!p || !tile || !out) return fail(TETRIS_EINVAL, "null argument");
-  Geom g;
-  const int rc = make_geom(p, N, H, W, stride, pad, *tile, &g);
+  Choice c;
+  const int rc = find_choice(p, N, H, W, stride, pad, *tile, &c);
   if (rc) return rc;
-  MatGeom m, pool;
-  if (choose_matrix(p, N, H, W, stride, pad, tile, g, &m, &pool)) {
+  const Geom& g = c.geom;
+  const MatGeom& m = c.mat;
+  if (c.matrix) {
     *out = {m.ptiles * m.mtiles * m.csplit, m.ptiles, m.mtiles, m.csplit, m.chunks, 64, 5, mat_lds_bytes(m),
             (int64_t)partial_bytes_of(m)};
     return TETRIS_OK;

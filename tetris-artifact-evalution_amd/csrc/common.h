@@ -191,6 +191,17 @@ constexpr int kMatTasks = 4;        // most blocks of 64 staged pixels x 8 chann
 constexpr int kMatLds = 160 * 1024;
 constexpr long long kMatCopies = 32 << 20;  // most bytes of partial sums of a split layer
 
+// Which kernel runs a layer, and how: decided on the host from shape, tile, options and tables.
+struct Choice {
+  Geom geom{};         // of the walking kernels
+  bool matrix = false; // the matrix kernel runs it instead, as `mat` says (`mat_pool`: where it pools; N = 0: it cannot)
+  MatGeom mat{}, mat_pool{};
+};
+struct Chosen {
+  int key[14];  // as Plan::key, then the options and the state of the loaded tables that it was decided under
+  Choice choice;
+};
+
 // A launch plan: everything run_launch derives from (input shape, tile) for one pack, kept for the next call.
 struct Plan {
   int key[12];  // N, H, W, stride, pad, lanes_w, quads, oc_per_wave, waves, tile_ic, csplit, walk (see find_plan)
@@ -227,6 +238,7 @@ struct tetris_g950 {
   int32_t* d_zero_pair = nullptr;  // [groups*stages] zeros: the pair counts of the unpaired arrangement
   int64_t n_paired_entries = 0;
   std::vector<tetris::Plan> plans;  // few per pack; searched linearly, most recent first
+  std::vector<tetris::Chosen> chosen;  // decisions, for plans and queries to come; likewise
   // partial sums of layers whose channel reduction is split over workgroups: [csplit][N][K][OH][OW], one buffer per
   // stream the pack is launched on, made by tetris_g950_prepare or by the first such launch; a buffer that had to
   // grow is kept (`retired`) until the pack is destroyed, because a captured graph may still hold its address
@@ -286,6 +298,7 @@ int make_geom(const tetris_g950* p, int N, int H, int W, int stride, int pad, co
 int choose_tile(int N, int H, int W, int C, int K, int ks, int stride, int pad, tetris_tile* t, bool* loaded = nullptr);
 // reads rows in the format of tuned_tiles.inc; choose_tile looks them up before the built-in table
 int load_tile_table(const char* path, int* rows_out);
+unsigned loaded_tables();  // how many were loaded so far
 // every tile shape the kernel can run for the layer, cheapest first by the selector's time model
 // (density: fraction of non-zero weights when the caller knows the filter, else 0)
 int rank_tiles(int N, int H, int W, int C, int K, int ks, int stride, int pad, std::vector<tetris_tile>* ranked,
@@ -312,7 +325,10 @@ int launch_conv(const Geom& g, const float* d_in, float* d_out, float* d_scratch
 int add_copies(const float* d_copies, float* d_out, int N, int K, int OH, int OW, int slices, int act, hipStream_t stream);
 
 // matrix_conv.hip
-bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out);
+// staged (may be null): of the same layer, what earlier calls found (zeros: nothing yet)
+using StagedPixels = std::array<int, 2>;  // of the largest tile of 64 and of 128 pixels
+bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out,
+                   StagedPixels* staged = nullptr);
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      MatGeom* g, MatGeom* pool);
 int mat_lds_bytes(const MatGeom& g);

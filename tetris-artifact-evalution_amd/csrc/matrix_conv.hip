@@ -365,7 +365,8 @@ int staged_pixels(const MatGeom& g, int P) {
 }  // namespace
 
 // Cuts a layer into workgroups of configuration `cfg` with `csplit` slices of the channels; false: it cannot be run so.
-bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out) {
+bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out,
+                   StagedPixels* staged) {
   MatGeom g{};
   if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || K <= 0 || cfg < 0 || cfg >= kMatConfigs || csplit < 1 || csplit > kMaxSplit) return false;
   g.N = N; g.C = C; g.H = H; g.W = W; g.K = K; g.ks = ks; g.pad = pad;
@@ -403,7 +404,10 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
   const int P = 32 * c.nb * (4 / c.wm);
   g.ptiles = ceil_div(g.npix, P);
   g.mtiles = ceil_div(g.mblocks, c.wm);
-  g.lpad = ceil_div(staged_pixels(g, P), 64) * 64;
+  StagedPixels one{};
+  int& most = (staged ? *staged : one)[P / 128];  // tiles are of 64 or 128 pixels
+  if (!most) most = staged_pixels(g, P);
+  g.lpad = ceil_div(most, 64) * 64;
   if (g.kgs * g.lpad / 64 > 4 * kMatTasks || lds_bytes(g) > kMatLds) return false;
   if ((long long)g.ptiles * g.mtiles * csplit >= (1ll << 28)) return false;
   // multiply-high divisions: dividend * divisor below 2^32
@@ -474,10 +478,11 @@ bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int 
   if (C < 16) return false;  // most of a chunk of 16 channels would be padding
   const bool pools = walk.OH >= 2 && walk.OW >= 2 && (walk.csplit > 1 || geom_pools_in_kernel(walk));
   std::vector<std::pair<double, MatGeom>> found;
+  StagedPixels staged{};
   const double limit = 0.93 * walk_time(walk, nnz);
   for (int cfg = 0; cfg < kMatConfigs; ++cfg) {
     MatGeom m;
-    if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, 1, false, &m)) continue;
+    if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, 1, false, &m, &staged)) continue;
     for (const int slices : {1, 2, 3, 4, 6, 8}) {
       if (slices > m.chunks || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
       m.csplit = slices;

@@ -464,6 +464,7 @@ const Tuned kTuned[] = {
 // Rows a caller loaded at run time (tetris_tile_table_load); they are looked up before the built-in ones.
 std::mutex g_loaded_mu;
 std::vector<Tuned> g_loaded;
+std::atomic<unsigned> g_tables{0};
 
 // trust a table row only as far as the kernel's own checks go
 bool usable(const Tuned& e) {
@@ -480,6 +481,8 @@ bool same_shape(const Tuned& e, int N, int H, int W, int C, int K, int ks, int s
   return e.N == N && e.H == H && e.W == W && e.C == C && e.K == K && e.ks == ks && e.stride == stride && e.pad == pad;
 }
 }  // namespace
+
+unsigned loaded_tables() { return g_tables.load(); }
 
 int load_tile_table(const char* path, int* rows_out) {
   FILE* fp = std::fopen(path, "r");
@@ -498,6 +501,7 @@ int load_tile_table(const char* path, int* rows_out) {
   std::fclose(fp);
   std::lock_guard<std::mutex> lock(g_loaded_mu);
   g_loaded.insert(g_loaded.begin(), rows.begin(), rows.end());
+  g_tables.fetch_add(1);
   if (rows_out) *rows_out = (int)rows.size();
   return TETRIS_OK;
 }
