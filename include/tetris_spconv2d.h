@@ -269,9 +269,11 @@ int tetris_g950_prepare(tetris_g950* p, int batch, int img_h, int img_w, int str
  * must exist already (tetris_g950_prepare or an earlier tetris_spconv2d_launch with the same shape and tile, else
  * TETRIS_ENOTFOUND), and the partial sums of a split layer go to a static device array of
  * TETRIS_NOALLOC_SCRATCH_BYTES that every GPU the library runs on holds until the process ends (64 KiB of it are the
- * split layers' tickets).  A layer whose partial sums need more is refused with TETRIS_EINVAL.  All calls on one GPU share that array: calls that overlap in
+ * split layers' tickets).  A layer whose partial sums need more is refused with TETRIS_EINVAL; one that the matrix cores
+ * would run in slices, after tetris_g950_prepare, only where the walking kernel's sums do not fit either (it then runs
+ * the layer, whose sums are added in another order: the one case in which the bits differ from a launch's).  All calls on one GPU share that array: calls that overlap in
  * time on one GPU (different streams or threads) race; calls on one stream are ordered by the stream.  Results are
- * bit-identical to tetris_spconv2d_launch's. */
+ * otherwise bit-identical to tetris_spconv2d_launch's. */
 #define TETRIS_NOALLOC_SCRATCH_BYTES (64u << 20)
 int tetris_spconv2d_launch_noalloc(tetris_g950* p, const float* d_input, float* d_output, int batch, int img_h,
                                    int img_w, int stride, int padding, const tetris_tile* tile, void* stream);

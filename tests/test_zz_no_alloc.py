@@ -89,3 +89,36 @@ def test_noalloc_covers_a_split_layer_and_refuses_what_does_not_fit(env):
         assert T.noalloc_scratch_limit(0) == 64 << 20
     assert conv(T, torch, pk, x, K, tile, True).tobytes() == got.tobytes()
     pk.close()
+
+
+def test_noalloc_under_a_limit_that_only_the_walking_kernel_meets(env):
+    """A layer that the matrix cores run in slices, whose walking kernel needs no scratch, runs under any limit."""
+    T, torch, O = env
+    N, C, H, W, K, ks = 5, 163, 41, 54, 81, 3
+    rng = np.random.default_rng(33)
+    w, x = sparse_filter(rng, K, C, ks, 0.7), relu_like(rng, (N, C, H, W))
+    tile = T.tile_select(N, H, W, C, K, ks, 1, 1)
+    pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+    shape = pk.launch_shape(N, H, W, 1, 1, tile)
+    assert shape.kernel == 5 and shape.csplit > 1
+    pk.prepare(N, H, W, 1, 1, tile)
+    dx = torch.from_numpy(x).cuda()
+
+    def run(fn):
+        y = torch.full((N, K, H, W), float("nan"), device="cuda")
+        fn(dx.data_ptr(), y.data_ptr(), N, H, W, 1, 1, tile)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    matrix = run(pk.launch)
+    assert run(pk.launch_noalloc).tobytes() == matrix.tobytes()
+    try:
+        T.noalloc_scratch_limit(4096)
+        walk = run(pk.launch_noalloc)
+        assert run(pk.launch).tobytes() == matrix.tobytes()
+    finally:
+        T.noalloc_scratch_limit(0)
+    assert run(pk.launch_noalloc).tobytes() == matrix.tobytes()
+    ref = O.host_conv2d(x, w, 1, 1, threads=8)
+    assert walk.tobytes() != matrix.tobytes() and max_rel_err(walk, ref) <= 1e-4 and max_rel_err(matrix, ref) <= 1e-4
+    pk.close()

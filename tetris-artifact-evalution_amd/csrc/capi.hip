@@ -988,6 +988,13 @@ int tetris_g950_prepare(tetris_g950* p, int N, int H, int W, int stride, int pad
   size_t bytes = 0;
   rc = plan_scratch(p, plan, stream, &d_partial, &bytes);
   if (rc) return rc;
+  // The walking kernel's plan as well where it needs less scratch: tetris_spconv2d_launch_noalloc takes it when the matrix
+  // kernel's slices do not fit under tetris_noalloc_scratch_limit.
+  if (plan.parts && partial_bytes_of(plan.mat) > partial_bytes_of(plan.geom)) {
+    Plan walk;
+    rc = find_plan(p, N, H, W, stride, pad, tile, stream, true, true, &walk);
+    if (rc) return rc;
+  }
   float* s = nullptr;
   return static_scratch(&s);  // looks the static scratch array of this GPU up, for tetris_spconv2d_launch_noalloc
 }
@@ -1016,10 +1023,14 @@ int tetris_spconv2d_launch_noalloc(tetris_g950* p, const float* d_in, float* d_o
   Plan plan;
   int rc = find_plan(p, N, H, W, stride, pad, tile, stream, false, false, &plan);
   if (rc) return rc;
+  const size_t limit = g_scratch_limit.load();
+  Plan walk;
+  if (plan.parts && partial_bytes_of(plan.mat) > limit && partial_bytes_of(plan.geom) <= limit &&
+      find_plan(p, N, H, W, stride, pad, tile, stream, false, true, &walk) == TETRIS_OK)
+    plan = walk;
   float* d_partial = nullptr;
   if (slices_of(plan) > 1) {
     const size_t need = plan.parts ? partial_bytes_of(plan.mat) : partial_bytes_of(plan.geom);
-    const size_t limit = g_scratch_limit.load();
     if (need > limit)
       return fail(TETRIS_EINVAL, "this layer needs %zu bytes of tickets and partial sums, the static scratch holds %zu: "
                   "use tetris_spconv2d_launch", need, limit);
@@ -1028,7 +1039,7 @@ int tetris_spconv2d_launch_noalloc(tetris_g950* p, const float* d_in, float* d_o
   }
   // Every element of the partial sums that are added is written by this launch's conv kernel first, so
   // what an earlier call left in the array needs no clearing.
-  return launch_plan(plan, d_in, d_out, d_partial, g_scratch_limit.load(), p->d_oc_order, 0, stream);
+  return launch_plan(plan, d_in, d_out, d_partial, limit, p->d_oc_order, 0, stream);
 }
 
 int tetris_spconv2d_launch_spf_arrays(const float* d_in, const int32_t* d_offsets, const int32_t* d_stage_len,
