@@ -64,16 +64,18 @@ def test_parts_keep_every_bit():
     N, C, H, K = 2, 64, 20, 96
     rng = np.random.default_rng(4)
     w = np.zeros((K, C, 1, 1), np.float32)
-    w[np.arange(K), np.arange(K) % C] = 1.0
-    x = (rng.standard_normal((N, C, H, H)) * np.exp2(rng.integers(-60, 60, (N, C, H, H)))).astype(np.float32)
-    w[:, :, 0, 0] += (rng.random((K, C)) < 0.4) * np.float32(2.0 ** -149)  # dense enough; below every product that is kept
+    w[np.arange(K), np.arange(K) % 48] = 1.0
+    w[:, 48:] = sparse_filter(rng, K, 16, 1, 0.2, False)  # dense enough for the matrix cores, and x is zero there
+    x = (rng.standard_normal((N, C, H, H)) * np.exp2(rng.integers(-145, 125, (N, C, H, H)))).astype(np.float32)
+    x[:, 48:] = 0
     tile = T.tile_select(N, H, H, C, K, 1, 1, 0)
     pk = T.G950Filter.for_tile(w, tile)
     assert pk.launch_shape(N, H, H, 1, 0, tile).kernel == 5
-    dx, y = torch.from_numpy(x).cuda(), torch.empty((N, K, H, H), device="cuda")
-    pk.launch(dx.data_ptr(), y.data_ptr(), N, H, H, 1, 0, tile)
-    torch.cuda.synchronize()
-    assert np.array_equal(y.cpu().numpy(), x[:, np.arange(K) % C])
+    for each in (x, np.clip(x, -2.0 ** 60, 2.0 ** 60)):  # with numbers whose tiles are computed again, and without
+        dx, y = torch.from_numpy(each).cuda(), torch.empty((N, K, H, H), device="cuda")
+        pk.launch(dx.data_ptr(), y.data_ptr(), N, H, H, 1, 0, tile)
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy(), each[:, np.arange(K) % 48])
     pk.close()
 
 
@@ -151,3 +153,85 @@ def test_queries_tell_what_launches_run(C, matrix, oracle):
         T.options_set(options)
     assert max_rel_err(out, oracle.host_conv2d(x, w, 1, 1, threads=8)) <= 1e-4
     pk.close()
+
+
+def conv64(x, w, stride, pad, terms=False):
+    """float64 on the CPU; with `terms`: also the sum of the terms' magnitudes, which bounds what any order of sums can lose"""
+    import torch
+
+    f = lambda a, b: torch.nn.functional.conv2d(torch.from_numpy(a).double(), torch.from_numpy(b).double(),  # noqa: E731
+                                                stride=stride, padding=pad).numpy()
+    return (f(x, w), f(np.abs(x), np.abs(w))) if terms else f(x, w)
+
+
+def run_both(w, x, stride, pad, act=0):
+    """The layer as the library runs it, on the matrix cores, and on a walking tile of the same pack"""
+    import torch
+    import tetris_amd as T
+
+    N, C, H, W = x.shape
+    K, _, ks, _ = w.shape
+    tile = T.tile_select(N, H, W, C, K, ks, stride, pad)
+    pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+    assert pk.launch_shape(N, H, W, stride, pad, tile).kernel == 5
+    other = T.Tile(tile.lanes_w, tile.quads, tile.oc_per_wave, tile.waves, tile.tile_ic, 1 if tile.csplit != 1 else 0)
+    dx, outs = torch.from_numpy(x).cuda(), []
+    for t in (tile, other):
+        y = torch.full((N, K, T.out_extent(H, pad, ks, stride), T.out_extent(W, pad, ks, stride)), float("nan"), device="cuda")
+        pk.launch_act(dx.data_ptr(), y.data_ptr(), N, H, W, stride, pad, t, act)
+        torch.cuda.synchronize()
+        outs.append(y.cpu().numpy())
+    pk.close()
+    return outs
+
+
+RANGE_LAYERS = [
+    (6, 25, 55, 77, 72, 1, 1, 0), (5, 163, 41, 54, 81, 3, 1, 1), (2, 23, 67, 45, 161, 5, 1, 2), (3, 38, 53, 25, 279, 2, 1, 1),
+    (2, 16, 38, 137, 11, 3, 2, 1), (1, 194, 46, 8, 10, 3, 1, 1), (4, 17, 5, 7, 40, 1, 2, 0), (3, 28, 7, 47, 5, 1, 1, 0)]
+
+
+@pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad", RANGE_LAYERS)
+def test_values_out_of_range_give_what_the_walk_gives(N, C, H, W, K, ks, stride, pad):
+    """Infinities, NaN, the largest numbers and sums that overflow, a few among ordinary values: they reach the outputs
+    whose window holds them with a weight that is not zero, and no others."""
+    rng = np.random.default_rng(C * K)
+    w, x = sparse_filter(rng, K, C, ks, 0.7), relu_like(rng, (N, C, H, W)) - np.float32(0.25)
+    odd = np.array([np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 2.0 ** 100, -2.0 ** 90, 1e-45], np.float32)
+    at = rng.permutation(x.size)[:48]
+    x.reshape(-1)[at] = np.tile(odd, 6)
+    for act in (0, 1):
+        with np.errstate(all="ignore"):
+            matrix, walk = run_both(w, x, stride, pad, act)
+            assert np.array_equal(np.isnan(matrix), np.isnan(walk)) and np.array_equal(np.isinf(matrix), np.isinf(walk))
+            assert act or (np.isnan(walk).any() and np.isinf(walk).any())
+            ok = np.isfinite(walk)
+            assert np.array_equal(np.sign(matrix[~ok]), np.sign(walk[~ok]), equal_nan=True)
+            tame = np.where(np.isfinite(x), x, 0)
+            _, terms = conv64(tame, w, stride, pad, True)
+            n = C * ks * ks
+            assert (np.abs(matrix[ok].astype(np.float64) - walk[ok]) <= 2 * n * 2.0 ** -24 * terms[ok]).all()
+
+
+def test_weights_out_of_range_stay_with_the_walk(oracle):
+    import torch
+    import tetris_amd as T
+
+    N, C, H, K = 2, 64, 20, 96
+    for value, kernel5 in [(1.0, True), (2.0 ** 63, True), (2.0 ** -149, True), (2.0 ** 64, False), (np.inf, False), (np.nan, False)]:
+        rng = np.random.default_rng(6)
+        w, x = sparse_filter(rng, K, C, 1, 0.6), relu_like(rng, (N, C, H, H))
+        w[5, 7] = value
+        tile = T.tile_select(N, H, H, C, K, 1, 1, 0)
+        pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+        assert (pk.launch_shape(N, H, H, 1, 0, tile).kernel == 5) == kernel5, value
+        assert pk.host_arrays()["nnz"] == int((w != 0).sum())
+        dx, y = torch.from_numpy(x).cuda(), torch.empty((N, K, H, H), device="cuda")
+        pk.launch(dx.data_ptr(), y.data_ptr(), N, H, H, 1, 0, tile)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        if np.isfinite(value):
+            ref, terms = conv64(x, w, 1, 0, True)
+            assert (np.abs(got - ref) <= C * 2.0 ** -24 * terms).all(), value
+        else:
+            assert np.isfinite(np.delete(got, 5, 1)).all()
+        pk.close()

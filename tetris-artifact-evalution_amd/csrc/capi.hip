@@ -46,6 +46,7 @@ int upload(const std::vector<T>& v, T** d) {
 // tile that was measured, where this is a prediction) and an option that picks a form of the walking kernels.
 bool choose_matrix(const tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile* tile, const Geom& walk,
                    MatGeom* g, MatGeom* pool) {
+  if (p->huge) return false;
   if (options() & (TETRIS_OPT_PAIRS | TETRIS_OPT_NO_BANK_RULE | TETRIS_OPT_ADD_IN_KERNEL)) return false;
   tetris_tile own{};
   bool loaded = false;

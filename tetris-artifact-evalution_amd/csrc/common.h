@@ -221,6 +221,7 @@ struct tetris_g950 {
   int slots = 0;            // K rounded up to a multiple of kSlotPad
   int groups = 0;           // slots / g
   int64_t n_entries = 0, nnz = 0;
+  bool huge = false;        // a weight of 2^64 or more, or not finite: the matrix kernel does not take it
   // two allocations: grp_off, grp_nnz and oc_order; position and values
   int32_t* d_grp_off = nullptr;   // [groups*stages+1] entry index, multiples of 8; then the number of non-zeros
   int32_t* d_grp_nnz = nullptr;   // [groups*stages]

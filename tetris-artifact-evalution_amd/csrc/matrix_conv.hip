@@ -22,8 +22,11 @@
 // products at 2.1 GHz, where the vendor's bf16 GEMM of 8192^3 reaches 1.32; half of the rest is the last, partly filled
 // round of workgroups); on small ones the latency of a round: weights from L2, input from HBM, barrier.
 //
-// Not finite inputs: a zero weight is multiplied here, so an infinity or NaN makes every output NaN whose window holds it,
-// as in a dense convolution; the walking kernels leave those out whose weight is zero.
+// Range: parts are made of numbers scaled by 2^32, inputs and weights, so that the lowest bit of every fp32 number, subnormal
+// ones too, is a normal bf16 number's, and sums are scaled back as they are stored.  What is out of that range upwards
+// (an infinity, NaN, an input of 2^96 or more, a sum of 2^64 or more) makes every sum that it enters infinite or NaN,
+// whatever the weight: a wave that finds such a sum computes its tile once more as the walking kernels do, with FMAs on
+// the non-zero weights, in their order.  Packs with weights of 2^64 or more, or not finite, stay with those kernels.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -41,11 +44,13 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kOutside = 0x7ff00000;  // a byte offset beyond every tensor this path takes (1 GiB): loads give 0, stores are dropped
 
-// three bf16 parts of eight floats
+constexpr float kScale = 0x1p32f, kUnscale = 0x1p-64f;
+
+// three bf16 parts of eight floats, scaled
 __device__ __forceinline__ void cut(const float (&x)[8], u32x4& hi, u32x4& mid, u32x4& lo) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const f32x2 v = {x[2 * i], x[2 * i + 1]};
+    const f32x2 v = {x[2 * i] * kScale, x[2 * i + 1] * kScale};
     const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
     const float r0 = v.x - __builtin_bit_cast(float, h << 16), r1 = v.y - __builtin_bit_cast(float, h & 0xffff0000u);
     const unsigned m = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
@@ -155,27 +160,36 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
 
   if (c_beg < c_end) fetch(c_beg);
 
-  // where this lane's pixels lie: in LDS and in the output
+  // where this lane's pixels lie: in the output's images, in LDS and in the output
+  struct Pixel { bool in_range; int t; unsigned n, dq, uy, oy, ox, w; };  // ox: in its strip, w: in its image
+  auto pixel = [&](int b, int lane) {
+    Pixel p;
+    const int t = (wn * NB + b) * 32 + (lane & 31);
+    p.in_range = pt * P + t < g.npix;
+    p.t = p.in_range ? t : g.npix - 1 - pt * P;
+    const unsigned x = ox0 + (p.t >> psh);
+    const unsigned dy = __umulhi(x, g.m_uw), ux = g.uw == 1 ? 0 : x - dy * g.uw;
+    const unsigned y = oy0 + (g.uw == 1 ? x : dy);
+    p.dq = g.uh == 1 ? y : __umulhi(y, g.m_uh);
+    p.uy = y - p.dq * g.uh;
+    p.oy = (p.uy << dbl) + (g.pool ? (p.t >> 1) & 1 : 0);
+    p.ox = (ux << dbl) + (g.pool ? p.t & 1 : 0);
+    const unsigned q = q0 + p.dq;
+    p.n = g.strips == 1 ? q : __umulhi(q, g.m_strips);
+    p.w = (q - p.n * g.strips) * g.ws + p.ox;
+    return p;
+  };
   int bpos[NB], ooff[NB];
   const int ohw = g.pool ? (g.OH >> 1) * (g.OW >> 1) : g.OH * g.OW;
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const int t = (wn * NB + b) * 32 + (lane & 31);
-    const bool in_range = pt * P + t < g.npix;
-    const int tt = in_range ? t : g.npix - 1 - pt * P;
-    const unsigned x = ox0 + (tt >> psh);
-    const unsigned dy = __umulhi(x, g.m_uw), ux = g.uw == 1 ? 0 : x - dy * g.uw;
-    const unsigned y = oy0 + (g.uw == 1 ? x : dy);
-    const unsigned dq = g.uh == 1 ? y : __umulhi(y, g.m_uh), uy = y - dq * g.uh;
-    const unsigned oy = (uy << dbl) + (g.pool ? (tt >> 1) & 1 : 0), ox = (ux << dbl) + (g.pool ? tt & 1 : 0);
-    bpos[b] = ((int)(dq * g.ihs + oy * g.stride) - row0) * g.wp + (int)ox * g.stride - col0 + (lane >> 5) * 3 * g.lpad;
-    const unsigned q = q0 + dq, n = g.strips == 1 ? q : __umulhi(q, g.m_strips), strip = q - n * g.strips;
-    const unsigned w = strip * g.ws + ox;
+    const Pixel p = pixel(b, lane);
+    bpos[b] = ((int)(p.dq * g.ihs + p.oy * g.stride) - row0) * g.wp + (int)p.ox * g.stride - col0 + (lane >> 5) * 3 * g.lpad;
     if (g.pool)
-      ooff[b] = in_range && (tt & 3) == 0 && (w >> 1) < (unsigned)(g.OW >> 1)
-                    ? 4 * (int)((n * g.K + 4 * (lane >> 5)) * ohw + uy * (g.OW >> 1) + (w >> 1)) : kOutside;
+      ooff[b] = p.in_range && (p.t & 3) == 0 && (p.w >> 1) < (unsigned)(g.OW >> 1)
+                    ? 4 * (int)((p.n * g.K + 4 * (lane >> 5)) * ohw + p.uy * (g.OW >> 1) + (p.w >> 1)) : kOutside;
     else
-      ooff[b] = in_range && w < (unsigned)g.OW ? 4 * (int)((n * g.K + 4 * (lane >> 5)) * ohw + oy * g.OW + w) : kOutside;
+      ooff[b] = p.in_range && p.w < (unsigned)g.OW ? 4 * (int)((p.n * g.K + 4 * (lane >> 5)) * ohw + p.oy * g.OW + p.w) : kOutside;
   }
 
   // The products of the leading parts and the five small ones are summed apart: a sum of its own is rounded once per 16
@@ -259,11 +273,16 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
     if (oc + 4 * (lane >> 5) < g.K && ooff[b] != kOutside)
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), orsrc, ooff[b], oc * ohw * 4, 0);
   };
+  float odd = 0;  // NaN once a sum is infinite or NaN
+  auto finish = [&](int i, int b, float v) {
+    odd = fmaf(v, 0.f, odd);
+    store(i, b, v * kUnscale);
+  };
   if constexpr (KW == 1) {
 #pragma unroll
     for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) store(i, b, acc[b][i] + low[b][i]);
+      for (int b = 0; b < NB; ++b) finish(i, b, acc[b][i] + low[b][i]);
   } else {
     // every team leaves its sums in LDS and adds a share of all of them
     float* sums = reinterpret_cast<float*>(all_lds) + wave * 1024 * NB + lane;
@@ -280,8 +299,42 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
         float v = sums[(i * NB + b) * 64];
 #pragma unroll
         for (int k = 1; k < KW; ++k) v += sums[k * 4096 * NB + (i * NB + b) * 64];
-        store(i, b, v);
+        finish(i, b, v);
       }
+    }
+  }
+  if (__ballot(odd != 0.f) == 0) return;
+  // Out of range: the wave's sums once more, over what was stored.  (A lane's stores to one address keep their order.)
+  int again = lane;  // (unknown to the compiler, which would else keep the pixels' places in registers all the while)
+  asm("" : "+v"(again));
+  const int ch0 = slice * g.chunks / g.csplit * 8 * g.kgs, ch1 = min(g.C, (slice + 1) * g.chunks / g.csplit * 8 * g.kgs);
+  const unsigned short* rows = reinterpret_cast<const unsigned short*>(weights + (size_t)min(mt * WM + wm, g.mblocks - 1) * g.steps * 192);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const Pixel p = pixel(b, again);
+#pragma nounroll
+    for (int i = team * (16 / KW); i < (team + 1) * (16 / KW); ++i) {
+      const int row = 8 * (i / 4) + 4 * (lane >> 5) + i % 4;
+      float sum = 0;
+#pragma nounroll
+      for (int c = ch0; c < ch1; ++c) {
+        const int kg = c >> 3, chunk = kg / g.kgs, k = kg - chunk * g.kgs;
+#pragma nounroll
+        for (int r = 0; r < g.ks; ++r)
+#pragma nounroll
+          for (int s = 0; s < g.ks; ++s) {
+            const int step = (chunk * g.ks * g.ks + r * g.ks + s) * halves + (k >> 1);
+            const unsigned short* d = rows + ((size_t)step * 192 + (k & 1) * 32 + row) * 8 + (c & 7);
+            const float w = __builtin_bit_cast(float, (unsigned)d[0] << 16) + __builtin_bit_cast(float, (unsigned)d[512] << 16) +
+                            __builtin_bit_cast(float, (unsigned)d[1024] << 16);
+            const int iy = (int)(p.oy * g.stride + r) * g.sub - g.pad, ix = (int)(p.w * g.stride + s) * g.sub - g.pad;
+            const bool inside = iy >= 0 && iy < g.H && ix >= 0 && ix < g.W && p.n < (unsigned)g.N;
+            const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                irsrc, inside ? 4 * (int)(((p.n * g.C + c) * g.H + iy) * g.W + ix) : kOutside, 0, 0));
+            if (w != 0.f) sum = fmaf(v, w * (1 / kScale), sum);
+          }
+      }
+      store(i, b, sum);
     }
   }
 }

@@ -30,19 +30,26 @@ __global__ __launch_bounds__(256) void count_kernel(const float* __restrict__ fi
   const int c0 = st * tile_ic;
   const int n = min(tile_ic, C - c0) * kk * G;
   int cnt = 0;
+  bool huge = false;
   for (int i = lane; i < n; i += 64) {
     const int p = i / G, l = i - p * G;
     const int oc = oc_order[grp * G + l];
-    if (oc >= 0) cnt += (filter[((size_t)oc * C + c0) * kk + p] != 0.f) ? 1 : 0;
+    if (oc >= 0) {
+      const float w = filter[((size_t)oc * C + c0) * kk + p];
+      cnt += (w != 0.f) ? 1 : 0;
+      huge |= !(fabsf(w) < 0x1p64f);
+    }
   }
+  huge = __ballot(huge) != 0;
   for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
   if (lane == 0) {
     grp_nnz[sid] = cnt;
-    grp_pad[sid] = (cnt + kBatch - 1) / kBatch * kBatch;
+    grp_pad[sid] = (cnt + kBatch - 1) / kBatch * kBatch | (huge ? 1 : 0);
   }
 }
 
-// exclusive scan of grp_pad into grp_off[0..n], single workgroup; nnz != nullptr: grp_off[n + 1] = the sum of nnz[0..n)
+// exclusive scan of grp_pad (multiples of kBatch, and a flag in bit 0) into grp_off[0..n], single workgroup; nnz != nullptr:
+// grp_off[n + 1] = the sum of nnz[0..n), with bit 31 set where any flag is
 __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ grp_pad, int32_t* __restrict__ grp_off,
                                                     int n, const int32_t* __restrict__ nnz = nullptr) {
   __shared__ int part[1024];
@@ -50,7 +57,7 @@ __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ 
   const int chunk = (n + 1023) / 1024;
   const int b = min(n, tid * chunk), e = min(n, b + chunk);
   int s = 0;
-  for (int i = b; i < e; ++i) s += grp_pad[i];
+  for (int i = b; i < e; ++i) s += grp_pad[i] & -kBatch;
   part[tid] = s;
   __syncthreads();
   for (int off = 1; off < 1024; off <<= 1) {
@@ -62,20 +69,24 @@ __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ 
   int run = tid ? part[tid - 1] : 0;
   for (int i = b; i < e; ++i) {
     grp_off[i] = run;
-    run += grp_pad[i];
+    run += grp_pad[i] & -kBatch;
   }
   if (tid == 1023) grp_off[n] = part[1023];
   if (!nnz) return;
   s = 0;
-  for (int i = tid; i < n; i += 1024) s += nnz[i];
+  int flag = 0;
+  for (int i = tid; i < n; i += 1024) {
+    s += nnz[i];
+    flag |= grp_pad[i] & 1;
+  }
+  flag = __syncthreads_or(flag);  // part has been read
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  __syncthreads();  // part has been read
   if ((tid & 63) == 0) part[tid >> 6] = s;
   __syncthreads();
   if (tid == 0) {
     s = 0;
     for (int i = 0; i < 16; ++i) s += part[i];
-    grp_off[n + 1] = s;
+    grp_off[n + 1] = flag ? (int)(s | 0x80000000u) : s;
   }
 }
 
@@ -184,11 +195,12 @@ int pack_device(const float* d_filter, int C, int K, int ks, int tile_ic, int G,
                      ks, tile_ic, p->stages, G, nseg);
   hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, stream, d_pad, p->d_grp_off, nseg, p->d_grp_nnz);
   HIPC(hipGetLastError());
-  int32_t total[2] = {0, 0};  // entries, non-zeros
+  int32_t total[2] = {0, 0};  // entries; non-zeros and whether a weight is huge
   HIPC(hipMemcpyAsync(total, p->d_grp_off + nseg, sizeof total, hipMemcpyDeviceToHost, stream));
   HIPC(hipStreamSynchronize(stream));
   p->n_entries = total[0];
-  p->nnz = total[1];
+  p->nnz = total[1] & 0x7fffffff;
+  p->huge = total[1] < 0;
   // one spare batch so that a kernel may prefetch the batch after the last one
   const size_t room = (size_t)total[0] + kBatch;
   HIPC(hipMalloc(&p->d_position, 2 * sizeof(int32_t) * room));
