@@ -212,6 +212,27 @@ def test_values_out_of_range_give_what_the_walk_gives(N, C, H, W, K, ks, stride,
             assert (np.abs(matrix[ok].astype(np.float64) - walk[ok]) <= 2 * n * 2.0 ** -24 * terms[ok]).all()
 
 
+@pytest.mark.parametrize("scale_x,scale_w", [(-120, 0), (-140, 4), (0, -130), (-70, -60), (40, 20), (80, -100), (120, -10)])
+def test_precision_at_any_scale(scale_x, scale_w):
+    """Outputs of one term each, inputs and weights of full 24-bit significands at either end of fp32's exponents: as exact
+    as one rounding of the product, and to the last bit of a subnormal one."""
+    N, C, H, K = 2, 64, 20, 96
+    rng = np.random.default_rng(5)
+    w = np.zeros((K, C, 1, 1), np.float32)
+    w[:, 48:] = sparse_filter(rng, K, 16, 1, 0.2, False)  # dense enough for the matrix cores, and x is zero there
+    w[np.arange(K), np.arange(K) % 48, 0, 0] = np.ldexp(1 + rng.random(K, dtype=np.float32), scale_w)
+    x = np.zeros((N, C, H, H), np.float32)
+    x[:, :48] = np.ldexp((1 + rng.random((N, 48, H, H))).astype(np.float32), scale_x)
+    matrix, walk = run_both(w, x, 1, 0)
+    ref = conv64(x, w, 1, 0)
+    # half a unit in the last place; for the matrix cores also the rounding of the smaller products' sum, which is 2^-8 of
+    # the product, and of a subnormal output first that of the scaled sum and then its own
+    normal = np.abs(ref) >= 2.0 ** -126
+    half = np.where(normal, np.abs(ref) * 2.0 ** -24, 2.0 ** -150)
+    assert (np.abs(walk - ref) <= half * 1.0001).all()
+    assert (np.abs(matrix - ref) <= half * (1 + 2.0 ** -5) + np.where(normal, 0, np.abs(ref) * 2.0 ** -24)).all()
+
+
 def test_weights_out_of_range_stay_with_the_walk(oracle):
     import torch
     import tetris_amd as T

@@ -3,11 +3,11 @@
 //
 // A vector FMA with a scalar weight does 16 multiply-adds a cycle and SIMD and the walk reaches two thirds of that, on the
 // non-zeros only.  The matrix cores do 512 a cycle and SIMD in bf16.  An fp32 number is the sum of three bf16 numbers,
-// exactly (8 + 8 + 8 bits of significand, each part rounded to nearest, so that the next one is at most 2^-9 of it), and
-// of the nine products of two such sums the six with weight 2^-18 or more are formed here; the other three are below
-// 2^-26 of the product, a quarter of what rounding it to fp32 costs.  Sums stay in fp32.  That is 85 fp32 multiply-adds a cycle
-// and SIMD on ALL weights, zeros included: ahead of the walk up to some 85 % of zeros on large layers, and everywhere
-// where the walk's stages are too short to fill its waves.
+// exactly (8 + 8 + 8 bits of significand, each part rounded to nearest: the second is at most 2^-8 of the first, the
+// third 2^-17), and of the nine products of two such sums all but the last, low times low, are formed here: that one is
+// 2^-34 of the product at most.  (Without mid times low and low times mid, up to 2^-25 each, an output of one term was
+// off by up to 8.6e-8 of itself where one rounding to fp32 is off by 6.0e-8.)  Sums stay in fp32.  That is 64 fp32
+// multiply-adds a cycle and SIMD on ALL weights, zeros included.
 //
 // Workgroup: KW teams of four waves on one tile of 32*WM output channels x P = 32*NB*(4/WM) output pixels.  The input of P
 // pixels (with its halo) of 8*kgs channels at a time is read from the NCHW image, cut into its three parts once, and
@@ -192,8 +192,8 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
       ooff[b] = p.in_range && p.w < (unsigned)g.OW ? 4 * (int)((p.n * g.K + 4 * (lane >> 5)) * ohw + p.oy * g.OW + p.w) : kOutside;
   }
 
-  // The products of the leading parts and the five small ones are summed apart: a sum of its own is rounded once per 16
-  // k-values, not six times, and the small ones are 2^-8 of it.
+  // The products of the leading parts and the seven small ones are summed apart: a sum of its own is rounded once per 16
+  // k-values, not eight times, and the small ones are 2^-8 of it.
   f32x16 acc[NB], low[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -226,8 +226,8 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
           half = 0;
           if (++s == g.ks) { s = 0; ++r; }
         }
-        // the six products, smallest first
-        constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
+        // the eight products, smallest first
+        constexpr int pa[8] = {2, 1, 2, 1, 0, 1, 0, 0}, pb[8] = {1, 2, 0, 1, 2, 0, 1, 0};
         if constexpr (KW < 4) {
           u32x4 v[NB][3];
 #pragma unroll
@@ -235,10 +235,10 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
 #pragma unroll
             for (int p = 0; p < 3; ++p) v[b][p] = src[bpos[b] + p * g.lpad];
 #pragma unroll
-          for (int t = 0; t < 6; ++t)
+          for (int t = 0; t < 8; ++t)
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-              f32x16& sum = t == 5 ? acc[b] : low[b];
+              f32x16& sum = t == 7 ? acc[b] : low[b];
               sum = product(w[pa[t]], v[b][pb[t]], sum);
             }
         } else {
@@ -248,8 +248,8 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
 #pragma unroll
             for (int p = 0; p < 3; ++p) v[p] = src[bpos[b] + p * g.lpad];
 #pragma unroll
-            for (int t = 0; t < 6; ++t) {
-              f32x16& sum = t == 5 ? acc[b] : low[b];
+            for (int t = 0; t < 8; ++t) {
+              f32x16& sum = t == 7 ? acc[b] : low[b];
               sum = product(w[pa[t]], v[pb[t]], sum);
             }
           }
@@ -489,10 +489,10 @@ double matrix_time(const MatGeom& g) {
   const int wgs = g.ptiles * g.mtiles * g.csplit, rounds = ceil_div(ceil_div(g.chunks, g.csplit), c.kw);
   const int steps = g.ks * g.ks * g.kgs / 2, staging = ceil_div(g.kgs * g.lpad, 256);
   // cycles of n workgroups on a CU: start and end; a round's staging and barrier; a step, which waits for its weights or,
-  // with enough waves, for the matrix core (6 * nb products of 32 cycles per team and SIMD)
+  // with enough waves, for the matrix core (8 * nb products of 32 cycles per team and SIMD)
   auto cycles = [&](int n) {
     if (n == 0) return 0.0;
-    const double step = std::max(g.ks == 1 ? 193.0 : 539.0, 1.205 * 192 * c.nb * c.kw * n);
+    const double step = std::max(g.ks == 1 ? 193.0 : 539.0, 1.205 * 256 * c.nb * c.kw * n);
     return 3958.0 + 349.0 * c.nb * n * c.kw + rounds * ((g.ks == 1 ? 1031.0 : 2033.0) + 321.0 * staging * c.kw * n + steps * step);
   };
   const int full = wgs / (256 * fit), rest = wgs % (256 * fit);
