@@ -1167,3 +1167,69 @@ int64_t tetris_tensor_first_mismatch(const float* x, const float* y, int64_t len
 }
 
 }  // extern "C"
+
+#ifdef TETRIS_FIT
+// What tetris_amd/kernel_times.py measures and fits the two time models with.  Only in the library `make fit` builds.
+extern "C" {
+
+// the configuration's geometry (16 numbers, see kernel_times.py) and predicted microseconds; TETRIS_EINVAL: it cannot be run
+int tetris_fit_matrix_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, int* out,
+                           double* predicted) {
+  MatGeom g;
+  if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, csplit, false, &g)) return fail(TETRIS_EINVAL, "not a configuration");
+  if (csplit > 1 && 4ll * g.out_floats * csplit > kMatCopies) return fail(TETRIS_EINVAL, "too many slices");
+  const int v[16] = {g.ptiles, g.mtiles, g.csplit, g.chunks, g.kgs, g.lpad, g.OH, g.OW, mat_lds_bytes(g), g.mblocks, g.steps};
+  std::copy(v, v + 16, out);
+  *predicted = matrix_time(g);
+  return TETRIS_OK;
+}
+
+int tetris_fit_walk_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const tetris_tile* tile, long long nnz,
+                         int* out, double* predicted) {
+  tetris_g950 shape;
+  shape.C = C; shape.K = K; shape.ks = ks; shape.tile_ic = tile->tile_ic; shape.g = tile->oc_per_wave;
+  shape.stages = ceil_div(C, tile->tile_ic);
+  shape.slots = ceil_div(K, kSlotPad) * kSlotPad;
+  Geom g;
+  const int rc = make_geom(&shape, N, H, W, stride, pad, *tile, &g);
+  if (rc) return rc;
+  const bool one = g.waves == 16 || (g.waves == 8 && g.buf_bytes != kHalfBufBytes && g.buf_bytes != kFlatHalfBufBytes);
+  const int v[16] = {g.ugroups, g.kblocks, g.csplit, g.stages, g.waves, g.nq, g.g, g.ver, g.OH, g.OW, one};
+  std::copy(v, v + 16, out);
+  *predicted = walk_time(g, nnz);
+  return TETRIS_OK;
+}
+
+// microseconds of a launch: configuration `cfg` of the matrix kernel, or (cfg < 0) the walking kernel of `tile`
+int tetris_fit_time(tetris_g950* p, const float* d_in, float* d_out, int N, int H, int W, int stride, int pad,
+                    const tetris_tile* tile, int cfg, int csplit, int warm, int repeat, float* us) {
+  Plan plan;
+  float* d_scratch = nullptr;
+  size_t bytes = 0;
+  int rc = TETRIS_OK;
+  if (cfg < 0) {
+    rc = find_plan(p, N, H, W, stride, pad, tile, nullptr, true, true, &plan);
+  } else {
+    if (!make_mat_geom(N, p->C, H, W, p->K, p->ks, stride, pad, cfg, csplit, false, &plan.mat)) return fail(TETRIS_EINVAL, "not a configuration");
+    rc = matrix_weights(p, plan.mat, nullptr, &plan.parts);
+  }
+  if (rc == TETRIS_OK) rc = plan_scratch(p, plan, nullptr, &d_scratch, &bytes);
+  if (rc) return rc;
+  hipEvent_t a, b;
+  TETRIS_HIP(hipEventCreate(&a));
+  TETRIS_HIP(hipEventCreate(&b));
+  for (int i = -warm; i < repeat && rc == TETRIS_OK; ++i) {
+    if (i == 0) TETRIS_HIP(hipEventRecord(a, nullptr));
+    rc = launch_plan(plan, d_in, d_out, d_scratch, bytes, p->d_oc_order, 0, nullptr);
+  }
+  TETRIS_HIP(hipEventRecord(b, nullptr));
+  TETRIS_HIP(hipEventSynchronize(b));
+  TETRIS_HIP(hipEventElapsedTime(us, a, b));
+  *us *= 1e3f / repeat;
+  (void)hipEventDestroy(a);
+  (void)hipEventDestroy(b);
+  return rc;
+}
+
+}  // extern "C"
+#endif

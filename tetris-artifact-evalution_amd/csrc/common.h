@@ -332,6 +332,9 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
                    StagedPixels* staged = nullptr);
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      MatGeom* g, MatGeom* pool);
+// predicted microseconds of a launch
+double matrix_time(const MatGeom& g);
+double walk_time(const Geom& g, long long nnz);
 int mat_lds_bytes(const MatGeom& g);
 size_t mat_weight_bytes(const MatGeom& g);
 int mat_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* dst);

@@ -477,11 +477,12 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
   return true;
 }
 
-namespace {
-
-// Microseconds of a launch, fitted to 10 600 timed launches (325 layers: those of the benchmark's suites at batch 1, 2 and
-// 16, and random ones; every configuration and slice count): 11 % off (standard deviation), and the configuration that it
-// names is 2.7 % slower than the fastest one.
+// Microseconds of a launch.  The constants were fitted to the times of a kernel with six products a step, whose cycles
+// were then scaled by 8/6.  Against 13 469 timed launches of 424 layers -- those of the benchmark's suites at batch 1, 4
+// and 16 and 160 random ones, every configuration and slice count: profiles/kernel_times.txt, measured and checked by
+// tetris_amd/kernel_times.py -- they are 11 % off (standard deviation), and the configuration that they name is 3.1 %
+// slower than the fastest one.  A fit to these times, with a term for the weights' bytes, is 11 % off as well, 2.6 %
+// slower than the fastest, and not faster in any network (VGG19 at batch 1: 408 us, 400 with these).
 double matrix_time(const MatGeom& g) {
   const Config& c = kConfigs[g.cfg];
   const int by_regs = c.nb == 4 ? 2 / c.kw : c.nb == 2 ? std::max(1, 3 / c.kw) : c.kw == 1 ? 5 : c.kw == 2 ? 2 : 1;
@@ -502,8 +503,7 @@ double matrix_time(const MatGeom& g) {
   return 2.2 + std::max(compute, memory) + (g.csplit > 1 ? 2.5 + out * (g.csplit + 1) / 4.07e6 : 0);
 }
 
-// The same for the kernels that walk the non-zeros, fitted to the same layers: 10 % off on the layers of the table of
-// measured tiles, 22 % elsewhere.
+// The same for the kernels that walk the non-zeros: 15 % off.
 double walk_time(const Geom& g, long long nnz) {
   const int family = g.ver - 2;  // one LDS tile, three LDS buffers, flat
   constexpr double start[] = {12362, 12723, 9370}, stage[] = {2346, 5171, 1186}, busy[] = {1.872, 0.955, 1.442}, alone[] = {60.8, 55.6, 60};
@@ -521,11 +521,12 @@ double walk_time(const Geom& g, long long nnz) {
   return std::max(compute, (in + out) / 6.9e6) + (g.csplit > 1 ? 1.5 + out * (g.csplit + 1) / 4.1e6 : 0);
 }
 
-}  // namespace
-
 // Whether the matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and
-// slice count of least predicted time, if that is 7 % below the walking kernel's (about what the two predictions
-// err by).  Where the walking kernel can pool its outputs, so must the matrix kernel.
+// slice count of least predicted time, if that is 7 % below the walking kernel's.  Of the 424 timed layers 185 then go to
+// the matrix cores; over all of them that is 1.147 times the walk's speed, 2.5 % short of the best choice, and 18 lose
+// more than 3 %.  (Without a margin: 228, 1.148 times, 38 lose; with 10 %: 164, 1.150 times, 7 lose, but networks are
+// slower: ResNet-50 at batch 16 1.50 ms, 1.48 with 7 %.)  Where the walking kernel can pool its outputs, so must the
+// matrix kernel.
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      MatGeom* g, MatGeom* pool) {
   if (C < 16) return false;  // most of a chunk of 16 channels would be padding
