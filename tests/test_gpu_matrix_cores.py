@@ -21,6 +21,20 @@ pytestmark = pytest.mark.gpu
     (1, 53, 14, 5, 105, 2, 1, 1),      # tiles of rows shorter than a quad
     (4, 17, 5, 7, 40, 1, 2, 0),        # strided pointwise, one tile over all images
     (3, 28, 7, 47, 5, 1, 1, 0),        # odd rows and columns to pool
+    # the remaining configurations of tile and teams, kernel sizes and strides
+    (2, 44, 71, 53, 129, 1, 1, 0),     # 128 channels by 64 pixels, two teams
+    (10, 120, 40, 32, 89, 3, 2, 1),    # ... in four slices
+    (4, 80, 51, 42, 66, 3, 1, 1),      # 128 by 128, two teams, three slices
+    (14, 56, 48, 7, 271, 2, 1, 1),     # 64 by 128, four teams
+    (11, 152, 57, 18, 17, 2, 1, 0),    # ... in three slices
+    (3, 200, 48, 21, 19, 1, 4, 0),     # every fourth pixel
+    (15, 60, 22, 7, 130, 2, 3, 0),     # stride 3: pixels that are staged and not used
+    (2, 196, 8, 11, 128, 4, 1, 0),
+    (7, 169, 71, 12, 59, 4, 2, 0),
+    (4, 143, 11, 9, 117, 6, 1, 0),
+    (1, 82, 19, 18, 274, 6, 2, 0),
+    (2, 95, 9, 27, 244, 7, 1, 3),
+    (3, 60, 31, 7, 30, 7, 2, 3),
 ])
 def test_layer_on_the_matrix_cores(N, C, H, W, K, ks, stride, pad, oracle):
     import torch
@@ -165,7 +179,8 @@ def conv64(x, w, stride, pad, terms=False):
 
 
 def run_both(w, x, stride, pad, act=0):
-    """The layer as the library runs it, on the matrix cores, and on a walking tile of the same pack"""
+    """The layer as the library runs it, on the matrix cores, and on a walking tile of the same pack; None where one of the
+    two cannot pool"""
     import torch
     import tetris_amd as T
 
@@ -175,9 +190,12 @@ def run_both(w, x, stride, pad, act=0):
     pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
     assert pk.launch_shape(N, H, W, stride, pad, tile).kernel == 5
     other = T.Tile(tile.lanes_w, tile.quads, tile.oc_per_wave, tile.waves, tile.tile_ic, 1 if tile.csplit != 1 else 0)
-    dx, outs = torch.from_numpy(x).cuda(), []
+    if not all(pk.act_supported(N, H, W, stride, pad, t, act) for t in (tile, other)):
+        return None
+    dx, outs, div = torch.from_numpy(x).cuda(), [], 2 if act == T.ACT_RELU_POOL2 else 1
     for t in (tile, other):
-        y = torch.full((N, K, T.out_extent(H, pad, ks, stride), T.out_extent(W, pad, ks, stride)), float("nan"), device="cuda")
+        y = torch.full((N, K, T.out_extent(H, pad, ks, stride) // div, T.out_extent(W, pad, ks, stride) // div), float("nan"),
+                       device="cuda")
         pk.launch_act(dx.data_ptr(), y.data_ptr(), N, H, W, stride, pad, t, act)
         torch.cuda.synchronize()
         outs.append(y.cpu().numpy())
@@ -199,15 +217,21 @@ def test_values_out_of_range_give_what_the_walk_gives(N, C, H, W, K, ks, stride,
     odd = np.array([np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 2.0 ** 100, -2.0 ** 90, 1e-45], np.float32)
     at = rng.permutation(x.size)[:48]
     x.reshape(-1)[at] = np.tile(odd, 6)
-    for act in (0, 1):
+    for act in (0, 1, 2):
         with np.errstate(all="ignore"):
-            matrix, walk = run_both(w, x, stride, pad, act)
+            both = run_both(w, x, stride, pad, act)
+            if both is None:
+                continue
+            matrix, walk = both
             assert np.array_equal(np.isnan(matrix), np.isnan(walk)) and np.array_equal(np.isinf(matrix), np.isinf(walk))
             assert act or (np.isnan(walk).any() and np.isinf(walk).any())
             ok = np.isfinite(walk)
             assert np.array_equal(np.sign(matrix[~ok]), np.sign(walk[~ok]), equal_nan=True)
             tame = np.where(np.isfinite(x), x, 0)
             _, terms = conv64(tame, w, stride, pad, True)
+            if act == 2:  # of a maximum: the largest bound of the four
+                k, oh, ow = walk.shape[1:]
+                terms = terms[:, :, :2 * oh, :2 * ow].reshape(N, k, oh, 2, ow, 2).max(axis=(3, 5))
             n = C * ks * ks
             assert (np.abs(matrix[ok].astype(np.float64) - walk[ok]) <= 2 * n * 2.0 ** -24 * terms[ok]).all()
 
@@ -256,3 +280,71 @@ def test_weights_out_of_range_stay_with_the_walk(oracle):
         else:
             assert np.isfinite(np.delete(got, 5, 1)).all()
         pk.close()
+
+
+SPLIT = (5, 163, 41, 54, 81, 3, 1, 1)  # runs on the matrix cores in slices
+
+
+def split_layer(seed):
+    import torch
+    import tetris_amd as T
+
+    N, C, H, W, K, ks, stride, pad = SPLIT
+    rng = np.random.default_rng(seed)
+    w = sparse_filter(rng, K, C, ks, 0.7)
+    tile = T.tile_select(N, H, W, C, K, ks, stride, pad)
+    pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+    shape = pk.launch_shape(N, H, W, stride, pad, tile)
+    assert shape.kernel == 5 and shape.csplit > 1
+    xs = [torch.from_numpy(relu_like(rng, (N, C, H, W))).cuda() for _ in range(2)]
+
+    def launch(x, y, stream=0):
+        pk.launch(x.data_ptr(), y.data_ptr(), N, H, W, stride, pad, tile, stream)
+
+    want = []
+    for x in xs:
+        y = torch.full((N, K, H, W), float("nan"), device="cuda")
+        launch(x, y)
+        torch.cuda.synchronize()
+        want.append(y.cpu().numpy())
+    return pk, tile, launch, xs, want
+
+
+def test_graph_of_a_split_matrix_layer():
+    import torch
+
+    N, C, H, W, K, ks, stride, pad = SPLIT
+    pk, tile, launch, xs, want = split_layer(21)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    pk.prepare(N, H, W, stride, pad, tile, side.cuda_stream)
+    x, y, other = xs[0].clone(), torch.empty((N, K, H, W), device="cuda"), torch.empty((N, K, H, W), device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        launch(x, y, torch.cuda.current_stream().cuda_stream)
+    for i in range(6):
+        x.copy_(xs[i % 2])
+        y.fill_(float("nan"))
+        graph.replay()
+        launch(xs[1 - i % 2], other)  # eager, on another stream, with sums of its own
+        torch.cuda.synchronize()
+        assert y.cpu().numpy().tobytes() == want[i % 2].tobytes(), i
+        assert other.cpu().numpy().tobytes() == want[1 - i % 2].tobytes(), i
+    del graph
+    pk.close()
+
+
+def test_two_streams_of_a_split_matrix_layer():
+    import torch
+
+    N, C, H, W, K, ks, stride, pad = SPLIT
+    pk, tile, launch, xs, want = split_layer(22)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    ys = [[torch.full((N, K, H, W), float("nan"), device="cuda") for _ in range(8)] for _ in streams]
+    torch.cuda.synchronize()
+    for i in range(8):
+        for x, y, s in zip(xs, ys, streams):
+            launch(x, y[i], s.cuda_stream)
+    torch.cuda.synchronize()
+    for each, ref in zip(ys, want):
+        assert all(y.cpu().numpy().tobytes() == ref.tobytes() for y in each)
+    pk.close()
