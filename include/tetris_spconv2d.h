@@ -121,7 +121,12 @@ typedef struct tetris_tile {
 /* Unmeasured selection: a built-in table of tiles measured on MI355X for the layer shapes of the benchmark
  * suites (csrc/tuned_tiles.inc, made by tetris_amd/tune.py); for other shapes the tile of the most similar
  * measured layer of the same kernel size and stride, refitted to the image width; else the first choice of a
- * cycle model. */
+ * cycle model.
+ * A launch with the library's own choice -- a NULL tile, or the one named here, unless a loaded row names it -- may run on
+ * the matrix cores instead of walking the non-zeros, where a time model says that this is at least 7 % faster: the same
+ * fp32 convolution, each number cut into three bf16 parts and eight of the nine products formed, with fp32 sums.  Its
+ * error against 64-bit sums is no larger than the walking kernels', and infinities, NaN and numbers at either end of
+ * fp32's range give what they give there.  tetris_launch_shape_of says which kernel runs; any other tile is obeyed. */
 int tetris_tile_select(int batch, int img_h, int img_w, int in_channel, int out_channel, int kernel_size, int stride,
                        int padding, tetris_tile* out);
 
@@ -293,9 +298,12 @@ size_t tetris_noalloc_scratch_limit(size_t bytes);
  * SparseFilter's TILE_IC (a template argument of the reference launcher) and entries per lane and step: 4
  * (apply_vectorize), 1, or 0 for the keep-as-is layout of apply_reorder = false (spconv2d_utils.h:38-61; then
  * d_oc_permutation may be NULL) -- the format of the reference's CSR-like baseline variant.  n_entries: how many
- * entries d_position and d_values hold (0: not known).  Before any kernel reads the arrays the offsets are copied to
- * the host and checked -- they start at 0, never decrease, step by multiples of vec_width and span at most n_entries
- * entries -- so a wrong out_channel, tile_ic or vec_width is TETRIS_EINVAL, not an out-of-range read on the device.
+ * entries d_position and d_values hold (0: not known).  Arrays that have not been decoded before (or whose content has
+ * changed) are read by no kernel until the offsets have been copied to the host and checked -- they start at 0, never
+ * decrease, step by multiples of vec_width and span at most n_entries entries -- so a wrong out_channel, tile_ic or
+ * vec_width is TETRIS_EINVAL, not an out-of-range read on the device.  For arrays decoded before, with the same shape
+ * arguments, the hash kernel compares the last offset with the number of entries that was checked then, and reads no
+ * further where they differ.
  * tile: NULL = the library chooses.  Not capturable into a HIP graph (it synchronises); capture
  * tetris_spconv2d_launch instead.  With TETRIS_OPT_TRUST_SPF_ARRAYS a set of arrays seen before is neither read back
  * nor hashed (see there). */

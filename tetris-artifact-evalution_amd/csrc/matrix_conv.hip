@@ -16,11 +16,11 @@
 // the parts are made once for all ks*ks taps.  Weights were cut when the plan was made and lie in the order the lanes load
 // them (1 KiB per 32 channels, 16 k-values and part): they go from L2 to registers, past LDS, because the four waves along
 // the channels share none.  The teams take the chunks of channels in turn and add their sums in LDS at the end: four waves
-// on every SIMD also where a layer has one tile per CU (16 x 128 x 28 x 28, 3x3: 28 us with one team, 26 with two).
+// on every SIMD also where a layer has one tile per CU (16 x 128 x 28 x 28, 3x3: 36 us with one team, 31 with two).
 //
-// What bounds it: on large layers the matrix cores (128 -> 256 channels, 52x52, batch 16: 130 us, 1.18 PFLOP/s of bf16
-// products at 2.1 GHz, where the vendor's bf16 GEMM of 8192^3 reaches 1.32; half of the rest is the last, partly filled
-// round of workgroups); on small ones the latency of a round: weights from L2, input from HBM, barrier.
+// What bounds it: on large layers the matrix cores (128 -> 256 channels, 52x52, batch 16: 148 us, 1.38 PFLOP/s of bf16
+// products, where the vendor's bf16 GEMM of 8192^3 reaches 1.37); on small ones the latency of a round: weights from L2,
+// input from HBM, barrier.
 //
 // Range: parts are made of numbers scaled by 2^32, inputs and weights, so that the lowest bit of every fp32 number, subnormal
 // ones too, is a normal bf16 number's, and sums are scaled back as they are stored.  What is out of that range upwards
