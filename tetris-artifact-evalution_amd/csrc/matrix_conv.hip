@@ -25,8 +25,8 @@
 // Range: parts are made of numbers scaled by 2^32, inputs and weights, so that the lowest bit of every fp32 number, subnormal
 // ones too, is a normal bf16 number's, and sums are scaled back as they are stored.  What is out of that range upwards
 // (an infinity, NaN, an input of 2^96 or more, a sum of 2^64 or more) makes every sum that it enters infinite or NaN,
-// whatever the weight: a wave that finds such a sum computes its tile once more as the walking kernels do, with FMAs on
-// the non-zero weights, in their order.  Packs with weights of 2^64 or more, or not finite, stay with those kernels.
+// whatever the weight: a wave that finds such a sum computes its outputs once more as the walking kernels do, with FMAs on
+// the non-zero weights only.  Packs with weights of 2^64 or more, or not finite, stay with those kernels.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -308,34 +308,44 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
   int again = lane;  // (unknown to the compiler, which would else keep the pixels' places in registers all the while)
   asm("" : "+v"(again));
   const int ch0 = slice * g.chunks / g.csplit * 8 * g.kgs, ch1 = min(g.C, (slice + 1) * g.chunks / g.csplit * 8 * g.kgs);
-  const unsigned short* rows = reinterpret_cast<const unsigned short*>(weights + (size_t)min(mt * WM + wm, g.mblocks - 1) * g.steps * 192);
+  const u32x4* block = weights + (size_t)min(mt * WM + wm, g.mblocks - 1) * g.steps * 192;
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const Pixel p = pixel(b, again);
+    float sum[16 / KW];
+#pragma unroll
+    for (int j = 0; j < 16 / KW; ++j) sum[j] = 0;
 #pragma nounroll
-    for (int i = team * (16 / KW); i < (team + 1) * (16 / KW); ++i) {
-      const int row = 8 * (i / 4) + 4 * (lane >> 5) + i % 4;
-      float sum = 0;
+    for (int c = ch0; c < ch1; c += 8) {
+      const int kg = c >> 3, chunk = kg / g.kgs, k = kg - chunk * g.kgs;
 #pragma nounroll
-      for (int c = ch0; c < ch1; ++c) {
-        const int kg = c >> 3, chunk = kg / g.kgs, k = kg - chunk * g.kgs;
+      for (int r = 0; r < g.ks; ++r)
 #pragma nounroll
-        for (int r = 0; r < g.ks; ++r)
-#pragma nounroll
-          for (int s = 0; s < g.ks; ++s) {
-            const int step = (chunk * g.ks * g.ks + r * g.ks + s) * halves + (k >> 1);
-            const unsigned short* d = rows + ((size_t)step * 192 + (k & 1) * 32 + row) * 8 + (c & 7);
-            const float w = __builtin_bit_cast(float, (unsigned)d[0] << 16) + __builtin_bit_cast(float, (unsigned)d[512] << 16) +
-                            __builtin_bit_cast(float, (unsigned)d[1024] << 16);
-            const int iy = (int)(p.oy * g.stride + r) * g.sub - g.pad, ix = (int)(p.w * g.stride + s) * g.sub - g.pad;
-            const bool inside = iy >= 0 && iy < g.H && ix >= 0 && ix < g.W && p.n < (unsigned)g.N;
-            const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                irsrc, inside ? 4 * (int)(((p.n * g.C + c) * g.H + iy) * g.W + ix) : kOutside, 0, 0));
-            if (w != 0.f) sum = fmaf(v, w * (1 / kScale), sum);
+        for (int s = 0; s < g.ks; ++s) {
+          const int iy = (int)(p.oy * g.stride + r) * g.sub - g.pad, ix = (int)(p.w * g.stride + s) * g.sub - g.pad;
+          const bool inside = iy >= 0 && iy < g.H && ix >= 0 && ix < g.W && p.n < (unsigned)g.N;
+          const int at = 4 * (int)(((p.n * g.C + c) * g.H + iy) * g.W + ix);
+          float v[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                 irsrc, inside && c + q < ch1 ? at + q * hw4 : kOutside, 0, 0));
+          const u32x4* d = block + (size_t)((chunk * g.ks * g.ks + r * g.ks + s) * halves + (k >> 1)) * 192 + (k & 1) * 32 + 4 * (again >> 5);
+#pragma unroll
+          for (int j = 0; j < 16 / KW; ++j) {
+            const int i = team * (16 / KW) + j, row = 8 * (i / 4) + i % 4;
+            const u32x4 h = d[row], m = d[row + 64], l = d[row + 128];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+              auto part = [&](u32x4 x) { return __builtin_bit_cast(float, q & 1 ? x[q / 2] & 0xffff0000u : x[q / 2] << 16); };
+              const float w = part(h) + part(m) + part(l);
+              if (w != 0.f) sum[j] = fmaf(v[q], w * (1 / kScale), sum[j]);
+            }
           }
-      }
-      store(i, b, sum);
+        }
     }
+#pragma unroll
+    for (int j = 0; j < 16 / KW; ++j) store(team * (16 / KW) + j, b, sum[j]);
   }
 }
 
