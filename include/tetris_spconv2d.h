@@ -158,9 +158,9 @@ int tetris_tile_table_load(const char* path, int* rows_out);
 #define TETRIS_OPT_TRUST_SPF_ARRAYS 8u
 /* Layers whose channel reduction is split over workgroups add their partial sums inside the conv kernel -- the last
  * wave of every (output tile, wave) pair to finish reads the slices back through L2 and adds them -- instead of in a
- * second kernel.  Same bits either way.  Measured slower on every suite (the adding wave's loads are a chain of L2
- * round trips at the end of the kernel, where nothing hides them), so it is a switch for comparing the two, off by
- * default. */
+ * second kernel.  Same bits either way.  Measured faster only for a layer launched again and again where two slices
+ * meet (16 x 128 x 28 x 28, 3x3: 30.7 us, 32.8 with the second kernel), slower with four or eight, which one wave then
+ * reads alone, and up to 2 us slower per layer in a network, so it is a switch for comparing the two, off by default. */
 #define TETRIS_OPT_ADD_IN_KERNEL 16u
 /* Whether split layers add their slices inside the conv kernel on the current GPU: TETRIS_OPT_ADD_IN_KERNEL is on and
  * the workgroups whose ids are equal modulo 8 run on one XCD (they then share an L2), which a probe kernel checks once
