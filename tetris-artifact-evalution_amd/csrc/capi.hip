@@ -96,7 +96,7 @@ bool known_plan(tetris_g950* p, const Key& key, Plan* out) {
 }
 
 // Decides which kernel runs (input shape, tile); `t`: the tile, given or chosen.  Remembered, so that a query and the
-// plan that follows it decide once (0.3 ms for an image of 211 x 223).
+// plan that follows it decide once (some 20 us on images of 211 x 223).
 int choose_kernel(tetris_g950* p, int N, int H, int W, int stride, int pad, const tetris_tile& t, bool given, bool walk,
                   Choice* out) {
   const Key shape = plan_key(N, H, W, stride, pad, given ? &t : nullptr, walk);
