@@ -1,0 +1,164 @@
+"""The kernel that writes filter and input as three fp16 parts and multiplies them with the matrix cores' sparse instructions
+(csrc/matrix_half.hip), through the public entry points, on layers that the library gives to it."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def filter_of(rng, K, C, ks, density):
+    """normally distributed weights, of which exactly `density` are not zero"""
+    w = rng.standard_normal(K * C * ks * ks).astype(np.float32)
+    w[rng.permutation(w.size)[int(density * w.size):]] = 0
+    return w.reshape(K, C, ks, ks)
+
+
+def conv64(x, w, stride, pad):
+    """float64 on the CPU, and the sum of the terms' magnitudes"""
+    import torch
+
+    f = lambda a, b: torch.nn.functional.conv2d(torch.from_numpy(a).double(), torch.from_numpy(b).double(),  # noqa: E731
+                                                stride=stride, padding=pad).numpy()
+    return f(x, w), f(np.abs(x), np.abs(w))
+
+
+class Layer:
+    def __init__(self, w, shape, stride, pad):
+        import tetris_amd as T
+
+        N, C, H, W = shape
+        K, _, ks, _ = w.shape
+        self.at = (N, H, W, stride, pad)
+        self.out = (N, K, T.out_extent(H, pad, ks, stride), T.out_extent(W, pad, ks, stride))
+        self.tile = T.tile_select(N, H, W, C, K, ks, stride, pad)
+        self.pack = T.G950Filter.for_tile(w, self.tile, oc_order="balanced")
+        self.shape = self.pack.launch_shape(*self.at, self.tile)
+        # (LDS: whole KiB of input, then what this kernel alone keeps there)
+        assert self.shape.kernel == 5 and self.shape.lds_bytes % 1024
+
+    def walk(self):
+        import tetris_amd as T
+
+        t = self.tile
+        return T.Tile(t.lanes_w, t.quads, t.oc_per_wave, t.waves, t.tile_ic, 1 if t.csplit != 1 else 0)
+
+    def __call__(self, x, tile=None):
+        import torch
+
+        dx, y = torch.from_numpy(x).cuda(), torch.full(self.out, float("nan"), device="cuda")
+        self.pack.launch(dx.data_ptr(), y.data_ptr(), *self.at, tile or self.tile)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad,density", [
+    (9, 16, 21, 21, 7, 2, 3, 0, 0.15),     # 256 channels by 64 pixels, one chunk of them; stride 3
+    (15, 18, 21, 41, 131, 5, 1, 2, 0.3),   # ... chunks of 16 channels, the last of two; blocks that come twice
+    (6, 39, 5, 9, 4, 7, 2, 3, 0.3),        # ... 7 x 7, in slices; four output channels
+    (3, 42, 40, 77, 81, 3, 1, 1, 0.15),    # 128 by 64, two teams, a chunk each and ten channels more; two strips
+    (4, 17, 70, 26, 166, 6, 1, 0, 0.3),    # ... 6 x 6
+    (12, 53, 27, 35, 7, 4, 1, 0, 0.15),    # 64 by 64, two teams
+    (1, 21, 8, 8, 3, 7, 1, 3, 0.3),        # ... an image of one tile
+    (8, 19, 79, 28, 275, 3, 1, 0, 0.3),    # 256 by 128
+    (12, 17, 73, 24, 85, 2, 3, 1, 0.15),   # short chunks: 256 by 64
+    (3, 95, 9, 8, 3, 4, 3, 0, 0.3),        # ... in slices
+    (5, 17, 67, 31, 74, 4, 1, 2, 0.2),     # ... 128 by 64, two teams
+    (10, 17, 14, 6, 6, 2, 3, 0, 0.15),     # ... 64 by 64
+    (1, 20, 28, 8, 10, 4, 1, 0, 0.3),      # ... two teams
+    (8, 117, 38, 38, 183, 1, 1, 0, 0.15),  # pointwise
+])
+def test_layer(N, C, H, W, K, ks, stride, pad, density):
+    rng = np.random.default_rng(N * C + K)
+    w = filter_of(rng, K, C, ks, density)
+    x = np.maximum(rng.standard_normal((N, C, H, W)), -0.25).astype(np.float32)
+    layer = Layer(w, x.shape, stride, pad)
+    got, walk = layer(x), layer(x, layer.walk())
+    ref, terms = conv64(x, w, stride, pad)
+    # in any order of fp32 sums an output is off by a rounding per term at most, each of the terms' magnitude; and the parts
+    # lose no more than the walking kernel's FMAs do
+    assert (np.abs(got - ref) <= C * ks * ks * 2.0 ** -24 * terms).all()
+    assert np.linalg.norm(got - ref) <= 1.05 * np.linalg.norm(walk - ref)
+    layer.pack.close()
+
+
+LAYER = (3, 42, 40, 77, 81, 3, 1, 1, 0.15)
+
+
+@pytest.mark.parametrize("what", ["as it is", "2^40", "2^-60", "zero where it is looked at", "tiny beside ones", "2^120", "subnormal", "infinite"])
+def test_inputs_of_any_scale(what):
+    """Inputs are scaled by what some of them show; what fp16 parts do not hold then is computed with bf16 parts, and what those
+    do not hold with FMAs."""
+    N, C, H, W, K, ks, stride, pad, density = LAYER
+    rng = np.random.default_rng(1)
+    w = filter_of(rng, K, C, ks, density)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    if what == "2^40":
+        x *= np.float32(2.0 ** 40)
+    elif what == "2^-60":
+        x *= np.float32(2.0 ** -60)
+    elif what == "zero where it is looked at":
+        x[:, :, ::2] = 0
+        x[:, ::11] = 0
+    elif what == "tiny beside ones":
+        x[:, :, :, 30:] *= np.float32(2.0 ** -80)
+    elif what == "2^120":
+        x *= np.float32(2.0 ** 120)
+    elif what == "subnormal":
+        x *= np.float32(2.0 ** -130)
+    odd = None
+    if what == "infinite":
+        x[1, 20, 13, 50], x[2, 3, 30, 7] = np.inf, np.nan
+        odd = ~np.isfinite(x)
+    layer = Layer(w, x.shape, stride, pad)
+    got = layer(x)
+    ref, terms = conv64(np.where(np.isfinite(x), x, 0), w, stride, pad)
+    # (a subnormal output is rounded as such, twice)
+    off = np.abs(got - ref) <= C * ks * ks * 2.0 ** -24 * terms + 2.0 ** -149
+    if odd is not None:
+        reached = conv64(odd.astype(np.float32), np.abs(w), stride, pad)[0] > 0
+        assert reached.any() and not np.isfinite(got[reached]).any()
+        off |= reached
+    assert off.all()
+    layer.pack.close()
+
+
+@pytest.mark.parametrize("value,count", [(2.0 ** -20, 1), (2.0 ** -40, 60), (2.0 ** -40, 3000), (2.0 ** -100, 1), (2.0 ** -149, 2), (2.0 ** 63, 1)])
+def test_small_weights(value, count):
+    """Weights far below the largest of their row: multiplied one by one; all with bf16 parts where they are many, or where their
+    products would underflow."""
+    N, C, H, W, K, ks, stride, pad, density = LAYER
+    rng = np.random.default_rng(2)
+    w = filter_of(rng, K, C, ks, density)
+    there = np.flatnonzero(w)
+    w.reshape(-1)[rng.permutation(there)[:count]] = np.float32(value)
+    only = np.zeros_like(x := rng.standard_normal((N, C, H, W)).astype(np.float32))
+    layer = Layer(w, x.shape, stride, pad)
+    for each in (x, only):
+        if each is only:  # an input that meets nothing but small weights in a row of the filter
+            k, c, r, s = np.argwhere(w == np.float32(value))[0]
+            w2 = w[k:k + 1]
+            keep = [i for i in range(C) if not (np.abs(w2[0, i]) > abs(value)).any()]
+            each[:, keep] = x[:, keep]
+        got = layer(each)
+        ref, terms = conv64(each, w, stride, pad)
+        assert (np.abs(got - ref) <= C * ks * ks * 2.0 ** -24 * terms + 2.0 ** -149).all(), value
+    layer.pack.close()
+
+
+def test_outputs_that_do_not_lie_on_16_bytes():
+    """Outputs go out four pixels at a time where they lie so in memory, one by one elsewhere: the same bits."""
+    import torch
+
+    N, C, H, W, K, ks, stride, pad, density = 12, 53, 27, 35, 7, 4, 1, 0, 0.15
+    rng = np.random.default_rng(3)
+    w, x = filter_of(rng, K, C, ks, density), rng.standard_normal((N, C, H, W)).astype(np.float32)
+    layer = Layer(w, x.shape, stride, pad)
+    count = int(np.prod(layer.out))
+    dx, y = torch.from_numpy(x).cuda(), torch.full((2 * count + 16,), float("nan"), device="cuda")
+    for first in (0, count + 1):
+        layer.pack.launch(dx.data_ptr(), y.data_ptr() + 4 * first, *layer.at, layer.tile)
+    torch.cuda.synchronize()
+    y = y.cpu().numpy()
+    assert count % 4 == 0 and y[:count].tobytes() == y[count + 1:2 * count + 1].tobytes()
+    assert np.isnan(y[count]) and np.isnan(y[2 * count + 1:]).all()
+    layer.pack.close()

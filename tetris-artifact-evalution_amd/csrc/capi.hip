@@ -58,22 +58,22 @@ bool choose_matrix(const tetris_g950* p, int N, int H, int W, int stride, int pa
 }
 
 // the weights of pack `p` as the matrix kernel loads them, made on first use
-int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const void** out) {
+int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const MatWeights** out) {
   std::lock_guard<std::mutex> lock(p->mu);
-  auto it = p->parts.find(g.kgs);
+  const int key = g.kgs | g.half << 8;
+  auto it = p->parts.find(key);
   if (it == p->parts.end()) {
     void* d = nullptr;
+    MatWeights w{};
     TETRIS_HIP(hipMalloc(&d, mat_weight_bytes(g)));
-    int rc = mat_weights(p, g, stream, d);
-    // launches on other streams may follow at once
-    if (rc == TETRIS_OK && hipStreamSynchronize(stream) != hipSuccess) rc = fail(TETRIS_EHIP, "making a matrix plan failed");
+    const int rc = mat_weights(p, g, stream, d, &w);
     if (rc) {
       (void)hipFree(d);
       return rc;
     }
-    it = p->parts.emplace(g.kgs, d).first;
+    it = p->parts.emplace(key, w).first;
   }
-  *out = it->second;
+  *out = &it->second;  // (a map's entries stay where they are)
   return TETRIS_OK;
 }
 
@@ -212,10 +212,10 @@ int launch_plan(const Plan& p, const float* d_in, float* d_out, float* d_scratch
     return fail(TETRIS_EINVAL, "2x2 pooling needs an output of at least 2 x 2");
   if (p.mat.csplit == 1) {
     if (act == 2 && !p.mat_pool.N) return fail(TETRIS_EUNSUPPORTED, "this layer cannot pool its outputs");
-    return launch_matrix(act == 2 ? p.mat_pool : p.mat, d_in, d_out, p.parts, act != 0, stream);
+    return launch_matrix(act == 2 ? p.mat_pool : p.mat, d_in, d_out, *p.parts, act != 0, stream);
   }
   float* copies = d_scratch + kTicketBytes / sizeof(float);
-  const int rc = launch_matrix(p.mat, d_in, copies, p.parts, 0, stream);
+  const int rc = launch_matrix(p.mat, d_in, copies, *p.parts, 0, stream);
   if (rc) return rc;
   return add_copies(copies, d_out, p.mat.N, p.mat.K, p.mat.OH, p.mat.OW, p.mat.csplit, act, stream);
 }
@@ -1174,13 +1174,13 @@ extern "C" {
 
 // the configuration's geometry (16 numbers, see kernel_times.py) and predicted microseconds; TETRIS_EINVAL: it cannot be run
 int tetris_fit_matrix_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, int* out,
-                           double* predicted) {
+                           long long nnz, double* predicted) {
   MatGeom g;
   if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, csplit, false, &g)) return fail(TETRIS_EINVAL, "not a configuration");
   if (csplit > 1 && 4ll * g.out_floats * csplit > kMatCopies) return fail(TETRIS_EINVAL, "too many slices");
-  const int v[16] = {g.ptiles, g.mtiles, g.csplit, g.chunks, g.kgs, g.lpad, g.OH, g.OW, mat_lds_bytes(g), g.mblocks, g.steps};
+  const int v[16] = {g.ptiles, g.mtiles, g.csplit, g.chunks, g.kgs, g.lpad, g.OH, g.OW, mat_lds_bytes(g), g.mblocks, g.half};
   std::copy(v, v + 16, out);
-  *predicted = matrix_time(g);
+  *predicted = matrix_time(g, nnz);
   return TETRIS_OK;
 }
 

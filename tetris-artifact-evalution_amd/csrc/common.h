@@ -177,16 +177,32 @@ struct MatDiv { unsigned m; int shift; };  // x / d == x * m >> shift for x < 2^
 struct MatGeom {
   int N, C, H, W, K, OH, OW, ks, stride, pad, sub;  // stride, in staged pixels, of the outputs; sub, in input pixels, of the staged ones
   int in_bytes, out_floats;  // input bytes; floats of the output, or of one slice's copy of it
-  int pool, relu;
+  int pool, relu, quads;     // quads: outputs are stored four pixels at a time (relu, quads: set per launch)
   int strips, ws, wp, ihs;   // strips per image; output columns of one; staged columns and rows of one
   int uw, uh, upq, npix;     // columns, rows and pixels of a strip's outputs (2x2 blocks when pooling); all outputs
-  int kgs, chunks, steps;    // groups of 8 channels staged together; such chunks; products of 16 k-values
+  int kgs, chunks;           // groups of 8 channels staged together; such chunks
+  int half, steps, smax;     // which matrix kernel; matrix_kernel: products of 16 k-values; half_kernel: most steps of a chunk
   int mblocks, mtiles, ptiles, csplit, cfg;
   int lpad;                  // staged pixels of a tile, to a multiple of 64
+  int lds_rows;              // bytes in front of the rows' exponents in LDS
   unsigned m_uw, m_uh, m_wp, m_ihs, m_strips;
   MatDiv d_tiles, d_mtiles, d_upq, d_uw, d_blocks;
 };
-constexpr int kMatConfigs = 11;
+// A filter's weights as a matrix kernel loads them (device memory).  matrix_kernel: `base` only.  half_kernel: per 32 output
+// channels and chunk of input channels up to MatGeom::smax steps, each a 32 x 32 matrix of which two in four consecutive values of a row are kept.
+struct MatWeights {
+  void* base;           // the allocation that holds them all
+  const char* steps;    // fp16 parts
+  const char* slots;    // the same weights in fp32
+  const int* first;     // first step of every (32 output channels, chunk)
+  const int* row_exp;   // per output channel: the power of two that its sums are multiplied by
+  const int* loose_count;  // per 32 output channels: weights that fp16 parts do not hold
+  const int2* loose;    // ... which: row, tap and input channel; the scaled weight
+  const float* dense;   // [output channel][tap][input channel, to a multiple of the chunk]
+  int step_bytes;       // of all steps
+  int wide;             // some weight is not the sum of its fp16 parts
+};
+constexpr int kMatConfigs = 21;
 constexpr int kMatTasks = 4;        // most blocks of 64 staged pixels x 8 channels that a wave holds at a time
 constexpr int kMatLds = 160 * 1024;
 constexpr long long kMatCopies = 32 << 20;  // most bytes of partial sums of a split layer
@@ -209,7 +225,7 @@ struct Plan {
   const int2* entries;        // the pack's entries bound to the geometry
   const int32_t* grp_off;     // [groups*stages+1] first entry of every stream in `entries`
   const int32_t* grp_pair;    // [groups*stages] entries of the stream's leading segment of pairs (0 when unpaired)
-  const void* parts = nullptr;  // the weights of the matrix kernel: set where it runs the layer instead
+  const MatWeights* parts = nullptr;  // the weights of the matrix kernel (the pack's): set where it runs the layer instead
   MatGeom mat, mat_pool;
 };
 }  // namespace tetris
@@ -230,7 +246,7 @@ struct tetris_g950 {
   float* d_values = nullptr;      // [n_entries + 8]
   // (LDS byte offset | accumulator index << 16 | 0xC << 28, value) pairs for one tile geometry, made on first use
   std::map<tetris::BoundKey, int2*> bound;
-  std::map<int, void*> parts;  // the weights as the matrix kernel loads them, by MatGeom::kgs
+  std::map<int, tetris::MatWeights> parts;  // the weights as the matrix kernel loads them, by MatGeom::kgs
   // Paired arrangement of the streams (made on the first paired bind; depends on the pack only): two consecutive
   // entries of a stream that share their position become a pair; per stream first all pairs, padded to a multiple
   // of 8 entries, then the entries left single, padded likewise.
@@ -327,18 +343,18 @@ int add_copies(const float* d_copies, float* d_out, int N, int K, int OH, int OW
 
 // matrix_conv.hip
 // staged (may be null): of the same layer, what earlier calls found (zeros: nothing yet)
-using StagedPixels = std::array<int, 2>;  // of the largest tile of 64 and of 128 pixels
+using StagedPixels = std::array<int, 3>;  // of the largest tile of 64 and of 128 pixels
 bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out,
                    StagedPixels* staged = nullptr);
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      MatGeom* g, MatGeom* pool);
 // predicted microseconds of a launch
-double matrix_time(const MatGeom& g);
+double matrix_time(const MatGeom& g, long long nnz);
 double walk_time(const Geom& g, long long nnz);
 int mat_lds_bytes(const MatGeom& g);
 size_t mat_weight_bytes(const MatGeom& g);
-int mat_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* dst);
-int launch_matrix(const MatGeom& g, const float* d_in, float* d_out, const void* weights, int relu, hipStream_t stream);
+int mat_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* base, MatWeights* out);  // waits for them
+int launch_matrix(const MatGeom& g, const float* d_in, float* d_out, const MatWeights& weights, int relu, hipStream_t stream);
 
 // whether workgroups with the same blockIdx.x % 8 run on one XCD of the current device (probed once per device):
 // what lets the slices of a split layer exchange their partial sums through that XCD's L2

@@ -32,44 +32,13 @@
 #include <cmath>
 #include <numeric>
 
-#include "common.h"
+#include "matrix.h"
 
 namespace tetris {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kOutside = 0x7ff00000;  // a byte offset beyond every tensor this path takes (1 GiB): loads give 0, stores are dropped
-
-constexpr float kScale = 0x1p32f, kUnscale = 0x1p-64f;
-
-// three bf16 parts of eight floats, scaled
-__device__ __forceinline__ void cut(const float (&x)[8], u32x4& hi, u32x4& mid, u32x4& lo) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const f32x2 v = {x[2 * i] * kScale, x[2 * i + 1] * kScale};
-    const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
-    const float r0 = v.x - __builtin_bit_cast(float, h << 16), r1 = v.y - __builtin_bit_cast(float, h & 0xffff0000u);
-    const unsigned m = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
-    const float s0 = r0 - __builtin_bit_cast(float, m << 16), s1 = r1 - __builtin_bit_cast(float, m & 0xffff0000u);
-    hi[i] = h;
-    mid[i] = m;
-    lo[i] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{s0, s1}, bf16x2));
-  }
-}
-
 __device__ __forceinline__ f32x16 product(u32x4 a, u32x4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// maximum over the four lanes of a quad
-__device__ __forceinline__ float quad_max(float v) {
-  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true)));
-  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true)));
 }
 
 // x / d for x below 2^30
@@ -379,15 +348,12 @@ __global__ __launch_bounds__(256) void parts_kernel(const int32_t* __restrict__ 
   }
 }
 
-struct Config { int wm, nb, kw; };
-constexpr Config kConfigs[] = {{4, 4, 1}, {4, 4, 2}, {4, 2, 1}, {4, 2, 2}, {4, 2, 4}, {2, 2, 1}, {2, 2, 2}, {2, 2, 4}, {2, 1, 1}, {2, 1, 2}, {2, 1, 4}};
-static_assert(sizeof kConfigs / sizeof *kConfigs == kMatConfigs);
-
 // input buffers, or what the teams' sums need
-int lds_bytes(const MatGeom& g) {
-  const Config& c = kConfigs[g.cfg];
-  return std::max(c.kw * 96 * g.kgs * g.lpad, c.kw > 1 ? c.kw * 16384 * c.nb : 0);
+int lds_main(const MatGeom& g) {
+  const MatShape& c = kMatShapes[g.cfg];
+  return std::max(c.kw * 96 * g.kgs * g.lpad, c.kw > 1 ? c.kw * c.wm * c.wn * 4096 * c.nb : 0);
 }
+int lds_bytes(const MatGeom& g) { return lds_main(g) + (g.half ? 128 * kMatShapes[g.cfg].wm + 16 : 0); }
 
 template <int WM, int NB, int KW, int TM>
 int launch_one(const MatGeom& g, const float* d_in, float* d_out, const void* weights, hipStream_t stream) {
@@ -459,22 +425,35 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
   g.upq = g.uw * g.uh;
   if ((long long)N * g.strips * g.upq * (pool ? 4 : 1) >= (1ll << 30)) return false;
   g.npix = N * g.strips * g.upq * (pool ? 4 : 1);
+  g.half = kMatShapes[cfg].half;
   g.kgs = ks == 1 ? 4 : 2;
+  if (g.half) {
+    // (A step's words have room for 8 groups, and for 2 where ks > 4.)  Long chunks: fewer barriers, and fewer steps that are not
+    // full; short ones: more workgroups on a CU, and tiles whose halo would not fit else.
+    g.kgs = C <= 16 || ks > 4 ? 2 : C <= 32 || ks > 1 ? 4 : 8;
+    if (kMatShapes[cfg].brief) {
+      if (g.kgs == 2) return false;
+      g.kgs /= 2;
+    }
+  }
   g.chunks = ceil_div(C, 8 * g.kgs);
   if (csplit > g.chunks) return false;
   g.csplit = csplit;
   g.steps = g.chunks * ks * ks * (g.kgs / 2);
   g.mblocks = ceil_div(K, 32);
-  const Config c = kConfigs[cfg];
+  const MatShape c = kMatShapes[cfg];
   g.cfg = cfg;
-  const int P = 32 * c.nb * (4 / c.wm);
+  g.smax = ceil_div(2 * g.kgs * ks * ks, 4);
+  if (g.half && (g.chunks / csplit < c.kw || ((long long)g.mblocks * g.chunks * g.smax + 3) * kStepBytes >= (1ll << 31))) return false;
+  const int P = 32 * c.nb * c.wn;
   g.ptiles = ceil_div(g.npix, P);
   g.mtiles = ceil_div(g.mblocks, c.wm);
   StagedPixels one{};
-  int& most = (staged ? *staged : one)[P / 128];  // tiles are of 64 or 128 pixels
+  int& most = (staged ? *staged : one)[P / 128];  // tiles are of 64, 128 or 256 pixels
   if (!most) most = staged_pixels(g, P);
   g.lpad = ceil_div(most, 64) * 64;
-  if (g.kgs * g.lpad / 64 > 4 * kMatTasks || lds_bytes(g) > kMatLds) return false;
+  if (g.kgs * g.lpad / 64 > c.wm * c.wn * (g.half && c.nb == 4 ? 2 : kMatTasks) || lds_bytes(g) > kMatLds) return false;
+  g.lds_rows = lds_main(g);
   if ((long long)g.ptiles * g.mtiles * csplit >= (1ll << 28)) return false;
   // multiply-high divisions: dividend * divisor below 2^32
   const long long lim = 1ll << 32;
@@ -491,13 +470,12 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
 }
 
 // Microseconds of a launch.  The constants were fitted to the times of a kernel with six products a step, whose cycles
-// were then scaled by 8/6.  Against 13 469 timed launches of 424 layers -- those of the benchmark's suites at batch 1, 4
+// were then scaled by 8/6.  Against 13 413 timed launches of 424 layers -- those of the benchmark's suites at batch 1, 4
 // and 16 and 160 random ones, every configuration and slice count: profiles/kernel_times.txt, measured and checked by
-// tetris_amd/kernel_times.py -- they are 11 % off (standard deviation), and the configuration that they name is 3.1 %
-// slower than the fastest one.  A fit to these times, with a term for the weights' bytes, is 11 % off as well, 2.6 %
-// slower than the fastest, and not faster in any network (VGG19 at batch 1: 408 us, 400 with these).
-double matrix_time(const MatGeom& g) {
-  const Config& c = kConfigs[g.cfg];
+// tetris_amd/kernel_times.py -- they are 11 % off (standard deviation).  A fit to these times, with a term for the weights'
+// bytes, is 11 % off as well and not faster in any network (VGG19 at batch 1: 408 us, 400 with these).
+double plain_time(const MatGeom& g) {
+  const MatShape& c = kMatShapes[g.cfg];
   const int by_regs = c.nb == 4 ? 2 / c.kw : c.nb == 2 ? std::max(1, 3 / c.kw) : c.kw == 1 ? 5 : c.kw == 2 ? 2 : 1;
   const int fit = std::max(1, std::min(by_regs, kMatLds / lds_bytes(g)));  // workgroups per CU
   const int wgs = g.ptiles * g.mtiles * g.csplit, rounds = ceil_div(ceil_div(g.chunks, g.csplit), c.kw);
@@ -515,6 +493,32 @@ double matrix_time(const MatGeom& g) {
   const double memory = (in * (1 + 0.19 * std::sqrt(g.mtiles - 1.0)) + out * g.csplit) / 4.17e6;
   return 2.2 + std::max(compute, memory) + (g.csplit > 1 ? 2.5 + out * (g.csplit + 1) / 4.07e6 : 0);
 }
+
+// The same for half_kernel, fitted to 11 063 launches of the same layers: 9 % off.
+double half_time(const MatGeom& g, long long nnz) {
+  const MatShape& c = kMatShapes[g.cfg];
+  const int team = c.wm * c.wn, waves = team * c.kw;
+  const int by_regs = std::max(1, (c.nb >= 2 ? 8 : 12) / waves);
+  const int fit = std::max(1, std::min(by_regs, kMatLds / lds_bytes(g)));  // workgroups per CU
+  const int wgs = g.ptiles * g.mtiles * g.csplit, rounds = ceil_div(ceil_div(g.chunks, g.csplit), c.kw);
+  // steps of a chunk: its blocks, those of them again that hold more than two weights in a group of four, four to a step
+  const double density = std::min(1.0, (double)nnz / ((double)g.K * g.C * g.ks * g.ks)), more = density * density * density * (4 - 3 * density);
+  const double blocks = (double)ceil_div(g.C, 8) * g.ks * g.ks / g.chunks, staging = (double)g.kgs * g.lpad / 64 / team;
+  const double steps = blocks * (2 - std::pow(1 - more, 64)) / 4 + 0.375;
+  // cycles of n workgroups on a CU: start and end; a round's staging and barrier; a step, as long as one wave takes or, with
+  // enough waves, the matrix core (6 * nb products of 32 cycles per wave)
+  auto cycles = [&](int n) {
+    if (n == 0) return 0.0;
+    const double per_simd = n * waves / 4.0, products = 192.0 * c.nb;
+    const double step = std::max(202.0 + 1.823 * products, (100.0 + 1.276 * products) * per_simd);
+    return 5339.0 + 1160.0 * c.nb * per_simd + rounds * ((g.ks == 1 ? 275.0 : 799.0) + 638.0 * staging * per_simd + steps * step);
+  };
+  const int full = wgs / (256 * fit), rest = wgs % (256 * fit);
+  const double out = 4.0 * g.N * g.K * g.OH * g.OW;
+  return 1.54 + (full * cycles(fit) + cycles(ceil_div(rest, 256))) / 2.3e3 + (g.csplit > 1 ? 2.59 + out * (g.csplit + 1) / 4.52e6 : 0);
+}
+
+double matrix_time(const MatGeom& g, long long nnz) { return g.half ? half_time(g, nnz) : plain_time(g); }
 
 // The same for the kernels that walk the non-zeros: 15 % off.
 double walk_time(const Geom& g, long long nnz) {
@@ -534,27 +538,29 @@ double walk_time(const Geom& g, long long nnz) {
   return std::max(compute, (in + out) / 6.9e6) + (g.csplit > 1 ? 1.5 + out * (g.csplit + 1) / 4.1e6 : 0);
 }
 
-// Whether the matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and
-// slice count of least predicted time, if that is 7 % below the walking kernel's.  Of the 424 timed layers 185 then go to
-// the matrix cores; over all of them that is 1.147 times the walk's speed, 2.5 % short of the best choice, and 18 lose
-// more than 3 %.  (Without a margin: 228, 1.148 times, 38 lose; with 10 %: 164, 1.150 times, 7 lose, but networks are
-// slower: ResNet-50 at batch 16 1.50 ms, 1.48 with 7 %.)  Where the walking kernel can pool its outputs, so must the
-// matrix kernel.
+// Whether a matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and slice
+// count of least predicted time, if that is 7 % below the walking kernel's; half_kernel's, if that is 16 % below the walking
+// kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's.  Of the 424 timed layers 138
+// then go to matrix_kernel and 69 to half_kernel; over all of them that is 1.173 times the walk's speed, 2.8 % short of the
+// best choice, 10 layers lose more than 3 % to the walk and one to what matrix_kernel and the walk alone would give it.
+// (Without half_kernel 1.142 times.  With 14 %: one layer in 424 less well chosen; with 10 % and no advantage asked over
+// matrix_kernel 13 of them, and networks are slower: yolov3's backbone at batch 16 4.82 ms, 4.70 so.)  Where the walking
+// kernel can pool its outputs, so must the matrix kernel.
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      MatGeom* g, MatGeom* pool) {
   if (C < 16) return false;  // most of a chunk of 16 channels would be padding
   const bool pools = walk.OH >= 2 && walk.OW >= 2 && (walk.csplit > 1 || geom_pools_in_kernel(walk));
   std::vector<std::pair<double, MatGeom>> found;
   StagedPixels staged{};
-  const double limit = 0.93 * walk_time(walk, nnz);
+  const double walking = walk_time(walk, nnz);
   for (int cfg = 0; cfg < kMatConfigs; ++cfg) {
     MatGeom m;
     if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, 1, false, &m, &staged)) continue;
     for (const int slices : {1, 2, 3, 4, 6, 8}) {
-      if (slices > m.chunks || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
+      if (m.chunks / slices < (m.half ? kMatShapes[cfg].kw : 1) || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
       m.csplit = slices;
-      const double t = matrix_time(m);
-      if (t < limit) found.emplace_back(t, m);
+      const double t = matrix_time(m, nnz);
+      if (t < (m.half ? 0.84 : 0.93) * walking) found.emplace_back(m.half ? 1.05 * t : t, m);
     }
   }
   std::stable_sort(found.begin(), found.end(),
@@ -574,26 +580,32 @@ bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int 
 
 int mat_lds_bytes(const MatGeom& g) { return lds_bytes(g); }
 
-size_t mat_weight_bytes(const MatGeom& g) { return (size_t)g.mblocks * g.steps * 192 * 16; }
+size_t mat_weight_bytes(const MatGeom& g) { return g.half ? half_weight_bytes(g) : (size_t)g.mblocks * g.steps * 192 * 16; }
 
-int mat_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* dst) {
+int mat_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* dst, MatWeights* out) {
+  if (g.half) return half_weights(p, g, stream, dst, out);
   TETRIS_HIP(hipMemsetAsync(dst, 0, mat_weight_bytes(g), stream));
   const int nstream = p->groups * p->stages;
   hipLaunchKernelGGL(parts_kernel, dim3(ceil_div(nstream, 4)), dim3(256), 0, stream, p->d_grp_off, p->d_grp_nnz, p->d_oc_order,
                      p->d_position, p->d_values, static_cast<unsigned short*>(dst), p->K, p->ks, p->tile_ic, p->stages, p->g,
                      nstream, g.kgs, g.steps);
   TETRIS_HIP(hipGetLastError());
+  TETRIS_HIP(hipStreamSynchronize(stream));  // launches on other streams may follow at once
+  *out = MatWeights{};
+  out->base = dst;
   return TETRIS_OK;
 }
 
-int launch_matrix(const MatGeom& g, const float* d_in, float* d_out, const void* weights, int relu, hipStream_t stream) {
+int launch_matrix(const MatGeom& g, const float* d_in, float* d_out, const MatWeights& w, int relu, hipStream_t stream) {
+  if (g.half) return launch_half(g, d_in, d_out, w, relu, stream);
+  const void* weights = w.base;
   MatGeom k = g;
   k.relu = relu;
   const bool two = g.kgs * g.lpad / 64 <= 8;
 #define TETRIS_MAT(WM, NB, KW) \
   if (c.wm == WM && c.nb == NB && c.kw == KW) \
     return two ? launch_one<WM, NB, KW, 2>(k, d_in, d_out, weights, stream) : launch_one<WM, NB, KW, kMatTasks>(k, d_in, d_out, weights, stream);
-  const Config& c = kConfigs[g.cfg];
+  const MatShape& c = kMatShapes[g.cfg];
   TETRIS_MAT(4, 4, 1) TETRIS_MAT(4, 4, 2) TETRIS_MAT(4, 2, 1) TETRIS_MAT(4, 2, 2) TETRIS_MAT(4, 2, 4) TETRIS_MAT(2, 2, 1)
   TETRIS_MAT(2, 2, 2) TETRIS_MAT(2, 2, 4) TETRIS_MAT(2, 1, 1) TETRIS_MAT(2, 1, 2) TETRIS_MAT(2, 1, 4)
 #undef TETRIS_MAT

@@ -596,7 +596,7 @@ int tetris_g950_create_balanced(const float* h_filter, int C, int K, int ks, con
 void tetris_g950_destroy(tetris_g950* p) {
   if (!p) return;
   for (auto& kv : p->bound) (void)hipFree(kv.second);
-  for (auto& kv : p->parts) (void)hipFree(kv.second);
+  for (auto& kv : p->parts) (void)hipFree(kv.second.base);
   (void)hipFree(p->d_grp_off);   // with the counts and the channel order
   (void)hipFree(p->d_position);  // with the values
   (void)hipFree(p->d_pgrp_off);

@@ -1,5 +1,5 @@
-"""Times the walking kernels and every configuration of the matrix kernel on a set of layers, and checks or fits the two time
-models that the library chooses between them with (matrix_time and walk_time in csrc/matrix_conv.hip).
+"""Times the walking kernels and every configuration of the two matrix kernels on a set of layers, and checks the time models that
+the library chooses between them with, or fits those of half_kernel and of the walk (csrc/matrix_conv.hip).
 
     make fit                                                  the library with the entry points used here
     TETRIS_SPCONV2D_LIB=$PWD/build_fit/libtetris_spconv2d.so python -m tetris_amd.kernel_times --measure FILE     (GPU)
@@ -21,8 +21,15 @@ import numpy as np
 import tetris_amd as T
 from tetris_amd import workloads as W
 
-CONFIGS = [(4, 4, 1), (4, 4, 2), (4, 2, 1), (4, 2, 2), (4, 2, 4), (2, 2, 1), (2, 2, 2), (2, 2, 4), (2, 1, 1), (2, 1, 2),
-           (2, 1, 4)]  # 32-channel blocks, pixel blocks per wave, teams: kConfigs
+# kMatShapes in csrc/matrix.h: a team's waves along the channels and along the pixels, pixel blocks of a wave, teams; those of
+# matrix_kernel, then those of half_kernel, four with long and six with short chunks of channels
+CONFIGS = [(4, 1, 4, 1), (4, 1, 4, 2), (4, 1, 2, 1), (4, 1, 2, 2), (4, 1, 2, 4), (2, 2, 2, 1), (2, 2, 2, 2), (2, 2, 2, 4),
+           (2, 2, 1, 1), (2, 2, 1, 2), (2, 2, 1, 4),
+           (8, 1, 2, 1), (4, 1, 2, 2), (2, 2, 1, 2), (8, 1, 4, 1),
+           (8, 1, 2, 1), (4, 1, 2, 2), (2, 2, 1, 1), (2, 2, 1, 2), (8, 1, 4, 1), (4, 2, 4, 1)]
+# half_kernel is taken where it is predicted to be faster than matrix_kernel by this, and its margin to the walking kernel is larger
+# by that (choose_mat_geom)
+BIAS, MORE = 1.05, 0.09
 SLICES = (1, 2, 3, 4, 6, 8)
 I16 = C.c_int * 16
 
@@ -53,7 +60,6 @@ def measure(path, count):
 
     time = T._lib.tetris_fit_time
     time.argtypes = [C.c_void_p] * 3 + [C.c_int] * 5 + [C.POINTER(T.Tile)] + [C.c_int] * 4 + [C.POINTER(C.c_float)]
-    settle = True
     with open(path, "w") as f:
         f.write("# N C H W K ks stride pad nnz  lanes_w quads oc_per_wave waves tile_ic csplit  walk  us per configuration %s "
                 "with %s slices\n" % (CONFIGS, SLICES))
@@ -61,6 +67,7 @@ def measure(path, count):
             n, c, h, w, k, ks, stride, pad = key
             rng = np.random.default_rng(i)
             filt = (rng.standard_normal((k, c, ks, ks)) * 0.05 * (rng.random((k, c, ks, ks)) >= sparsity)).astype(np.float32)
+            nnz = int(np.count_nonzero(filt))
             tile = T.tile_select(n, h, w, c, k, ks, stride, pad)
             pk = T.G950Filter.for_tile(filt, tile, oc_order="balanced")
             x = torch.rand((n, c, h, w), device="cuda").sub_(0.5).clamp_(min=0)
@@ -73,16 +80,13 @@ def measure(path, count):
                           C.byref(us))
                 return us.value if rc == 0 else None
 
-            if settle:  # the shader clock needs some 30 ms of work
-                run(-1, 1, 2000, 10)
-                settle = False
             out, info, pred = [], I16(), C.c_double()
-            best = run(-1, 1, 3, 10)
-            walk = min(best, run(-1, 1, 1, 10))
+            run(-1, 1, int(4e4 / run(-1, 1, 3, 5)), 1)  # after the pause for the filter the shader clock needs some 30 ms of work
+            best = walk = min(run(-1, 1, 3, 10), run(-1, 1, 1, 10))
             for cfg in range(len(CONFIGS)):
                 row = []
                 for s in SLICES:
-                    ok = T._lib.tetris_fit_matrix_geom(n, c, h, w, k, ks, stride, pad, cfg, s, info, C.byref(pred)) == 0
+                    ok = T._lib.tetris_fit_matrix_geom(n, c, h, w, k, ks, stride, pad, cfg, s, info, C.c_longlong(nnz), C.byref(pred)) == 0
                     first = run(cfg, s, 2, 5) if ok else None
                     if first is None or first > 3 * best:
                         row.append("-")
@@ -91,7 +95,6 @@ def measure(path, count):
                         best = min(best, first)
                         row.append("%.1f" % first)
                 out.append("|".join(row))
-            nnz = int(np.count_nonzero(filt))
             t = [tile.lanes_w, tile.quads, tile.oc_per_wave, tile.waves, tile.tile_ic, tile.csplit]
             f.write(" ".join(map(str, list(key) + [nnz] + t)) + " %.1f " % walk + " ".join(out) + "\n")
             f.flush()
@@ -117,8 +120,8 @@ def read(path):
         for cfg, field in enumerate(v[16:]):
             for s, us in zip(SLICES, field.split("|")):
                 if us != "-":
-                    T._check(T._lib.tetris_fit_matrix_geom(*order, cfg, s, info, C.byref(pred)))
-                    names = "ptiles mtiles csplit chunks kgs lpad OH OW lds mblocks steps".split()
+                    T._check(T._lib.tetris_fit_matrix_geom(*order, cfg, s, info, C.c_longlong(nnz), C.byref(pred)))
+                    names = "ptiles mtiles csplit chunks kgs lpad OH OW lds mblocks half".split()
                     rows.append((dict(layer, cfg=cfg, **dict(zip(names, info))), float(us), pred.value))
         out.append((walk, rows))
     return out
@@ -135,28 +138,31 @@ def filled(wgs, fit, cycles):
     return full * cycles(fit) + np.where(last > 0, cycles(last), 0)
 
 
-MATRIX0 = dict(start=3214, team=733, round1=1213, round3=2935, staging=293, step=469, product=1.08, launch=2.06,
-               reread=0.72, rate=4.26, weights=2.9, add=2.37, add_rate=3.95)
+HALF0 = dict(start=5339, team=1160, round1=275, round3=799, staging=638, step=202, issue=1.823, product=1.276, work=100,
+             launch=1.54, add=2.59, add_rate=4.52)
 
 
-def matrix_model(p, f):
-    wm, nb, kw = (np.array([CONFIGS[int(c)][i] for c in f["cfg"]]) for i in range(3))
-    regs = np.select([nb == 4, nb == 2, kw == 1, kw == 2], [2 // kw, np.maximum(1, 3 // kw), 5, 2], 1)
+def half_model(p, f):
+    wm, wn, nb, kw = (np.array([CONFIGS[int(c)][i] for c in f["cfg"]], np.float64) for i in range(4))
+    team = wm * wn
+    waves = team * kw
+    regs = np.maximum(1, np.floor(np.where(nb >= 2, 8, 12) / waves))
     fit = np.maximum(1, np.minimum(regs, np.floor(160 * 1024 / f["lds"])))
     rounds = np.ceil(np.ceil(f["chunks"] / f["csplit"]) / kw)
-    steps, staging = f["ks"] ** 2 * f["kgs"] / 2, np.ceil(f["kgs"] * f["lpad"] / 256)
+    density = np.minimum(1, f["nnz"] / (f["K"] * f["C"] * f["ks"] ** 2))
+    more = density ** 3 * (4 - 3 * density)
+    steps = np.ceil(f["C"] / 8) * f["ks"] ** 2 / f["chunks"] * (2 - (1 - more) ** 64) / 4 + 0.375
+    staging = f["kgs"] * f["lpad"] / 64 / team
     one = f["ks"] == 1
 
     def cycles(n):
-        step = np.maximum(np.where(one, 0, p["step"]), p["product"] * 256 * nb * kw * n)
-        return (p["start"] + p["team"] * nb * n * kw +
-                rounds * (np.where(one, p["round1"], p["round3"]) + p["staging"] * staging * kw * n + steps * step))
+        w = n * waves / 4
+        step = np.maximum(p["step"] + p["issue"] * 192 * nb, (p["work"] + p["product"] * 192 * nb) * w)
+        return p["start"] + p["team"] * nb * w + rounds * (np.where(one, p["round1"], p["round3"]) + p["staging"] * staging * w + steps * step)
 
-    compute = filled(f["ptiles"] * f["mtiles"] * f["csplit"], fit, cycles) / 2.2e3
     out = 4 * f["N"] * f["K"] * f["OH"] * f["OW"]
-    inp = 4 * f["N"] * f["C"] * np.where(one, f["OH"], f["H"]) * f["W"]
-    memory = (inp * (1 + p["reread"] * np.sqrt(f["mtiles"] - 1)) + out * f["csplit"] + p["weights"] * 3072 * f["mblocks"] * f["steps"]) / (p["rate"] * 1e6)
-    return p["launch"] + np.maximum(compute, memory) + np.where(f["csplit"] > 1, p["add"] + out * (f["csplit"] + 1) / (p["add_rate"] * 1e6), 0)
+    return p["launch"] + filled(f["ptiles"] * f["mtiles"] * f["csplit"], fit, cycles) / 2.3e3 + np.where(
+        f["csplit"] > 1, p["add"] + out * (f["csplit"] + 1) / (p["add_rate"] * 1e6), 0)
 
 
 WALK0 = dict(start2=9249, start3=10770, start4=8002, stage2=2913, stage3=5287, stage4=1239, busy2=1.55, busy3=0.905,
@@ -191,29 +197,34 @@ def fit(model, start, features, us, weight):
 
 def report(data, predict_matrix, predict_walk, margins):
     """what choosing by the two predictions gives over all layers, against the walk alone and the best of what was timed"""
-    off_m = np.log([predict_matrix(f, p) / us for _, rows in data for f, us, p in rows])
+    for half, name in ((0, "matrix_kernel"), (1, "half_kernel")):
+        off = np.log([predict_matrix(f, p) / us for _, rows in data for f, us, p in rows if f["half"] == half])
+        if len(off):
+            print("%s: %d times, predictions %+.1f %% on average, standard deviation %.1f %%" % (name, len(off), 100 * off.mean(), 100 * off.std()))
     off_w = np.log([predict_walk(w[0], w[2]) / w[1] for w, _ in data])
-    print("matrix kernel: %d times, predictions %+.1f %% on average, standard deviation %.1f %%" % (len(off_m), 100 * off_m.mean(), 100 * off_m.std()))
+    weighed = lambda f, p: predict_matrix(f, p) * (BIAS if f["half"] else 1)  # noqa: E731
     print("walking kernels: %d times, predictions %+.1f %% on average, standard deviation %.1f %%" % (len(off_w), 100 * off_w.mean(), 100 * off_w.std()))
     named = []
     for walk, rows in data:
         if rows:
-            us, pred = np.array([r[1] for r in rows]), np.array([predict_matrix(r[0], r[2]) for r in rows])
+            us, pred = np.array([r[1] for r in rows]), np.array([weighed(r[0], r[2]) for r in rows])
             named.append(us[pred.argmin()] / us.min())
     print("the configuration of least predicted time is %.1f %% slower than the fastest" % (100 * (np.exp(np.mean(np.log(named))) - 1)))
     for m in margins:
-        lost, gain, taken, slower = [], [], 0, []
+        lost, gain, taken, slower = [], [], [0, 0], []
         for walk, rows in data:
-            pw, pm = predict_walk(walk[0], walk[2]), [predict_matrix(r[0], r[2]) for r in rows]
-            use = rows and min(pm) < (1 - m) * pw
-            us = rows[int(np.argmin(pm))][1] if use else walk[1]
+            pw = predict_walk(walk[0], walk[2])
+            below = [r for r in rows if predict_matrix(r[0], r[2]) < (1 - m - (MORE if r[0]["half"] else 0)) * pw]
+            use = min(below, key=lambda r: weighed(r[0], r[2]), default=None)
+            us = use[1] if use else walk[1]
             lost.append(us / min([walk[1]] + [r[1] for r in rows]))
             gain.append(walk[1] / us)
-            taken += bool(use)
+            if use:
+                taken[int(use[0]["half"])] += 1
             if us > 1.03 * walk[1]:
                 slower.append(us / walk[1])
-        print("margin %.2f: matrix kernel on %d of %d layers; %.3f x the walk on (geometric) average, %.1f %% from the best choice; "
-              "%d layers more than 3 %% slower than the walk (worst %.2f x)" % (m, taken, len(data), np.exp(np.mean(np.log(gain))),
+        print("margin %.2f: matrix_kernel on %d and half_kernel on %d of %d layers; %.3f x the walk on (geometric) average, %.1f %% from the best choice; "
+              "%d layers more than 3 %% slower than the walk (worst %.2f x)" % (m, taken[0], taken[1], len(data), np.exp(np.mean(np.log(gain))),
               100 * (np.exp(np.mean(np.log(lost))) - 1), len(slower), max(slower, default=1)))
 
 
@@ -236,13 +247,15 @@ def main():
         for walk, rows in data:
             best = min([r[1] for r in rows], default=0)
             for f, us, _ in rows:
+                if not f["half"]:
+                    continue
                 fm.append(f), um.append(us), wm.append((best / us) ** 2 / math.sqrt(len(rows)))
-        pm = fit(matrix_model, MATRIX0, fm, um, np.array(wm))
+        pm = fit(half_model, HALF0, fm, um, np.array(wm))
         pw = fit(walk_model, WALK0, [w[0] for w, _ in data], [w[1] for w, _ in data], 1.0)
-        for name, p in (("matrix_time", pm), ("walk_time", pw)):
+        for name, p in (("half_time", pm), ("walk_time", pw)):
             print(name, ", ".join("%s %.4g" % kv for kv in p.items()))
-        one = lambda model, p: lambda f, _: float(model(p, columns([f]))[0])  # noqa: E731
-        report(data, one(matrix_model, pm), one(walk_model, pw), margins)
+        one = lambda model, p: lambda f, built: float(model(p, columns([f]))[0]) if f.get("half", 1) else built  # noqa: E731
+        report(data, one(half_model, pm), one(walk_model, pw), margins)
     else:
         sys.exit("one of --measure, --fit, --check")
 
