@@ -16,6 +16,11 @@ constexpr MatShape kMatShapes[] = {
     {8, 1, 2, 1, true, true}, {4, 1, 2, 2, true, true}, {2, 2, 1, 1, true, true}, {2, 2, 1, 2, true, true}, {8, 1, 4, 1, true, true}, {4, 2, 4, 1, true, true}};
 static_assert(sizeof kMatShapes / sizeof *kMatShapes == kMatConfigs);
 
+// whether four consecutive pixels of a tile lie side by side in memory, in one image and on 16 bytes
+inline bool stores_quads(const MatGeom& g, const float* d_out) {
+  return !g.pool && g.strips == 1 && g.OH * g.OW % 4 == 0 && reinterpret_cast<uintptr_t>(d_out) % 16 == 0;
+}
+
 // matrix_half.hip
 constexpr int kStepBytes = 3 * 1024 + 256, kSlotBytes = 2048;  // of a step's weights: fp16 parts and a word per lane; fp32
 size_t half_weight_bytes(const MatGeom& g);
@@ -49,10 +54,31 @@ __device__ __forceinline__ void cut(const float (&x)[8], u32x4& hi, u32x4& mid, 
   }
 }
 
+__device__ __forceinline__ unsigned bits_of(float x) { return __builtin_bit_cast(unsigned, x); }
+
 // maximum over the four lanes of a quad
 __device__ __forceinline__ float quad_max(float v) {
   v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true)));
   return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true)));
+}
+
+// value k of lane q of four neighbours becomes value q of lane k
+__device__ __forceinline__ void transpose_quad(float (&v)[4], int lane) {
+  auto from = [](float x, auto lanes) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(lanes)::value, 0xf, 0xf, true));
+  };
+  constexpr std::integral_constant<int, 0xB1> beside;  // lane ^ 1
+  constexpr std::integral_constant<int, 0x4E> across;  // lane ^ 2
+  const bool odd = lane & 1, high = lane & 2;
+  float o[4], a[4];  // (the exchanges outside of the choices: all lanes take part)
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = from(v[k ^ 1], beside);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = odd == (k & 1) ? v[k] : o[k];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = from(a[k ^ 2], across);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = high == (k >> 1) ? a[k] : o[k];
 }
 
 }  // namespace

@@ -240,19 +240,39 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
     const int oc = oc0 + 8 * (i / 4) + i % 4;
     if (g.pool) v = quad_max(v);
     if (g.relu) v = fmaxf(v, 0.f);
-    if (oc + 4 * (lane >> 5) < g.K && ooff[b] != kOutside)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), orsrc, ooff[b], oc * ohw * 4, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), orsrc, oc + 4 * (lane >> 5) < g.K ? ooff[b] : kOutside, oc * ohw * 4, 0);
   };
   float odd = 0;  // NaN once a sum is infinite or NaN
-  auto finish = [&](int i, int b, float v) {
-    odd = fmaf(v, 0.f, odd);
-    store(i, b, v * kUnscale);
+  auto finish = [&](int i, int b, float (&v)[4]) {  // sums i to i + 3
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      odd = fmaf(v[k], 0.f, odd);
+      v[k] *= kUnscale;
+    }
+    if (g.quads) {
+      // Four pixels of a channel to a lane instead of four channels of a pixel: a store of 16 bytes instead of four.  The
+      // stores, 16 cycles each for the address unit of a CU, are what the end of a tile waits for.
+      transpose_quad(v, lane);
+      u32x4 d;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[k] = bits_of(g.relu ? fmaxf(v[k], 0.f) : v[k]);
+      const bool inside = oc0 + 2 * i + 4 * (lane >> 5) + (lane & 3) < g.K && ooff[b] != kOutside;
+      __builtin_amdgcn_raw_buffer_store_b128(d, orsrc, inside ? ooff[b] + 4 * (lane & 3) * (ohw - 1) : kOutside, (oc0 + 2 * i) * ohw * 4, 0);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) store(i + k, b, v[k]);
+    }
   };
   if constexpr (KW == 1) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
+    for (int i = 0; i < 16; i += 4)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) finish(i, b, acc[b][i] + low[b][i]);
+      for (int b = 0; b < NB; ++b) {
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = acc[b][i + k] + low[b][i + k];
+        finish(i, b, v);
+      }
   } else {
     // every team leaves its sums in LDS and adds a share of all of them
     float* sums = reinterpret_cast<float*>(all_lds) + wave * 1024 * NB + lane;
@@ -262,13 +282,17 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
       for (int b = 0; b < NB; ++b) sums[team * 4096 * NB + (i * NB + b) * 64] = acc[b][i] + low[b][i];
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < 16; i += 4) {
       if (i / (16 / KW) != team) continue;
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        float v = sums[(i * NB + b) * 64];
+        float v[4];
 #pragma unroll
-        for (int k = 1; k < KW; ++k) v += sums[k * 4096 * NB + (i * NB + b) * 64];
+        for (int j = 0; j < 4; ++j) {
+          v[j] = sums[((i + j) * NB + b) * 64];
+#pragma unroll
+          for (int k = 1; k < KW; ++k) v[j] += sums[k * 4096 * NB + ((i + j) * NB + b) * 64];
+        }
         finish(i, b, v);
       }
     }
@@ -601,6 +625,7 @@ int launch_matrix(const MatGeom& g, const float* d_in, float* d_out, const MatWe
   const void* weights = w.base;
   MatGeom k = g;
   k.relu = relu;
+  k.quads = stores_quads(g, d_out);
   const bool two = g.kgs * g.lpad / 64 <= 8;
 #define TETRIS_MAT(WM, NB, KW) \
   if (c.wm == WM && c.nb == NB && c.kw == KW) \

@@ -49,7 +49,6 @@ typedef unsigned u32x8 __attribute__((ext_vector_type(8)));
 // of the largest would still be the sum of their parts, but of subnormal ones, whose left-out products are not small any more.)
 constexpr float kMid = 256.f, kLow = 128.f;  // from h to m, from m to l
 
-__device__ __forceinline__ unsigned bits_of(float x) { return __builtin_bit_cast(unsigned, x); }
 // (A bit cast of a vector's element itself, instead of its value, is compiled to one of the vector's first element.)
 __device__ __forceinline__ float float_of(unsigned x) { return __builtin_bit_cast(float, x); }
 
@@ -110,25 +109,6 @@ __device__ __forceinline__ unsigned wave_max(unsigned v) {
   step(std::integral_constant<int, 0x142>{});
   step(std::integral_constant<int, 0x143>{});
   return __builtin_amdgcn_readlane(v, 63);
-}
-
-// value k of lane q of four neighbours becomes value q of lane k
-__device__ __forceinline__ void transpose_quad(float (&v)[4], int lane) {
-  auto from = [](float x, auto lanes) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(lanes)::value, 0xf, 0xf, true));
-  };
-  constexpr std::integral_constant<int, 0xB1> beside;  // lane ^ 1
-  constexpr std::integral_constant<int, 0x4E> across;  // lane ^ 2
-  const bool odd = lane & 1, high = lane & 2;
-  float o[4], a[4];  // (the exchanges outside of the choices: all lanes take part)
-#pragma unroll
-  for (int k = 0; k < 4; ++k) o[k] = from(v[k ^ 1], beside);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) a[k] = odd == (k & 1) ? v[k] : o[k];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) o[k] = from(a[k ^ 2], across);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) v[k] = high == (k >> 1) ? a[k] : o[k];
 }
 
 // x / d through magic_reciprocal(d), which is 0 for d = 1
@@ -855,8 +835,7 @@ int half_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, voi
 int launch_half(const MatGeom& g, const float* d_in, float* d_out, const MatWeights& weights, int relu, hipStream_t stream) {
   MatGeom k = g;
   k.relu = relu;
-  // four consecutive pixels of a tile lie side by side in memory, in one image and 16-byte aligned
-  k.quads = !g.pool && g.strips == 1 && g.OH * g.OW % 4 == 0 && reinterpret_cast<uintptr_t>(d_out) % 16 == 0;
+  k.quads = stores_quads(g, d_out);
   const MatShape& c = kMatShapes[g.cfg];
   const bool two = g.kgs * g.lpad / 64 <= 2 * c.wm * c.wn;
 #define TETRIS_MAT(WM, WN, NB, KW) \
