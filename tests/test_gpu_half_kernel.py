@@ -59,7 +59,10 @@ class Layer:
     (4, 17, 70, 26, 166, 6, 1, 0, 0.3),    # ... 6 x 6
     (12, 53, 27, 35, 7, 4, 1, 0, 0.15),    # 64 by 64, two teams
     (1, 21, 8, 8, 3, 7, 1, 3, 0.3),        # ... an image of one tile
-    (8, 19, 79, 28, 275, 3, 1, 0, 0.3),    # 256 by 128
+    (8, 33, 47, 63, 68, 5, 1, 0, 0.3),     # 256 by 96: an odd number of blocks of pixels
+    (11, 120, 18, 70, 11, 7, 2, 0, 0.2),   # ... in slices; 7 x 7
+    (12, 111, 23, 78, 21, 3, 2, 1, 0.15),  # ... short chunks
+    (8, 19, 79, 28, 275, 3, 1, 0, 0.3),    # 128 by 192
     (12, 17, 73, 24, 85, 2, 3, 1, 0.15),   # short chunks: 256 by 64
     (3, 95, 9, 8, 3, 4, 3, 0, 0.3),        # ... in slices
     (5, 17, 67, 31, 74, 4, 1, 2, 0.2),     # ... 128 by 64, two teams
@@ -78,6 +81,32 @@ def test_layer(N, C, H, W, K, ks, stride, pad, density):
     # lose no more than the walking kernel's FMAs do
     assert (np.abs(got - ref) <= C * ks * ks * 2.0 ** -24 * terms).all()
     assert np.linalg.norm(got - ref) <= 1.05 * np.linalg.norm(walk - ref)
+    layer.pack.close()
+
+
+@pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad,density", [
+    (3, 42, 40, 77, 81, 3, 1, 1, 0.15), (8, 33, 47, 63, 68, 5, 1, 0, 0.3), (11, 120, 18, 70, 11, 7, 2, 0, 0.2),
+    (8, 19, 79, 28, 275, 3, 1, 0, 0.3), (1, 20, 28, 8, 10, 4, 1, 0, 0.3)])
+def test_activations(N, C, H, W, K, ks, stride, pad, density):
+    import torch
+    import tetris_amd as T
+
+    rng = np.random.default_rng(K)
+    w, x = filter_of(rng, K, C, ks, density), rng.standard_normal((N, C, H, W)).astype(np.float32)
+    layer = Layer(w, x.shape, stride, pad)
+    ref, terms = conv64(x, w, stride, pad)
+    bound = C * ks * ks * 2.0 ** -24 * terms
+    dx, (oh, ow) = torch.from_numpy(x).cuda(), layer.out[2:]
+    y = torch.full(layer.out, float("nan"), device="cuda")
+    layer.pack.launch_act(dx.data_ptr(), y.data_ptr(), *layer.at, layer.tile, T.ACT_RELU)
+    torch.cuda.synchronize()
+    assert (np.abs(y.cpu().numpy() - np.maximum(ref, 0)) <= bound).all()
+    if layer.pack.act_supported(*layer.at, layer.tile, T.ACT_RELU_POOL2):
+        pooled = torch.full((N, K, oh // 2, ow // 2), float("nan"), device="cuda")
+        layer.pack.launch_act(dx.data_ptr(), pooled.data_ptr(), *layer.at, layer.tile, T.ACT_RELU_POOL2)
+        torch.cuda.synchronize()
+        most = lambda a: a[:, :, :oh // 2 * 2, :ow // 2 * 2].reshape(N, K, oh // 2, 2, ow // 2, 2).max((3, 5))  # noqa: E731
+        assert (np.abs(pooled.cpu().numpy() - np.maximum(most(ref), 0)) <= most(bound)).all()
     layer.pack.close()
 
 

@@ -202,7 +202,7 @@ struct MatWeights {
   int step_bytes;       // of all steps
   int wide;             // some weight is not the sum of its fp16 parts
 };
-constexpr int kMatConfigs = 21;
+constexpr int kMatConfigs = 23;
 constexpr int kMatTasks = 4;        // most blocks of 64 staged pixels x 8 channels that a wave holds at a time
 constexpr int kMatLds = 160 * 1024;
 constexpr long long kMatCopies = 32 << 20;  // most bytes of partial sums of a split layer
@@ -343,7 +343,7 @@ int add_copies(const float* d_copies, float* d_out, int N, int K, int OH, int OW
 
 // matrix_conv.hip
 // staged (may be null): of the same layer, what earlier calls found (zeros: nothing yet)
-using StagedPixels = std::array<int, 3>;  // of the largest tile of 64 and of 128 pixels
+using StagedPixels = std::array<int, 9>;  // of the largest tile of 32, 64, ... pixels
 bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out,
                    StagedPixels* staged = nullptr);
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,

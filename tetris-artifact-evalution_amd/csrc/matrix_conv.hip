@@ -473,7 +473,7 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
   g.ptiles = ceil_div(g.npix, P);
   g.mtiles = ceil_div(g.mblocks, c.wm);
   StagedPixels one{};
-  int& most = (staged ? *staged : one)[P / 128];  // tiles are of 64, 128 or 256 pixels
+  int& most = (staged ? *staged : one)[P / 32];
   if (!most) most = staged_pixels(g, P);
   g.lpad = ceil_div(most, 64) * 64;
   if (g.kgs * g.lpad / 64 > c.wm * c.wn * (g.half && c.nb == 4 ? 2 : kMatTasks) || lds_bytes(g) > kMatLds) return false;
@@ -494,7 +494,7 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
 }
 
 // Microseconds of a launch.  The constants were fitted to the times of a kernel with six products a step, whose cycles
-// were then scaled by 8/6.  Against 13 413 timed launches of 424 layers -- those of the benchmark's suites at batch 1, 4
+// were then scaled by 8/6.  Against 13 462 timed launches of 424 layers -- those of the benchmark's suites at batch 1, 4
 // and 16 and 160 random ones, every configuration and slice count: profiles/kernel_times.txt, measured and checked by
 // tetris_amd/kernel_times.py -- they are 11 % off (standard deviation).  A fit to these times, with a term for the weights'
 // bytes, is 11 % off as well and not faster in any network (VGG19 at batch 1: 408 us, 400 with these).
@@ -518,7 +518,7 @@ double plain_time(const MatGeom& g) {
   return 2.2 + std::max(compute, memory) + (g.csplit > 1 ? 2.5 + out * (g.csplit + 1) / 4.07e6 : 0);
 }
 
-// The same for half_kernel, fitted to 11 063 launches of the same layers: 9 % off.
+// The same for half_kernel, fitted to 13 801 launches of the same layers: 9 % off.
 double half_time(const MatGeom& g, long long nnz) {
   const MatShape& c = kMatShapes[g.cfg];
   const int team = c.wm * c.wn, waves = team * c.kw;
@@ -534,12 +534,12 @@ double half_time(const MatGeom& g, long long nnz) {
   auto cycles = [&](int n) {
     if (n == 0) return 0.0;
     const double per_simd = n * waves / 4.0, products = 192.0 * c.nb;
-    const double step = std::max(202.0 + 1.823 * products, (100.0 + 1.276 * products) * per_simd);
-    return 5339.0 + 1160.0 * c.nb * per_simd + rounds * ((g.ks == 1 ? 275.0 : 799.0) + 638.0 * staging * per_simd + steps * step);
+    const double step = std::max(165.0 + 2.032 * products, (87.0 + 1.231 * products) * per_simd);
+    return 4973.0 + 1257.0 * c.nb * per_simd + rounds * ((g.ks == 1 ? 221.0 : 722.0) + 681.0 * staging * per_simd + steps * step);
   };
   const int full = wgs / (256 * fit), rest = wgs % (256 * fit);
   const double out = 4.0 * g.N * g.K * g.OH * g.OW;
-  return 1.54 + (full * cycles(fit) + cycles(ceil_div(rest, 256))) / 2.3e3 + (g.csplit > 1 ? 2.59 + out * (g.csplit + 1) / 4.52e6 : 0);
+  return 1.67 + (full * cycles(fit) + cycles(ceil_div(rest, 256))) / 2.3e3 + (g.csplit > 1 ? 2.48 + out * (g.csplit + 1) / 4.3e6 : 0);
 }
 
 double matrix_time(const MatGeom& g, long long nnz) { return g.half ? half_time(g, nnz) : plain_time(g); }
@@ -564,11 +564,11 @@ double walk_time(const Geom& g, long long nnz) {
 
 // Whether a matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and slice
 // count of least predicted time, if that is 7 % below the walking kernel's; half_kernel's, if that is 16 % below the walking
-// kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's.  Of the 424 timed layers 138
-// then go to matrix_kernel and 69 to half_kernel; over all of them that is 1.173 times the walk's speed, 2.8 % short of the
-// best choice, 10 layers lose more than 3 % to the walk and one to what matrix_kernel and the walk alone would give it.
-// (Without half_kernel 1.142 times.  With 14 %: one layer in 424 less well chosen; with 10 % and no advantage asked over
-// matrix_kernel 13 of them, and networks are slower: yolov3's backbone at batch 16 4.82 ms, 4.70 so.)  Where the walking
+// kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's.  Of the 424 timed layers 125
+// then go to matrix_kernel and 96 to half_kernel; over all of them that is 1.196 times the walk's speed, 2.8 % short of the
+// best choice, 10 layers lose more than 3 % to the walk and two to what matrix_kernel and the walk alone would give them.
+// (Without half_kernel 1.152 times.  With 12 % to the walk eight layers lose so, with 10 % and no advantage asked over
+// matrix_kernel 22.)  Where the walking
 // kernel can pool its outputs, so must the matrix kernel.
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      MatGeom* g, MatGeom* pool) {

@@ -23,7 +23,7 @@
 // of the time); for small layers the start, 5400 cycles, in which arguments, lists and input arrive one after the other.
 // Microseconds, matrix_conv.hip's best against this, the walk in brackets: 16 x 128 -> 128 28x28 3x3 of 85 % zeros 30.3, 23.8
 // (31.3); 16 x 256 -> 256 28x28 to 14x14 of 85 % 44.9, 33.9 (45.0); 4 x 256 -> 256 28x28 of 90 % 35.3, 25.9 (33.3); 16 x 256 ->
-// 512 26x26 of 85 % 155, 125 (124).
+// 512 26x26 of 85 % 148, 103 (125) -- of 226 tiles of 96 pixels; 170 of 128 pixels leave a third of the CUs idle: 125.
 //
 // Range: inputs are scaled by what a few of them, the same for all waves, show; where some input is then not the sum of its parts
 // (smaller than 2^-28 of those few, or 2^4 times as large) the workgroup makes a second pass with bf16 parts, which hold every
@@ -344,7 +344,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int i = 0; i < 16; ++i) sum[0][b][i] = sum[1][b][i] = 0.f;
-  constexpr int kSets = F16 ? NB == 4 ? 2 : 3 : 1;
+  constexpr int kSets = F16 ? NB > 2 ? 2 : 3 : 1;
   Step ahead[kSets];
 #pragma unroll
   for (int i = 0; F16 && i < kSets; ++i) {
@@ -391,7 +391,9 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     place_of(ahead[0].word);
     read(input[0], 0);
   }
-  auto step = [&](Step& now, Step& next) {
+  // Where a wave has an odd number of blocks, more than one, two steps take turns with the two places for a block's input.
+  auto step = [&](Step& now, Step& next, auto turn) {
+    constexpr int kFirst = NB > 1 && NB % 2 ? decltype(turn)::value % 2 : 0, kNext = (kFirst + (NB > 1 ? NB : 0)) % 2;
     if constexpr (!F16) {
       fetch_weights(now);
       place_of(now.word);
@@ -399,7 +401,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     }
     const unsigned word = now.word;
     const bool last = __builtin_amdgcn_readfirstlane(word) >> 31, more = round + 1 < mine;
-    if constexpr (NB > 1) read(input[1], 1);
+    if constexpr (NB > 1) read(input[1 - kFirst], 1);
     if constexpr (F16) __builtin_amdgcn_sched_barrier(0);
     u32x4 a[F16 ? 6 : 3];
     if constexpr (F16) {
@@ -427,10 +429,10 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     };
 #pragma unroll
     for (int b = 0; b < (NB > 1 ? NB - 1 : 1); ++b) {
-      products(input[b & 1], b);
+      products(input[(kFirst + b) % 2], b);
       if (b > 0 || NB > 2) {
         if constexpr (F16) __builtin_amdgcn_sched_barrier(0);
-        if (b + 2 < NB) read(input[b & 1], b + 2);
+        if (b + 2 < NB) read(input[(kFirst + b) % 2], b + 2);
         if constexpr (F16) __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -448,15 +450,15 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
       if constexpr (F16) {
         __builtin_amdgcn_sched_barrier(0);
         place_of(next.word);
-        read(input[0], 0);
+        read(input[kNext], 0);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (NB > 1) products(input[1], NB - 1);
+      if constexpr (NB > 1) products(input[(kFirst + NB - 1) % 2], NB - 1);
       refill();
       return;
     }
     // the chunk's last
-    if constexpr (NB > 1) products(input[1], NB - 1);
+    if constexpr (NB > 1) products(input[(kFirst + NB - 1) % 2], NB - 1);
     refill();
     if (!F16 && more) fetch(c_beg + round + 1);  // (the second pass is rare: fewer registers instead of less waiting)
     if (more) keep(buf ^ 1);
@@ -467,17 +469,20 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     __syncthreads();
     if constexpr (F16) {
       place_of(next.word);
-      read(input[0], 0);
+      read(input[kNext], 0);
     }
   };
   for (int left = steps; left > 0; left -= kSets) {
-    step(ahead[0], ahead[1 % kSets]);
-#pragma unroll
-    for (int i = 1; i < kSets; ++i) {
-      // (Waiting for all loads when the steps run out costs nothing that matters, and tells the compiler that at the head
-      // of the loop the first set's loads are the oldest.)
-      if (left > i) step(ahead[i], ahead[(i + 1) % kSets]);
+    step(ahead[0], ahead[1 % kSets], std::integral_constant<int, 0>{});
+    // (Waiting for all loads when the steps run out costs nothing that matters, and tells the compiler that at the head of the
+    // loop the first set's loads are the oldest.)
+    if constexpr (kSets > 1) {
+      if (left > 1) step(ahead[1], ahead[2 % kSets], std::integral_constant<int, 1>{});
       else __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    }
+    if constexpr (kSets > 2) {
+      if (left > 2) step(ahead[2], ahead[0], std::integral_constant<int, 2>{});
+      else __builtin_amdgcn_s_waitcnt(0x0f70);
     }
   }
   if (round < rounds) {  // a team with a chunk less
@@ -842,7 +847,8 @@ int launch_half(const MatGeom& g, const float* d_in, float* d_out, const MatWeig
   if (c.wm == WM && c.wn == WN && c.nb == NB && c.kw == KW) \
     return two ? launch_one<WM, WN, NB, KW, 2>(k, d_in, d_out, weights, stream) \
                : launch_one<WM, WN, NB, KW, NB == 4 ? 2 : kMatTasks>(k, d_in, d_out, weights, stream);
-  TETRIS_MAT(8, 1, 2, 1) TETRIS_MAT(4, 1, 2, 2) TETRIS_MAT(2, 2, 1, 1) TETRIS_MAT(2, 2, 1, 2) TETRIS_MAT(8, 1, 4, 1) TETRIS_MAT(4, 2, 4, 1)
+  TETRIS_MAT(8, 1, 2, 1) TETRIS_MAT(4, 1, 2, 2) TETRIS_MAT(2, 2, 1, 1) TETRIS_MAT(2, 2, 1, 2) TETRIS_MAT(8, 1, 3, 1) TETRIS_MAT(4, 2, 3, 1) TETRIS_MAT(8, 1, 4, 1)
+  TETRIS_MAT(4, 2, 4, 1)
 #undef TETRIS_MAT
   return fail(TETRIS_EINVAL, "no matrix kernel of configuration %d", g.cfg);
 }

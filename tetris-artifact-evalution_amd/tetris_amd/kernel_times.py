@@ -22,11 +22,11 @@ import tetris_amd as T
 from tetris_amd import workloads as W
 
 # kMatShapes in csrc/matrix.h: a team's waves along the channels and along the pixels, pixel blocks of a wave, teams; those of
-# matrix_kernel, then those of half_kernel, four with long and six with short chunks of channels
+# matrix_kernel, then those of half_kernel, four with long and eight with short chunks of channels
 CONFIGS = [(4, 1, 4, 1), (4, 1, 4, 2), (4, 1, 2, 1), (4, 1, 2, 2), (4, 1, 2, 4), (2, 2, 2, 1), (2, 2, 2, 2), (2, 2, 2, 4),
            (2, 2, 1, 1), (2, 2, 1, 2), (2, 2, 1, 4),
-           (8, 1, 2, 1), (4, 1, 2, 2), (2, 2, 1, 2), (8, 1, 4, 1),
-           (8, 1, 2, 1), (4, 1, 2, 2), (2, 2, 1, 1), (2, 2, 1, 2), (8, 1, 4, 1), (4, 2, 4, 1)]
+           (8, 1, 2, 1), (8, 1, 3, 1), (4, 1, 2, 2), (2, 2, 1, 2),
+           (8, 1, 2, 1), (8, 1, 3, 1), (8, 1, 4, 1), (4, 2, 3, 1), (4, 2, 4, 1), (4, 1, 2, 2), (2, 2, 1, 1), (2, 2, 1, 2)]
 # half_kernel is taken where it is predicted to be faster than matrix_kernel by this, and its margin to the walking kernel is larger
 # by that (choose_mat_geom)
 BIAS, MORE = 1.05, 0.09
@@ -138,8 +138,8 @@ def filled(wgs, fit, cycles):
     return full * cycles(fit) + np.where(last > 0, cycles(last), 0)
 
 
-HALF0 = dict(start=5339, team=1160, round1=275, round3=799, staging=638, step=202, issue=1.823, product=1.276, work=100,
-             launch=1.54, add=2.59, add_rate=4.52)
+HALF0 = dict(start=4973, team=1257, round1=221, round3=722, staging=681, step=165, issue=2.032, product=1.231, work=87,
+             launch=1.67, add=2.48, add_rate=4.3)
 
 
 def half_model(p, f):
