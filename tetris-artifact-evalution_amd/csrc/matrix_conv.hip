@@ -574,7 +574,8 @@ bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int 
                      MatGeom* g, MatGeom* pool) {
   if (C < 16) return false;  // most of a chunk of 16 channels would be padding
   const bool pools = walk.OH >= 2 && walk.OW >= 2 && (walk.csplit > 1 || geom_pools_in_kernel(walk));
-  std::vector<std::pair<double, MatGeom>> found;
+  struct Found { double t; int cfg, slices; };
+  std::vector<Found> found;
   StagedPixels staged{};
   const double walking = walk_time(walk, nnz);
   for (int cfg = 0; cfg < kMatConfigs; ++cfg) {
@@ -584,20 +585,17 @@ bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int 
       if (m.chunks / slices < (m.half ? kMatShapes[cfg].kw : 1) || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
       m.csplit = slices;
       const double t = matrix_time(m, nnz);
-      if (t < (m.half ? 0.84 : 0.93) * walking) found.emplace_back(m.half ? 1.05 * t : t, m);
+      if (t < (m.half ? 0.84 : 0.93) * walking) found.push_back({m.half ? 1.05 * t : t, cfg, slices});
     }
   }
-  std::stable_sort(found.begin(), found.end(),
-                   [](const std::pair<double, MatGeom>& a, const std::pair<double, MatGeom>& b) { return a.first < b.first; });
-  for (const auto& f : found) {
+  std::stable_sort(found.begin(), found.end(), [](const Found& a, const Found& b) { return a.t < b.t; });
+  for (const Found& f : found) {
     *pool = MatGeom{};
-    if (f.second.csplit == 1 && walk.OH >= 2 && walk.OW >= 2 &&
-        !make_mat_geom(N, C, H, W, K, ks, stride, pad, f.second.cfg, 1, true, pool)) {
+    if (f.slices == 1 && walk.OH >= 2 && walk.OW >= 2 && !make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool)) {
       *pool = MatGeom{};
       if (pools) continue;
     }
-    *g = f.second;
-    return true;
+    return make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, f.slices, false, g, &staged);
   }
   return false;
 }
