@@ -125,7 +125,7 @@ typedef struct tetris_tile {
  * A launch with the library's own choice -- a NULL tile, or the one named here, unless a loaded row names it -- may run on
  * the matrix cores instead of walking the non-zeros, where a time model says that this is at least 7 % faster: the same
  * fp32 convolution, each number cut into three 16-bit parts (eight of the nine products formed of bf16 parts, six of fp16
- * ones, which is all that 2^-30 of a product needs), with fp32 sums.  Its
+ * ones, of numbers for which those leave out less than 2^-28 of a product), with fp32 sums.  Its
  * error against 64-bit sums is no larger than the walking kernels', and infinities, NaN and numbers at either end of
  * fp32's range give what they give there.  tetris_launch_shape_of says which kernel runs; any other tile is obeyed. */
 int tetris_tile_select(int batch, int img_h, int img_w, int in_channel, int out_channel, int kernel_size, int stride,

@@ -151,6 +151,35 @@ def test_inputs_of_any_scale(what):
     layer.pack.close()
 
 
+@pytest.mark.parametrize("what,large,small", [
+    ("8 bits", 0, -38), ("8 bits", 0, -40), ("one bit", 0, -44), ("bf16", 0, -36),  # their parts add up to them, and are not enough
+    ("24 bits", 0, -24), ("24 bits", 0, -27), ("24 bits", 0, -28), ("24 bits", 0, -29), ("24 bits", 0, -34),
+    ("24 bits", 44, -126), ("24 bits", 60, -110), ("24 bits", 72, -100), ("24 bits", 110, -60), ("24 bits", 100, -130)])  # lost in its scale
+@pytest.mark.parametrize("at", [LAYER, (8, 19, 79, 28, 275, 3, 1, 1, 0.3)])
+def test_small_inputs_beside_large_ones(at, what, large, small):
+    """Stripes of small inputs between stripes of large ones, which the whole tile is scaled by: where an output is a sum of small ones
+    alone, it is as exact as the walk's, whatever their size and their number of significant bits."""
+    N, C, H, W, K, ks, stride, pad, density = at
+    rng = np.random.default_rng(4)
+    w = filter_of(rng, K, C, ks, density)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    tiny = {"8 bits": rng.integers(0, 256, x.shape) / 256, "one bit": rng.integers(0, 2, x.shape),
+            "bf16": (x.view(np.uint32) & 0xffff0000).view(np.float32), "24 bits": x}[what].astype(np.float32)
+    stripe = np.arange(W) // 6 % 2 == 1
+    x = np.where(stripe, np.ldexp(tiny, small), np.ldexp(x, large)).astype(np.float32)
+    layer = Layer(w, x.shape, stride, pad)
+    got, walk = layer(x), layer(x, layer.walk())
+    alone = conv64((x != 0) * ~stripe * np.float32(1), (w != 0).astype(np.float32), stride, pad)[0] == 0
+    x[..., ~stripe] = 0
+    ref, terms = conv64(x, w, stride, pad)
+    assert alone.mean() > 0.2
+    count = (w != 0).reshape(K, -1).sum(1).reshape(1, K, 1, 1)
+    assert (np.abs(got - ref) <= count * 2.0 ** -24 * terms + 2.0 ** -149)[alone].all()
+    if small > -120:  # (a subnormal output is rounded twice)
+        assert np.linalg.norm((got - ref)[alone]) <= 1.05 * np.linalg.norm((walk - ref)[alone])
+    layer.pack.close()
+
+
 @pytest.mark.parametrize("value,count", [(2.0 ** -20, 1), (2.0 ** -40, 60), (2.0 ** -40, 3000), (2.0 ** -100, 1), (2.0 ** -149, 2), (2.0 ** 63, 1)])
 def test_small_weights(value, count):
     """Weights far below the largest of their row: multiplied one by one; all with bf16 parts where they are many, or where their

@@ -6,7 +6,8 @@
 //     so that h times h has 16: sums of such products are rounded hardly ever, which is what keeps the whole as exact as bf16
 //     parts do.  With eleven bits in h an output was off twice as far (1.9e-7 of the largest against 1.0e-7, 16 x 128 channels
 //     3x3).  To need six products nevertheless, a weight is also written as near + off, eleven bits and the rest, made in
-//     registers from its parts: h xh + 2^-8 (m xh + l xh + off xm + near xm + near xl), which leaves out less than 2^-30.
+//     registers from its parts: h xh + 2^-8 (m xh + l xh + off xm + near xm + near xl).  What that leaves out, off xl, is less than
+//     2^-29.5 of the product, of the smallest inputs that are multiplied so (below) 2^-28.
 //   * k-values: v_smfmac takes a left operand of which two in four consecutive k-values are kept, at the rate of a dense
 //     product of half as many (32 cycles for 32 x 32 x 32, measured: 3.3 PFLOP/s of what it stands for, 1.7 dense).  Blocks --
 //     one tap of 8 channels for 32 output channels -- with three or four weights in a group of four come twice, blocks of
@@ -25,10 +26,12 @@
 // (31.3); 16 x 256 -> 256 28x28 to 14x14 of 85 % 44.9, 33.9 (45.0); 4 x 256 -> 256 28x28 of 90 % 35.3, 25.9 (33.3); 16 x 256 ->
 // 512 26x26 of 85 % 148, 103 (125) -- of 226 tiles of 96 pixels; 170 of 128 pixels leave a third of the CUs idle: 125.
 //
-// Range: inputs are scaled by what a few of them, the same for all waves, show; where some input is then not the sum of its parts
-// (smaller than 2^-28 of those few, or 2^4 times as large) the workgroup makes a second pass with bf16 parts, which hold every
-// number (see matrix_conv.hip for those, and for what is out of their range: the third pass).  Weights that fp16 parts do not
-// hold are few: FMAs add them at the end.
+// Range: inputs are scaled by what a few of them, the same for all waves, show.  Where some input is 2^4 times as large as those, or
+// smaller than 2^-27 of the largest of them and not zero, the workgroup makes a second pass with bf16 parts, which hold every number
+// (see matrix_conv.hip for those, and for what is out of their range: the third pass).  An input's size decides, and not
+// whether its parts add up to it: with few significant bits they do so far below, where m has lost bits to fp16's smallest
+// exponent, l carries the number, and off xl is 2^-17 of the product and more.  Weights that fp16 parts do not hold are few: FMAs
+// add them at the end.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -48,6 +51,7 @@ typedef unsigned u32x8 __attribute__((ext_vector_type(8)));
 // brings the largest of its row to [2^14, 2^15) likewise.  h has eight bits, m eleven, l the rest.  (With 2^-19 l inputs of 2^-32
 // of the largest would still be the sum of their parts, but of subnormal ones, whose left-out products are not small any more.)
 constexpr float kMid = 256.f, kLow = 128.f;  // from h to m, from m to l
+constexpr float kSmall = 0x1p-16f;  // the smallest scaled input that is multiplied in parts: from here on all 24 bits are in them
 
 // (A bit cast of a vector's element itself, instead of its value, is compiled to one of the vector's first element.)
 __device__ __forceinline__ float float_of(unsigned x) { return __builtin_bit_cast(float, x); }
@@ -226,15 +230,20 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
       }
     }
   };
-  unsigned rest = 0;
+  unsigned rest = 0, least = ~0u;  // least: of the inputs' bits without the sign, doubled, less one: zeros come out on top
   float scale = 1.f;
   auto keep = [&](int buf) {
 #pragma unroll
     for (int k = 0; k < TM; ++k) {
       if (wave + TW * k >= tasks) break;
       u32x4 h, m, l;
-      if constexpr (F16) cut16(x[k], scale, h, m, l, rest);
-      else cut(x[k], h, m, l);
+      if constexpr (F16) {
+        cut16(x[k], scale, h, m, l, rest);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) least = min(least, (bits_of(x[k][j]) << 1) - 1);
+      } else {
+        cut(x[k], h, m, l);
+      }
       u32x4* d = lds + buf * 3 * at.kgs * at.lpad + gslot[k];
       d[0] = h;
       d[1] = m;
@@ -352,7 +361,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     __builtin_amdgcn_sched_barrier(0);  // in this order: the loop waits for the first set only
   }
   if constexpr (F16) {
-    // Their largest is scaled to [2^11, 2^12): with 4 bits to spare above, an input is the sum of its parts down to 2^-30 of it.
+    // Their largest is scaled to [2^11, 2^12): with 4 bits to spare above, down to 2^-27 or 2^-28 of it.
     unsigned most = max(max(some[0] & 0x7fffffff, some[1] & 0x7fffffff), max(some[2] & 0x7fffffff, some[3] & 0x7fffffff));
     most = wave_max(most);
     const int shift = most ? min(max(138 - (int)(most >> 23), -100), 100) : 6;
@@ -362,6 +371,9 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   if (F16 && thread == 0) *inexact = w.wide;
   keep(0);
   __syncthreads();
+  // whether the inputs that were staged are what six products can be formed of: the sums of their parts, and none but zeros below
+  // kSmall / scale (looked at before it is scaled, where it may underflow)
+  auto held = [&]() { return __ballot(rest != 0 || least < 2 * (bits_of(kSmall) + bits_of(1.f) - bits_of(scale)) - 1) == 0; };
   const int wp3 = 3 * at.wp, lpad3 = 3 * at.lpad;
   const bool large = g.ks > 4;
   int buf = 0, round = 0;
@@ -415,7 +427,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
       cut(v, a[0], a[1], a[2]);
     }
     // The products, smallest first.  Of bf16 parts all but low times low.  Of fp16 parts, with a weight w = h + m + l =
-    // near + off: h h + m h + near m + l h + off m + near l, which leaves out less than 2^-30 of the whole.
+    // near + off: h h + m h + near m + l h + off m + near l.  That leaves out off l.
     auto products = [&](const Input& in, int b) {
       if constexpr (F16) {
         constexpr int pa[6] = {2, 0, 1, 5, 3, 4}, pb[6] = {0, 0, 0, 1, 1, 2}, to[6] = {1, 0, 1, 1, 1, 1};
@@ -462,7 +474,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     refill();
     if (!F16 && more) fetch(c_beg + round + 1);  // (the second pass is rare: fewer registers instead of less waiting)
     if (more) keep(buf ^ 1);
-    if (F16 && round + 1 == rounds && __ballot(rest != 0)) *inexact = 1;
+    if (F16 && round + 1 == rounds && !held()) *inexact = 1;
     buf ^= 1;
     fresh = true;
     ++round;
@@ -486,7 +498,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     }
   }
   if (round < rounds) {  // a team with a chunk less
-    if (F16 && __ballot(rest != 0)) *inexact = 1;
+    if (F16 && !held()) *inexact = 1;
     __syncthreads();
   }
   if constexpr (F16) {
