@@ -203,6 +203,30 @@ def test_small_weights(value, count):
     layer.pack.close()
 
 
+def test_small_weights_of_more_channels_than_their_places_hold():
+    """The library would give this layer to half_kernel, whose lists of small weights name channels below 2^20."""
+    import torch
+    import tetris_amd as T
+
+    C, K, H = 2 ** 20 + 24, 4, 10
+    rng = np.random.default_rng(5)
+    w = np.zeros((K, C, 1, 1), np.float32)
+    w.reshape(-1)[rng.permutation(K * C)[:K * C // 20]] = 1
+    at = [7, 2 ** 19 + 3, 2 ** 20 - 1, 2 ** 20, C - 1]
+    for k in range(K):
+        w[k, at, 0, 0] = np.ldexp(1 + k + np.arange(5), -20).astype(np.float32)
+    tile = T.tile_select(1, H, H, C, K, 1, 1, 0)
+    pack = T.G950Filter.for_tile(w, tile, oc_order="balanced")
+    x, y = torch.zeros((1, C, H, H), device="cuda"), torch.empty((1, K, H, H), device="cuda")
+    for c in at:
+        x[0, c] = 3
+        pack.launch(x.data_ptr(), y.data_ptr(), 1, H, H, 1, 0, tile)
+        torch.cuda.synchronize()
+        x[0, c] = 0
+        assert (y.cpu().numpy()[0] == 3 * w[:, c]).all(), c
+    pack.close()
+
+
 def test_outputs_that_do_not_lie_on_16_bytes():
     """Outputs go out four pixels at a time where they lie so in memory, one by one elsewhere: the same bits."""
     import torch

@@ -452,6 +452,7 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
   g.half = kMatShapes[cfg].half;
   g.kgs = ks == 1 ? 4 : 2;
   if (g.half) {
+    if (C > kMostChannels) return false;
     // (A step's words have room for 8 groups, and for 2 where ks > 4.)  Long chunks: fewer barriers, and fewer steps that are not
     // full; short ones: more workgroups on a CU, and tiles whose halo would not fit else.
     g.kgs = C <= 16 || ks > 4 ? 2 : C <= 32 || ks > 1 ? 4 : 8;
