@@ -227,6 +227,51 @@ def test_small_weights_of_more_channels_than_their_places_hold():
     pack.close()
 
 
+NO_ROOM = """
+#include <dlfcn.h>
+#include <stddef.h>
+#include <stdio.h>
+int hipMalloc(void** p, size_t n) {
+  int (*real)(void**, size_t) = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOLOAD | RTLD_LAZY), "hipMalloc");
+  if (n > 4000000 && n < 4800000) { fprintf(stderr, "no room for %zu bytes\\n", n); return 2; }
+  return real(p, n);
+}
+"""
+CHILD = """
+import ctypes, sys
+ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+import numpy as np
+import tetris_amd as T
+a = np.load(sys.argv[2])
+y = T.CudaSparseConv2d(a["x"], a["w"], 4, 28, 28, 128, 256, 3, 1, 1)[0]
+np.save(sys.argv[3], y)
+"""
+
+
+def test_no_room_for_the_plan(tmp_path):
+    """Where the weights in parts cannot be allocated the layer runs on the walk, which needs a tenth of their room.  (In a process of
+    its own, where an allocation of 4 to 4.8 MB is refused: of this layer, the plan's alone.)"""
+    import os
+    import subprocess
+    import sys
+
+    import tetris_amd as T
+
+    N, C, H, W, K, ks, stride, pad = 4, 128, 28, 28, 256, 3, 1, 1
+    rng = np.random.default_rng(6)
+    w, x = filter_of(rng, K, C, ks, 0.15), rng.standard_normal((N, C, H, W)).astype(np.float32)
+    layer = Layer(w, x.shape, stride, pad)
+    walk = layer(x, layer.walk())
+    layer.pack.close()
+    (tmp_path / "no_room.c").write_text(NO_ROOM)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", tmp_path / "no_room.so", tmp_path / "no_room.c", "-ldl"])
+    np.savez(tmp_path / "in.npz", x=x, w=w)
+    run = subprocess.run([sys.executable, "-c", CHILD, tmp_path / "no_room.so", tmp_path / "in.npz", tmp_path / "out.npy"], timeout=100,
+                         env=dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(T.__file__))), capture_output=True, text=True)
+    assert run.returncode == 0 and "no room" in run.stderr, run.stderr
+    assert np.linalg.norm(np.load(tmp_path / "out.npy") - walk) <= 1e-6 * np.linalg.norm(walk)
+
+
 def test_outputs_that_do_not_lie_on_16_bytes():
     """Outputs go out four pixels at a time where they lie so in memory, one by one elsewhere: the same bits."""
     import torch

@@ -57,7 +57,8 @@ bool choose_matrix(const tetris_g950* p, int N, int H, int W, int stride, int pa
   return choose_mat_geom(N, p->C, H, W, p->K, p->ks, stride, pad, walk, p->nnz, g, pool);
 }
 
-// the weights of pack `p` as the matrix kernel loads them, made on first use
+// The weights of pack `p` as the matrix kernel loads them, made on first use; null where the device has no room for them (up to 14.5
+// bytes a weight, zeros included): the walk, which needs 8 a non-zero, runs the layer then.
 int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const MatWeights** out) {
   std::lock_guard<std::mutex> lock(p->mu);
   const int key = g.kgs | g.half << 8;
@@ -65,7 +66,13 @@ int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const M
   if (it == p->parts.end()) {
     void* d = nullptr;
     MatWeights w{};
-    TETRIS_HIP(hipMalloc(&d, mat_weight_bytes(g)));
+    const hipError_t e = hipMalloc(&d, mat_weight_bytes(g));
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();  // launches ask for it
+      *out = nullptr;
+      return TETRIS_OK;
+    }
+    TETRIS_HIP(e);
     const int rc = mat_weights(p, g, stream, d, &w);
     if (rc) {
       (void)hipFree(d);
@@ -167,9 +174,9 @@ int find_plan(tetris_g950* p, int N, int H, int W, int stride, int pad, const te
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
     return fail(TETRIS_EINVAL, "the first launch of a shape allocates: call tetris_g950_prepare before capturing");
-  if (choice.matrix) {
-    rc = matrix_weights(p, plan.mat, stream, &plan.parts);
-  } else {
+  if (choice.matrix) rc = matrix_weights(p, plan.mat, stream, &plan.parts);
+  if (rc) return rc;
+  if (!plan.parts) {
     rc = g950_bind(p, plan.geom, geom_walks_pairs(plan.geom), stream, &plan.entries, &plan.grp_off, &plan.grp_pair,
                    &plan.geom.heads_off);
   }

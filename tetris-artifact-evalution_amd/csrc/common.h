@@ -246,7 +246,7 @@ struct tetris_g950 {
   float* d_values = nullptr;      // [n_entries + 8]
   // (LDS byte offset | accumulator index << 16 | 0xC << 28, value) pairs for one tile geometry, made on first use
   std::map<tetris::BoundKey, int2*> bound;
-  std::map<int, tetris::MatWeights> parts;  // the weights as the matrix kernel loads them, by MatGeom::kgs
+  std::map<int, tetris::MatWeights> parts;  // the weights as the matrix kernel loads them, by MatGeom::kgs and, above it, ::half
   // Paired arrangement of the streams (made on the first paired bind; depends on the pack only): two consecutive
   // entries of a stream that share their position become a pair; per stream first all pairs, padded to a multiple
   // of 8 entries, then the entries left single, padded likewise.
