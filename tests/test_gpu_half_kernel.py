@@ -69,6 +69,7 @@ class Layer:
     (10, 17, 14, 6, 6, 2, 3, 0, 0.15),     # ... 64 by 64
     (1, 20, 28, 8, 10, 4, 1, 0, 0.3),      # ... two teams
     (8, 117, 38, 38, 183, 1, 1, 0, 0.15),  # pointwise
+    (1, 2048, 4, 4, 1056, 2, 1, 0, 0.1),   # lists of steps too many to be added up where they are filled
 ])
 def test_layer(N, C, H, W, K, ks, stride, pad, density):
     rng = np.random.default_rng(N * C + K)

@@ -196,11 +196,10 @@ struct MatWeights {
   const char* slots;    // the same weights in fp32
   const int* first;     // first step of every (32 output channels, chunk)
   const int* row_exp;   // per output channel: the power of two that its sums are multiplied by
-  const int* loose_count;  // per 32 output channels: weights that fp16 parts do not hold
+  const int* loose_count;  // per 32 output channels: weights that fp16 parts do not hold; -1 where they are too many or too small
   const int2* loose;    // ... which: row, tap and input channel; the scaled weight
   const float* dense;   // [output channel][tap][input channel, to a multiple of the chunk]
   int step_bytes;       // of all steps
-  int wide;             // some weight is not the sum of its fp16 parts
 };
 constexpr int kMatConfigs = 23;
 constexpr int kMatTasks = 4;        // most blocks of 64 staged pixels x 8 channels that a wave holds at a time

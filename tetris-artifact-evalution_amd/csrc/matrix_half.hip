@@ -179,9 +179,9 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   // Weights: the steps of a wave follow one another; they are asked for three steps ahead of their products.
   struct Step { u32x4 p[F16 ? 3 : 2]; unsigned word; };
   int next_step = w.first[block * g.chunks + c_beg];
-  // (With weights that fp16 parts cannot hold the first pass has no steps.  With a branch around it the compiler would spill
-  // registers of it.)
-  const int steps = F16 && w.wide ? 0 : w.first[block * g.chunks + c_beg + mine] - next_step, loose = F16 ? w.loose_count[block] : 0;
+  // (With weights that fp16 parts cannot hold, `loose` below zero, the first pass has no steps.  With a branch around it the compiler
+  // would spill registers of it.)
+  const int loose = F16 ? w.loose_count[block] : 0, steps = loose < 0 ? 0 : w.first[block * g.chunks + c_beg + mine] - next_step;
   const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(w.steps), 0, w.step_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(w.slots), 0, w.step_bytes / kStepBytes * kSlotBytes, 0x00020000);
   auto fetch_weights = [&](Step& s) {
@@ -368,7 +368,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     scale = __builtin_bit_cast(float, (127 + shift) << 23);
     if (thread < 32 * WM) row_exp[thread] = exponent - shift;
   }
-  if (F16 && thread == 0) *inexact = w.wide;
+  if (F16 && thread == 0) *inexact = loose < 0;
   keep(0);
   __syncthreads();
   // whether the inputs that were staged are what six products can be formed of: the sums of their parts, and none but zeros below
@@ -627,43 +627,56 @@ __global__ __launch_bounds__(256) void dense_kernel(const int32_t* __restrict__ 
   }
 }
 
-// exponent of the largest weight of a row, a wave per row, 16 bytes to a lane (4 bytes: 15 us on average over four layers,
-// 3.6 so)
-__global__ __launch_bounds__(64) void row_kernel(const float* __restrict__ dense, int* __restrict__ row_exp, int K, int per_row) {
-  float most = 0;
-  if ((int)blockIdx.x < K) {
-    const float4* row = reinterpret_cast<const float4*>(dense + (size_t)blockIdx.x * per_row);
-#pragma unroll 4
-    for (int i = threadIdx.x; i < per_row / 4; i += 64) {
-      const float4 f = row[i];
-      most = fmaxf(fmaxf(fmaxf(most, fabsf(f.x)), fmaxf(fabsf(f.y), fabsf(f.z))), fabsf(f.w));
-    }
-  }
-  for (int d = 32; d; d >>= 1) most = fmaxf(most, __shfl_xor(most, d));
-  if (threadIdx.x == 0) row_exp[blockIdx.x] = most > 0 ? ilogbf(most) - 14 : 0;
-}
+// What making a plan writes.
+struct MatLists {
+  int* wide;      // not zero: some weight is not the sum of its parts
+  int* count;     // steps of every (32 output channels, chunk)
+  int* first;     // the sums before them, and of them all
+  int* row_exp;
+  int* loose_count;
+  int2* loose;
+  char* steps;
+  char* slots;
+};
+constexpr int kMostCounts = 2048;  // of a plan whose workgroups each add up the counts before their own
 
 // A workgroup per 32 output channels and chunk of 8*kgs input channels.  The chunk's blocks -- one tap of 8 channels -- are put
 // four to a step; a block with three or four weights in a group of four channels comes twice, the second time with the
 // third and the fourth.  Blocks of zeros are left out.
-// FILL false: counts the steps only.
+// FILL false: counts the steps only; the workgroups beyond those find the exponents of the rows' largest weights, a wave per row.
+// Latency of a workgroup's few rounds bounds both, so 1024 threads: 6 and 16 us on average over four layers, with 256 8 and 18.
 template <bool FILL>
-__global__ __launch_bounds__(256) void steps_kernel(const MatWeights w, int* __restrict__ first, char* __restrict__ steps,
-                                                    char* __restrict__ slots, int* __restrict__ loose_count, int2* __restrict__ loose,
-                                                    int* __restrict__ wide, int K, int ks, int kgs, int chunks) {
-  constexpr int kMost = 256;
+__global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const MatLists out, int K, int ks, int kgs, int chunks, int mblocks) {
+  constexpr int kMost = 256, kThreads = 1024;
   __shared__ int layers[kMost];
   __shared__ int list[2 * kMost];
   __shared__ int listed;
-  const int chunk = blockIdx.x, block = blockIdx.y, taps = ks * ks, subs = kgs * taps;
+  __shared__ int before[kThreads / 64];
+  const int id = blockIdx.x, counts = chunks * mblocks, block = id / chunks, chunk = id - block * chunks, taps = ks * ks, subs = kgs * taps;
+  if (!FILL && id >= counts) {
+    const int row = (id - counts) * (kThreads / 64) + threadIdx.x / 64, per_row = taps * chunks * 8 * kgs;
+    if (row >= 32 * mblocks) return;
+    float most = 0;
+    if (row < K) {
+      const float4* values = reinterpret_cast<const float4*>(w.dense + (size_t)row * per_row);
+#pragma unroll 4
+      for (int i = threadIdx.x & 63; i < per_row / 4; i += 64) {
+        const float4 f = values[i];
+        most = fmaxf(fmaxf(fmaxf(most, fabsf(f.x)), fmaxf(fabsf(f.y), fabsf(f.z))), fabsf(f.w));
+      }
+    }
+    for (int d = 32; d; d >>= 1) most = fmaxf(most, __shfl_xor(most, d));
+    if ((threadIdx.x & 63) == 0) out.row_exp[row] = most > 0 ? ilogbf(most) - 14 : 0;
+    return;
+  }
   auto weights = [&](int row, int sub, int group) {  // four channels of a block
     const int oc = block * 32 + row, tap = sub / kgs;
     const float4* d = reinterpret_cast<const float4*>(w.dense + (((size_t)oc * taps + tap) * chunks + chunk) * 8 * kgs);
     return oc < K ? d[2 * (sub - tap * kgs) + group] : make_float4(0.f, 0.f, 0.f, 0.f);
   };
-  for (int i = threadIdx.x; i < subs; i += 256) layers[i] = 0;
+  for (int i = threadIdx.x; i < subs; i += kThreads) layers[i] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < subs * 64; i += 256) {
+  for (int i = threadIdx.x; i < subs * 64; i += kThreads) {
     const int sub = i >> 6, row = i & 31, group = i >> 5 & 1;
     const float4 f = weights(row, sub, group);
     const int n = (f.x != 0.f) + (f.y != 0.f) + (f.z != 0.f) + (f.w != 0.f);
@@ -676,15 +689,29 @@ __global__ __launch_bounds__(256) void steps_kernel(const MatWeights w, int* __r
       for (int sub = 0; sub < subs; ++sub)
         if (layers[sub] > layer) list[n++] = sub | layer << 16;
     listed = n;
-    if (!FILL) first[block * chunks + chunk] = max(1, (n + 3) / 4);
+    if (!FILL) out.count[id] = max(1, (n + 3) / 4);
   }
   if (!FILL) return;
+  // the steps before these: summed here, or where they are many by first_kernel
+  int first = 0;
+  if (counts <= kMostCounts) {
+    for (int i = threadIdx.x; i < id; i += kThreads) first += out.count[i];
+    for (int d = 32; d; d >>= 1) first += __shfl_xor(first, d);
+    if ((threadIdx.x & 63) == 0) before[threadIdx.x / 64] = first;
+  }
   __syncthreads();
   const int n = listed, steps_here = max(1, (n + 3) / 4), items = steps_here * 64;
-  if (block == (int)gridDim.y - 1 && chunk == chunks - 1 && threadIdx.x < 192)  // what is read ahead of the end names a block that exists
-    *reinterpret_cast<unsigned*>(steps + (size_t)(first[block * chunks + chunk] + steps_here + (int)threadIdx.x / 64) * kStepBytes + 3072 +
-                                 threadIdx.x % 64 * 4) = 0;
-  for (int i = threadIdx.x; i < items; i += 256) {
+  if (counts <= kMostCounts) {
+    first = 0;
+    for (int i = 0; i < kThreads / 64; ++i) first += before[i];
+    if (threadIdx.x == 0) out.first[id] = first;
+    if (threadIdx.x == 0 && id == counts - 1) out.first[counts] = first + steps_here;
+  } else {
+    first = out.first[id];
+  }
+  if (id == counts - 1 && threadIdx.x < 192)  // what is read ahead of the end names a block that exists
+    *reinterpret_cast<unsigned*>(out.steps + (size_t)(first + steps_here + (int)threadIdx.x / 64) * kStepBytes + 3072 + threadIdx.x % 64 * 4) = 0;
+  for (int i = threadIdx.x; i < items; i += kThreads) {
     const int step = i >> 6, lane = i & 63, row = lane & 31, half = lane >> 5;
     // eight slots: blocks 2 half and 2 half + 1 of the step, two groups of four channels each, two slots a group
     unsigned index = 0;
@@ -716,9 +743,9 @@ __global__ __launch_bounds__(256) void steps_kernel(const MatWeights w, int* __r
         v[2 * k + slot] = value[slot];
         scaled[2 * k + slot] = ldexpf(value[slot], shift);
         if (value[slot] == 0.f || fabsf(scaled[2 * k + slot]) >= kLeast) continue;
-        const int tap = sub / kgs, n = atomicAdd(loose_count + block, 1);
-        if (n >= kMostLoose || !(fabsf(scaled[2 * k + slot]) >= kLeastLoose)) atomicOr(wide, 1);
-        else loose[kMostLoose * block + n] = make_int2(row | tap / ks << 5 | tap % ks << 8 |
+        const int tap = sub / kgs, n = atomicAdd(out.loose_count + block, 1);
+        if (n >= kMostLoose || !(fabsf(scaled[2 * k + slot]) >= kLeastLoose)) *out.wide = 1;
+        else out.loose[kMostLoose * block + n] = make_int2(row | tap / ks << 5 | tap % ks << 8 |
                                                            ((chunk * kgs + sub - tap * kgs) * 8 + 4 * (k & 1) + place[slot]) << 11,
                                                        (int)bits_of(scaled[2 * k + slot]));
         scaled[2 * k + slot] = 0;
@@ -731,25 +758,30 @@ __global__ __launch_bounds__(256) void steps_kernel(const MatWeights w, int* __r
       const int bits = ks > 4 ? 3 : 2;  // seven bits: column and row of the tap, channel group
       code[r] = (unsigned)(tap % ks | tap / ks << bits | kg << 2 * bits);
     }
-    const size_t out = first[block * chunks + chunk] + step;
-    char* dst = steps + out * kStepBytes;
+    const size_t to = first + step;
+    char* dst = out.steps + to * kStepBytes;
     *reinterpret_cast<unsigned*>(dst + 3072 + lane * 4) = index | code[0] << 16 | code[1] << 24 | (step + 1 == steps_here ? 0x80000000u : 0u);
     u32x4 h, m, l;
     unsigned rest = 0;
     cut16(scaled, 1.f, h, m, l, rest);
-    if (rest) atomicOr(wide, 1);
+    if (rest) *out.wide = 1;
     l = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, l) * (f16x8)(_Float16)(1 / kLow));
     *reinterpret_cast<u32x4*>(dst + lane * 16) = h;
     *reinterpret_cast<u32x4*>(dst + 1024 + lane * 16) = m;
     *reinterpret_cast<u32x4*>(dst + 2048 + lane * 16) = l;
-    char* raw = slots + out * kSlotBytes + lane * 16;
+    char* raw = out.slots + to * kSlotBytes + lane * 16;
     *reinterpret_cast<u32x4*>(raw) = u32x4{bits_of(v[0]), bits_of(v[1]), bits_of(v[2]), bits_of(v[3])};
     *reinterpret_cast<u32x4*>(raw + 1024) = u32x4{bits_of(v[4]), bits_of(v[5]), bits_of(v[6]), bits_of(v[7])};
   }
 }
 
-// puts a block's loose weights in order, so that sums do not depend on who came first
-__global__ __launch_bounds__(64) void loose_kernel(const int* __restrict__ loose_count, int2* __restrict__ loose) {
+// Puts a block's loose weights in order, so that sums do not depend on who came first; their count is -1 where the first pass cannot
+// be made.
+__global__ __launch_bounds__(64) void loose_kernel(const int* __restrict__ wide, int* __restrict__ loose_count, int2* __restrict__ loose) {
+  if (*wide) {
+    if (threadIdx.x == 0) loose_count[blockIdx.x] = -1;
+    return;
+  }
   __shared__ int2 list[kMostLoose];
   const int n = min(loose_count[blockIdx.x], kMostLoose), i = threadIdx.x;
   int2* all = loose + kMostLoose * blockIdx.x;
@@ -762,11 +794,11 @@ __global__ __launch_bounds__(64) void loose_kernel(const int* __restrict__ loose
 }
 
 // counts -> the first step of every (32 output channels, chunk)
-__global__ __launch_bounds__(1024) void first_kernel(int* __restrict__ first, int n) {
+__global__ __launch_bounds__(1024) void first_kernel(const int* __restrict__ count, int* __restrict__ first, int n) {
   __shared__ int sums[1024];
   int before = 0;
   for (int at = 0; at < n; at += 1024) {
-    const int i = at + (int)threadIdx.x, mine = i < n ? first[i] : 0;
+    const int i = at + (int)threadIdx.x, mine = i < n ? count[i] : 0;
     sums[threadIdx.x] = mine;
     __syncthreads();
     for (int d = 1; d < 1024; d <<= 1) {
@@ -798,26 +830,38 @@ int launch_one(const MatGeom& g, const float* d_in, float* d_out, const MatWeigh
 
 size_t dense_bytes(const MatGeom& g) { return (size_t)g.K * g.ks * g.ks * g.chunks * 8 * g.kgs * sizeof(float); }
 
-// one allocation: the flag, the rows' exponents, the chunks' steps, the dense filter, the steps, their weights as they are
-MatWeights mat_weights_at(const MatGeom& g, void* base, size_t* bytes) {
-  size_t at = 256;
+// one allocation: first what has to be zero (flag, counts of loose weights, dense filter), then the rows' exponents, the steps' counts
+// and sums, the loose weights, the steps, their weights as they are
+MatWeights mat_weights_at(const MatGeom& g, void* base, size_t* bytes, size_t* zeros = nullptr, MatLists* lists = nullptr) {
+  size_t at = 0;
   auto take = [&](size_t n) {
     char* p = static_cast<char*>(base) + at;
     at += (n + 255) / 256 * 256;
     return p;
   };
   const size_t steps = (size_t)g.mblocks * g.chunks * g.smax + 3;  // (waves read ahead)
+  MatLists l{};
+  l.wide = reinterpret_cast<int*>(take(sizeof(int)));
+  l.loose_count = reinterpret_cast<int*>(take((size_t)g.mblocks * 4));
   MatWeights w{};
   w.base = base;
-  w.row_exp = reinterpret_cast<const int*>(take((size_t)g.mblocks * 32 * 4));
-  w.first = reinterpret_cast<const int*>(take(((size_t)g.mblocks * g.chunks + 1) * 4));
   w.dense = reinterpret_cast<const float*>(take(dense_bytes(g)));
-  w.loose_count = reinterpret_cast<const int*>(take((size_t)g.mblocks * 4));
-  w.loose = reinterpret_cast<const int2*>(take((size_t)g.mblocks * kMostLoose * 8));
-  w.steps = take(steps * kStepBytes);
-  w.slots = take(steps * kSlotBytes);
+  if (zeros) *zeros = at;
+  l.row_exp = reinterpret_cast<int*>(take((size_t)g.mblocks * 32 * 4));
+  l.count = reinterpret_cast<int*>(take((size_t)g.mblocks * g.chunks * 4));
+  l.first = reinterpret_cast<int*>(take(((size_t)g.mblocks * g.chunks + 1) * 4));
+  l.loose = reinterpret_cast<int2*>(take((size_t)g.mblocks * kMostLoose * 8));
+  l.steps = take(steps * kStepBytes);
+  l.slots = take(steps * kSlotBytes);
+  w.row_exp = l.row_exp;
+  w.first = l.first;
+  w.loose_count = l.loose_count;
+  w.loose = l.loose;
+  w.steps = l.steps;
+  w.slots = l.slots;
   w.step_bytes = (int)(steps * kStepBytes);
   if (bytes) *bytes = at;
+  if (lists) *lists = l;
   return w;
 }
 
@@ -830,26 +874,19 @@ size_t half_weight_bytes(const MatGeom& g) {
 }
 
 int half_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* base, MatWeights* out) {
-  MatWeights w = mat_weights_at(g, base, nullptr);
-  TETRIS_HIP(hipMemsetAsync(base, 0, 256, stream));
-  TETRIS_HIP(hipMemsetAsync(const_cast<int*>(w.loose_count), 0, (size_t)g.mblocks * 4, stream));
-  TETRIS_HIP(hipMemsetAsync(const_cast<float*>(w.dense), 0, dense_bytes(g), stream));
-  const int nstream = p->groups * p->stages;
+  MatLists l;
+  size_t zeros = 0;
+  const MatWeights w = mat_weights_at(g, base, nullptr, &zeros, &l);
+  TETRIS_HIP(hipMemsetAsync(base, 0, zeros, stream));
+  const int nstream = p->groups * p->stages, counts = g.chunks * g.mblocks;
   hipLaunchKernelGGL(dense_kernel, dim3(ceil_div(nstream, 4)), dim3(256), 0, stream, p->d_grp_off, p->d_grp_nnz, p->d_oc_order,
                      p->d_position, p->d_values, const_cast<float*>(w.dense), p->C, p->K, p->ks, p->tile_ic, p->stages, p->g, nstream,
                      8 * g.kgs * g.chunks);
-  hipLaunchKernelGGL(row_kernel, dim3(32 * g.mblocks), dim3(64), 0, stream, w.dense, const_cast<int*>(w.row_exp), g.K,
-                     8 * g.kgs * g.chunks * g.ks * g.ks);
-  int* first = const_cast<int*>(w.first);
-  char *steps = const_cast<char*>(w.steps), *slots = const_cast<char*>(w.slots);
-  hipLaunchKernelGGL(steps_kernel<false>, dim3(g.chunks, g.mblocks), dim3(256), 0, stream, w, first, steps, slots,
-                     const_cast<int*>(w.loose_count), const_cast<int2*>(w.loose), static_cast<int*>(base), g.K, g.ks, g.kgs, g.chunks);
-  hipLaunchKernelGGL(first_kernel, dim3(1), dim3(1024), 0, stream, first, g.chunks * g.mblocks);
-  hipLaunchKernelGGL(steps_kernel<true>, dim3(g.chunks, g.mblocks), dim3(256), 0, stream, w, first, steps, slots,
-                     const_cast<int*>(w.loose_count), const_cast<int2*>(w.loose), static_cast<int*>(base), g.K, g.ks, g.kgs, g.chunks);
-  hipLaunchKernelGGL(loose_kernel, dim3(g.mblocks), dim3(64), 0, stream, w.loose_count, const_cast<int2*>(w.loose));
+  hipLaunchKernelGGL(steps_kernel<false>, dim3(counts + 2 * g.mblocks), dim3(1024), 0, stream, w, l, g.K, g.ks, g.kgs, g.chunks, g.mblocks);
+  if (counts > kMostCounts) hipLaunchKernelGGL(first_kernel, dim3(1), dim3(1024), 0, stream, l.count, l.first, counts);
+  hipLaunchKernelGGL(steps_kernel<true>, dim3(counts), dim3(1024), 0, stream, w, l, g.K, g.ks, g.kgs, g.chunks, g.mblocks);
+  hipLaunchKernelGGL(loose_kernel, dim3(g.mblocks), dim3(64), 0, stream, l.wide, l.loose_count, l.loose);
   TETRIS_HIP(hipGetLastError());
-  TETRIS_HIP(hipMemcpyAsync(&w.wide, base, sizeof(int), hipMemcpyDeviceToHost, stream));
   // launches on other streams may follow at once
   TETRIS_HIP(hipStreamSynchronize(stream));
   *out = w;
