@@ -56,18 +56,22 @@ constexpr float kSmall = 0x1p-16f;  // the smallest scaled input that is multipl
 // (A bit cast of a vector's element itself, instead of its value, is compiled to one of the vector's first element.)
 __device__ __forceinline__ float float_of(unsigned x) { return __builtin_bit_cast(float, x); }
 
-// three fp16 parts of eight floats, scaled; `rest` gets a bit that is not zero where they do not add up to the floats
-__device__ __forceinline__ void cut16(const float (&x)[8], float scale, u32x4& hi, u32x4& mid, u32x4& lo, unsigned& rest) {
+// Three fp16 parts of eight floats, scaled; `zeros` becomes NaN where an h is infinite or NaN, `rest` (if any) gets a bit that is not
+// zero where the parts do not add up to the floats.  (h is the bf16 number itself from 2^-16 of its scale on, so what is left of x
+// takes full-rate FMAs; with inputs tested by `rest` and taken off h in fp16 workgroups were 1 % slower.)
+__device__ __forceinline__ void cut16(const float (&x)[8], float scale, u32x4& hi, u32x4& mid, u32x4& lo, f16x2& zeros, unsigned* rest) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float a = x[2 * i], b = x[2 * i + 1];
     const unsigned t = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a * scale, b * scale}), bf16x2));
-    const f16x2 h = __builtin_convertvector((f32x2{__builtin_bit_cast(float, t << 16), __builtin_bit_cast(float, t & 0xffff0000u)}), f16x2);
-    const float r0 = fmaf((float)h.x, -kMid, a * (scale * kMid)), r1 = fmaf((float)h.y, -kMid, b * (scale * kMid));
+    const float h0 = __builtin_bit_cast(float, t << 16), h1 = __builtin_bit_cast(float, t & 0xffff0000u);
+    const f16x2 h = __builtin_convertvector((f32x2{h0, h1}), f16x2);
+    const float r0 = fmaf(h0, -kMid, a * (scale * kMid)), r1 = fmaf(h1, -kMid, b * (scale * kMid));
     const f16x2 m = __builtin_convertvector((f32x2{r0, r1}), f16x2);
     const float s0 = fmaf((float)m.x, -kLow, r0 * kLow), s1 = fmaf((float)m.y, -kLow, r1 * kLow);
     const f16x2 l = __builtin_convertvector((f32x2{s0, s1}), f16x2);
-    rest |= bits_of(fmaf((float)l.x, -1.f, s0)) | bits_of(fmaf((float)l.y, -1.f, s1));
+    zeros = __builtin_elementwise_fma(h, f16x2{0, 0}, zeros);
+    if (rest) *rest |= bits_of(fmaf((float)l.x, -1.f, s0)) | bits_of(fmaf((float)l.y, -1.f, s1));
     hi[i] = __builtin_bit_cast(unsigned, h);
     mid[i] = __builtin_bit_cast(unsigned, m);
     lo[i] = __builtin_bit_cast(unsigned, l);
@@ -230,7 +234,8 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
       }
     }
   };
-  unsigned rest = 0, least = ~0u;  // least: of the inputs' bits without the sign, doubled, less one: zeros come out on top
+  f16x2 zeros = {0, 0};
+  unsigned least = ~0u;  // least: of the inputs' bits without the sign, doubled, less one: zeros come out on top
   float scale = 1.f;
   auto keep = [&](int buf) {
 #pragma unroll
@@ -238,7 +243,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
       if (wave + TW * k >= tasks) break;
       u32x4 h, m, l;
       if constexpr (F16) {
-        cut16(x[k], scale, h, m, l, rest);
+        cut16(x[k], scale, h, m, l, zeros, nullptr);
 #pragma unroll
         for (int j = 0; j < 8; ++j) least = min(least, (bits_of(x[k][j]) << 1) - 1);
       } else {
@@ -371,9 +376,12 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   if (F16 && thread == 0) *inexact = loose < 0;
   keep(0);
   __syncthreads();
-  // whether the inputs that were staged are what six products can be formed of: the sums of their parts, and none but zeros below
-  // kSmall / scale (looked at before it is scaled, where it may underflow)
-  auto held = [&]() { return __ballot(rest != 0 || least < 2 * (bits_of(kSmall) + bits_of(1.f) - bits_of(scale)) - 1) == 0; };
+  // whether the inputs that were staged are what six products can be formed of: no h is infinite, and none but zeros are below
+  // kSmall / scale (looked at before they are scaled, where they may underflow)
+  auto held = [&]() {
+    const bool infinite = __builtin_bit_cast(unsigned, zeros) & 0x7fff7fff;
+    return __builtin_amdgcn_ballot_w64(infinite || least < 2 * (bits_of(kSmall) + bits_of(1.f) - bits_of(scale)) - 1) == 0;
+  };
   const int wp3 = 3 * at.wp, lpad3 = 3 * at.lpad;
   const bool large = g.ks > 4;
   int buf = 0, round = 0;
@@ -763,7 +771,8 @@ __global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const M
     *reinterpret_cast<unsigned*>(dst + 3072 + lane * 4) = index | code[0] << 16 | code[1] << 24 | (step + 1 == steps_here ? 0x80000000u : 0u);
     u32x4 h, m, l;
     unsigned rest = 0;
-    cut16(scaled, 1.f, h, m, l, rest);
+    f16x2 zeros = {0, 0};
+    cut16(scaled, 1.f, h, m, l, zeros, &rest);
     if (rest) *out.wide = 1;
     l = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, l) * (f16x8)(_Float16)(1 / kLow));
     *reinterpret_cast<u32x4*>(dst + lane * 16) = h;
