@@ -36,6 +36,14 @@ class Layer:
         # (LDS: whole KiB of input, then what this kernel alone keeps there)
         assert self.shape.kernel == 5 and self.shape.lds_bytes % 1024
 
+    def runs(self, channels, pixels, slices):
+        """whether workgroups take tiles of this size (what the grid's numbers say)"""
+        N, K, oh, ow = self.out
+        strips = -(-ow // 64)
+        columns = ow if strips == 1 else -(-ow // strips) + 1 & ~1
+        return (self.shape.channel_blocks, self.shape.unit_groups, self.shape.csplit) == (
+            -(--(-K // 32) // (channels // 32)), -(-N * strips * columns * oh // pixels), slices)
+
     def walk(self):
         import tetris_amd as T
 
@@ -51,43 +59,55 @@ class Layer:
         return y.cpu().numpy()
 
 
-@pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad,density", [
-    (9, 16, 21, 21, 7, 2, 3, 0, 0.15),     # 256 channels by 64 pixels, one chunk of them; stride 3
-    (15, 18, 21, 41, 131, 5, 1, 2, 0.3),   # ... chunks of 16 channels, the last of two; blocks that come twice
-    (6, 39, 5, 9, 4, 7, 2, 3, 0.3),        # ... 7 x 7, in slices; four output channels
-    (3, 42, 40, 77, 81, 3, 1, 1, 0.15),    # 128 by 64, two teams, a chunk each and ten channels more; two strips
-    (4, 17, 70, 26, 166, 6, 1, 0, 0.3),    # ... 6 x 6
-    (12, 53, 27, 35, 7, 4, 1, 0, 0.15),    # 64 by 64, two teams
-    (1, 21, 8, 8, 3, 7, 1, 3, 0.3),        # ... an image of one tile
-    (8, 33, 47, 63, 68, 5, 1, 0, 0.3),     # 256 by 96: an odd number of blocks of pixels
-    (11, 120, 18, 70, 11, 7, 2, 0, 0.2),   # ... in slices; 7 x 7
-    (12, 111, 23, 78, 21, 3, 2, 1, 0.15),  # ... short chunks
-    (8, 19, 79, 28, 275, 3, 1, 0, 0.3),    # 128 by 192
-    (12, 17, 73, 24, 85, 2, 3, 1, 0.15),   # short chunks: 256 by 64
-    (3, 95, 9, 8, 3, 4, 3, 0, 0.3),        # ... in slices
-    (5, 17, 67, 31, 74, 4, 1, 2, 0.2),     # ... 128 by 64, two teams
-    (10, 17, 14, 6, 6, 2, 3, 0, 0.15),     # ... 64 by 64
-    (1, 20, 28, 8, 10, 4, 1, 0, 0.3),      # ... two teams
-    (8, 117, 38, 38, 183, 1, 1, 0, 0.15),  # pointwise
-    (1, 2048, 4, 4, 1056, 2, 1, 0, 0.1),   # lists of steps too many to be added up where they are filled
-])
-def test_layer(N, C, H, W, K, ks, stride, pad, density):
+LAYERS = [  # N, C, H, W, K, ks, stride, pad, density of the filter; channels, pixels and slices of the tiles it runs in
+    (9, 16, 21, 21, 7, 2, 3, 0, 0.15, (256, 64, 1)),      # one chunk of channels; stride 3
+    (15, 18, 21, 41, 131, 5, 1, 2, 0.3, (256, 64, 1)),    # chunks of 16 channels, the last of two; blocks that come twice
+    (6, 39, 5, 9, 4, 7, 2, 3, 0.3, (256, 64, 3)),         # 7 x 7; four output channels
+    (3, 42, 40, 77, 81, 3, 1, 1, 0.15, (128, 64, 1)),     # two teams, a chunk each and ten channels more; two strips
+    (4, 17, 70, 26, 166, 6, 1, 0, 0.3, (128, 64, 1)),     # 6 x 6
+    (12, 53, 27, 35, 7, 4, 1, 0, 0.15, (64, 64, 1)),      # two teams
+    (1, 21, 8, 8, 3, 7, 1, 3, 0.3, (64, 64, 1)),          # an image of one tile
+    (8, 33, 47, 63, 68, 5, 1, 0, 0.3, (256, 96, 1)),      # an odd number of blocks of pixels
+    (11, 120, 18, 70, 11, 7, 2, 0, 0.2, (256, 96, 8)),    # ... 7 x 7
+    (12, 111, 23, 78, 21, 3, 2, 1, 0.15, (256, 96, 4)),   # ... short chunks
+    (8, 19, 79, 28, 275, 3, 1, 0, 0.3, (128, 192, 1)),
+    (12, 17, 73, 24, 85, 2, 3, 1, 0.15, (256, 64, 1)),    # short chunks
+    (3, 95, 9, 8, 3, 4, 3, 0, 0.3, (256, 64, 6)),
+    (5, 17, 67, 31, 74, 4, 1, 2, 0.2, (128, 64, 1)),      # two teams
+    (10, 17, 14, 6, 6, 2, 3, 0, 0.15, (64, 64, 1)),
+    (1, 20, 28, 8, 10, 4, 1, 0, 0.3, (64, 64, 1)),        # two teams
+    (8, 117, 38, 38, 183, 1, 1, 0, 0.15, (256, 64, 1)),   # pointwise
+    (1, 2048, 4, 4, 1056, 2, 1, 0, 0.1, (64, 64, 8)),     # lists of steps too many to be added up where they are filled
+    (4, 18, 69, 92, 175, 3, 1, 0, 0.15, (256, 128, 1)),   # four blocks of pixels a wave, which leave registers for two sets of weights
+    (6, 19, 88, 50, 199, 3, 1, 0, 0.2, (256, 128, 1)),    # ... outputs four pixels at a time
+    (3, 85, 45, 63, 228, 3, 1, 1, 0.3, (256, 128, 3)),
+    (4, 17, 52, 80, 258, 3, 1, 1, 0.15, (128, 256, 1)),
+    (8, 19, 79, 28, 275, 3, 1, 1, 0.3, (128, 256, 1)),
+    (6, 68, 60, 57, 69, 3, 1, 1, 0.2, (128, 256, 3)),
+]
+
+
+@pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad,density,tile", LAYERS)
+def test_layer(N, C, H, W, K, ks, stride, pad, density, tile):
     rng = np.random.default_rng(N * C + K)
     w = filter_of(rng, K, C, ks, density)
     x = np.maximum(rng.standard_normal((N, C, H, W)), -0.25).astype(np.float32)
     layer = Layer(w, x.shape, stride, pad)
+    assert layer.runs(*tile)
     got, walk = layer(x), layer(x, layer.walk())
     ref, terms = conv64(x, w, stride, pad)
     # in any order of fp32 sums an output is off by a rounding per term at most, each of the terms' magnitude; and the parts
     # lose no more than the walking kernel's FMAs do
-    assert (np.abs(got - ref) <= C * ks * ks * 2.0 ** -24 * terms).all()
+    count = (w != 0).reshape(K, -1).sum(1).reshape(1, K, 1, 1)
+    assert (np.abs(got - ref) <= count * 2.0 ** -24 * terms).all()
     assert np.linalg.norm(got - ref) <= 1.05 * np.linalg.norm(walk - ref)
     layer.pack.close()
 
 
 @pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad,density", [
     (3, 42, 40, 77, 81, 3, 1, 1, 0.15), (8, 33, 47, 63, 68, 5, 1, 0, 0.3), (11, 120, 18, 70, 11, 7, 2, 0, 0.2),
-    (8, 19, 79, 28, 275, 3, 1, 0, 0.3), (1, 20, 28, 8, 10, 4, 1, 0, 0.3)])
+    (8, 19, 79, 28, 275, 3, 1, 0, 0.3), (1, 20, 28, 8, 10, 4, 1, 0, 0.3),
+    (6, 19, 88, 50, 199, 3, 1, 0, 0.2), (4, 17, 52, 80, 258, 3, 1, 1, 0.15), (6, 68, 60, 57, 69, 3, 1, 1, 0.2)])
 def test_activations(N, C, H, W, K, ks, stride, pad, density):
     import torch
     import tetris_amd as T
@@ -156,7 +176,7 @@ def test_inputs_of_any_scale(what):
     ("8 bits", 0, -38), ("8 bits", 0, -40), ("one bit", 0, -44), ("bf16", 0, -36),  # their parts add up to them, and are not enough
     ("24 bits", 0, -24), ("24 bits", 0, -27), ("24 bits", 0, -28), ("24 bits", 0, -29), ("24 bits", 0, -34),
     ("24 bits", 44, -126), ("24 bits", 60, -110), ("24 bits", 72, -100), ("24 bits", 110, -60), ("24 bits", 100, -130)])  # lost in its scale
-@pytest.mark.parametrize("at", [LAYER, (8, 19, 79, 28, 275, 3, 1, 1, 0.3)])
+@pytest.mark.parametrize("at", [LAYER, (8, 19, 79, 28, 275, 3, 1, 1, 0.3)])  # (tiles of 128 x 64 and of 128 x 256)
 def test_small_inputs_beside_large_ones(at, what, large, small):
     """Stripes of small inputs between stripes of large ones, which the whole tile is scaled by: where an output is a sum of small ones
     alone, it is as exact as the walk's, whatever their size and their number of significant bits."""
@@ -178,6 +198,73 @@ def test_small_inputs_beside_large_ones(at, what, large, small):
     assert (np.abs(got - ref) <= count * 2.0 ** -24 * terms + 2.0 ** -149)[alone].all()
     if small > -120:  # (a subnormal output is rounded twice)
         assert np.linalg.norm((got - ref)[alone]) <= 1.05 * np.linalg.norm((walk - ref)[alone])
+    layer.pack.close()
+
+
+@pytest.mark.parametrize("scale_x,scale_w", [(0, 0), (-10, 3), (-120, 0), (-140, 4), (0, -130), (-70, -60), (40, 20), (80, -100), (120, -10)])
+def test_outputs_of_one_term(scale_x, scale_w):
+    """Inputs and weights of full 24-bit significands, one product an output: as exact as one rounding of it."""
+    N, C, H, W, K, ks, stride, pad, density = 8, 117, 38, 38, 183, 1, 1, 0, 0.15
+    rng = np.random.default_rng(8)
+    w = np.zeros((K, C), np.float32)
+    rest = np.zeros(K * (C - 48), np.float32)  # as many weights as make the library choose half_kernel, and x is zero there
+    rest[rng.permutation(rest.size)[:int(density * K * C) - K]] = 1
+    w[:, 48:] = rest.reshape(K, C - 48) * (1 + rng.random((K, C - 48)))
+    w[np.arange(K), np.arange(K) % 48] = 1 + rng.random(K)
+    w = np.ldexp(w, scale_w).astype(np.float32).reshape(K, C, 1, 1)
+    x = np.zeros((N, C, H, W), np.float32)
+    x[:, :48] = np.ldexp((1 + rng.random((N, 48, H, W))).astype(np.float32), scale_x)
+    layer = Layer(w, x.shape, stride, pad)
+    assert layer.runs(256, 64, 1)
+    got = layer(x)
+    ref = conv64(x, w, stride, pad)[0]
+    # Half a unit in the last place, and what is left out, 2^-28, and the roundings of the smaller products' sum, which is 2^-8 of the
+    # product; of a subnormal output first that of the scaled sum and then its own.
+    normal = np.abs(ref) >= 2.0 ** -126
+    half = np.where(normal, np.abs(ref) * 2.0 ** -24, 2.0 ** -150)
+    assert (np.abs(got - ref) <= half * (1 + 2.0 ** -3) + np.where(normal, 0, np.abs(ref) * 2.0 ** -24)).all()
+    layer.pack.close()
+
+
+@pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad,density", [
+    (12, 53, 27, 35, 7, 4, 1, 0, 0.15), (8, 117, 38, 38, 183, 1, 1, 0, 0.15), (8, 19, 79, 28, 275, 3, 1, 1, 0.3),
+    (6, 19, 88, 50, 199, 3, 1, 0, 0.2), (11, 120, 18, 70, 11, 7, 2, 0, 0.2), (5, 163, 41, 54, 81, 3, 1, 1, 0.3)])
+def test_values_out_of_range_give_what_the_walk_gives(N, C, H, W, K, ks, stride, pad, density):
+    """Infinities, NaN and the largest numbers reach the outputs whose window holds them with a weight that is not zero, and no others:
+    a wave stores what its passes give over what the pass before has stored, also where that is four pixels at a time (all of these
+    layers but the last)."""
+    import torch
+    import tetris_amd as T
+
+    rng = np.random.default_rng(9)
+    w = filter_of(rng, K, C, ks, density)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    x.reshape(-1)[rng.permutation(x.size)[:48]] = np.tile(np.array([np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 2.0 ** 100, -2.0 ** 90, 1e-45], np.float32), 6)
+    layer = Layer(w, x.shape, stride, pad)
+    assert (-(-layer.out[3] // 64) == 1 and layer.out[2] * layer.out[3] % 4 == 0) == (C != 163)
+    dx = torch.from_numpy(x).cuda()
+    terms = conv64(np.where(np.isfinite(x), x, 0), w, stride, pad)[1]
+    count = (w != 0).reshape(K, -1).sum(1).reshape(1, K, 1, 1)
+    for act in (T.ACT_NONE, T.ACT_RELU, T.ACT_RELU_POOL2):
+        if not all(layer.pack.act_supported(*layer.at, t, act) for t in (layer.tile, layer.walk())):
+            continue
+        n, k, oh, ow = layer.out
+        outs, half = [], 2 if act == T.ACT_RELU_POOL2 else 1
+        for t in (layer.tile, layer.walk()):
+            y = torch.full((n, k, oh // half, ow // half), float("nan"), device="cuda")
+            layer.pack.launch_act(dx.data_ptr(), y.data_ptr(), *layer.at, t, act)
+            torch.cuda.synchronize()
+            outs.append(y.cpu().numpy())
+        got, walk = outs
+        assert np.array_equal(np.isnan(got), np.isnan(walk)) and np.array_equal(np.isinf(got), np.isinf(walk))
+        assert act or (np.isnan(walk).any() and np.isinf(walk).any())
+        ok = np.isfinite(walk)
+        assert np.array_equal(np.sign(got[~ok]), np.sign(walk[~ok]), equal_nan=True)
+        bound = 2 * count * 2.0 ** -24 * terms
+        if half == 2:  # of a maximum: the largest bound of the four
+            bound = bound[:, :, :oh // 2 * 2, :ow // 2 * 2].reshape(n, k, oh // 2, 2, ow // 2, 2).max((3, 5))
+        with np.errstate(all="ignore"):
+            assert (np.abs(got.astype(np.float64) - walk)[ok] <= bound[ok]).all()
     layer.pack.close()
 
 

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad", [
     (6, 25, 55, 77, 72, 1, 1, 0),      # pointwise, two strips, C and K over a multiple of 8 and 32
-    (5, 163, 41, 54, 81, 3, 1, 1),     # 128 pixels a tile, slices
+    (5, 163, 41, 54, 81, 3, 1, 1),     # half_kernel: 192 pixels a tile, slices
     (2, 23, 67, 45, 161, 5, 1, 2),     # 512 staged pixels; every slice of the input in one buffer
     (3, 38, 53, 25, 279, 2, 1, 1),     # four teams, more channel blocks than fill the last workgroup
     (7, 61, 31, 32, 5, 3, 1, 0),       # fewer output channels than lanes
@@ -282,20 +282,22 @@ def test_weights_out_of_range_stay_with_the_walk(oracle):
         pk.close()
 
 
-SPLIT = (5, 163, 41, 54, 81, 3, 1, 1)  # runs on the matrix cores in slices
+# run on the matrix cores in slices: by half_kernel and by matrix_kernel (LDS: whole KiB of input, then what half_kernel alone keeps there)
+SPLIT = [((5, 163, 41, 54, 81, 3, 1, 1), True), ((10, 120, 40, 32, 89, 3, 2, 1), False)]
 
 
-def split_layer(seed):
+def split_layer(seed, layer, half):
     import torch
     import tetris_amd as T
 
-    N, C, H, W, K, ks, stride, pad = SPLIT
+    N, C, H, W, K, ks, stride, pad = layer
     rng = np.random.default_rng(seed)
     w = sparse_filter(rng, K, C, ks, 0.7)
     tile = T.tile_select(N, H, W, C, K, ks, stride, pad)
     pk = T.G950Filter.for_tile(w, tile, oc_order="balanced")
     shape = pk.launch_shape(N, H, W, stride, pad, tile)
-    assert shape.kernel == 5 and shape.csplit > 1
+    assert shape.kernel == 5 and shape.csplit > 1 and (shape.lds_bytes % 1024 != 0) == half
+    oh, ow = T.out_extent(H, pad, ks, stride), T.out_extent(W, pad, ks, stride)
     xs = [torch.from_numpy(relu_like(rng, (N, C, H, W))).cuda() for _ in range(2)]
 
     def launch(x, y, stream=0):
@@ -303,21 +305,22 @@ def split_layer(seed):
 
     want = []
     for x in xs:
-        y = torch.full((N, K, H, W), float("nan"), device="cuda")
+        y = torch.full((N, K, oh, ow), float("nan"), device="cuda")
         launch(x, y)
         torch.cuda.synchronize()
         want.append(y.cpu().numpy())
     return pk, tile, launch, xs, want
 
 
-def test_graph_of_a_split_matrix_layer():
+@pytest.mark.parametrize("layer,half", SPLIT)
+def test_graph_of_a_split_matrix_layer(layer, half):
     import torch
 
-    N, C, H, W, K, ks, stride, pad = SPLIT
-    pk, tile, launch, xs, want = split_layer(21)
+    N, C, H, W, K, ks, stride, pad = layer
+    pk, tile, launch, xs, want = split_layer(21, layer, half)
     side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     pk.prepare(N, H, W, stride, pad, tile, side.cuda_stream)
-    x, y, other = xs[0].clone(), torch.empty((N, K, H, W), device="cuda"), torch.empty((N, K, H, W), device="cuda")
+    x, y, other = xs[0].clone(), torch.empty(want[0].shape, device="cuda"), torch.empty(want[0].shape, device="cuda")
     torch.cuda.synchronize()
     with torch.cuda.graph(graph, stream=side):
         launch(x, y, torch.cuda.current_stream().cuda_stream)
@@ -333,13 +336,13 @@ def test_graph_of_a_split_matrix_layer():
     pk.close()
 
 
-def test_two_streams_of_a_split_matrix_layer():
+@pytest.mark.parametrize("layer,half", SPLIT)
+def test_two_streams_of_a_split_matrix_layer(layer, half):
     import torch
 
-    N, C, H, W, K, ks, stride, pad = SPLIT
-    pk, tile, launch, xs, want = split_layer(22)
+    pk, tile, launch, xs, want = split_layer(22, layer, half)
     streams = [torch.cuda.Stream() for _ in range(2)]
-    ys = [[torch.full((N, K, H, W), float("nan"), device="cuda") for _ in range(8)] for _ in streams]
+    ys = [[torch.full(want[0].shape, float("nan"), device="cuda") for _ in range(8)] for _ in streams]
     torch.cuda.synchronize()
     for i in range(8):
         for x, y, s in zip(xs, ys, streams):
