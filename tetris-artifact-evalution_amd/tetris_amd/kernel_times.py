@@ -1,5 +1,5 @@
 """Times the walking kernels and every configuration of the two matrix kernels on a set of layers, and checks the time models that
-the library chooses between them with, or fits those of half_kernel and of the walk (csrc/matrix_conv.hip).
+the library chooses between them with, or fits them (csrc/matrix_conv.hip).
 
     make fit                                                  the library with the entry points used here
     TETRIS_SPCONV2D_LIB=$PWD/build_fit/libtetris_spconv2d.so python -m tetris_amd.kernel_times --measure FILE     (GPU)
@@ -138,6 +138,30 @@ def filled(wgs, fit, cycles):
     return full * cycles(fit) + np.where(last > 0, cycles(last), 0)
 
 
+PLAIN0 = dict(start=3214, team=733, round1=1213, round3=2935, staging=293, step=469, product=1.08, launch=2.06,
+              reread=0.72, rate=4.26, weights=2.9, add=2.37, add_rate=3.95)
+
+
+def plain_model(p, f):
+    wm, wn, nb, kw = (np.array([CONFIGS[int(c)][i] for c in f["cfg"]]) for i in range(4))
+    regs = np.select([nb == 4, nb == 2, kw == 1, kw == 2], [2 // kw, np.maximum(1, 3 // kw), 5, 2], 1)
+    fit = np.maximum(1, np.minimum(regs, np.floor(160 * 1024 / f["lds"])))
+    rounds = np.ceil(np.ceil(f["chunks"] / f["csplit"]) / kw)
+    steps, staging = f["ks"] ** 2 * f["kgs"] / 2, np.ceil(f["kgs"] * f["lpad"] / 256)
+    one = f["ks"] == 1
+
+    def cycles(n):
+        step = np.maximum(np.where(one, 0, p["step"]), p["product"] * 256 * nb * kw * n)
+        return (p["start"] + p["team"] * nb * n * kw +
+                rounds * (np.where(one, p["round1"], p["round3"]) + p["staging"] * staging * kw * n + steps * step))
+
+    compute = filled(f["ptiles"] * f["mtiles"] * f["csplit"], fit, cycles) / 2.2e3
+    out = 4 * f["N"] * f["K"] * f["OH"] * f["OW"]
+    inp = 4 * f["N"] * f["C"] * np.where(one, f["OH"], f["H"]) * f["W"]
+    memory = (inp * (1 + p["reread"] * np.sqrt(f["mtiles"] - 1)) + out * f["csplit"] + p["weights"] * 3072 * f["mblocks"] * f["chunks"] * steps) / (p["rate"] * 1e6)
+    return p["launch"] + np.maximum(compute, memory) + np.where(f["csplit"] > 1, p["add"] + out * (f["csplit"] + 1) / (p["add_rate"] * 1e6), 0)
+
+
 HALF0 = dict(start=4973, team=1257, round1=221, round3=722, staging=681, step=165, issue=2.032, product=1.231, work=87,
              launch=1.67, add=2.48, add_rate=4.3)
 
@@ -243,19 +267,20 @@ def main():
     elif a.fit:
         data = read(a.fit)
         # the fastest configurations of a layer decide, and are weighed accordingly
-        fm, um, wm = [], [], []
-        for walk, rows in data:
-            best = min([r[1] for r in rows], default=0)
-            for f, us, _ in rows:
-                if not f["half"]:
-                    continue
-                fm.append(f), um.append(us), wm.append((best / us) ** 2 / math.sqrt(len(rows)))
-        pm = fit(half_model, HALF0, fm, um, np.array(wm))
+        models = {}
+        for half, name, model, start in ((0, "plain_time", plain_model, PLAIN0), (1, "half_time", half_model, HALF0)):
+            fm, um, wm = [], [], []
+            for walk, rows in data:
+                best = min([r[1] for r in rows], default=0)
+                for f, us, _ in rows:
+                    if f["half"] == half:
+                        fm.append(f), um.append(us), wm.append((best / us) ** 2 / math.sqrt(len(rows)))
+            models[half] = model, fit(model, start, fm, um, np.array(wm))
+            print(name, ", ".join("%s %.4g" % kv for kv in models[half][1].items()))
         pw = fit(walk_model, WALK0, [w[0] for w, _ in data], [w[1] for w, _ in data], 1.0)
-        for name, p in (("half_time", pm), ("walk_time", pw)):
-            print(name, ", ".join("%s %.4g" % kv for kv in p.items()))
-        one = lambda model, p: lambda f, built: float(model(p, columns([f]))[0]) if f.get("half", 1) else built  # noqa: E731
-        report(data, one(half_model, pm), one(walk_model, pw), margins)
+        print("walk_time", ", ".join("%s %.4g" % kv for kv in pw.items()))
+        one = lambda model, p, f: float(model(p, columns([f]))[0])  # noqa: E731
+        report(data, lambda f, _: one(*models[f["half"]], f), lambda f, _: one(walk_model, pw, f), margins)
     else:
         sys.exit("one of --measure, --fit, --check")
 
