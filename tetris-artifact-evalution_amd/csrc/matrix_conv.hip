@@ -298,9 +298,11 @@ __global__ __launch_bounds__(256 * KW, KW == 4 ? 4 : 2) void matrix_kernel(const
     }
   }
   if (__ballot(odd != 0.f) == 0) return;
-  // Out of range: the wave's sums once more, over what was stored.  (A lane's stores to one address keep their order.)
+  // Out of range: the wave's sums once more, over what was stored.  (Not always by the same lane: where outputs went out four pixels
+  // at a time an output's lane was its neighbour.  So the wave waits until they are there.)
   // Latency of the loads bounds this, and it is here to be right: 1.7 ms with one infinity in the input of the layer above
   // (128 -> 256 channels, 52x52, batch 16), 3.9 ms with nothing but.
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   int again = lane;  // (unknown to the compiler, which would else keep the pixels' places in registers all the while)
   asm("" : "+v"(again));
   const int ch0 = slice * g.chunks / g.csplit * 8 * g.kgs, ch1 = min(g.C, (slice + 1) * g.chunks / g.csplit * 8 * g.kgs);

@@ -616,6 +616,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW, NB == 1 ? 3 : 2) void half_kerne
   asm("" : "+s"(arguments), "+v"(thread));  // so that nothing that a pass computed is kept for the next
   if (matrix_pass<1, WM, WN, NB, KW, TM>(arguments, thread)) return;
   asm("" : "+s"(arguments), "+v"(thread));
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the last pass stores over what the second has stored, by other lanes
   matrix_pass<2, WM, WN, NB, KW, TM>(arguments, thread);
 }
 
