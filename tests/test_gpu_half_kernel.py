@@ -201,6 +201,45 @@ def test_small_inputs_beside_large_ones(at, what, large, small):
     layer.pack.close()
 
 
+@pytest.mark.parametrize("tiny_weights", [False, True])
+@pytest.mark.parametrize("N,C,H,W,K,ks,stride,pad,density", [
+    (3, 42, 40, 77, 81, 3, 1, 1, 0.15), (8, 33, 47, 63, 68, 5, 1, 0, 0.3), (11, 120, 18, 70, 11, 7, 2, 0, 0.2), (12, 111, 23, 78, 21, 3, 2, 1, 0.15),
+    (8, 117, 38, 38, 183, 1, 1, 0, 0.15), (1, 20, 28, 8, 10, 4, 1, 0, 0.3), (6, 19, 88, 50, 199, 3, 1, 0, 0.2), (4, 17, 52, 80, 258, 3, 1, 1, 0.15)])
+def test_a_few_inputs_out_of_range(N, C, H, W, K, ks, stride, pad, density, tiny_weights):
+    """Single inputs that fp16 parts do not hold, in the first and the last channels, at an edge and inside: the outputs that they do
+    not reach keep the bits that they have without them (so nothing is computed again), and the others are as exact as any."""
+    import torch
+    import tetris_amd as T
+
+    rng = np.random.default_rng(10)
+    w = filter_of(rng, K, C, ks, density)
+    if tiny_weights:  # the second of every eighth row, multiplied one by one too
+        for k in range(0, K, 8):
+            w.reshape(K, -1)[k, np.flatnonzero(w.reshape(K, -1)[k])[1]] *= np.float32(2.0 ** -22)
+    without = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    at = [(0, C - 1, 5, W - 1, -30), (0, 0, H - 1, 2, -50), (N - 1, C // 2, H // 2, W // 3, 8), (N - 1, 1, H - 2, W // 2, 25)]
+    # (The small ones alone.  A large one where a tile's scale is taken from, at the start of a row, would put more than itself out of range.)
+    for n, c, y, x, e in at:
+        without[n, c if e > 0 else slice(None), max(y - ks, 0):y + ks + 1, max(x - ks, 0):x + ks + 1] = 0
+    few = without.copy()
+    for n, c, y, x, e in at:
+        few[n, c, y, x] = np.ldexp(1 + rng.random(), e)
+    layer = Layer(w, few.shape, stride, pad)
+    got, again, base = layer(few), layer(few), layer(without)
+    reached = conv64((few != without).astype(np.float32), (w != 0).astype(np.float32), stride, pad)[0] != 0
+    assert reached.any() and np.array_equal(got, again) and np.array_equal(got[~reached], base[~reached])
+    ref, terms = conv64(few, w, stride, pad)
+    bound = (w != 0).reshape(K, -1).sum(1).reshape(1, K, 1, 1) * 2.0 ** -24 * terms
+    assert (np.abs(got - ref) <= bound).all()
+    if layer.pack.act_supported(*layer.at, layer.tile, T.ACT_RELU_POOL2):
+        n, k, oh, ow = layer.out
+        dx, y = torch.from_numpy(few).cuda(), torch.full((n, k, oh // 2, ow // 2), float("nan"), device="cuda")
+        layer.pack.launch_act(dx.data_ptr(), y.data_ptr(), *layer.at, layer.tile, T.ACT_RELU_POOL2)
+        quads = lambda a: a[:, :, :oh // 2 * 2, :ow // 2 * 2].reshape(n, k, oh // 2, 2, ow // 2, 2).max((3, 5))  # noqa: E731
+        assert (np.abs(y.cpu().numpy() - np.maximum(quads(ref), 0)) <= quads(bound)).all()
+    layer.pack.close()
+
+
 @pytest.mark.parametrize("scale_x,scale_w", [(0, 0), (-10, 3), (-120, 0), (-140, 4), (0, -130), (-70, -60), (40, 20), (80, -100), (120, -10)])
 def test_outputs_of_one_term(scale_x, scale_w):
     """Inputs and weights of full 24-bit significands, one product an output: as exact as one rounding of it."""

@@ -25,6 +25,7 @@ inline bool stores_quads(const MatGeom& g, const float* d_out) {
 
 // matrix_half.hip
 constexpr int kMostChannels = 1 << 20;  // input channels of a layer: a loose weight's place is an int, 20 bits of which name its channel
+constexpr int kAsideBytes = 64 + 64 * 8;  // of LDS: inputs that are multiplied one by one
 constexpr int kStepBytes = 3 * 1024 + 256, kSlotBytes = 2048;  // of a step's weights: fp16 parts and a word per lane; fp32
 size_t half_weight_bytes(const MatGeom& g);
 int half_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* base, MatWeights* out);  // waits for them

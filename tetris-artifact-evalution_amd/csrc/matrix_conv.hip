@@ -379,7 +379,7 @@ int lds_main(const MatGeom& g) {
   const MatShape& c = kMatShapes[g.cfg];
   return std::max(c.kw * 96 * g.kgs * g.lpad, c.kw > 1 ? c.kw * c.wm * c.wn * 4096 * c.nb : 0);
 }
-int lds_bytes(const MatGeom& g) { return lds_main(g) + (g.half ? 128 * kMatShapes[g.cfg].wm + 16 : 0); }
+int lds_bytes(const MatGeom& g) { return lds_main(g) + (g.half ? 128 * kMatShapes[g.cfg].wm + kAsideBytes : 0); }
 
 template <int WM, int NB, int KW, int TM>
 int launch_one(const MatGeom& g, const float* d_in, float* d_out, const void* weights, hipStream_t stream) {

@@ -26,12 +26,17 @@
 // (31.3); 16 x 256 -> 256 28x28 to 14x14 of 85 % 44.9, 33.9 (45.0); 4 x 256 -> 256 28x28 of 90 % 35.3, 25.9 (33.3); 16 x 256 ->
 // 512 26x26 of 85 % 148, 103 (125) -- of 226 tiles of 96 pixels; 170 of 128 pixels leave a third of the CUs idle: 125.
 //
-// Range: inputs are scaled by what a few of them, the same for all waves, show.  Where some input is 2^4 times as large as those, or
-// smaller than 2^-27 of the largest of them and not zero, the workgroup makes a second pass with bf16 parts, which hold every number
-// (see matrix_conv.hip for those, and for what is out of their range: the third pass).  An input's size decides, and not
-// whether its parts add up to it: with few significant bits they do so far below, where m has lost bits to fp16's smallest
-// exponent, l carries the number, and off xl is 2^-17 of the product and more.  Weights that fp16 parts do not hold are few: FMAs
-// add them at the end.
+// Range: inputs are scaled by what a few of them, the same for all waves, show.  Inputs 2^6 times as large as those, or smaller than
+// 2^-25 of the largest of them and not zero, are staged as zeros and multiplied one by one with FMAs in the end, up to eight of a workgroup.
+// Where they are more, or infinite, it makes a second pass with bf16 parts, which hold every number (see matrix_conv.hip for those,
+// and for what is out of their range: the third pass).  An input's size decides, and not whether its parts add up to it:
+// with few significant bits they do so far below, where m has lost bits to fp16's smallest exponent, l carries the number, and off xl
+// is 2^-17 of the product and more.  Weights that fp16 parts do not hold are few: FMAs add them at the end as well.
+// Single inputs out of range are ordinary: one in 10^7 of normally distributed ones is below 2^-25 of the largest, which is one
+// workgroup or two of 226 on 256 channels, and a launch ends with its slowest.  Microseconds with a second pass for each such workgroup
+// and now, in brackets the walk: 16 x 256 -> 512 26x26 of 85 % zeros, channels that differ in scale by e^(normal) 198, 106 (124); SiLU of
+// normal inputs 123, 112; softmax over the channels, where the first chunk shows that they are many, 246, 147; exp(3 normal) 245, 229.
+// Testing and listing costs 0 to 0.35 us a launch.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -51,7 +56,9 @@ typedef unsigned u32x8 __attribute__((ext_vector_type(8)));
 // brings the largest of its row to [2^14, 2^15) likewise.  h has eight bits, m eleven, l the rest.  (With 2^-19 l inputs of 2^-32
 // of the largest would still be the sum of their parts, but of subnormal ones, whose left-out products are not small any more.)
 constexpr float kMid = 256.f, kLow = 128.f;  // from h to m, from m to l
-constexpr float kSmall = 0x1p-16f;  // the smallest scaled input that is multiplied in parts: from here on all 24 bits are in them
+// Exponents of scaled inputs: the smallest that is multiplied in parts, from which on all 24 bits are in them; below the largest that
+// h holds; the smallest that is listed where it is not, and above the largest.
+constexpr int kSmall = -16, kLarge = 15, kLeastListed = -60, kMostListed = 40;
 
 // (A bit cast of a vector's element itself, instead of its value, is compiled to one of the vector's first element.)
 __device__ __forceinline__ float float_of(unsigned x) { return __builtin_bit_cast(float, x); }
@@ -138,6 +145,12 @@ static_assert(kStepBytes == 3 * 1024 + 256);
 constexpr float kLeast = 0x1p-3f, kLeastLoose = 0x1p-60f;
 constexpr int kMostLoose = 64;
 
+// Inputs that fp16 parts do not hold, or not well enough, are multiplied one by one as well: a wave stages zeros in their place and
+// lists them, if they are 2^-60 to 2^40 in the tile's scale.  Where a workgroup has more than kMostAside, or others, it makes the second
+// pass, and at once where a wave's first chunk already shows that.
+constexpr unsigned kMostAside = 8, kNotListed = 1u << 24;
+static_assert(kAsideBytes == 2 * 8 * 4 + 8 * 8 * kMostAside);  // of eight waves: counts after the first chunk and in the end, lists
+
 struct MatArguments { const float* in; float* out; MatWeights w; MatGeom g; };
 typedef const MatArguments __attribute__((address_space(4))) * Arguments;  // the kernel's, read through the scalar cache
 
@@ -149,8 +162,8 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   constexpr int TW = WM * WN, P = 32 * NB * WN;
   const auto& g = arguments->g;
   // What the places of the pixels are worked out with, read at once: each first touch of a line is a trip to L2.
-  const struct { unsigned m_uw, m_uh, m_wp, m_ihs, m_strips; int upq, uw, uh, wp, ihs, strips, ws, stride, sub, pad, pool, npix, H, W, C, N, kgs, lpad; } at = {
-      g.m_uw, g.m_uh, g.m_wp, g.m_ihs, g.m_strips, g.upq, g.uw, g.uh, g.wp, g.ihs, g.strips, g.ws, g.stride, g.sub, g.pad, g.pool, g.npix, g.H, g.W, g.C, g.N, g.kgs, g.lpad};
+  const struct { unsigned m_uw, m_uh, m_wp, m_ihs, m_strips; int upq, uw, uh, wp, ihs, strips, ws, stride, sub, pad, pool, npix, H, W, C, N, ks, kgs, lpad; } at = {
+      g.m_uw, g.m_uh, g.m_wp, g.m_ihs, g.m_strips, g.upq, g.uw, g.uh, g.wp, g.ihs, g.strips, g.ws, g.stride, g.sub, g.pad, g.pool, g.npix, g.H, g.W, g.C, g.N, g.ks, g.kgs, g.lpad};
   const auto& w = arguments->w;
   const float* const in = arguments->in;
   extern __shared__ u32x4 all_lds[];  // [KW][2][kgs][lpad][3], then the exponents of the tile's rows
@@ -158,7 +171,8 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   const int team = wave_id / TW, wave = wave_id % TW;
   u32x4* const lds = all_lds + team * 6 * g.kgs * g.lpad;
   int* const row_exp = reinterpret_cast<int*>(reinterpret_cast<char*>(all_lds) + g.lds_rows);
-  int* const inexact = row_exp + 32 * WM;  // set where an input's parts do not add up to it
+  unsigned* const asides = reinterpret_cast<unsigned*>(row_exp + 32 * WM);  // per wave: how many inputs are set aside
+  int2* const aside = reinterpret_cast<int2*>(asides + 16);                 // ... which: channel and staged pixel; the input
   // workgroup ids go round-robin to the XCDs: each XCD gets a contiguous range of logical ids.  Channel blocks of one pixel
   // tile are neighbours (they read the same input), slices outermost (they share nothing).
   const int per = gridDim.x >> 3;
@@ -183,9 +197,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   // Weights: the steps of a wave follow one another; they are asked for three steps ahead of their products.
   struct Step { u32x4 p[F16 ? 3 : 2]; unsigned word; };
   int next_step = w.first[block * g.chunks + c_beg];
-  // (With weights that fp16 parts cannot hold, `loose` below zero, the first pass has no steps.  With a branch around it the compiler
-  // would spill registers of it.)
-  const int loose = F16 ? w.loose_count[block] : 0, steps = loose < 0 ? 0 : w.first[block * g.chunks + c_beg + mine] - next_step;
+  const int loose = F16 ? w.loose_count[block] : 0, steps = w.first[block * g.chunks + c_beg + mine] - next_step;
   const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(w.steps), 0, w.step_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(w.slots), 0, w.step_bytes / kStepBytes * kSlotBytes, 0x00020000);
   auto fetch_weights = [&](Step& s) {
@@ -234,18 +246,51 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
       }
     }
   };
-  f16x2 zeros = {0, 0};
-  unsigned least = ~0u;  // least: of the inputs' bits without the sign, doubled, less one: zeros come out on top
   float scale = 1.f;
-  auto keep = [&](int buf) {
+  // the exponent bits of 2^e in the tile's scale, of a number that is not scaled yet (where it may underflow)
+  auto unscaled = [&](int e) { return (unsigned)min(max(2 * 127 + e - (int)(bits_of(scale) >> 23), 0), 255) << 23; };
+  // inputs of a lane that six products cannot be formed of: listed, and zero in its parts
+  unsigned own_asides = loose < 0 ? kNotListed : 0;
+  auto set_aside = [&](const float (&x)[8], u32x4& h, u32x4& m, u32x4& l, int slot, int channel) {
+    unsigned which = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const unsigned u = bits_of(x[j]) & 0x7fffffff;
+      if (u - 1 < unscaled(kSmall) - 1 || u >= unscaled(kLarge)) which |= 1u << j;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned held = (which >> 2 * i & 1 ? 0 : 0xffffu) | (which >> 2 * i & 2 ? 0 : 0xffff0000u);
+      h[i] &= held;
+      m[i] &= held;
+      l[i] &= held;
+    }
+    while (const unsigned long long lanes = __builtin_amdgcn_ballot_w64(which != 0)) {
+      const int j = __builtin_ctz(which | 256);
+      float v = x[0];
+#pragma unroll
+      for (int q = 1; q < 8; ++q) v = j == q ? x[q] : v;
+      const unsigned u = bits_of(v) & 0x7fffffff, n = own_asides + __builtin_amdgcn_mbcnt_hi(lanes >> 32, __builtin_amdgcn_mbcnt_lo(lanes, 0));
+      const bool listed = u >= unscaled(kLeastListed) && u < unscaled(kMostListed);
+      if (which && n < kMostAside) aside[wave_id * kMostAside + n] = make_int2((channel + j) << 10 | slot, (int)bits_of(v));
+      own_asides = min(own_asides + (__builtin_amdgcn_ballot_w64(which && !listed) ? kNotListed : __builtin_popcountll(lanes)), kNotListed);
+      which &= which - 1;
+    }
+  };
+  auto keep = [&](int buf, int chunk) {
 #pragma unroll
     for (int k = 0; k < TM; ++k) {
       if (wave + TW * k >= tasks) break;
       u32x4 h, m, l;
       if constexpr (F16) {
+        f16x2 zeros = {0, 0};
         cut16(x[k], scale, h, m, l, zeros, nullptr);
+        unsigned least = ~0u;  // of the inputs' bits without the sign, doubled, less one: zeros come out on top
 #pragma unroll
         for (int j = 0; j < 8; ++j) least = min(least, (bits_of(x[k][j]) << 1) - 1);
+        const bool infinite = __builtin_bit_cast(unsigned, zeros) & 0x7fff7fff;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(infinite || least < 2 * unscaled(kSmall) - 1) != 0, 0))
+          set_aside(x[k], h, m, l, gslot[k] / 3 - gkg[k] * at.lpad, (chunk * at.kgs + gkg[k]) * 8);
       } else {
         cut(x[k], h, m, l);
       }
@@ -369,24 +414,19 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     __builtin_amdgcn_sched_barrier(0);  // in this order: the loop waits for the first set only
   }
   if constexpr (F16) {
-    // Their largest is scaled to [2^11, 2^12): with 4 bits to spare above, down to 2^-27 or 2^-28 of it.
+    // Their largest is scaled to [2^9, 2^10).  (To [2^11, 2^12), with 4 bits to spare above, channels that differ in scale often had more
+    // than a few inputs too large: 150 us for the 106 named above.)
     unsigned most = max(max(some[0] & 0x7fffffff, some[1] & 0x7fffffff), max(some[2] & 0x7fffffff, some[3] & 0x7fffffff));
     most = wave_max(most);
-    const int shift = most ? min(max(138 - (int)(most >> 23), -100), 100) : 6;
+    const int shift = most ? min(max(136 - (int)(most >> 23), -100), 100) : 6;
     scale = __builtin_bit_cast(float, (127 + shift) << 23);
     if (thread < 32 * WM) row_exp[thread] = exponent - shift;
   }
-  if (F16 && thread == 0) *inexact = loose < 0;
-  keep(0);
+  keep(0, c_beg);
+  if (F16) asides[8 + wave_id] = own_asides > kMostAside || (own_asides > 2 && own_asides * (unsigned)rounds > kMostAside);
   __syncthreads();
-  // whether the inputs that were staged are what six products can be formed of: no h is infinite, and none but zeros are below
-  // kSmall / scale (looked at before they are scaled, where they may underflow)
-  auto held = [&]() {
-    const bool infinite = __builtin_bit_cast(unsigned, zeros) & 0x7fff7fff;
-    return __builtin_amdgcn_ballot_w64(infinite || least < 2 * (bits_of(kSmall) + bits_of(1.f) - bits_of(scale)) - 1) == 0;
-  };
   const int wp3 = 3 * at.wp, lpad3 = 3 * at.lpad;
-  const bool large = g.ks > 4;
+  const bool large = at.ks > 4;
   int buf = 0, round = 0;
   bool fresh = true;  // the chunk's first step
   // A step reads the input of its two blocks of pixels one after the other, each while the products of the one before run: the
@@ -413,6 +453,7 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
   if constexpr (F16) {
     place_of(ahead[0].word);
     read(input[0], 0);
+    if (__builtin_amdgcn_ballot_w64(asides[8 + (lane & (TW * KW - 1))] != 0)) return false;
   }
   // Where a wave has an odd number of blocks, more than one, two steps take turns with the two places for a block's input.
   auto step = [&](Step& now, Step& next, auto turn) {
@@ -484,8 +525,8 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     if constexpr (NB > 1) products(input[(kFirst + NB - 1) % 2], NB - 1);
     refill();
     if (!F16 && more) fetch(c_beg + round + 1);  // (the second pass is rare: fewer registers instead of less waiting)
-    if (more) keep(buf ^ 1);
-    if (F16 && round + 1 == rounds && !held()) *inexact = 1;
+    if (more) keep(buf ^ 1, c_beg + round + 1);
+    if (F16 && round + 1 == rounds) asides[wave_id] = own_asides;
     buf ^= 1;
     fresh = true;
     ++round;
@@ -509,11 +550,13 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
     }
   }
   if (round < rounds) {  // a team with a chunk less
-    if (F16 && !held()) *inexact = 1;
+    if (F16) asides[wave_id] = own_asides;
     __syncthreads();
   }
   if constexpr (F16) {
-    if (*inexact) return false;
+    const unsigned listed = asides[lane / kMostAside & (TW * KW - 1)];  // by the wave whose list this lane may read
+    const unsigned long long some_listed = __builtin_amdgcn_ballot_w64(lane < TW * KW * (int)kMostAside && lane % kMostAside < listed);
+    if (__builtin_popcountll(some_listed) > (int)kMostAside || __builtin_amdgcn_ballot_w64(listed > kMostAside)) return false;
     // the weights that fp16 parts do not hold: few blocks have any
     int again = lane;  // (unknown to the compiler, which would else keep the pixels' places in registers all the while)
     asm("" : "+v"(again));
@@ -532,6 +575,37 @@ __device__ __forceinline__ bool matrix_pass(Arguments arguments, int thread) {
 #pragma unroll
         for (int i = 0; i < 16; ++i)
           if (i == (row >> 3) * 4 + (row & 3)) sum[0][b][i] = fmaf(v, weight, sum[0][b][i]);
+      }
+    }
+    // The inputs that are set aside, with the weights that are not among those, in the order of their places: sums do not depend on
+    // who came first.
+    if (some_listed) {
+      const int2 own = some_listed >> again & 1 ? aside[again] : make_int2(0x7fffffff, 0);
+      const int all = __builtin_popcountll(some_listed);
+      int before = 0;
+      for (unsigned long long left = some_listed; left; left &= left - 1) before += __builtin_amdgcn_readlane(own.x, __builtin_ctzll(left)) < own.x;
+      const int shift = (int)(bits_of(scale) >> 23) - 127, cpad = 8 * at.kgs * g.chunks;
+      for (int e = 0; e < all; ++e) {
+        const int from = __builtin_ctzll(__builtin_amdgcn_ballot_w64(before == e));
+        const int where = __builtin_amdgcn_readlane(own.x, from), c = where >> 10, chunk = c / (8 * at.kgs);
+        if (chunk < c_beg || chunk >= c_beg + mine) continue;
+        const float v = float_of(__builtin_amdgcn_readlane(own.y, from)) * scale;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          int tap = -1;  // of the lane's pixel that reads it
+          for (int r = 0; r < g.ks; ++r) {
+            const int s = 3 * (where & 1023) - bpos[b] - 3 * r * at.wp;
+            if (s >= 0 && s < 3 * g.ks) tap = r * g.ks + s / 3;
+          }
+          if (!__builtin_amdgcn_ballot_w64(tap >= 0)) continue;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int row = 8 * (i / 4) + 4 * (again >> 5) + i % 4, oc = oc0 + row;
+            const float weight = tap >= 0 && oc < g.K ? w.dense[((size_t)oc * g.ks * g.ks + tap) * cpad + c] : 0.f;
+            const float scaled = ldexpf(weight, -(row_exp[wm * 32 + row] + shift));
+            sum[0][b][i] = fmaf(v, fabsf(scaled) >= kLeast ? scaled : 0.f, sum[0][b][i]);
+          }
+        }
       }
     }
   }
