@@ -521,7 +521,7 @@ double plain_time(const MatGeom& g) {
   return 2.2 + std::max(compute, memory) + (g.csplit > 1 ? 2.5 + out * (g.csplit + 1) / 4.07e6 : 0);
 }
 
-// The same for half_kernel, fitted to 13 801 launches of the same layers: 9 % off.
+// The same for half_kernel, fitted to launches of the same layers before inputs out of range were listed: 9 % off on 13 749 since.
 double half_time(const MatGeom& g, long long nnz) {
   const MatShape& c = kMatShapes[g.cfg];
   const int team = c.wm * c.wn, waves = team * c.kw;
@@ -568,11 +568,12 @@ double walk_time(const Geom& g, long long nnz) {
 // Whether a matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and slice
 // count of least predicted time, if that is 7 % below the walking kernel's; half_kernel's, if that is 16 % below the walking
 // kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's.  Of the 424 timed layers 125
-// then go to matrix_kernel and 96 to half_kernel; over all of them that is 1.196 times the walk's speed, 2.8 % short of the
-// best choice, 10 layers lose more than 3 % to the walk and two to what matrix_kernel and the walk alone would give them.
-// (Without half_kernel 1.152 times.  With 12 % to the walk eight layers lose so, with 10 % and no advantage asked over
-// matrix_kernel 22.)  Where the walking
-// kernel can pool its outputs, so must the matrix kernel.
+// then go to matrix_kernel and 96 to half_kernel; over all of them that is 1.192 times the walk's speed, 3.0 % short of the
+// best choice.  10 layers lose more than 3 % to the walk, all on matrix_kernel and pointwise or of one image, two of them half
+// as much again (1 x 512 -> 1024 28x28 15.6 us, 10.6; 1 x 1024 -> 255 13x13 15.4, 10.5; with 10 % instead of 7 % two layers lose, 9 % at
+// most, and 1.191 times), and six to what matrix_kernel and the walk alone would give them.  (Without half_kernel 1.152 times.  With
+// 12 % to the walk 13 layers lose so, with 10 % and no advantage asked over matrix_kernel 27.)  Where the walking kernel can pool its
+// outputs, so must the matrix kernel.
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      MatGeom* g, MatGeom* pool) {
   if (C < 16) return false;  // most of a chunk of 16 channels would be padding
