@@ -699,19 +699,31 @@ __device__ __forceinline__ void compute_again(Arguments arguments, const Work& w
   const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(w.steps), 0, w.step_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(w.slots), 0, w.step_bytes / kBytes * kSlotBytes, 0x00020000);
   int next_step = w.first[block * g.chunks + work.c_beg];
+  struct { u32x4 v[2]; unsigned word; } ahead;
+  auto fetch_slots = [&](int step) {
+    ahead.v[0] = __builtin_amdgcn_raw_buffer_load_b128(srsrc, lane * 16, step * kSlotBytes, 0);
+    ahead.v[1] = __builtin_amdgcn_raw_buffer_load_b128(srsrc, lane * 16 + 1024, step * kSlotBytes, 0);
+    ahead.word = __builtin_amdgcn_raw_buffer_load_b32(wrsrc, lane * 4 + 2048, step * kBytes, 0);
+  };
+  fetch_slots(next_step);
   const int end = w.first[block * g.chunks + work.c_beg + work.rounds];
   for (int round = 0; round < work.rounds; ++round) {
     __syncthreads();
     for (int task = wave_id * 64 + lane; task < at.kgs * tile.staged; task += 512) {
       const int kg = task / tile.staged, quad = task - kg * tile.staged, c = ((work.c_beg + round) * at.kgs + kg) * 8;
       unsigned inside;
-      const int off = source_of(at, tile, quad, inside);
-#pragma nounroll
+      const int from = source_of(at, tile, quad, inside) + c * hw4;
+      u32x4 x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_raw_buffer_load_b128(irsrc, c + j < at.C ? max(from, 0) + j * hw4 : kOutside, 0, 0);
+      for (int p = 0; p < 3; ++p)  // (read from the tensor's first pixel on instead of from before it)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = from + 4 * p < 0 ? u32x4{0, x[j][0], x[j][1], x[j][2]} : x[j];
+#pragma unroll
       for (int e = 0; e < 4; ++e) {
         float v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          v[j] = float_of(__builtin_amdgcn_raw_buffer_load_b32(irsrc, inside >> e & 1 && c + j < at.C ? off + 4 * e + (c + j) * hw4 : kOutside, 0, 0));
+        for (int j = 0; j < 8; ++j) v[j] = inside >> e & 1 ? float_of(x[j][e]) : 0.f;
         u32x4 part[3];
         cut(v, part[0], part[1], part[2]);
 #pragma unroll
@@ -719,9 +731,10 @@ __device__ __forceinline__ void compute_again(Arguments arguments, const Work& w
       }
     }
     __syncthreads();
-    for (bool last = false; !last && next_step < end; ++next_step) {
-      const u32x4 w0 = __builtin_amdgcn_raw_buffer_load_b128(srsrc, lane * 16, next_step * kSlotBytes, 0), w1 = __builtin_amdgcn_raw_buffer_load_b128(srsrc, lane * 16 + 1024, next_step * kSlotBytes, 0);
-      const unsigned word = __builtin_amdgcn_raw_buffer_load_b32(wrsrc, lane * 4 + 2048, next_step * kBytes, 0);
+    for (bool last = false; !last && next_step < end;) {
+      const u32x4 w0 = ahead.v[0], w1 = ahead.v[1];
+      const unsigned word = ahead.word;
+      fetch_slots(++next_step);  // (none behind the last: zeros)
       last = __builtin_amdgcn_readfirstlane(word) >> 31;
       int place[2];
 #pragma unroll
