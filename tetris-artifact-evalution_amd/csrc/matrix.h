@@ -28,7 +28,7 @@ inline bool stores_quads(const MatGeom& g, const float* d_out) {
 // matrix_half.hip
 constexpr int kMostChannels = 1 << 20;  // input channels of a layer: a loose weight's place is an int, 20 bits of which name its channel
 constexpr int kRelayPart = 60 * 1024;  // of LDS: a part of the inputs that relay_kernel stages
-constexpr int kRelayBytes = 4 * 4 + 3 * 8 * 4 + 48 * 4 + 3 * 64 * 8;  // ... behind those
+constexpr int kRelayBytes = 4 * 4 + 3 * 8 * 4 + 48 * 4 + 2 * 4 + 3 * 64 * 8;  // ... behind those
 constexpr int kAsideBytes = 64 + 64 * 8;  // of LDS: inputs that are multiplied one by one
 constexpr int kStepBytes = 3 * 1024 + 256, kStepBytes2 = 2 * 1024 + 256, kSlotBytes = 2048;  // of a step's weights: three or two fp16 parts and a word per lane; fp32
 size_t half_weight_bytes(const MatGeom& g);

@@ -12,11 +12,12 @@
 // 12 products, and a step takes 1100 to 1350 cycles of two waves, whose products alone are 792 -- and in between they stage what is
 // multiplied next: the first chunk of the next tile too, so that of the 18 000 cycles that a workgroup takes to its first product
 // (tiles, the inputs' scale, two trips to memory, a barrier) a run of tiles pays once.  The halves of the workgroup, of which a SIMD has one
-// wave each, stage at different times.  Sums are cleared every eight steps into a second set that is rounded less often: 1.92e-7 becomes
+// wave each, stage at different times, and no barrier ends a chunk (Stage::arrive): a wave whose channels have fewer steps goes ahead of the others
+// by up to a third of one, 141 against 134 us on 16 x 512 -> 512 28x28, 78 against 77 on 16 x 256 -> 512 26x26.  Sums are cleared every eight steps into a second set that is rounded less often: 1.92e-7 becomes
 // 1.49e-7 on 16 x 512 -> 512 28x28 (with the two kinds of small products summed apart instead 2.3e-7; clearing every two steps 1.89e-7).
 //
-// Microseconds, the walk and this: 16 x 256 -> 256 56x56, 10 % of the weights, 159 and 138 to 142 (large layers run at 1.5 to 1.8 GHz here,
-// held back by power); 15 % 222 and 163; 16 x 512 -> 512 28x28 175 and 131 to 142; 16 x 256 -> 512 26x26, 15 %, 124 and 73; 9 x 157 -> 152 134x134
+// Microseconds, the walk and this: 16 x 256 -> 256 56x56, 10 % of the weights, 159 and 132 to 140 (large layers run at 1.5 to 1.8 GHz here,
+// held back by power); 15 % 222 and 163; 16 x 512 -> 512 28x28 175 and 128 to 136; 16 x 256 -> 512 26x26, 15 %, 124 and 71; 9 x 157 -> 152 134x134
 // 5x5, 20 %, 1060 and 633.  Half of the waves staging for the others, which then multiply twelve blocks a step, took 5 to 20 % longer, and so
 // did one loop for all counts of blocks in a tile.
 #include "matrix_half.h"
@@ -205,6 +206,7 @@ struct Shared {
   int* shift;        // [4] inputs of a tile are multiplied by two to this
   unsigned* most;    // [3][kWaves] the largest of a few of them, per wave
   unsigned* asides;  // [3][16] per wave: how many inputs are set aside; 8: whether they are too many after the first chunk
+  int* counts;       // [2] chunks that waves have staged, all waves' added up, from a workgroup's second on; chunks that they have multiplied
   int2* aside;       // [3][kWaves][kMostAside] ... which: channel and staged pixel; the input
   float* sums;       // [kWaves][1024] of a block of pixels
 };
@@ -213,11 +215,12 @@ __device__ __forceinline__ Shared shared_of(Arguments arguments, u32x4* lds) {
   s.shift = reinterpret_cast<int*>(reinterpret_cast<char*>(lds) + arguments->g.lds_rows);
   s.most = reinterpret_cast<unsigned*>(s.shift + 4);
   s.asides = s.most + 3 * kWaves;
-  s.aside = reinterpret_cast<int2*>(s.asides + 48);
+  s.counts = reinterpret_cast<int*>(s.asides + 48);
+  s.aside = reinterpret_cast<int2*>(s.counts + 2);
   s.sums = reinterpret_cast<float*>(s.aside + 3 * kWaves * kMostAside);
   return s;
 }
-static_assert(kRelayBytes == 4 * 4 + 3 * kWaves * 4 + 48 * 4 + 3 * kWaves * kMostAside * 8);
+static_assert(kRelayBytes == 4 * 4 + 3 * kWaves * 4 + 48 * 4 + 2 * 4 + 3 * kWaves * kMostAside * 8);
 constexpr int kPart = kRelayPart / 16;  // A part of all staged inputs lies a fixed distance from the other, which reads have room for in their offsets.
 
 // whether a tile that is all staged has more inputs set aside than are multiplied one by one
@@ -237,6 +240,7 @@ struct Task {
   int c, off;       // first channel; where its first pixel lies there
 };
 constexpr int kNowhere = -1;
+constexpr int kStaged = 0, kMultiplied = 1;
 
 // What a wave asks for, and when: a tile's chunks one after the other, then the next tile's.
 template <int WN>
@@ -256,6 +260,7 @@ struct Stage {
   unsigned own_asides = 0;
   bool begins = false;  // what was asked for is a tile's first chunk
   int asked_tile = 0, asked_chunk = 0;
+  int done = 0;         // chunks that the wave has multiplied
   bool unread = false;  // the tensor's first pixels, with columns outside of the image before them
 
   __device__ __forceinline__ bool more() const { return tile < work.tiles; }
@@ -399,11 +404,22 @@ struct Stage {
     }
     return odd;
   }
-  __device__ __forceinline__ void end_chunk(int buf, bool odd) {
+  // how many inputs of a chunk are set aside (the count counts only once the tile's last chunk is staged)
+  __device__ __forceinline__ void publish() const {
     const int slot = asked_tile % 3;
-    if (__builtin_expect(odd, 0)) set_aside(buf);
     if (begins) shared.asides[16 * slot + 8 + wave] = own_asides > kMostAside || (own_asides > 2 && own_asides * (unsigned)work.rounds > kMostAside);
-    shared.asides[16 * slot + wave] = own_asides;  // (counts only once the tile's last chunk is staged)
+    shared.asides[16 * slot + wave] = own_asides;
+  }
+  // A wave goes on as soon as what it needs is there, not when the last one has done all that it has to: it multiplies a chunk once all have
+  // staged their part of it, and stages the next one once all have multiplied the one before, which the buffer held.
+  __device__ __forceinline__ void arrive(int which) const {
+    if (lane == 0) __hip_atomic_fetch_add(shared.counts + which, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ void wait_for(int which, int chunks) const {
+    for (int i = 0; i < 1 << 22; ++i) {  // (all waves are resident, and none waits for what comes after its own: the bound is never met)
+      if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(shared.counts + which, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) >= kWaves * chunks) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
   }
 };
 
@@ -488,15 +504,27 @@ __device__ __forceinline__ void multiply(Stage<WN>& stage, int k, unsigned some,
             sum[0][b][k] = 0.f;
           }
       }
-      if (i == max(when, 1) && stages) odd_inputs = stage.keep(buf ^ 1);
+      if (i == max(when, 1) && stages) {
+        stage.wait_for(kMultiplied, stage.done);
+        odd_inputs = stage.keep(buf ^ 1);
+        if (!odd_inputs) {
+          stage.publish();
+          stage.arrive(kStaged);
+        }
+      }
       if (i >= pairs) break;
       step(ahead[0], ahead[1], even, true);
       step(ahead[1], ahead[0], odd, i + 1 < pairs);
     }
     if (stages) {
-      stage.end_chunk(buf ^ 1, odd_inputs);
+      if (__builtin_expect(odd_inputs, 0)) {
+        stage.set_aside(buf ^ 1);
+        stage.publish();
+        stage.arrive(kStaged);
+      }
       if (round + 1 == stage.work.rounds && k + 2 < stage.work.tiles) stage.keep_sample(k + 2, some);
-      __syncthreads();
+      stage.arrive(kMultiplied);
+      stage.wait_for(kStaged, ++stage.done);
     }
     buf ^= 1;
   }
@@ -598,8 +626,10 @@ __device__ __forceinline__ unsigned long long multiply_all(Arguments arguments, 
   int buf = 0;
   stage.keep_sample(0, some_first[0]);
   if (work.tiles > 1) stage.keep_sample(1, some_first[1]);
+  if (wave == 0 && lane < 2) shared.counts[lane] = 0;
   __syncthreads();
-  stage.end_chunk(0, stage.keep(0));
+  if (stage.keep(0)) stage.set_aside(0);
+  stage.publish();
   __syncthreads();
   for (int k = 0; k < work.tiles; ++k) {
     const int slot = k % 3;
@@ -615,7 +645,11 @@ __device__ __forceinline__ unsigned long long multiply_all(Arguments arguments, 
       if (stage.tile == k || work.rounds == 1) stage.begin(k + 1);
       if (stage.more()) {
         stage.ask();
-        stage.end_chunk(buf ^ 1, stage.keep(buf ^ 1));
+        if (stage.keep(buf ^ 1)) stage.set_aside(buf ^ 1);
+        stage.publish();
+        stage.arrive(kStaged);
+        stage.arrive(kMultiplied);
+        ++stage.done;
       }
       __syncthreads();
       buf ^= 1;
