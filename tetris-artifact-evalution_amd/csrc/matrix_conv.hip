@@ -636,62 +636,71 @@ double walk_time(const Geom& g, long long nnz) {
   return std::max(compute, (in + out) / 6.9e6) + (g.csplit > 1 ? 1.5 + out * (g.csplit + 1) / 4.1e6 : 0);
 }
 
+// relay_kernel: only where a sum of the walk, in a slice of the channels, has kLeastTerms weights on average, and its own at most twice as many:
+// there it is as exact.  Its error from 64 bits, in the outputs' 2-norm over the walk's, is 0.38 to 0.98 on 6414 random layers that
+// this rule picks (inputs after a ReLU), and 1.1 to 1.3 on layers with 57 terms.  Walks of one, two and four quads of accumulators a lane take 0.95, 0.83 and
+// 0.72 of their prediction on such layers, and relay_margin says what of that relay_kernel's prediction may be at most.
+constexpr double kLeastTerms = 112;
+
+// The prediction errs by the kind of layer: of 4800 random layers of predictions between 0.8 and 1.15 of the walk's, those of 3x3 and stride 1
+// take 1.10 of relay_kernel's and 1.15 of the walk's, of 3x3 and stride 2 1.00 and 1.01, of 5x5 1.08 and 1.05, and where two thirds
+// of a workgroup's output channels are padding the walk is faster as often as not.  With these limits 927 of 1520 layers with zeros at random are
+// picked, 15 of them lose more than 3 %, 3 more than 10 %; with 0.9 for all 870, 32 and 8.  16 x 128 -> 256 52x52, 10 % of the weights: 87 us, 76.
+double relay_margin(const MatGeom& g) {
+  const int padded = 32 * kMatShapes[g.cfg].wm * g.mtiles;
+  if (3 * g.K < padded) return 0.85;
+  if (g.ks >= 5) return 0.87;
+  return g.stride == 1 && g.K >= 48 && 9 * padded <= 20 * g.K ? 0.97 : 0.9;
+}
+
 // Whether a matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and slice
 // count of least predicted time, if that is 7 % below the walking kernel's; half_kernel's, if that is 16 % below the walking
-// kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's; where neither is, relay_kernel's, if that is
-// 10 % below the walk's (below).  Of the 424 timed layers 125
+// kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's; where neither is, relay_kernel's (below).  Of the 424 timed layers 125
 // then go to matrix_kernel and 96 to half_kernel; over all of them that is 1.192 times the walk's speed, 3.0 % short of the
 // best choice.  10 layers lose more than 3 % to the walk, all on matrix_kernel and pointwise or of one image, two of them half
 // as much again (1 x 512 -> 1024 28x28 15.6 us, 10.6; 1 x 1024 -> 255 13x13 15.4, 10.5; with 10 % instead of 7 % two layers lose, 9 % at
 // most, and 1.191 times), and six to what matrix_kernel and the walk alone would give them.  (Without half_kernel 1.152 times.  With
 // 12 % to the walk 13 layers lose so, with 10 % and no advantage asked over matrix_kernel 27.)  Where the walking kernel can pool its
 // outputs, so must the matrix kernel.
-// relay_kernel: only where a sum of the walk, in a slice of the channels, has kLeastTerms weights on average, and its own at most twice as many:
-// there it is as exact.  Its error from 64 bits, in the outputs' 2-norm over the walk's, is 0.38 to 0.98 on 6414 random layers that
-// this rule picks (inputs after a ReLU), and 1.1 to 1.3 on layers with 57 terms.  Walks of one, two and four quads of accumulators a lane take 0.95, 0.83 and
-// 0.72 of their prediction on such layers.  Of 2614 random ones that it picks it is 1.49 times as fast as the walk (geometric mean) and loses
-// more than 3 % on 73, most of them of fewer than 32 output channels (padded to 64 in the narrowest tile).
-constexpr double kLeastTerms = 112;
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
                      double crowded, MatGeom* g, MatGeom* pool) {
   if (C < 16) return false;  // most of a chunk of 16 channels would be padding
   const bool pools = walk.OH >= 2 && walk.OW >= 2 && (walk.csplit > 1 || geom_pools_in_kernel(walk));
   struct Found { double t; int cfg, slices; };
-  std::vector<Found> found, relays;
   StagedPixels staged{};
   const double walking = walk_time(walk, nnz), terms = (double)nnz / K / walk.csplit;
-  for (int cfg = 0; cfg < kMatConfigs; ++cfg) {
-    MatGeom m;
-    const bool relay = kMatShapes[cfg].relay;
-    if (relay && (!found.empty() || terms < kLeastTerms)) break;
-    if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, 1, false, &m, &staged)) continue;
-    for (const int slices : {1, 2, 3, 4, 6, 8}) {
-      if (m.chunks / slices < (m.half ? kMatShapes[cfg].kw : 1) || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
-      set_slices(m, slices);
-      const double t = matrix_time(m, nnz, crowded);
-      if (relay) {
-        if (t < 0.9 * (walk.nq == 1 ? 0.95 : walk.nq == 2 ? 0.83 : 0.72) * walking && slices * 2 >= walk.csplit) relays.push_back({t, cfg, slices});
-      } else if (t < (m.half ? 0.84 : 0.93) * walking) {
-        found.push_back({m.half ? 1.05 * t : t, cfg, slices});
+  const double walked = (walk.nq == 1 ? 0.95 : walk.nq == 2 ? 0.83 : 0.72) * walking;
+  auto choose = [&](bool relay) {
+    std::vector<Found> found;
+    for (int cfg = 0; cfg < kMatConfigs; ++cfg) {
+      MatGeom m;
+      if (kMatShapes[cfg].relay != relay || !make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, 1, false, &m, &staged)) continue;
+      for (const int slices : {1, 2, 3, 4, 6, 8}) {
+        if (m.chunks / slices < (m.half ? kMatShapes[cfg].kw : 1) || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
+        set_slices(m, slices);
+        const double t = matrix_time(m, nnz, crowded);
+        if (relay ? t < relay_margin(m) * walked && slices * 2 >= walk.csplit : t < (m.half ? 0.84 : 0.93) * walking)
+          found.push_back({m.half && !relay ? 1.05 * t : t, cfg, slices});
       }
     }
-  }
-  if (found.empty()) found = relays;
-  std::stable_sort(found.begin(), found.end(), [](const Found& a, const Found& b) { return a.t < b.t; });
-  for (const Found& f : found) {
-    *pool = MatGeom{};
-    if (f.slices == 1 && walk.OH >= 2 && walk.OW >= 2 && !make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool)) {
+    std::stable_sort(found.begin(), found.end(), [](const Found& a, const Found& b) { return a.t < b.t; });
+    for (const Found& f : found) {
       *pool = MatGeom{};
-      if (pools) continue;
+      if (f.slices == 1 && walk.OH >= 2 && walk.OW >= 2 && !make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool)) {
+        *pool = MatGeom{};
+        if (pools) continue;
+      }
+      if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, f.slices, false, g, &staged)) return false;
+      if (!pool->N || pool->kgs == g->kgs) return true;
+      // (relay_kernel's chunks: both are to read the same weights)
+      const int groups = std::min(pool->kgs, g->kgs);
+      return make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, false, g, nullptr, groups) &&
+             make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool, nullptr, groups);
     }
-    if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, f.slices, false, g, &staged)) return false;
-    if (!pool->N || pool->kgs == g->kgs) return true;
-    // (relay_kernel's chunks: both are to read the same weights)
-    const int groups = std::min(pool->kgs, g->kgs);
-    return make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, false, g, nullptr, groups) &&
-           make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool, nullptr, groups);
-  }
-  return false;
+    return false;
+  };
+  // (relay_kernel too where the others cannot pool: 16 x 64 -> 128 104x104, 20 % of the weights, 162 us, 107)
+  return choose(false) || (terms >= kLeastTerms && choose(true));
 }
 
 int mat_lds_bytes(const MatGeom& g) { return lds_bytes(g); }
