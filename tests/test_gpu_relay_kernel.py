@@ -12,7 +12,7 @@ LDS = 2 * 60 * 1024 + 1848 + 8 * 4096  # what this kernel alone asks for
 # N, C, H, W, K, ks, stride, pad, density of the filter; workgroups along the pixels and the channels, slices
 LAYERS = [
     (11, 41, 8, 146, 3, 5, 2, 5, 0.15, (85, 1, 3)),        # three channels; quads of columns outside of the image; two strips, stored in quads
-    (6, 34, 33, 19, 34, 6, 2, 3, 0.15, (16, 1, 3)),        # 6 x 6, stride 2; ragged channels on both sides
+    (6, 34, 33, 19, 100, 6, 2, 3, 0.2, (16, 1, 3)),        # 6 x 6, stride 2; ragged channels on both sides
     (1, 49, 28, 122, 352, 4, 2, 1, 0.15, (14, 2, 4)),      # eight waves along the channels
     (5, 108, 8, 91, 483, 5, 2, 0, 0.15, (7, 2, 8)),        # ... images of two rows
     (1, 103, 28, 28, 152, 7, 1, 0, 0.1, (2, 3, 8)),        # 7 x 7; two workgroups for an image
@@ -25,6 +25,9 @@ LAYERS = [
     (5, 23, 61, 61, 112, 6, 1, 3, 0.15, (155, 1, 1)),      # ... two chunks
     (13, 25, 6, 124, 204, 6, 1, 3, 0.15, (182, 1, 1)),     # eight; two strips
     (7, 119, 100, 6, 70, 6, 1, 3, 0.15, (32, 1, 8)),       # images of six columns
+    (16, 96, 40, 40, 250, 3, 1, 1, 0.15, (256, 1, 1)),     # runs of 3 blocks, 64 pairs of which share one: tiles of 4, 3 for half of the waves
+    (5, 96, 75, 71, 470, 3, 1, 1, 0.15, (128, 2, 1)),      # ... of 6, all of them; two channel blocks
+    (16, 192, 46, 46, 250, 3, 1, 1, 0.07, (256, 1, 1)),    # ... of 4: the last tile has two blocks, of which half of the waves store one
 ]
 
 
@@ -91,7 +94,7 @@ LAYER, SPLIT = LAYERS[10], LAYERS[2]
 
 @pytest.mark.parametrize("what", ["2^40", "2^-60", "zero where it is looked at", "tiny beside ones", "2^120", "subnormal", "few out of range",
                                   "many out of range", "infinite"])
-@pytest.mark.parametrize("at", [LAYERS[5], LAYER, SPLIT, LAYERS[12]])  # (2, 4, 8 and 8 waves along the channels)
+@pytest.mark.parametrize("at", [LAYERS[5], LAYER, SPLIT, LAYERS[12], LAYERS[14]])  # (2, 4, 8, 8 and 8 waves along the channels)
 def test_inputs_of_any_scale(at, what):
     """Inputs are scaled by what some of them show; a few that fp16 parts then do not hold are added one by one, a tile with more of them is
     computed with bf16 parts, and sums that are not finite with FMAs."""

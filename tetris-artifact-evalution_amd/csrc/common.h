@@ -186,6 +186,7 @@ struct MatGeom {
   int mblocks, mtiles, ptiles, csplit, cfg;
   int runs;                  // relay_kernel: workgroups that share the pixels of a channel block; `ptiles` counts blocks of pixels
   int run_blocks, run_rest;  // blocks of a workgroup; how many have one more
+  int run_halves;            // instead, that many pairs of neighbours share one, each for half of the output channels
   int lpad;                  // staged pixels of a tile, to a multiple of 64 (relay_kernel: of 4)
   int lds_rows;              // bytes in front of the rows' exponents in LDS
   unsigned m_uw, m_uh, m_wp, m_ihs, m_strips;

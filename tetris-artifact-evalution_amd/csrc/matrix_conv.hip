@@ -436,6 +436,7 @@ void set_slices(MatGeom& g, int csplit) {
     tiles = g.runs = std::max({1, std::min(256 / (g.mtiles * csplit), g.ptiles / 2), ceil_div(g.ptiles, 180)});
     g.run_blocks = g.ptiles / g.runs;
     g.run_rest = g.ptiles % g.runs;
+    g.run_halves = kMatShapes[g.cfg].wn == 1 && 2 * g.run_rest <= g.runs;
   }
   g.d_tiles = divider(tiles * g.mtiles);
 }
@@ -604,7 +605,8 @@ double half_time(const MatGeom& g, long long nnz) {
 // random sizes, the zeros of 60 % of them in output channels of unequal density (with the density of the whole filter instead of
 // `crowded` 16 % too short on those).
 double relay_time(const MatGeom& g, long long nnz, double crowded) {
-  const int blocks = ceil_div(g.ptiles, g.runs), tiles = ceil_div(blocks, kMatShapes[g.cfg].nb), rounds = ceil_div(g.chunks, g.csplit);
+  const int most = ceil_div(g.ptiles, g.runs), tiles = ceil_div(most, kMatShapes[g.cfg].nb), rounds = ceil_div(g.chunks, g.csplit);
+  const double blocks = g.run_halves && g.run_rest ? most - 0.5 : most;  // of a SIMD's two waves
   const double density = std::min(1.0, (double)nnz / ((double)g.K * g.C * g.ks * g.ks));
   const double more = crowded < 0 ? density * density * density * (4 - 3 * density) : std::min(1.0, crowded);
   const double steps = 2 * ((double)ceil_div(g.C, 8) * g.ks * g.ks / g.chunks * (2 - std::pow(1 - more, 64)) / 8 + 0.5);  // of a chunk, in pairs
@@ -643,14 +645,13 @@ double walk_time(const Geom& g, long long nnz) {
 constexpr double kLeastTerms = 112;
 
 // The prediction errs by the kind of layer: of 4800 random layers of predictions between 0.8 and 1.15 of the walk's, those of 3x3 and stride 1
-// take 1.10 of relay_kernel's and 1.15 of the walk's, of 3x3 and stride 2 1.00 and 1.01, of 5x5 1.08 and 1.05, and where two thirds
-// of a workgroup's output channels are padding the walk is faster as often as not.  With these limits 927 of 1520 layers with zeros at random are
-// picked, 15 of them lose more than 3 %, 3 more than 10 %; with 0.9 for all 870, 32 and 8.  16 x 128 -> 256 52x52, 10 % of the weights: 87 us, 76.
+// take 1.10 of relay_kernel's and 1.15 of the walk's, the others 1.00 to 1.08 of both, and where two thirds of a workgroup's output channels
+// are padding the walk is faster as often as not.  With these limits 981 of 1520 layers with zeros at random are picked, 23 of them
+// lose more than 3 %; with 0.9 for all 870 and 32, with 0.87 for 5x5 927 and 15.  16 x 128 -> 256 52x52, 10 % of the weights: 87 us, 76.
 double relay_margin(const MatGeom& g) {
   const int padded = 32 * kMatShapes[g.cfg].wm * g.mtiles;
   if (3 * g.K < padded) return 0.85;
-  if (g.ks >= 5) return 0.87;
-  return g.stride == 1 && g.K >= 48 && 9 * padded <= 20 * g.K ? 0.97 : 0.9;
+  return g.ks < 5 && g.stride == 1 && g.K >= 48 && 9 * padded <= 20 * g.K ? 0.97 : 0.9;
 }
 
 // Whether a matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and slice

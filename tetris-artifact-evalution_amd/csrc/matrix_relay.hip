@@ -46,6 +46,7 @@ __device__ __forceinline__ void cut2(const float (&x)[8], float scale, u32x4& hi
 struct Work {
   int slice, mt, c_beg, rounds;  // rounds: chunks of the slice, from c_beg on
   int first, blocks, tiles;      // blocks of 32*WN pixels, cut into tiles of four and three, seldom two
+  int shared;                    // of the run's blocks the last is the next run's, too (1), or the first that of the run before (2): see own_of
 };
 struct Tile {
   int block, count;                 // first block of pixels and how many
@@ -65,8 +66,10 @@ __device__ __forceinline__ Work work_of(Arguments arguments) {
   w.mt = id - w.slice * all - run * g.mtiles;
   w.c_beg = w.slice * g.chunks / g.csplit;
   w.rounds = (w.slice + 1) * g.chunks / g.csplit - w.c_beg;
-  w.first = run * g.run_blocks + min(run, g.run_rest);
-  w.blocks = g.run_blocks + (run < g.run_rest);
+  const int rest = g.run_rest << g.run_halves;
+  w.first = run * g.run_blocks + (min(run, rest) >> g.run_halves);
+  w.blocks = g.run_blocks + (run < rest);
+  w.shared = g.run_halves && run < rest ? 1 + (run & 1) : 0;
   w.tiles = (w.blocks + kTile - 1) / kTile;
   return w;
 }
@@ -99,6 +102,20 @@ __device__ __forceinline__ Tile tile_of(Arguments arguments, const Work& w, int 
   const int last = ((q - t.q0) * g.ihs + ((y << dbl) + dbl) * g.stride - t.row0) * g.wp + ((x << dbl) + dbl) * g.stride - t.col0;
   t.staged = (last + (g.ks - 1) * (g.wp + 1) + 4) >> 2;
   return t;
+}
+
+// Which blocks of a tile a wave multiplies and which of them it stores.  Where runs are a block longer than others, a launch takes as long as
+// if all were.  So two neighbours share a block instead, each for half of the output channels: the first for those of its first four waves, the
+// second for those of the others.  (A SIMD has one wave of each half.)  Microseconds before and with it: 126 and 120 on 16 x 512 -> 512 28x28,
+// 10 % of the weights (128 runs of 3 blocks for each half of the channels, 8 of which had 4), 111 and 107 on 16 x 256 -> 256 48x48 (4.5 blocks), 134 and 132 on
+// 56x56 (6.125): power holds the others back while all CUs are busy.  Where more than half of the runs have one more there is nothing to share.
+struct Own { int first, count, stores; };  // stores: a bit each
+__device__ __forceinline__ Own own_of(const Work& w, const Tile& t, int k, int wave) {
+  const bool half = wave >= kWaves / 2;
+  const int lead = w.shared == 2 && !half && k == 0, trail = w.shared == 1 && half && k == w.tiles - 1;
+  const int stored = t.count - lead - trail;
+  if (stored < 2) return {0, t.count, ((1 << stored) - 1) << lead};
+  return {lead, stored, (1 << stored) - 1};
 }
 
 // The geometry's numbers that places are worked out with, read at once: each first touch of a line is a trip to L2.
@@ -532,7 +549,7 @@ __device__ __forceinline__ void multiply(Stage<WN>& stage, int k, unsigned some,
 
 // What is added to a tile's sums with FMAs: few tiles have any.  `sums`: room for a block of them, per wave.
 template <int WM, int WN>
-__device__ __forceinline__ void add_singles(Arguments arguments, const Work& work, const Places& at, const Shared& shared, const Tile& tile, int block, int slot,
+__device__ __forceinline__ void add_singles(Arguments arguments, const Work& work, const Places& at, const Shared& shared, const Tile& tile, const Own& own_blocks, int block, int slot,
                                             unsigned long long listed, const int (&bpos)[kTile], f32x16 (&sum)[2][kTile], float* sums, int wave, int lane) {
   asm volatile("" : "+v"(lane));  // (unknown to the compiler, which else would keep much of this in registers all the while)
   const auto& g = arguments->g;
@@ -546,10 +563,10 @@ __device__ __forceinline__ void add_singles(Arguments arguments, const Work& wor
   for (unsigned long long left = listed; left; left &= left - 1) before += __builtin_amdgcn_readlane(own.x, __builtin_ctzll(left)) < own.x;
 #pragma unroll
   for (int b = 0; b < kTile; ++b) {
-    if (b >= tile.count) break;
+    if (b >= own_blocks.count) break;
 #pragma unroll
     for (int i = 0; i < 16; ++i) sums[i * 64 + lane] = sum[0][b][i];
-    const Pixel p = pixel_of<WN>(at, work, tile, wn * tile.count + b, lane);
+    const Pixel p = pixel_of<WN>(at, work, tile, wn * tile.count + own_blocks.first + b, lane);
     // weights that fp16 parts do not hold
 #pragma nounroll
     for (int e = 0; e < loose; ++e) {
@@ -656,19 +673,20 @@ __device__ __forceinline__ unsigned long long multiply_all(Arguments arguments, 
       continue;
     }
     const Tile tile = tile_of<WN>(arguments, work, k);
+    const Own own = own_of(work, tile, k, wave);
     int bpos[kTile];
     f32x16 sum[2][kTile];
 #pragma unroll
     for (int b = 0; b < kTile; ++b) {
-      bpos[b] = lds_of(at, tile, pixel_of<WN>(at, work, tile, wn * tile.count + min(b, tile.count - 1), lane));
+      bpos[b] = lds_of(at, tile, pixel_of<WN>(at, work, tile, wn * tile.count + own.first + min(b, own.count - 1), lane));
 #pragma unroll
       for (int i = 0; i < 16; ++i) sum[0][b][i] = sum[1][b][i] = 0.f;
     }
     if constexpr (kTile == 4) {
-      if (tile.count == 4) multiply<4>(stage, k, some, first, lds, weights, ahead, base, bpos, sum, buf);
+      if (own.count == 4) multiply<4>(stage, k, some, first, lds, weights, ahead, base, bpos, sum, buf);
     }
-    if (tile.count == 2) multiply<2>(stage, k, some, first, lds, weights, ahead, base, bpos, sum, buf);
-    else if (tile.count == 3) multiply<3>(stage, k, some, first, lds, weights, ahead, base, bpos, sum, buf);
+    if (own.count == 2) multiply<2>(stage, k, some, first, lds, weights, ahead, base, bpos, sum, buf);
+    else if (own.count == 3) multiply<3>(stage, k, some, first, lds, weights, ahead, base, bpos, sum, buf);
     first_weights();
     if (too_many(shared, slot, lane)) {
       again |= 1ull << k;
@@ -681,7 +699,7 @@ __device__ __forceinline__ unsigned long long multiply_all(Arguments arguments, 
     const unsigned listed = shared.asides[16 * slot + lane / kMostAside];  // by the wave whose list this lane may read
     const unsigned long long some_listed = __builtin_amdgcn_ballot_w64(lane % kMostAside < listed);
     if (some_listed || w.loose_count[block])
-      add_singles<WM, WN>(arguments, work, at, shared, tile, block, slot, some_listed, bpos, sum, sums, wave, lane);
+      add_singles<WM, WN>(arguments, work, at, shared, tile, own, block, slot, some_listed, bpos, sum, sums, wave, lane);
     const Stores stores = stores_of(arguments, work, oc0);
     const int shift = shared.shift[slot];
     int4 e[4];
@@ -691,8 +709,8 @@ __device__ __forceinline__ unsigned long long multiply_all(Arguments arguments, 
     asm volatile("" : "+v"(unknown));
 #pragma unroll
     for (int b = 0; b < kTile; ++b) {
-      if (b >= tile.count) break;
-      const int out = out_of(arguments, pixel_of<WN>(at, work, tile, wn * tile.count + b, unknown), unknown);
+      if (!(own.stores >> b & 1)) continue;
+      const int out = out_of(arguments, pixel_of<WN>(at, work, tile, wn * tile.count + own.first + b, unknown), unknown);
 #pragma unroll
       for (int i = 0; i < 16; i += 4) {
         float v[4];
@@ -718,12 +736,13 @@ __device__ __forceinline__ void compute_again(Arguments arguments, const Work& w
   const __amdgpu_buffer_rsrc_t irsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(arguments->in), 0, g.in_bytes, 0x00020000);
   const int hw4 = 4 * g.H * g.W, plane = at.kgs * at.lpad;
   const int wave = wave_id, wm = wave % WM, wn = wave / WM, block = min(work.mt * WM + wm, g.mblocks - 1), oc0 = (work.mt * WM + wm) * 32;
+  const Own own = own_of(work, tile, k, wave);
   f32x16 sum[2][NB];
   int bpos[NB], out[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const bool exists = b < tile.count;
-    const Pixel p = pixel_of<WN>(at, work, tile, wn * tile.count + min(b, tile.count - 1), lane);
+    const bool exists = own.stores >> b & 1;
+    const Pixel p = pixel_of<WN>(at, work, tile, wn * tile.count + own.first + min(b, own.count - 1), lane);
     bpos[b] = lds_of(at, tile, p);
     out[b] = exists ? out_of(arguments, p, lane) : kOutside;
 #pragma unroll
@@ -813,8 +832,9 @@ __device__ __forceinline__ void compute_again(Arguments arguments, const Work& w
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): what follows stores over what was stored, by other lanes
   const int ch0 = work.c_beg * 8 * g.kgs, ch1 = min(g.C, (work.c_beg + work.rounds) * 8 * g.kgs), cpad = 8 * g.kgs * g.chunks;
 #pragma nounroll
-  for (int b = 0; b < tile.count; ++b) {
-    const Pixel p = pixel_of<WN>(at, work, tile, wn * tile.count + b, lane);
+  for (int b = 0; b < own.count; ++b) {
+    if (!(own.stores >> b & 1)) continue;
+    const Pixel p = pixel_of<WN>(at, work, tile, wn * tile.count + own.first + b, lane);
     float sums[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) sums[i] = 0;
