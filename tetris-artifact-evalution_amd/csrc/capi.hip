@@ -54,14 +54,14 @@ bool choose_matrix(const tetris_g950* p, int N, int H, int W, int stride, int pa
   if (tile && (tile->lanes_w != own.lanes_w || tile->quads != own.quads || tile->oc_per_wave != own.oc_per_wave ||
                tile->waves != own.waves || tile->tile_ic != own.tile_ic || tile->csplit != own.csplit))
     return false;
-  return choose_mat_geom(N, p->C, H, W, p->K, p->ks, stride, pad, walk, p->nnz, p->crowded, g, pool);
+  return choose_mat_geom(N, p->C, H, W, p->K, p->ks, stride, pad, walk, p->nnz, g, pool);
 }
 
 // The weights of pack `p` as the matrix kernel loads them, made on first use; null where the device has no room for them (up to 14.5
 // bytes a weight, zeros included): the walk, which needs 8 a non-zero, runs the layer then.
 int matrix_weights(tetris_g950* p, const MatGeom& g, hipStream_t stream, const MatWeights** out) {
   std::lock_guard<std::mutex> lock(p->mu);
-  const int key = g.kgs | g.half << 8 | g.parts << 9;
+  const int key = g.kgs | g.half << 8;
   auto it = p->parts.find(key);
   if (it == p->parts.end()) {
     void* d = nullptr;
@@ -970,8 +970,7 @@ int tetris_launch_shape_of(tetris_g950* p, int N, int H, int W, int stride, int 
   const Geom& g = c.geom;
   const MatGeom& m = c.mat;
   if (c.matrix) {
-    const int tiles = m.runs ? m.runs : m.ptiles;
-    *out = {tiles * m.mtiles * m.csplit, tiles, m.mtiles, m.csplit, m.chunks, 64, 5, mat_lds_bytes(m),
+    *out = {m.ptiles * m.mtiles * m.csplit, m.ptiles, m.mtiles, m.csplit, m.chunks, 64, 5, mat_lds_bytes(m),
             (int64_t)partial_bytes_of(m)};
     return TETRIS_OK;
   }

@@ -181,18 +181,14 @@ struct MatGeom {
   int strips, ws, wp, ihs;   // strips per image; output columns of one; staged columns and rows of one
   int uw, uh, upq, npix;     // columns, rows and pixels of a strip's outputs (2x2 blocks when pooling); all outputs
   int kgs, chunks;           // groups of 8 channels staged together; such chunks
-  int half, parts;           // fp16 parts, and how many a number has: half_kernel and relay_kernel
-  int steps, smax;           // matrix_kernel: products of 16 k-values; half_kernel, relay_kernel: most steps of a chunk
+  int half, steps, smax;     // which matrix kernel; matrix_kernel: products of 16 k-values; half_kernel: most steps of a chunk
   int mblocks, mtiles, ptiles, csplit, cfg;
-  int runs;                  // relay_kernel: workgroups that share the pixels of a channel block; `ptiles` counts blocks of pixels
-  int run_blocks, run_rest;  // blocks of a workgroup; how many have one more
-  int run_halves;            // instead, that many pairs of neighbours share one, each for half of the output channels
-  int lpad;                  // staged pixels of a tile, to a multiple of 64 (relay_kernel: of 4)
+  int lpad;                  // staged pixels of a tile, to a multiple of 64
   int lds_rows;              // bytes in front of the rows' exponents in LDS
   unsigned m_uw, m_uh, m_wp, m_ihs, m_strips;
   MatDiv d_tiles, d_mtiles, d_upq, d_uw, d_blocks;
 };
-// A filter's weights as a matrix kernel loads them (device memory).  matrix_kernel: `base` only.  half_kernel, relay_kernel: per 32 output
+// A filter's weights as a matrix kernel loads them (device memory).  matrix_kernel: `base` only.  half_kernel: per 32 output
 // channels and chunk of input channels up to MatGeom::smax steps, each a 32 x 32 matrix of which two in four consecutive values of a row are kept.
 struct MatWeights {
   void* base;           // the allocation that holds them all
@@ -205,7 +201,7 @@ struct MatWeights {
   const float* dense;   // [output channel][tap][input channel, to a multiple of the chunk]
   int step_bytes;       // of all steps
 };
-constexpr int kMatConfigs = 26;
+constexpr int kMatConfigs = 23;
 constexpr int kMatTasks = 4;        // most blocks of 64 staged pixels x 8 channels that a wave holds at a time
 constexpr int kMatLds = 160 * 1024;
 constexpr long long kMatCopies = 32 << 20;  // most bytes of partial sums of a split layer
@@ -240,7 +236,6 @@ struct tetris_g950 {
   int slots = 0;            // K rounded up to a multiple of kSlotPad
   int groups = 0;           // slots / g
   int64_t n_entries = 0, nnz = 0;
-  double crowded = 0;       // share of groups of four consecutive input channels, of an output channel and a tap, with more than two weights, estimated
   bool huge = false;        // a weight of 2^64 or more, or not finite: the matrix kernel does not take it
   // two allocations: grp_off, grp_nnz and oc_order; position and values
   int32_t* d_grp_off = nullptr;   // [groups*stages+1] entry index, multiples of 8; then the number of non-zeros
@@ -250,7 +245,7 @@ struct tetris_g950 {
   float* d_values = nullptr;      // [n_entries + 8]
   // (LDS byte offset | accumulator index << 16 | 0xC << 28, value) pairs for one tile geometry, made on first use
   std::map<tetris::BoundKey, int2*> bound;
-  std::map<int, tetris::MatWeights> parts;  // the weights as the matrix kernel loads them, by MatGeom::kgs and, above it, ::half and ::parts
+  std::map<int, tetris::MatWeights> parts;  // the weights as the matrix kernel loads them, by MatGeom::kgs and, above it, ::half
   // Paired arrangement of the streams (made on the first paired bind; depends on the pack only): two consecutive
   // entries of a stream that share their position become a pair; per stream first all pairs, padded to a multiple
   // of 8 entries, then the entries left single, padded likewise.
@@ -347,14 +342,13 @@ int add_copies(const float* d_copies, float* d_out, int N, int K, int OH, int OW
 
 // matrix_conv.hip
 // staged (may be null): of the same layer, what earlier calls found (zeros: nothing yet)
-using StagedPixels = std::array<int, 17>;  // of the largest tile of 32, 64, ... pixels
-// most_groups: of 8 channels that relay_kernel stages together
+using StagedPixels = std::array<int, 9>;  // of the largest tile of 32, 64, ... pixels
 bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out,
-                   StagedPixels* staged = nullptr, int most_groups = 8);
+                   StagedPixels* staged = nullptr);
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
-                     double crowded, MatGeom* g, MatGeom* pool);
-// predicted microseconds of a launch; crowded: see tetris_g950 (below zero: of weights that are zero at random)
-double matrix_time(const MatGeom& g, long long nnz, double crowded = -1);
+                     MatGeom* g, MatGeom* pool);
+// predicted microseconds of a launch
+double matrix_time(const MatGeom& g, long long nnz);
 double walk_time(const Geom& g, long long nnz);
 int mat_lds_bytes(const MatGeom& g);
 size_t mat_weight_bytes(const MatGeom& g);

@@ -1,4 +1,4 @@
-// What the three matrix kernels (matrix_conv.hip, matrix_half.hip, matrix_relay.hip) share.
+// What the two matrix kernels (matrix_conv.hip, matrix_half.hip) share.
 #pragma once
 #include "common.h"
 
@@ -6,34 +6,29 @@ namespace tetris {
 
 // A workgroup of a configuration: waves along the channels and along the pixels of a team, pixel blocks of a wave, teams;
 // whether half_kernel runs it, and with short chunks of channels.  (half_kernel's: those that are left if of 22 and four more the
-// ones are dropped one after the other that the 424 layers of profiles/kernel_times.txt lose least without, 0.01 % in all.)  relay: run by
-// relay_kernel, eight waves and the largest tile of up to four blocks a wave.
+// ones are dropped one after the other that the 424 layers of profiles/kernel_times.txt lose least without, 0.01 % in all.)
 struct MatShape {
   int wm, wn, nb, kw;
-  bool half, brief, relay;
+  bool half, brief;
 };
 constexpr MatShape kMatShapes[] = {
     {4, 1, 4, 1}, {4, 1, 4, 2}, {4, 1, 2, 1}, {4, 1, 2, 2}, {4, 1, 2, 4}, {2, 2, 2, 1}, {2, 2, 2, 2}, {2, 2, 2, 4}, {2, 2, 1, 1}, {2, 2, 1, 2}, {2, 2, 1, 4},
     {8, 1, 2, 1, true}, {8, 1, 3, 1, true}, {4, 1, 2, 2, true}, {2, 2, 1, 2, true},
     {8, 1, 2, 1, true, true}, {8, 1, 3, 1, true, true}, {8, 1, 4, 1, true, true}, {4, 2, 3, 1, true, true}, {4, 2, 4, 1, true, true},
-    {4, 1, 2, 2, true, true}, {2, 2, 1, 1, true, true}, {2, 2, 1, 2, true, true},
-    {8, 1, 4, 1, true, false, true}, {4, 2, 4, 1, true, false, true}, {2, 4, 4, 1, true, false, true}};
+    {4, 1, 2, 2, true, true}, {2, 2, 1, 1, true, true}, {2, 2, 1, 2, true, true}};
 static_assert(sizeof kMatShapes / sizeof *kMatShapes == kMatConfigs);
 
-// whether four consecutive pixels of a tile, the first a multiple of four, lie side by side in memory, in one image and on 16 bytes
+// whether four consecutive pixels of a tile lie side by side in memory, in one image and on 16 bytes
 inline bool stores_quads(const MatGeom& g, const float* d_out) {
-  return !g.pool && (g.strips == 1 ? g.OH * g.OW % 4 == 0 : g.ws % 4 == 0 && g.OW % 4 == 0) && reinterpret_cast<uintptr_t>(d_out) % 16 == 0;
+  return !g.pool && g.strips == 1 && g.OH * g.OW % 4 == 0 && reinterpret_cast<uintptr_t>(d_out) % 16 == 0;
 }
 
 // matrix_half.hip
 constexpr int kMostChannels = 1 << 20;  // input channels of a layer: a loose weight's place is an int, 20 bits of which name its channel
-constexpr int kRelayPart = 60 * 1024;  // of LDS: a part of the inputs that relay_kernel stages
-constexpr int kRelayBytes = 4 * 4 + 3 * 8 * 4 + 48 * 4 + 2 * 4 + 3 * 64 * 8;  // ... behind those
 constexpr int kAsideBytes = 64 + 64 * 8;  // of LDS: inputs that are multiplied one by one
-constexpr int kStepBytes = 3 * 1024 + 256, kStepBytes2 = 2 * 1024 + 256, kSlotBytes = 2048;  // of a step's weights: three or two fp16 parts and a word per lane; fp32
+constexpr int kStepBytes = 3 * 1024 + 256, kSlotBytes = 2048;  // of a step's weights: fp16 parts and a word per lane; fp32
 size_t half_weight_bytes(const MatGeom& g);
 int half_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void* base, MatWeights* out);  // waits for them
-int launch_relay(const MatGeom& g, const float* d_in, float* d_out, const MatWeights& weights, int relu, hipStream_t stream);  // matrix_relay.hip
 int launch_half(const MatGeom& g, const float* d_in, float* d_out, const MatWeights& weights, int relu, hipStream_t stream);
 
 namespace {

@@ -377,13 +377,9 @@ __global__ __launch_bounds__(256) void parts_kernel(const int32_t* __restrict__ 
 // input buffers, or what the teams' sums need
 int lds_main(const MatGeom& g) {
   const MatShape& c = kMatShapes[g.cfg];
-  if (c.relay) return 2 * kRelayPart;
   return std::max(c.kw * 96 * g.kgs * g.lpad, c.kw > 1 ? c.kw * c.wm * c.wn * 4096 * c.nb : 0);
 }
-int lds_bytes(const MatGeom& g) {
-  const MatShape& c = kMatShapes[g.cfg];
-  return lds_main(g) + (c.relay ? kRelayBytes + 8 * 4096 : g.half ? 128 * c.wm + kAsideBytes : 0);
-}
+int lds_bytes(const MatGeom& g) { return lds_main(g) + (g.half ? 128 * kMatShapes[g.cfg].wm + kAsideBytes : 0); }
 
 template <int WM, int NB, int KW, int TM>
 int launch_one(const MatGeom& g, const float* d_in, float* d_out, const void* weights, hipStream_t stream) {
@@ -409,43 +405,26 @@ MatDiv divider(int d) {
   return r;
 }
 
-// channel groups of `lpad` staged pixels that relay_kernel has room for twice
-int relay_groups(int lpad) { return std::min(kRelayPart / (2 * 16), 2048) / lpad; }
-
-// staged pixels the largest tile of `P` pixels needs, where tiles begin at multiples of `apart`
-int staged_pixels(const MatGeom& g, int P, int apart) {
+// staged pixels the largest tile of `P` pixels needs
+int staged_pixels(const MatGeom& g, int P) {
   const int psh = g.pool ? 2 : 0, dbl = g.pool ? 1 : 0;
   auto at = [&](int u, int d) {
     const int q = u / g.upq, r = u - q * g.upq, y = r / g.uw, x = r - y * g.uw;
     return ((long long)q * g.ihs + (long long)((y << dbl) + d) * g.stride) * g.wp + (long long)((x << dbl) + d) * g.stride;
   };
   // (the tiles' starts repeat, relative to their strip, after upq / gcd tiles at the latest)
-  const int per = P >> psh, step = apart >> psh, tiles = std::min(ceil_div(g.npix, apart), g.upq / std::gcd(step, g.upq));
+  const int per = P >> psh, tiles = std::min(ceil_div(g.npix, P), g.upq / std::gcd(per, g.upq));
   long long most = 0;
   for (int t = 0; t < tiles; ++t)
-    most = std::max(most, at(t * step + per - 1, dbl) - at(t * step, 0) + (long long)(g.ks - 1) * (g.wp + 1) + 1);
+    most = std::max(most, at(t * per + per - 1, dbl) - at(t * per, 0) + (long long)(g.ks - 1) * (g.wp + 1) + 1);
   return (int)std::min<long long>(most, 1 << 28);
-}
-
-// `csplit` slices of the channels, and which workgroup does what
-void set_slices(MatGeom& g, int csplit) {
-  g.csplit = csplit;
-  int tiles = g.ptiles;
-  if (kMatShapes[g.cfg].relay) {
-    // a workgroup per CU, with 2 to 180 blocks of pixels each: the tiles that are computed again are bits of 64
-    tiles = g.runs = std::max({1, std::min(256 / (g.mtiles * csplit), g.ptiles / 2), ceil_div(g.ptiles, 180)});
-    g.run_blocks = g.ptiles / g.runs;
-    g.run_rest = g.ptiles % g.runs;
-    g.run_halves = kMatShapes[g.cfg].wn == 1 && 2 * g.run_rest <= g.runs;
-  }
-  g.d_tiles = divider(tiles * g.mtiles);
 }
 
 }  // namespace
 
 // Cuts a layer into workgroups of configuration `cfg` with `csplit` slices of the channels; false: it cannot be run so.
 bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, int cfg, int csplit, bool pool, MatGeom* out,
-                   StagedPixels* staged, int most_groups) {
+                   StagedPixels* staged) {
   MatGeom g{};
   if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || K <= 0 || cfg < 0 || cfg >= kMatConfigs || csplit < 1 || csplit > kMaxSplit) return false;
   g.N = N; g.C = C; g.H = H; g.W = W; g.K = K; g.ks = ks; g.pad = pad;
@@ -461,44 +440,15 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
   g.out_floats = pool ? N * K * (g.OH / 2) * (g.OW / 2) : N * K * g.OH * g.OW;
   // Images wider than 64 are cut into strips, which are images to everything below: a tile's pixels are consecutive in a
   // strip, row by row, and the rows above and below that it stages as well are a strip wide.
-  auto cut_strips = [&](int strips) {
-    g.strips = strips;
-    g.ws = ceil_div(g.OW, g.strips);
-    if (g.strips > 1 || pool) g.ws += g.ws & 1;
-    if (pool && g.strips == 1) g.ws = g.OW & ~1;
-    g.wp = (g.ws - 1) * g.stride + ks;
-    if (kMatShapes[cfg].relay) g.wp = ceil_div(g.wp, 4) * 4;  // rows of whole quads
-    g.ihs = (g.OH - 1) * g.stride + ks;
-    g.uw = pool ? g.ws / 2 : g.ws;
-    g.uh = pool ? g.OH / 2 : g.OH;
-    g.upq = g.uw * g.uh;
-  };
-  const MatShape c = kMatShapes[cfg];
-  const int P = 32 * c.nb * c.wn;
-  cut_strips(ceil_div(g.OW, 64));
-  if (c.relay) {
-    // Strips as narrow as eight columns: of a tile's rows the more are read, but its edges take room and time too.  Compared by the cycles
-    // that a tile takes to multiply a group of channels (66 to a block and step; or its reads: 16 pixels side by side at a time, more
-    // where rows end) and to stage it.  A pointwise layer has no halo, nor enough products for a staged input.
-    if (ks == 1) return false;
-    int best = 0;
-    double least = 0;
-    for (int strips = g.strips, last = 0; strips <= std::max(g.strips, ceil_div(g.OW, 8)); ++strips) {
-      cut_strips(strips);
-      if (g.ws == last) continue;
-      last = g.ws;
-      const int rows = P % g.ws ? (P + g.ws - 2) / g.ws + 1 : P / g.ws;
-      const int lpad = ((rows - 1) * g.stride + ks + (g.OH % rows ? ks - 1 : 0)) * g.wp;
-      const int kgs = std::min(relay_groups(lpad), 8);
-      if (kgs < 1) continue;
-      const double reads = 64 * (g.ws % 16 ? g.ws < 16 ? 2 : 1 + 15.0 / g.ws : 1);
-      const double multiply = ks * ks * 0.33 * c.nb * std::max(99.0, reads * g.stride), stage = 1.5 * lpad;
-      const double t = (double)strips * g.ws / g.OW * (std::max(multiply, stage) + 0.2 * std::min(multiply, stage) + 600 / kgs);
-      if (!best || t < least) { best = strips; least = t; }
-    }
-    if (!best) return false;
-    cut_strips(best);
-  }
+  g.strips = ceil_div(g.OW, 64);
+  g.ws = ceil_div(g.OW, g.strips);
+  if (g.strips > 1 || pool) g.ws += g.ws & 1;
+  if (pool && g.strips == 1) g.ws = g.OW & ~1;
+  g.wp = (g.ws - 1) * g.stride + ks;
+  g.ihs = (g.OH - 1) * g.stride + ks;
+  g.uw = pool ? g.ws / 2 : g.ws;
+  g.uh = pool ? g.OH / 2 : g.OH;
+  g.upq = g.uw * g.uh;
   if ((long long)N * g.strips * g.upq * (pool ? 4 : 1) >= (1ll << 30)) return false;
   g.npix = N * g.strips * g.upq * (pool ? 4 : 1);
   g.half = kMatShapes[cfg].half;
@@ -513,28 +463,23 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
       g.kgs /= 2;
     }
   }
-  g.cfg = cfg;
-  g.parts = c.relay ? 2 : g.half ? 3 : 0;
-  g.ptiles = ceil_div(g.npix, c.relay ? 32 * c.wn : P);
-  StagedPixels one{};
-  int& most = (staged && !c.relay ? *staged : one)[P / 32];
-  if (!most) most = staged_pixels(g, P, c.relay ? 32 * c.wn : P);
-  g.lpad = c.relay ? ceil_div(most + 3, 4) * 4 : ceil_div(most, 64) * 64;  // (the first quad may begin three pixels before)
-  if (c.relay) {
-    // as many groups at a time as LDS holds twice, of equal chunks
-    const int groups = ceil_div(C, 8);
-    g.kgs = std::min({ks > 4 ? 2 : 8, relay_groups(g.lpad), most_groups});
-    if (g.kgs < 1 || g.lpad > 1024) return false;
-    g.kgs = ceil_div(groups, ceil_div(groups, g.kgs));
-  }
   g.chunks = ceil_div(C, 8 * g.kgs);
   if (csplit > g.chunks) return false;
+  g.csplit = csplit;
   g.steps = g.chunks * ks * ks * (g.kgs / 2);
   g.mblocks = ceil_div(K, 32);
-  g.smax = ceil_div(2 * g.kgs * ks * ks, c.relay ? 8 : 4) * (c.relay ? 2 : 1);
+  const MatShape c = kMatShapes[cfg];
+  g.cfg = cfg;
+  g.smax = ceil_div(2 * g.kgs * ks * ks, 4);
   if (g.half && (g.chunks / csplit < c.kw || ((long long)g.mblocks * g.chunks * g.smax + 3) * kStepBytes >= (1ll << 31))) return false;
+  const int P = 32 * c.nb * c.wn;
+  g.ptiles = ceil_div(g.npix, P);
   g.mtiles = ceil_div(g.mblocks, c.wm);
-  if ((!c.relay && g.kgs * g.lpad / 64 > c.wm * c.wn * (g.half && c.nb == 4 ? 2 : kMatTasks)) || lds_bytes(g) > kMatLds) return false;
+  StagedPixels one{};
+  int& most = (staged ? *staged : one)[P / 32];
+  if (!most) most = staged_pixels(g, P);
+  g.lpad = ceil_div(most, 64) * 64;
+  if (g.kgs * g.lpad / 64 > c.wm * c.wn * (g.half && c.nb == 4 ? 2 : kMatTasks) || lds_bytes(g) > kMatLds) return false;
   g.lds_rows = lds_main(g);
   if ((long long)g.ptiles * g.mtiles * csplit >= (1ll << 28)) return false;
   // multiply-high divisions: dividend * divisor below 2^32
@@ -545,9 +490,8 @@ bool make_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pa
     return false;
   g.m_uw = magic_reciprocal(g.uw); g.m_uh = magic_reciprocal(g.uh); g.m_wp = magic_reciprocal(g.wp);
   g.m_ihs = magic_reciprocal(g.ihs); g.m_strips = magic_reciprocal(g.strips);
-  g.d_mtiles = divider(g.mtiles); g.d_upq = divider(g.upq);
-  g.d_uw = divider(g.uw); g.d_blocks = divider(std::max(g.lpad / 64, 1));
-  set_slices(g, csplit);
+  g.d_tiles = divider(g.ptiles * g.mtiles); g.d_mtiles = divider(g.mtiles); g.d_upq = divider(g.upq);
+  g.d_uw = divider(g.uw); g.d_blocks = divider(g.lpad / 64);
   *out = g;
   return true;
 }
@@ -601,24 +545,7 @@ double half_time(const MatGeom& g, long long nnz) {
   return 1.67 + (full * cycles(fit) + cycles(ceil_div(rest, 256))) / 2.3e3 + (g.csplit > 1 ? 2.48 + out * (g.csplit + 1) / 4.3e6 : 0);
 }
 
-// The same for relay_kernel, whose workgroups are one to a CU and take one tile after the other: 7 % off on 14 990 launches of 6301 layers of
-// random sizes, the zeros of 60 % of them in output channels of unequal density (with the density of the whole filter instead of
-// `crowded` 16 % too short on those).
-double relay_time(const MatGeom& g, long long nnz, double crowded) {
-  const int most = ceil_div(g.ptiles, g.runs), tiles = ceil_div(most, kMatShapes[g.cfg].nb), rounds = ceil_div(g.chunks, g.csplit);
-  const double blocks = g.run_halves && g.run_rest ? most - 0.5 : most;  // of a SIMD's two waves
-  const double density = std::min(1.0, (double)nnz / ((double)g.K * g.C * g.ks * g.ks));
-  const double more = crowded < 0 ? density * density * density * (4 - 3 * density) : std::min(1.0, crowded);
-  const double steps = 2 * ((double)ceil_div(g.C, 8) * g.ks * g.ks / g.chunks * (2 - std::pow(1 - more, 64)) / 8 + 0.5);  // of a chunk, in pairs
-  const double cycles = 2937 + tiles * (12313 + 1311.0 * rounds) + rounds * steps * ((g.stride == 2 ? 228.4 : 205.0) * blocks + 271.6 * tiles);
-  const double out = 4.0 * g.N * g.K * g.OH * g.OW, in = 4.0 * g.N * g.C * g.H * g.W;
-  return 2 + ceil_div(g.runs * g.mtiles * g.csplit, 256) * cycles / 2.1e3 + (in * g.mtiles + out * g.csplit) / 5.9e6 +
-         (g.csplit > 1 ? 2.5 + out * (g.csplit + 1) / 4.3e6 : 0);
-}
-
-double matrix_time(const MatGeom& g, long long nnz, double crowded) {
-  return kMatShapes[g.cfg].relay ? relay_time(g, nnz, crowded) : g.half ? half_time(g, nnz) : plain_time(g);
-}
+double matrix_time(const MatGeom& g, long long nnz) { return g.half ? half_time(g, nnz) : plain_time(g); }
 
 // The same for the kernels that walk the non-zeros: 15 % off.
 double walk_time(const Geom& g, long long nnz) {
@@ -638,25 +565,9 @@ double walk_time(const Geom& g, long long nnz) {
   return std::max(compute, (in + out) / 6.9e6) + (g.csplit > 1 ? 1.5 + out * (g.csplit + 1) / 4.1e6 : 0);
 }
 
-// relay_kernel: only where a sum of the walk, in a slice of the channels, has kLeastTerms weights on average, and its own at most twice as many:
-// there it is as exact.  Its error from 64 bits, in the outputs' 2-norm over the walk's, is 0.38 to 0.98 on 6414 random layers that
-// this rule picks (inputs after a ReLU), and 1.1 to 1.3 on layers with 57 terms.  Walks of one, two and four quads of accumulators a lane take 0.95, 0.83 and
-// 0.72 of their prediction on such layers, and relay_margin says what of that relay_kernel's prediction may be at most.
-constexpr double kLeastTerms = 112;
-
-// The prediction errs by the kind of layer: of 4800 random layers of predictions between 0.8 and 1.15 of the walk's, those of 3x3 and stride 1
-// take 1.10 of relay_kernel's and 1.15 of the walk's, the others 1.00 to 1.08 of both, and where two thirds of a workgroup's output channels
-// are padding the walk is faster as often as not.  With these limits 981 of 1520 layers with zeros at random are picked, 23 of them
-// lose more than 3 %; with 0.9 for all 870 and 32, with 0.87 for 5x5 927 and 15.  16 x 128 -> 256 52x52, 10 % of the weights: 87 us, 76.
-double relay_margin(const MatGeom& g) {
-  const int padded = 32 * kMatShapes[g.cfg].wm * g.mtiles;
-  if (3 * g.K < padded) return 0.85;
-  return g.ks < 5 && g.stride == 1 && g.K >= 48 && 9 * padded <= 20 * g.K ? 0.97 : 0.9;
-}
-
 // Whether a matrix kernel is worth running in place of the walking kernel of geometry `walk`, and how: the configuration and slice
 // count of least predicted time, if that is 7 % below the walking kernel's; half_kernel's, if that is 16 % below the walking
-// kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's; where neither is, relay_kernel's (below).  Of the 424 timed layers 125
+// kernel's -- predictions for large walks are 8 % too long -- and 5 % below matrix_kernel's.  Of the 424 timed layers 125
 // then go to matrix_kernel and 96 to half_kernel; over all of them that is 1.192 times the walk's speed, 3.0 % short of the
 // best choice.  10 layers lose more than 3 % to the walk, all on matrix_kernel and pointwise or of one image, two of them half
 // as much again (1 x 512 -> 1024 28x28 15.6 us, 10.6; 1 x 1024 -> 255 13x13 15.4, 10.5; with 10 % instead of 7 % two layers lose, 9 % at
@@ -664,44 +575,33 @@ double relay_margin(const MatGeom& g) {
 // 12 % to the walk 13 layers lose so, with 10 % and no advantage asked over matrix_kernel 27.)  Where the walking kernel can pool its
 // outputs, so must the matrix kernel.
 bool choose_mat_geom(int N, int C, int H, int W, int K, int ks, int stride, int pad, const Geom& walk, long long nnz,
-                     double crowded, MatGeom* g, MatGeom* pool) {
+                     MatGeom* g, MatGeom* pool) {
   if (C < 16) return false;  // most of a chunk of 16 channels would be padding
   const bool pools = walk.OH >= 2 && walk.OW >= 2 && (walk.csplit > 1 || geom_pools_in_kernel(walk));
   struct Found { double t; int cfg, slices; };
+  std::vector<Found> found;
   StagedPixels staged{};
-  const double walking = walk_time(walk, nnz), terms = (double)nnz / K / walk.csplit;
-  const double walked = (walk.nq == 1 ? 0.95 : walk.nq == 2 ? 0.83 : 0.72) * walking;
-  auto choose = [&](bool relay) {
-    std::vector<Found> found;
-    for (int cfg = 0; cfg < kMatConfigs; ++cfg) {
-      MatGeom m;
-      if (kMatShapes[cfg].relay != relay || !make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, 1, false, &m, &staged)) continue;
-      for (const int slices : {1, 2, 3, 4, 6, 8}) {
-        if (m.chunks / slices < (m.half ? kMatShapes[cfg].kw : 1) || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
-        set_slices(m, slices);
-        const double t = matrix_time(m, nnz, crowded);
-        if (relay ? t < relay_margin(m) * walked && slices * 2 >= walk.csplit : t < (m.half ? 0.84 : 0.93) * walking)
-          found.push_back({m.half && !relay ? 1.05 * t : t, cfg, slices});
-      }
+  const double walking = walk_time(walk, nnz);
+  for (int cfg = 0; cfg < kMatConfigs; ++cfg) {
+    MatGeom m;
+    if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, cfg, 1, false, &m, &staged)) continue;
+    for (const int slices : {1, 2, 3, 4, 6, 8}) {
+      if (m.chunks / slices < (m.half ? kMatShapes[cfg].kw : 1) || (slices > 1 && 4ll * m.out_floats * slices > kMatCopies)) break;
+      m.csplit = slices;
+      const double t = matrix_time(m, nnz);
+      if (t < (m.half ? 0.84 : 0.93) * walking) found.push_back({m.half ? 1.05 * t : t, cfg, slices});
     }
-    std::stable_sort(found.begin(), found.end(), [](const Found& a, const Found& b) { return a.t < b.t; });
-    for (const Found& f : found) {
+  }
+  std::stable_sort(found.begin(), found.end(), [](const Found& a, const Found& b) { return a.t < b.t; });
+  for (const Found& f : found) {
+    *pool = MatGeom{};
+    if (f.slices == 1 && walk.OH >= 2 && walk.OW >= 2 && !make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool)) {
       *pool = MatGeom{};
-      if (f.slices == 1 && walk.OH >= 2 && walk.OW >= 2 && !make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool)) {
-        *pool = MatGeom{};
-        if (pools) continue;
-      }
-      if (!make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, f.slices, false, g, &staged)) return false;
-      if (!pool->N || pool->kgs == g->kgs) return true;
-      // (relay_kernel's chunks: both are to read the same weights)
-      const int groups = std::min(pool->kgs, g->kgs);
-      return make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, false, g, nullptr, groups) &&
-             make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, 1, true, pool, nullptr, groups);
+      if (pools) continue;
     }
-    return false;
-  };
-  // (relay_kernel too where the others cannot pool: 16 x 64 -> 128 104x104, 20 % of the weights, 162 us, 107)
-  return choose(false) || (terms >= kLeastTerms && choose(true));
+    return make_mat_geom(N, C, H, W, K, ks, stride, pad, f.cfg, f.slices, false, g, &staged);
+  }
+  return false;
 }
 
 int mat_lds_bytes(const MatGeom& g) { return lds_bytes(g); }
@@ -723,7 +623,6 @@ int mat_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, void
 }
 
 int launch_matrix(const MatGeom& g, const float* d_in, float* d_out, const MatWeights& w, int relu, hipStream_t stream) {
-  if (kMatShapes[g.cfg].relay) return launch_relay(g, d_in, d_out, w, relu, stream);
   if (g.half) return launch_half(g, d_in, d_out, w, relu, stream);
   const void* weights = w.base;
   MatGeom k = g;

@@ -41,10 +41,118 @@
 #include <cmath>
 #include <numeric>
 
-#include "matrix_half.h"
+#include "matrix.h"
 
 namespace tetris {
 namespace {
+
+typedef __bf16 bf16x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x8 __attribute__((ext_vector_type(8)));
+
+// fp16 parts: an input times a power of two of the workgroup's is h + 2^-8 m + 2^-15 l, a weight times the power of two that
+// brings the largest of its row to [2^14, 2^15) likewise.  h has eight bits, m eleven, l the rest.  (With 2^-19 l inputs of 2^-32
+// of the largest would still be the sum of their parts, but of subnormal ones, whose left-out products are not small any more.)
+constexpr float kMid = 256.f, kLow = 128.f;  // from h to m, from m to l
+// Exponents of scaled inputs: the smallest that is multiplied in parts, from which on all 24 bits are in them; below the largest that
+// h holds; the smallest that is listed where it is not, and above the largest.
+constexpr int kSmall = -16, kLarge = 15, kLeastListed = -60, kMostListed = 40;
+
+// (A bit cast of a vector's element itself, instead of its value, is compiled to one of the vector's first element.)
+__device__ __forceinline__ float float_of(unsigned x) { return __builtin_bit_cast(float, x); }
+
+// Three fp16 parts of eight floats, scaled; `zeros` becomes NaN where an h is infinite or NaN, `rest` (if any) gets a bit that is not
+// zero where the parts do not add up to the floats.  (h is the bf16 number itself from 2^-16 of its scale on, so what is left of x
+// takes full-rate FMAs; with inputs tested by `rest` and taken off h in fp16 workgroups were 1 % slower.)
+__device__ __forceinline__ void cut16(const float (&x)[8], float scale, u32x4& hi, u32x4& mid, u32x4& lo, f16x2& zeros, unsigned* rest) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = x[2 * i], b = x[2 * i + 1];
+    const unsigned t = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a * scale, b * scale}), bf16x2));
+    const float h0 = __builtin_bit_cast(float, t << 16), h1 = __builtin_bit_cast(float, t & 0xffff0000u);
+    const f16x2 h = __builtin_convertvector((f32x2{h0, h1}), f16x2);
+    const float r0 = fmaf(h0, -kMid, a * (scale * kMid)), r1 = fmaf(h1, -kMid, b * (scale * kMid));
+    const f16x2 m = __builtin_convertvector((f32x2{r0, r1}), f16x2);
+    const float s0 = fmaf((float)m.x, -kLow, r0 * kLow), s1 = fmaf((float)m.y, -kLow, r1 * kLow);
+    const f16x2 l = __builtin_convertvector((f32x2{s0, s1}), f16x2);
+    zeros = __builtin_elementwise_fma(h, f16x2{0, 0}, zeros);
+    if (rest) *rest |= bits_of(fmaf((float)l.x, -1.f, s0)) | bits_of(fmaf((float)l.y, -1.f, s1));
+    hi[i] = __builtin_bit_cast(unsigned, h);
+    mid[i] = __builtin_bit_cast(unsigned, m);
+    lo[i] = __builtin_bit_cast(unsigned, l);
+  }
+}
+
+// From the parts of eight weights (the last one as it is kept, 2^-7 of it): `near`, the weights to eleven bits, `far`, 2^-7 of
+// those, and `off`, what `near` is off by.  Subnormal roundings of fp16 cost a weight of 2^-3 or more (in its scale, where its
+// row's largest is 2^14 or more) less than 2^-30 of it.
+__device__ __forceinline__ void near_and_off(u32x4 hi, u32x4 mid, u32x4 lo, u32x4& near, u32x4& far, u32x4& off) {
+  const f16x8 h = __builtin_bit_cast(f16x8, hi), m = __builtin_bit_cast(f16x8, mid);
+  const f16x8 n = __builtin_elementwise_fma(m, (f16x8)(_Float16)(1 / kMid), h);
+  near = __builtin_bit_cast(u32x4, n);
+  far = __builtin_bit_cast(u32x4, n * (f16x8)(_Float16)(1 / kLow));
+  u32x4 rest;  // h - near, which the compiler would take apart
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm("v_pk_add_f16 %0, %1, %2 neg_lo:[0,1] neg_hi:[0,1]" : "=v"(rest[i]) : "v"(hi[i]), "v"(near[i]));
+  const f16x8 o = __builtin_elementwise_fma(__builtin_bit_cast(f16x8, rest), (f16x8)(_Float16)kMid, m);  // times 2^8, exactly
+  const u32x4 o4 = __builtin_bit_cast(u32x4, o);
+  u32x4 both;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm("v_pk_add_f16 %0, %1, %2" : "=v"(both[i]) : "v"(o4[i]), "v"(lo[i]));
+  off = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, both) * (f16x8)(_Float16)(1 / kMid));
+}
+
+// c + a * b: a 32 x 32, of which four consecutive values of a row hold two (`index` says which), b 32 x 32
+template <bool F16>
+__device__ __forceinline__ f32x16 product(u32x4 a, u32x4 b0, u32x4 b1, int index, f32x16 c) {
+  const u32x8 b = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
+  if constexpr (F16)
+    return __builtin_amdgcn_smfmac_f32_32x32x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x16, b), c, index, 0, 0);
+  else
+    return __builtin_amdgcn_smfmac_f32_32x32x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x16, b), c, index, 0, 0);
+}
+
+// maximum over the wave
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+  auto step = [&](auto lanes) { v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, decltype(lanes)::value, 0xf, 0xf, true)); };
+  step(std::integral_constant<int, 0x111>{});  // one, two, four and eight lanes down in a row of 16, then the rows
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});
+  step(std::integral_constant<int, 0x143>{});
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// x / d through magic_reciprocal(d), which is 0 for d = 1
+__device__ __forceinline__ unsigned over(unsigned x, unsigned m) {
+  const unsigned q = __umulhi(x, m);
+  return m ? q : x;
+}
+
+// x / d for x below 2^30
+__device__ __forceinline__ int quotient(int x, const MatDiv __attribute__((address_space(4)))& d) { return (int)((unsigned long long)(unsigned)x * d.m >> d.shift); }
+
+// The weights of a step: three parts of eight slots per lane, then a word per lane (the slots' places in their groups of four,
+// two bits each; above them the two blocks that the lane reads the input of).
+static_assert(kStepBytes == 3 * 1024 + 256);
+
+// Smallest weight, in its row's scale, that is kept in parts.  Smaller ones -- one in 10^5 of normally distributed weights -- are
+// `loose`: multiplied one by one.  Where a block of 32 rows has more than kMostLoose, or one below kLeastLoose, whose
+// products could underflow in the scale of the sums, the layer runs with bf16 parts.
+constexpr float kLeast = 0x1p-3f, kLeastLoose = 0x1p-60f;
+constexpr int kMostLoose = 64;
+
+// Inputs that fp16 parts do not hold, or not well enough, are multiplied one by one as well: a wave stages zeros in their place and
+// lists them, if they are 2^-60 to 2^40 in the tile's scale.  Where a workgroup has more than kMostAside, or others, it makes the second
+// pass, and at once where a wave's first chunk already shows that.
+constexpr unsigned kMostAside = 8, kNotListed = 1u << 24;
+static_assert(kAsideBytes == 2 * 8 * 4 + 8 * 8 * kMostAside);  // of eight waves: counts after the first chunk and in the end, lists
+
+struct MatArguments { const float* in; float* out; MatWeights w; MatGeom g; };
+typedef const MatArguments __attribute__((address_space(4))) * Arguments;  // the kernel's, read through the scalar cache
 
 // One pass over a tile of outputs.  0: with fp16 parts; false: some input (or the weights) cannot be written so, and nothing was
 // stored.  1: with bf16 parts; false: some sum of the wave's is not finite.  2: the wave's outputs with FMAs.
@@ -624,13 +732,12 @@ constexpr int kMostCounts = 2048;  // of a plan whose workgroups each add up the
 // FILL false: counts the steps only; the workgroups beyond those find the exponents of the rows' largest weights, a wave per row.
 // Latency of a workgroup's few rounds bounds both, so 1024 threads: 6 and 16 us on average over four layers, with 256 8 and 18.
 template <bool FILL>
-__global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const MatLists out, int K, int ks, int kgs, int chunks, int mblocks, int parts) {
+__global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const MatLists out, int K, int ks, int kgs, int chunks, int mblocks) {
   constexpr int kMost = 256, kThreads = 1024;
   __shared__ int layers[kMost];
   __shared__ int list[2 * kMost];
   __shared__ int listed;
   __shared__ int before[kThreads / 64];
-  const int step_bytes = parts * 1024 + 256;
   const int id = blockIdx.x, counts = chunks * mblocks, block = id / chunks, chunk = id - block * chunks, taps = ks * ks, subs = kgs * taps;
   if (!FILL && id >= counts) {
     const int row = (id - counts) * (kThreads / 64) + threadIdx.x / 64, per_row = taps * chunks * 8 * kgs;
@@ -648,7 +755,6 @@ __global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const M
     if ((threadIdx.x & 63) == 0) out.row_exp[row] = most > 0 ? ilogbf(most) - 14 : 0;
     return;
   }
-  auto steps_of = [&](int n) { return parts == 2 ? max(2, (n + 7) / 8 * 2) : max(1, (n + 3) / 4); };  // (relay_kernel takes them in pairs)
   auto weights = [&](int row, int sub, int group) {  // four channels of a block
     const int oc = block * 32 + row, tap = sub / kgs;
     const float4* d = reinterpret_cast<const float4*>(w.dense + (((size_t)oc * taps + tap) * chunks + chunk) * 8 * kgs);
@@ -669,7 +775,7 @@ __global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const M
       for (int sub = 0; sub < subs; ++sub)
         if (layers[sub] > layer) list[n++] = sub | layer << 16;
     listed = n;
-    if (!FILL) out.count[id] = steps_of(n);
+    if (!FILL) out.count[id] = max(1, (n + 3) / 4);
   }
   if (!FILL) return;
   // the steps before these: summed here, or where they are many by first_kernel
@@ -680,7 +786,7 @@ __global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const M
     if ((threadIdx.x & 63) == 0) before[threadIdx.x / 64] = first;
   }
   __syncthreads();
-  const int n = listed, steps_here = steps_of(n), items = steps_here * 64;
+  const int n = listed, steps_here = max(1, (n + 3) / 4), items = steps_here * 64;
   if (counts <= kMostCounts) {
     first = 0;
     for (int i = 0; i < kThreads / 64; ++i) first += before[i];
@@ -690,7 +796,7 @@ __global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const M
     first = out.first[id];
   }
   if (id == counts - 1 && threadIdx.x < 192)  // what is read ahead of the end names a block that exists
-    *reinterpret_cast<unsigned*>(out.steps + (size_t)(first + steps_here + (int)threadIdx.x / 64) * step_bytes + parts * 1024 + threadIdx.x % 64 * 4) = 0;
+    *reinterpret_cast<unsigned*>(out.steps + (size_t)(first + steps_here + (int)threadIdx.x / 64) * kStepBytes + 3072 + threadIdx.x % 64 * 4) = 0;
   for (int i = threadIdx.x; i < items; i += kThreads) {
     const int step = i >> 6, lane = i & 63, row = lane & 31, half = lane >> 5;
     // eight slots: blocks 2 half and 2 half + 1 of the step, two groups of four channels each, two slots a group
@@ -739,27 +845,17 @@ __global__ __launch_bounds__(1024) void steps_kernel(const MatWeights w, const M
       code[r] = (unsigned)(tap % ks | tap / ks << bits | kg << 2 * bits);
     }
     const size_t to = first + step;
-    char* dst = out.steps + to * step_bytes;
-    *reinterpret_cast<unsigned*>(dst + parts * 1024 + lane * 4) = index | code[0] << 16 | code[1] << 24 | (step + 1 == steps_here ? 0x80000000u : 0u);
-    if (parts == 2) {
-      f16x8 near, off;
-      for (int k = 0; k < 8; ++k) {
-        near[k] = (_Float16)scaled[k];
-        off[k] = (_Float16)(scaled[k] - (float)near[k]);
-      }
-      *reinterpret_cast<f16x8*>(dst + lane * 16) = near;
-      *reinterpret_cast<f16x8*>(dst + 1024 + lane * 16) = off;
-    } else {
-      u32x4 h, m, l;
-      unsigned rest = 0;
-      f16x2 zeros = {0, 0};
-      cut16(scaled, 1.f, h, m, l, zeros, &rest);
-      if (rest) *out.wide = 1;
-      l = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, l) * (f16x8)(_Float16)(1 / kLow));
-      *reinterpret_cast<u32x4*>(dst + lane * 16) = h;
-      *reinterpret_cast<u32x4*>(dst + 1024 + lane * 16) = m;
-      *reinterpret_cast<u32x4*>(dst + 2048 + lane * 16) = l;
-    }
+    char* dst = out.steps + to * kStepBytes;
+    *reinterpret_cast<unsigned*>(dst + 3072 + lane * 4) = index | code[0] << 16 | code[1] << 24 | (step + 1 == steps_here ? 0x80000000u : 0u);
+    u32x4 h, m, l;
+    unsigned rest = 0;
+    f16x2 zeros = {0, 0};
+    cut16(scaled, 1.f, h, m, l, zeros, &rest);
+    if (rest) *out.wide = 1;
+    l = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, l) * (f16x8)(_Float16)(1 / kLow));
+    *reinterpret_cast<u32x4*>(dst + lane * 16) = h;
+    *reinterpret_cast<u32x4*>(dst + 1024 + lane * 16) = m;
+    *reinterpret_cast<u32x4*>(dst + 2048 + lane * 16) = l;
     char* raw = out.slots + to * kSlotBytes + lane * 16;
     *reinterpret_cast<u32x4*>(raw) = u32x4{bits_of(v[0]), bits_of(v[1]), bits_of(v[2]), bits_of(v[3])};
     *reinterpret_cast<u32x4*>(raw + 1024) = u32x4{bits_of(v[4]), bits_of(v[5]), bits_of(v[6]), bits_of(v[7])};
@@ -842,8 +938,7 @@ MatWeights mat_weights_at(const MatGeom& g, void* base, size_t* bytes, size_t* z
   l.count = reinterpret_cast<int*>(take((size_t)g.mblocks * g.chunks * 4));
   l.first = reinterpret_cast<int*>(take(((size_t)g.mblocks * g.chunks + 1) * 4));
   l.loose = reinterpret_cast<int2*>(take((size_t)g.mblocks * kMostLoose * 8));
-  const int step_bytes = g.parts * 1024 + 256;
-  l.steps = take(steps * step_bytes);
+  l.steps = take(steps * kStepBytes);
   l.slots = take(steps * kSlotBytes);
   w.row_exp = l.row_exp;
   w.first = l.first;
@@ -851,7 +946,7 @@ MatWeights mat_weights_at(const MatGeom& g, void* base, size_t* bytes, size_t* z
   w.loose = l.loose;
   w.steps = l.steps;
   w.slots = l.slots;
-  w.step_bytes = (int)(steps * step_bytes);
+  w.step_bytes = (int)(steps * kStepBytes);
   if (bytes) *bytes = at;
   if (lists) *lists = l;
   return w;
@@ -874,9 +969,9 @@ int half_weights(const tetris_g950* p, const MatGeom& g, hipStream_t stream, voi
   hipLaunchKernelGGL(dense_kernel, dim3(ceil_div(nstream, 4)), dim3(256), 0, stream, p->d_grp_off, p->d_grp_nnz, p->d_oc_order,
                      p->d_position, p->d_values, const_cast<float*>(w.dense), p->C, p->K, p->ks, p->tile_ic, p->stages, p->g, nstream,
                      8 * g.kgs * g.chunks);
-  hipLaunchKernelGGL(steps_kernel<false>, dim3(counts + 2 * g.mblocks), dim3(1024), 0, stream, w, l, g.K, g.ks, g.kgs, g.chunks, g.mblocks, g.parts);
+  hipLaunchKernelGGL(steps_kernel<false>, dim3(counts + 2 * g.mblocks), dim3(1024), 0, stream, w, l, g.K, g.ks, g.kgs, g.chunks, g.mblocks);
   if (counts > kMostCounts) hipLaunchKernelGGL(first_kernel, dim3(1), dim3(1024), 0, stream, l.count, l.first, counts);
-  hipLaunchKernelGGL(steps_kernel<true>, dim3(counts), dim3(1024), 0, stream, w, l, g.K, g.ks, g.kgs, g.chunks, g.mblocks, g.parts);
+  hipLaunchKernelGGL(steps_kernel<true>, dim3(counts), dim3(1024), 0, stream, w, l, g.K, g.ks, g.kgs, g.chunks, g.mblocks);
   hipLaunchKernelGGL(loose_kernel, dim3(g.mblocks), dim3(64), 0, stream, l.wide, l.loose_count, l.loose);
   TETRIS_HIP(hipGetLastError());
   // launches on other streams may follow at once

@@ -18,19 +18,10 @@
 namespace tetris {
 namespace {
 
-// Of four of `n` positions drawn at random, `count` of which hold a non-zero: how often more than two do.
-__device__ __forceinline__ float crowded_share(float count, float n) {
-  if (n < 4) return count * count * count * (4 * n - 3 * count) / (n * n * n * n);
-  const float three = count * (count - 1) * (count - 2) / (n * (n - 1) * (n - 2));
-  return 4 * three - 3 * three * (count - 3) / (n - 3);
-}
-
-// one wave per (group, stage); element i of the stage is (position i / G, slot i % G).  grp_crowd: crowded_share of each slot, times
-// its positions, added up (G divides 64, so that a lane counts the elements of one slot)
+// one wave per (group, stage); element i of the stage is (position i / G, slot i % G)
 __global__ __launch_bounds__(256) void count_kernel(const float* __restrict__ filter, const int32_t* __restrict__ oc_order,
-                                                    int32_t* __restrict__ grp_nnz, int32_t* __restrict__ grp_pad,
-                                                    float* __restrict__ grp_crowd, int C, int ks, int tile_ic, int stages, int G,
-                                                    int nstream) {
+                                                    int32_t* __restrict__ grp_nnz, int32_t* __restrict__ grp_pad, int C,
+                                                    int ks, int tile_ic, int stages, int G, int nstream) {
   const int sid = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (sid >= nstream) return;
@@ -50,24 +41,17 @@ __global__ __launch_bounds__(256) void count_kernel(const float* __restrict__ fi
     }
   }
   huge = __ballot(huge) != 0;
-  for (int off = 32; off >= G; off >>= 1) cnt += __shfl_xor(cnt, off);
-  float crowd = n && oc_order[grp * G + (lane & (G - 1))] >= 0 ? crowded_share(cnt, n / G) * (n / G) : 0.f;
-  for (int off = G >> 1; off > 0; off >>= 1) {
-    cnt += __shfl_xor(cnt, off);
-    crowd += __shfl_xor(crowd, off);
-  }
+  for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
   if (lane == 0) {
-    grp_crowd[sid] = crowd;
     grp_nnz[sid] = cnt;
     grp_pad[sid] = (cnt + kBatch - 1) / kBatch * kBatch | (huge ? 1 : 0);
   }
 }
 
 // exclusive scan of grp_pad (multiples of kBatch, and a flag in bit 0) into grp_off[0..n], single workgroup; nnz != nullptr:
-// grp_off[n + 1] = the sum of nnz[0..n), with bit 31 set where any flag is, and grp_off[n + 2] that of crowd[0..n), a float
+// grp_off[n + 1] = the sum of nnz[0..n), with bit 31 set where any flag is
 __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ grp_pad, int32_t* __restrict__ grp_off,
-                                                    int n, const int32_t* __restrict__ nnz = nullptr,
-                                                    const float* __restrict__ crowd = nullptr) {
+                                                    int n, const int32_t* __restrict__ nnz = nullptr) {
   __shared__ int part[1024];
   const int tid = threadIdx.x;
   const int chunk = (n + 1023) / 1024;
@@ -91,31 +75,18 @@ __global__ __launch_bounds__(1024) void scan_kernel(const int32_t* __restrict__ 
   if (!nnz) return;
   s = 0;
   int flag = 0;
-  float c = 0;
   for (int i = tid; i < n; i += 1024) {
     s += nnz[i];
-    c += crowd[i];
     flag |= grp_pad[i] & 1;
   }
   flag = __syncthreads_or(flag);  // part has been read
-  for (int off = 32; off > 0; off >>= 1) {
-    s += __shfl_xor(s, off);
-    c += __shfl_xor(c, off);
-  }
-  if ((tid & 63) == 0) {
-    part[tid >> 6] = s;
-    part[16 + (tid >> 6)] = __float_as_int(c);
-  }
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  if ((tid & 63) == 0) part[tid >> 6] = s;
   __syncthreads();
   if (tid == 0) {
     s = 0;
-    c = 0;
-    for (int i = 0; i < 16; ++i) {
-      s += part[i];
-      c += __int_as_float(part[16 + i]);
-    }
+    for (int i = 0; i < 16; ++i) s += part[i];
     grp_off[n + 1] = flag ? (int)(s | 0x80000000u) : s;
-    grp_off[n + 2] = __float_as_int(c);
   }
 }
 
@@ -211,27 +182,25 @@ int pack_device(const float* d_filter, int C, int K, int ks, int tile_ic, int G,
     if (e_ != hipSuccess)                                                                                       \
       return cleanup(fail(TETRIS_EHIP, "%s failed at %s:%d: %s", #call, __FILE__, __LINE__, hipGetErrorString(e_))); \
   } while (0)
-  // One allocation for what the layer's shape fixes -- offsets (and, after the last, the number of non-zeros and how crowded they
-  // are), counts, channel order, and the padded counts and sums that only packing needs -- and one for the entries; tetris_g950_host_arrays
+  // One allocation for what the layer's shape fixes -- offsets (and, after the last, the number of non-zeros), counts,
+  // channel order, and the padded counts that only packing needs -- and one for the entries; tetris_g950_host_arrays
   // copies each back as a whole.
-  HIPC(hipMalloc(&p->d_grp_off, sizeof(int32_t) * (4 * (size_t)nseg + 3 + p->slots)));
-  p->d_grp_nnz = p->d_grp_off + nseg + 3;
+  HIPC(hipMalloc(&p->d_grp_off, sizeof(int32_t) * (3 * (size_t)nseg + 2 + p->slots)));
+  p->d_grp_nnz = p->d_grp_off + nseg + 2;
   p->d_oc_order = p->d_grp_nnz + nseg;
   int32_t* const d_pad = p->d_oc_order + p->slots;
-  float* const d_crowd = reinterpret_cast<float*>(d_pad + nseg);
   HIPC(hipMemcpyAsync(p->d_oc_order, order.data(), sizeof(int32_t) * p->slots, hipMemcpyHostToDevice, stream));
   const int blocks = (nseg + 3) / 4;
-  hipLaunchKernelGGL(count_kernel, dim3(blocks), dim3(256), 0, stream, d_filter, p->d_oc_order, p->d_grp_nnz, d_pad, d_crowd,
-                     C, ks, tile_ic, p->stages, G, nseg);
-  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, stream, d_pad, p->d_grp_off, nseg, p->d_grp_nnz, d_crowd);
+  hipLaunchKernelGGL(count_kernel, dim3(blocks), dim3(256), 0, stream, d_filter, p->d_oc_order, p->d_grp_nnz, d_pad, C,
+                     ks, tile_ic, p->stages, G, nseg);
+  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, stream, d_pad, p->d_grp_off, nseg, p->d_grp_nnz);
   HIPC(hipGetLastError());
-  int32_t total[3] = {0, 0, 0};  // entries; non-zeros and whether a weight is huge; how crowded they are
+  int32_t total[2] = {0, 0};  // entries; non-zeros and whether a weight is huge
   HIPC(hipMemcpyAsync(total, p->d_grp_off + nseg, sizeof total, hipMemcpyDeviceToHost, stream));
   HIPC(hipStreamSynchronize(stream));
   p->n_entries = total[0];
   p->nnz = total[1] & 0x7fffffff;
   p->huge = total[1] < 0;
-  p->crowded = __builtin_bit_cast(float, total[2]) / ((double)K * C * ks * ks);
   // one spare batch so that a kernel may prefetch the batch after the last one
   const size_t room = (size_t)total[0] + kBatch;
   HIPC(hipMalloc(&p->d_position, 2 * sizeof(int32_t) * room));
@@ -642,7 +611,7 @@ int tetris_g950_host_arrays(tetris_g950* p, tetris_g950_arrays* out) {
   if (!p || !out) return tetris::fail(TETRIS_EINVAL, "null argument");
   const int nseg = p->groups * p->stages;
   std::lock_guard<std::mutex> lock(p->mu);
-  const size_t fixed = 2 * (size_t)nseg + 3 + p->slots, room = (size_t)p->n_entries + tetris::kBatch;
+  const size_t fixed = 2 * (size_t)nseg + 2 + p->slots, room = (size_t)p->n_entries + tetris::kBatch;
   if (!p->h_fixed) {
     std::unique_ptr<int32_t[]> h(new int32_t[fixed]), e(new int32_t[2 * room]);
     TETRIS_HIP(hipMemcpy(h.get(), p->d_grp_off, sizeof(int32_t) * fixed, hipMemcpyDeviceToHost));
@@ -652,10 +621,10 @@ int tetris_g950_host_arrays(tetris_g950* p, tetris_g950_arrays* out) {
   }
   const int32_t* h = p->h_fixed.get();
   out->grp_offsets = h; out->n_grp_offsets = nseg + 1;
-  out->grp_nnz = h + nseg + 3; out->n_grp_nnz = nseg;
+  out->grp_nnz = h + nseg + 2; out->n_grp_nnz = nseg;
   out->position = p->h_entries.get(); out->n_entries = p->n_entries;
   out->values = reinterpret_cast<const float*>(p->h_entries.get() + room);
-  out->oc_order = h + 2 * (size_t)nseg + 3; out->n_slots = p->slots;
+  out->oc_order = h + 2 * (size_t)nseg + 2; out->n_slots = p->slots;
   out->stages = p->stages; out->tile_ic = p->tile_ic; out->oc_per_wave = p->g; out->nnz = p->nnz;
   return TETRIS_OK;
 }

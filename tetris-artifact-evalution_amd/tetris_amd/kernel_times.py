@@ -1,4 +1,4 @@
-"""Times the walking kernels and every configuration of matrix_kernel and half_kernel on a set of layers, and checks the time models that
+"""Times the walking kernels and every configuration of the two matrix kernels on a set of layers, and checks the time models that
 the library chooses between them with, or fits them (csrc/matrix_conv.hip).
 
     make fit                                                  the library with the entry points used here
